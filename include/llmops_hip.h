@@ -166,7 +166,8 @@ int llmops_fc_Q4A_decode(const float* x, int64_t rows, int64_t K, const int8_t* 
  * [out_parts][rows][N_out / out_parts] (Ng % out_parts == 0, N_out == Ng*32): the strips of part p are strips
  * p*Ng/out_parts .. of weiq.  A q|k|v projection over weights stacked along N (chatllama/main.py:347-349 runs three
  * FCs on the same input) thus leaves q, k and v as the three dense [rows, H*S] matrices the attention op takes,
- * with one quantization of the input.  norm_w / eps / glu (0 or 2) as above; no residual, no sums of squares. */
+ * with one quantization of the input.  norm_w / eps / glu (0 or 2) as above; no residual, no sums of squares.
+ * workspace_bytes: the larger of llmops_fc_Q4A_workspace_bytes for Ng and for Ng / out_parts strips. */
 int llmops_fc_Q4A_decode_parts(const float* x, int64_t rows, int64_t K, const int8_t* weiq, int64_t Ng, int64_t Kg,
                                int group_k, int64_t N_out, const float* norm_w, float eps, int glu, int64_t out_parts,
                                float* y, void* workspace, size_t workspace_bytes, llmops_stream_t stream);

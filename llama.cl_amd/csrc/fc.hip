@@ -197,8 +197,15 @@ static int fc_decode_impl(const float* x, int64_t rows, int64_t K, const int8_t*
         LLMOPS_REQUIRE(glu != 1 && residual == nullptr && sumsq_out == nullptr && (Ng % out_parts) == 0 &&
                        N_out == Ng * kGroupN);
     const FcWorkspace lay = fc_layout(rows, Ng, Kg, group_k);
-    if (workspace_bytes < lay.total)
-        return fail(LLMOPS_EWORKSPACE, "fc_Q4A needs %zu workspace bytes, got %zu", lay.total, workspace_bytes);
+    // (parts are products of their own with fewer strips each, and fewer strips are split over K more often: a part can
+    // need more room for partial sums than the whole; the offsets in front of them are the same)
+    size_t need = lay.total;
+    if (out_parts > 1) {
+        const size_t part_need = fc_layout(rows, Ng / out_parts, Kg, group_k).total;
+        need = part_need > need ? part_need : need;
+    }
+    if (workspace_bytes < need)
+        return fail(LLMOPS_EWORKSPACE, "fc_Q4A needs %zu workspace bytes, got %zu", need, workspace_bytes);
     uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
     if (rows > kMaxGemvRows) {
         // More rows than the streaming kernel takes: the producer is folded into the quantization launch instead

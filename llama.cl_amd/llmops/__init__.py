@@ -312,7 +312,10 @@ def fc_Q4A_decode(input, weiq, N_out, norm=None, residual=None, glu=False, sumsq
             return out, sumsq
         return out
     lib = _lib.load()
-    ws = _workspace(input.device, lib.llmops_fc_Q4A_workspace_bytes(rows, K, Ng, Kg, g))
+    need = lib.llmops_fc_Q4A_workspace_bytes(rows, K, Ng, Kg, g)
+    if out_parts != 1:  # products over Ng / out_parts strips, which may need more room for partial sums than one over all
+        need = max(need, lib.llmops_fc_Q4A_workspace_bytes(rows, K, Ng // out_parts, Kg, g))
+    ws = _workspace(input.device, need)
     if out_parts != 1:
         _require(rows > 8 and not glu and residual is None and not want_sumsq and Ng % out_parts == 0 and N_out == Ng * 32,
                  "out_parts: more than 8 rows, whole strips per part, no residual, no sumsq")
