@@ -1,176 +1,25 @@
-// Q4_1 x Q8 fully-connected product for many activation rows (prefill): int8 MFMA.
+// Q4_1 x Q8 fully-connected product for many activation rows (prefill), group 128: int8 MFMA, and the planning and
+// launching of the product for both group sizes (group 32: fc_gemm_g32.hip).
 //
-// A wavefront owns two adjacent strips (64 output columns) and RT tiles of 16 activation rows.
-// Operand layout of v_mfma_i32_16x16x{64,32}_i8: lane = 16*g + jj; the A lane holds row jj,
-// the B lane holds column jj, both for the same set of k-values chosen by g.  The packed
-// format gives, per 16-byte load, 4 adjacent columns x 8 k-values of one k8-row.  So lane
-// (g, jj) loads the k8-rows that belong to g for columns 4*(jj&7)..+3 of strip (jj>>3); dword c
+// Operand layout of v_mfma_i32_16x16x64_i8: lane = 16*g + jj; the A lane holds row jj, the B lane holds column jj, both
+// for the same set of k-values chosen by g.  The packed format gives, per 16-byte load, 4 adjacent columns x 8 k-values
+// of one k8-row.  So lane (g, jj) takes the k8-rows that belong to g for columns 4*(jj&7)..+3 of strip (jj>>3); dword c
 // of that load is the lane's B operand for MFMA number c, whose 16 tile columns are
-// { strip (jj>>3), column 4*(jj&7)+c }.  Unpacking is two ANDs and a shift per dword; nothing is
-// shuffled between lanes and the weights never pass through LDS.
-//   G=128: one MFMA 16x16x64 covers 8 k8-rows (g owns rows 2g,2g+1 = 16 consecutive k);
-//          two of them make one k-group.
-//   G=32 : one MFMA 16x16x32 covers the group's 4 k8-rows (g owns row g = 8 consecutive k).
+// { strip (jj>>3), column 4*(jj&7)+c }.  Unpacking is two ANDs and a shift per dword; nothing is shuffled between lanes.
+// One MFMA covers 8 k8-rows (g owns rows 2g,2g+1 = 16 consecutive k); two of them make one k-group.
 // After every k-group the int32 tile is folded into fp32 accumulators:
 //   f += (d[n]*dx[row]) * float(acc) ; f += m[n]*gsum[row]        (fc_Q4A,
 //   /root/reference/ops/op_fc.hpp:381-412; min term is m * raw group sum).
-// The group-128 kernels with LDS tiles compute the first term as fma(fma(X, d, -B*d), dx, f): their
+// The first term is computed as fma(fma(X, d, -B*d), dx, f): the
 // int32 sums start at the bit pattern of the float B = 1.5 * 2^23, so the sum's register, read as a
 // float X, IS B + sum (|sum| <= 128*15*127 < 2^22), and X*d - B*d = sum*d is exact before the fma's
 // one rounding because B*d (2 significant bits times the 11 of an fp16) is itself a float.  Two
 // vector instructions per output element and k-group instead of three (convert, multiply, fma).
 // Result tile layout of the 16x16 MFMAs: lane holds column jj, rows 4*g+v in register v.
-#include "common.h"
+#include "gemm_device.h"
 #include "gemv_device.h"
 
 namespace llmops {
-
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-typedef float v2f __attribute__((ext_vector_type(2)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-
-constexpr int kFoldBiasBits = 0x4B400000;  // the float 1.5 * 2^23 ...
-constexpr float kFoldBias = 12582912.0f;   // ... whose low mantissa bits count in units of 1
-
-__device__ __forceinline__ uint32_t lo4(uint32_t w) { return w & 0x0F0F0F0Fu; }
-__device__ __forceinline__ uint32_t hi4(uint32_t w) { return (w >> 4) & 0x0F0F0F0Fu; }
-
-template <int G>
-struct GemmTraits;
-template <>
-struct GemmTraits<128> {
-    static constexpr int kSteps = 2;  // MFMAs per k-group
-};
-template <>
-struct GemmTraits<32> {
-    static constexpr int kSteps = 1;
-};
-
-// acc[t][c] += A(row tile t) x B(column set c) over one k-group
-template <int G, int RT>
-__device__ __forceinline__ void mma_group(const uint8_t* blk, const int8_t* const xrow[RT], int64_t kofs, int g, int q,
-                                          v4i acc[RT][4]) {
-    if (G == 128) {
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const uint4 wa = *reinterpret_cast<const uint4*>(blk + h * 1024 + (2 * g) * kRowBytes + q * 16);
-            const uint4 wb = *reinterpret_cast<const uint4*>(blk + h * 1024 + (2 * g + 1) * kRowBytes + q * 16);
-            const uint32_t* pa = reinterpret_cast<const uint32_t*>(&wa);
-            const uint32_t* pb = reinterpret_cast<const uint32_t*>(&wb);
-            v4i b[4];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                b[c][0] = (int)lo4(pa[c]);
-                b[c][1] = (int)hi4(pa[c]);
-                b[c][2] = (int)lo4(pb[c]);
-                b[c][3] = (int)hi4(pb[c]);
-            }
-#pragma unroll
-            for (int t = 0; t < RT; t++) {
-                const v4i a = *reinterpret_cast<const v4i*>(xrow[t] + kofs + h * 64 + g * 16);
-#pragma unroll
-                for (int c = 0; c < 4; c++) acc[t][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b[c], acc[t][c], 0, 0, 0);
-            }
-        }
-    } else {
-        const uint4 wa = *reinterpret_cast<const uint4*>(blk + g * kRowBytes + q * 16);
-        const uint32_t* pa = reinterpret_cast<const uint32_t*>(&wa);
-        long b[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) b[c] = (long)(((uint64_t)hi4(pa[c]) << 32) | (uint64_t)lo4(pa[c]));
-#pragma unroll
-        for (int t = 0; t < RT; t++) {
-            const long a = *reinterpret_cast<const long*>(xrow[t] + kofs + g * 8);
-#pragma unroll
-            for (int c = 0; c < 4; c++) acc[t][c] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b[c], acc[t][c], 0, 0, 0);
-        }
-    }
-}
-
-// grid: x = ceil(pairs/4) (4 waves = 4 strip pairs per workgroup), y = row blocks of RT*16, z = k splits
-template <int G, int RT>
-__global__ __launch_bounds__(256) void fc_gemm_kernel(const uint8_t* __restrict__ weiq, const int8_t* __restrict__ xq,
-                                                       const float* __restrict__ xd, const float* __restrict__ gs,
-                                                       float* __restrict__ out, int Ng, int Kg, int64_t ldo, int64_t N,
-                                                       int rows, int kb_per_split, int64_t split_stride) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int g = lane >> 4, jj = lane & 15, q = jj & 7, sp = jj >> 3;
-    const int pair = blockIdx.x * 4 + wave;
-    if (pair * 2 >= Ng) return;
-    const int strip = pair * 2 + sp;
-    const bool strip_ok = strip < Ng;
-    const int strip_c = strip_ok ? strip : Ng - 1;
-    const int row0 = blockIdx.y * (RT * 16);
-    const int kb0 = blockIdx.z * kb_per_split, kb1 = min(Kg, kb0 + kb_per_split);
-    const int64_t Kp = (int64_t)Kg * G;
-    const uint8_t* sbase = weiq + (int64_t)strip_c * Kg * block_bytes(G);
-
-    const int8_t* xrow[RT];
-    int vrow[RT][4];  // clamped global row of result register v
-#pragma unroll
-    for (int t = 0; t < RT; t++) {
-        xrow[t] = xq + (int64_t)min(rows - 1, row0 + t * 16 + jj) * Kp;
-#pragma unroll
-        for (int v = 0; v < 4; v++) vrow[t][v] = min(rows - 1, row0 + t * 16 + g * 4 + v);
-    }
-
-    float f[RT][4][4];
-#pragma unroll
-    for (int t = 0; t < RT; t++)
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) f[t][c][v] = 0.0f;
-
-    for (int kb = kb0; kb < kb1; kb++) {
-        const uint8_t* blk = sbase + (int64_t)kb * block_bytes(G);
-        v4i acc[RT][4];
-#pragma unroll
-        for (int t = 0; t < RT; t++)
-#pragma unroll
-            for (int c = 0; c < 4; c++) acc[t][c] = v4i{0, 0, 0, 0};
-        mma_group<G, RT>(blk, xrow, (int64_t)kb * G, g, q, acc);
-
-        const uint2 dh = *reinterpret_cast<const uint2*>(blk + (G / 8) * kRowBytes + q * 8);
-        const uint2 mh = *reinterpret_cast<const uint2*>(blk + (G / 8) * kRowBytes + 64 + q * 8);
-        float d[4], m[4];
-        d[0] = f16_bits_to_f32((uint16_t)(dh.x & 0xFFFFu));
-        d[1] = f16_bits_to_f32((uint16_t)(dh.x >> 16));
-        d[2] = f16_bits_to_f32((uint16_t)(dh.y & 0xFFFFu));
-        d[3] = f16_bits_to_f32((uint16_t)(dh.y >> 16));
-        m[0] = f16_bits_to_f32((uint16_t)(mh.x & 0xFFFFu));
-        m[1] = f16_bits_to_f32((uint16_t)(mh.x >> 16));
-        m[2] = f16_bits_to_f32((uint16_t)(mh.y & 0xFFFFu));
-        m[3] = f16_bits_to_f32((uint16_t)(mh.y >> 16));
-#pragma unroll
-        for (int t = 0; t < RT; t++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const float dx = xd[(int64_t)vrow[t][v] * Kg + kb];
-                const float gsum = gs[(int64_t)vrow[t][v] * Kg + kb];
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    f[t][c][v] = fmaf(d[c] * dx, (float)acc[t][c][v], f[t][c][v]);
-                    f[t][c][v] = fmaf(m[c], gsum, f[t][c][v]);
-                }
-            }
-    }
-
-    if (!strip_ok) return;
-    float* o = out + (int64_t)blockIdx.z * split_stride;
-    const int64_t n0 = (int64_t)strip * kGroupN + q * 4;
-#pragma unroll
-    for (int t = 0; t < RT; t++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int row = row0 + t * 16 + g * 4 + v;
-            if (row >= rows) continue;
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-                if (n0 + c < N) o[(int64_t)row * ldo + n0 + c] = f[t][c][v];
-        }
-}
 
 // ---- split-K without a second launch -------------------------------------------------------------------
 // Every split stores its tile of partial sums with device-scope (write-through) stores, waits for them and
@@ -272,7 +121,7 @@ __device__ __forceinline__ void splitk_finish(const v4f (&f)[RT][4], float* __re
 //   XS: (dx, gsum) of the BM rows for this k-group
 // The global loads of iteration kb+1 are issued before the MFMAs of iteration kb and written to the
 // other LDS buffer after them; one barrier per iteration.  Each wave owns 64 rows x 64 columns
-// (RT = BM/32 row tiles x 4 column sets); operand mapping as in mma_group above, but from LDS.
+// (RT = BM/32 row tiles x 4 column sets); operand mapping as at the top of this file.
 constexpr int kAStride = 144;
 constexpr int kBlk128 = 2176;
 
@@ -292,20 +141,10 @@ __device__ __forceinline__ v2f buf_ld_pair(buffer_rsrc r, uint32_t voff, uint32_
 // subnormals and the row could lose bits relative to its own size, above it hi overflows.  Zeros are exact.
 // When a lane of the wave does not qualify, the wave takes the round with fp32 MFMAs instead (four k-groups
 // each, exact products): the slow path, there for correctness on any input.
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-union Halves8 {
-    v8h h;
-    uint32_t u[4];
-};
-
 // What a lane fetches for one round of 32 k-groups (k32 .. k32+31, those below kb1): for its eight k-groups
 // kgs .. kgs+7 the group sums of its row in each of RT row tiles (32 contiguous bytes of the [row][kg] matrix, which
 // start on a 4-byte boundary only) and the mins of its four columns.  kgs is k32 + 8g unless that would read past
 // the end of a row: then it is Kg - 8, and the slots below k32 + 8g do not count (min_term_add).
-struct __attribute__((packed, aligned(4))) Float4U {
-    float v[4];
-};
 template <int RT>
 struct MinTermRound {
     Float4U ga[RT][2];
@@ -704,17 +543,6 @@ struct GemmPPSmem {
     float dx[2][BM];
 };
 
-__device__ __forceinline__ uint32_t lds_off(const void* p) {
-    return (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) void*)p);
-}
-// lane i's 16 (4) bytes at base + off (base the same for the whole wave, off a byte offset per lane)
-// land at lds_base + 16*i (4*i); counts in vmcnt like any load
-__device__ __forceinline__ void copy16_to_lds(const void* base, uint32_t off, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(lds_base) : "memory", "m0");
-}
-__device__ __forceinline__ void copy4_to_lds(const void* base, uint32_t off, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(lds_base) : "memory", "m0");
-}
 // 16-byte LDS read whose result may only be used after lds_ready<N>() on it, N = number of LDS
 // operations issued after this one that may still be pending (LDS operations complete in order).
 // Between the two calls the variable must not be touched.
@@ -1086,40 +914,14 @@ __global__ void gemm_reduce_kernel(const float* __restrict__ part, float* __rest
     }
 }
 
-// Integer core only, through the same mma_group: acc[row][n][kb]
-template <int G>
-__global__ __launch_bounds__(256) void fc_gemm_partials_kernel(const uint8_t* __restrict__ weiq,
-                                                                const int8_t* __restrict__ xq, int32_t* __restrict__ out,
-                                                                int Ng, int Kg, int rows) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int g = lane >> 4, jj = lane & 15, q = jj & 7, sp = jj >> 3;
-    const int pair = blockIdx.x * 4 + wave;
-    if (pair * 2 >= Ng) return;
-    const int strip = pair * 2 + sp;
-    const bool strip_ok = strip < Ng;
-    const int strip_c = strip_ok ? strip : Ng - 1;
-    const int row0 = blockIdx.y * 16;
-    const int kb = blockIdx.z;
-    const int64_t Kp = (int64_t)Kg * G;
-    const int64_t Np = (int64_t)Ng * kGroupN;
-    const uint8_t* blk = weiq + ((int64_t)strip_c * Kg + kb) * block_bytes(G);
-    const int8_t* xrow[1] = {xq + (int64_t)min(rows - 1, row0 + jj) * Kp};
-    v4i acc[1][4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) acc[0][c] = v4i{0, 0, 0, 0};
-    mma_group<G, 1>(blk, xrow, (int64_t)kb * G, g, q, acc);
-    if (!strip_ok) return;
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-        const int row = row0 + g * 4 + v;
-        if (row >= rows) continue;
-#pragma unroll
-        for (int c = 0; c < 4; c++) out[((int64_t)row * Np + strip * kGroupN + q * 4 + c) * Kg + kb] = acc[0][c][v];
-    }
-}
+int plan_gemm_g32(int64_t rows, int64_t Ng, int64_t Kg, int force_split, int* st_per_split);
+int launch_gemm_g32(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, const float2* xsT, float* out, int64_t Ng,
+                    int64_t Kg, int64_t ldo, int64_t N, int64_t rows, int st_per_split, int S, int64_t split_stride,
+                    const float* residual, hipStream_t st);
+int launch_gemm_g32_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg, hipStream_t st);
 
 struct GemmPlan {
-    int RT, S, kb_per_split;
+    int RT, S, kb_per_split;  // group 32: RT = 1 (32-row tiles), kb_per_split in stages of four k-groups
     bool lds;
 };
 
@@ -1142,8 +944,8 @@ static GemmPlan plan_gemm(int64_t rows, int64_t Ng, int64_t Kg, int G) {
     GemmPlan p;
     p.lds = (G == 128);
     if (!p.lds) {
-        p.RT = rows > 32 ? 4 : (rows > 16 ? 2 : 1);  // RT*16 rows per wave
-        gemm_split((((Ng + 1) / 2 + 3) / 4) * ((rows + p.RT * 16 - 1) / (p.RT * 16)), 512, Kg, p);
+        p.RT = 1;
+        p.S = plan_gemm_g32(rows, Ng, Kg, g_gemm_force_split, &p.kb_per_split);
         return p;
     }
     // Candidates: the 256-row kernel with two wave groups (one workgroup per CU) and the four-wave
@@ -1214,15 +1016,6 @@ size_t gemm_workspace_bytes(int64_t rows, int64_t Ng, int64_t Kg, int G) {
     return p.S > 1 ? (size_t)p.S * rows * Ng * kGroupN * sizeof(float) : 0;
 }
 
-template <int G, int RT>
-static void launch_gemm_t(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, float* out, int64_t Ng,
-                          int64_t Kg, int64_t ldo, int64_t N, int64_t rows, const GemmPlan& p, int64_t split_stride,
-                          hipStream_t st) {
-    dim3 grid((unsigned)(((Ng + 1) / 2 + 3) / 4), (unsigned)((rows + RT * 16 - 1) / (RT * 16)), (unsigned)p.S);
-    fc_gemm_kernel<G, RT><<<grid, 256, 0, st>>>(w, xq, xd, gs, out, (int)Ng, (int)Kg, ldo, N, (int)rows, p.kb_per_split,
-                                                split_stride);
-}
-
 template <int RT>
 static int launch_gemm_lds_t(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, const float2* xsT,
                              float* out, int64_t Ng, int64_t Kg, int64_t ldo, int64_t N, int64_t rows, const GemmPlan& p,
@@ -1261,8 +1054,6 @@ static int launch_gemm_pp(const uint8_t* w, const int8_t* xq, const float* xd, c
     return LLMOPS_OK;
 }
 
-int launch_add(float* a, const float* b, int64_t total, hipStream_t st);  // misc.hip
-
 // y = product (+ residual, fp32 [rows, N], may be y itself)
 int launch_gemm(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, const float2* xsT, float* y,
                 float* part, unsigned* counters, int64_t rows, int64_t Ng, int64_t Kg, int G, int64_t N, const float* residual,
@@ -1295,17 +1086,14 @@ int launch_gemm(const uint8_t* w, const int8_t* xq, const float* xd, const float
         else rc = launch_gemm_lds_t<1>(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, y, N, kcnt, st);
         if (rc) return rc;
     } else {
-        if (p.RT == 4) launch_gemm_t<32, 4>(w, xq, xd, gs, out, Ng, Kg, ldo, Nw, rows, p, ss, st);
-        else if (p.RT == 2) launch_gemm_t<32, 2>(w, xq, xd, gs, out, Ng, Kg, ldo, Nw, rows, p, ss, st);
-        else launch_gemm_t<32, 1>(w, xq, xd, gs, out, Ng, Kg, ldo, Nw, rows, p, ss, st);
+        const int rc = launch_gemm_g32(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p.kb_per_split, p.S, ss, kres, st);
+        if (rc) return rc;
     }
     LLMOPS_LAUNCH_CHECK();
     if (p.S > 1 && !fused_reduce) {
         const int64_t total = rows * ((N + 3) / 4);
         gemm_reduce_kernel<<<(unsigned)((total + 255) / 256), 256, 0, st>>>(part, y, rows, N, Np, ss, p.S, residual);
         LLMOPS_LAUNCH_CHECK();
-    } else if (residual != nullptr && !p.lds) {
-        return launch_add(y, residual, rows * N, st);  // the group-32 kernel has no residual in its stores
     }
     return LLMOPS_OK;
 }
@@ -1337,8 +1125,7 @@ int launch_gemm_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64
         fc_gemm_lds_kernel<2, true><<<grid, 256, sizeof(GemmSmem<2>), st>>>(w, xq, nullptr, nullptr, nullptr, nullptr, acc,
                                                                           (int)Ng, (int)Kg, 0, 0, (int)rows, (int)Kg, 0, nullptr, nullptr, 0, nullptr);
     } else {
-        dim3 grid((unsigned)(((Ng + 1) / 2 + 3) / 4), (unsigned)((rows + 15) / 16), (unsigned)Kg);
-        fc_gemm_partials_kernel<32><<<grid, 256, 0, st>>>(w, xq, acc, (int)Ng, (int)Kg, (int)rows);
+        return launch_gemm_g32_partials(w, xq, acc, rows, Ng, Kg, st);
     }
     LLMOPS_LAUNCH_CHECK();
     return LLMOPS_OK;

@@ -1,0 +1,317 @@
+// Q4_1 x Q8 fully-connected product for more than 8 activation rows, group 32: int8 MFMA (fc_Q4A,
+// /root/reference/ops/op_fc.hpp:381-412).
+//
+// What bounds it: with a group of 32 every v_mfma_i32_32x32x32_i8 (32 cycles) is a whole k-group of its tile, and its 16
+// results per lane are folded into the fp32 accumulators with 32 vector instructions: the vector ALU (about 60 ns per
+// step and SIMD in a loop of nothing else, against 14 ns of matrix core) is the limit, so everything else is kept off it
+// and out of its way:
+//   * tile 32 rows x 256 columns, four waves side by side (each 32 x 64 = two strips): a strip's weights are unpacked by
+//     one wave only, and the rows' codes and scales are read from LDS by all four.  (Sixty-four rows x 128 columns, two
+//     waves either way: 0 to 3 % slower at almost every size, 512 x 11008 x 4096 116.4 against 113.8 us; 128 x 128 with
+//     64 x 64 per wave 122 us: its 256 registers leave two waves per SIMD.)
+//   * a stage is four k-groups.  Codes, packed blocks, scales and sums are all copied to LDS asynchronously
+//     (global_load_lds) one stage ahead: no registers, no LDS store instructions, 16 bytes per lane where the layout has
+//     them.  (Weights taken straight from memory into operand registers, one dword per lane and load, cost more than
+//     all of the arithmetic: 203 against 124 us.)
+//   * the fold of one step runs while the next step's MFMA does: two accumulators, the order pinned.
+//   * f += d * dx * sum in two instructions: the sums start at the bit pattern of 1.5 * 2^23 (gemm_device.h), so the
+//     register read as a float X is bias + sum and fma(X, d, -bias * d) = sum * d, exact before its one rounding
+//     (|sum| <= 32 * 15 * 127 < 2^22; bias * d has 2 + 11 significant bits).
+//   * the min term, sum over k-groups of m[column] * gsum[row], is a product with K = number of k-groups: every eight
+//     k-groups one v_mfma_f32_32x32x16_f16 per strip on gsum = hi + lo (22 bits; fp32 MFMAs where the sums do not suit
+//     fp16), instead of a third vector instruction per element.
+// Measured (us for the whole call, before -- one wave per 64 rows x 64 columns, operands straight from memory, three
+// instructions per fold -- and now): 512 x 11008 x 4096 330 / 114, 512 x 4096 x 11008 230 / 103, 2048 x 4096^2 291 / 139,
+// 64 x 4096^2 40 / 21, 9 x 4096 x 11008 33 / 21, 300 x 1024 x 2048 35 / 19.
+#include "gemm_device.h"
+#include "gemv_device.h"
+
+namespace llmops {
+
+constexpr int kG32Blk = 640;       // bytes of a packed block: 512 of nibbles, 32 fp16 scales, 32 fp16 mins
+constexpr int kG32Rows = 32;       // rows and strips of a tile
+constexpr int kG32Strips = 8;
+constexpr int kG32Gps = 4;         // k-groups per stage
+
+// PARTIALS: test build that stores the int32 sums of every (row, column, k-group) into out_i ([rows][Ng*32][Kg])
+template <bool PARTIALS>
+__global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __restrict__ weiq, const int8_t* __restrict__ xq,
+                                                              const float* __restrict__ xd, const float* __restrict__ gs,
+                                                              const float2* __restrict__ xsT, float* __restrict__ out,
+                                                              int32_t* __restrict__ out_i, int Ng, int Kg, int64_t ldo, int64_t N,
+                                                              int rows, int st_per_split, int64_t split_stride,
+                                                              const float* __restrict__ residual) {
+    constexpr int BM = kG32Rows, STRIPS = kG32Strips, GPS = kG32Gps, BLK = kG32Blk;
+    __shared__ __align__(16) uint8_t sa[2][BM * 128];           // codes, 128 bytes per row
+    __shared__ __align__(16) uint8_t sbn[2][STRIPS * 2048];     // nibbles, 16 k8-rows of 128 bytes per strip
+    __shared__ __align__(16) float sx[2][GPS * BM];             // activation scales [k-group][row]
+    __shared__ __align__(16) uint16_t sdm[16 * STRIPS * 64];    // ring of 16 k-groups: [strip][32 scales, 32 mins]
+    __shared__ __align__(16) float sg[16 * BM];                 // ring of 16 k-groups: activation sums [row]
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, j = lane & 31;
+    // tile numbering: one contiguous run of tiles per XCD (workgroups go to the XCDs round robin), bands of 8 row blocks,
+    // rows fastest, so that what is resident on one XCD shares its L2
+    const int nbx = (Ng + STRIPS - 1) / STRIPS, nby = (rows + BM - 1) / BM;
+    int bx, by;
+    {
+        const int total = nbx * nby, per_xcd = (total + 7) / 8;
+        const int i = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+        if ((int)(blockIdx.x >> 3) >= per_xcd || i >= total) return;  // uniform for the workgroup
+        constexpr int kBand = 8;
+        const int band = i / (kBand * nbx), in_band = i % (kBand * nbx);
+        const int first = band * kBand, rows_in_band = min(kBand, nby - first);
+        by = first + in_band % rows_in_band;
+        bx = in_band / rows_in_band;
+    }
+    const int tstrip = bx * STRIPS, strip0 = tstrip + 2 * wave;  // the tile's and this wave's first strip (may lie beyond Ng)
+    const int row0 = by * BM;
+    const int nst = (Kg + GPS - 1) / GPS;
+    const int st0 = blockIdx.z * st_per_split, st1 = min(nst, st0 + st_per_split);
+    const int kg1 = min(Kg, st1 * GPS);
+    const int Kp = Kg * 32;
+
+    // ---- what this wave copies per stage.  Sources past the end (rows, strips, the last stage's k-groups) re-read the
+    // last one that exists. ----
+    // codes: rows 8*wave .. +7.  16-byte chunk c of row r lies at position c ^ key(r), key(r) = (r + ((r >> 3) & 1)) & 7: the
+    // 16 rows that one phase of a ds_read_b128 touches fall on 16 different bank groups
+    const uint8_t* abase = reinterpret_cast<const uint8_t*>(xq) + (int64_t)row0 * Kp;
+    const uint32_t arow = (uint32_t)(min(rows - 1, row0 + wave * 8 + (lane >> 3)) - row0) * (uint32_t)Kp;
+    const uint32_t achunk = (uint32_t)(((lane & 7) ^ (((lane >> 3) + (wave & 1)) & 7)) * 16);
+    const uint32_t lds_a = lds_off(&sa[0][0]), lds_b = lds_off(&sbn[0][0]), lds_x = lds_off(&sx[0][0]), lds_d = lds_off(&sdm[0]),
+                   lds_g = lds_off(&sg[0]);
+    // nibbles: two strips, 8 k8-rows to a copy, the two low bits of the row number exchanged: the rows 4s+2h+p that the lane
+    // halves h = 0, 1 read together lie side by side
+    const uint32_t sb = (uint32_t)Kg * (uint32_t)BLK;  // bytes of a strip
+    const uint8_t* bbase = weiq + (int64_t)tstrip * sb;
+    uint32_t boff[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int slot = (i & 1) * 8 + (lane >> 3), r = (slot & 12) | ((slot & 1) << 1) | ((slot >> 1) & 1);
+        boff[i] = (uint32_t)(min(Ng - 1, strip0 + (i >> 1)) - tstrip) * sb + (uint32_t)((r & 3) * kRowBytes + (lane & 7) * 16);
+    }
+    // scales and mins: k-group `wave` of the stage, 128 bytes per block, eight strips
+    const uint32_t doff = (uint32_t)(min(Ng - 1, tstrip + (lane >> 3)) - tstrip) * sb + (uint32_t)(512 + (lane & 7) * 16);
+    // activation scales (waves 0, 1) and sums (waves 2, 3): two k-groups of 32 rows to a copy
+    const int xrow = min(rows - 1, row0 + j);
+    auto copy_stage = [&](int st, int buf) {
+        const int kg0 = st * GPS, ring = (kg0 - st0 * GPS) & 15;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int kg = min(Kg - 1, kg0 + (i & 1) * 2 + h);
+            copy16_to_lds(bbase, boff[i] + (uint32_t)kg * (uint32_t)BLK, lds_b + buf * (STRIPS * 2048) + (wave * 4 + i) * 1024);
+        }
+        copy16_to_lds(abase, arow + min((uint32_t)st * 128u + achunk, (uint32_t)Kp - 16u), lds_a + buf * (BM * 128) + wave * 1024);
+        if (PARTIALS) return;
+        {
+            const int c = wave & 1, kg = min(Kg - 1, kg0 + 2 * c + h);
+            const bool sums = wave >= 2;  // uniform
+            const uint32_t dst = sums ? lds_g + (ring * BM + c * 64) * 4 : lds_x + (buf * GPS * BM + c * 64) * 4;
+            if (xsT) {
+                const int kgb = min(Kg - 1, kg0 + 2 * c);
+                copy4_to_lds(uniform_ptr(reinterpret_cast<const float*>(xsT + (int64_t)kgb * rows) + (sums ? 1 : 0)),
+                             (uint32_t)((kg - kgb) * rows + xrow) * 8u, dst);
+            } else {
+                copy4_to_lds(uniform_ptr((sums ? gs : xd) + (int64_t)row0 * Kg), (uint32_t)((xrow - row0) * Kg + kg) * 4u, dst);
+            }
+        }
+        copy16_to_lds(bbase + (int64_t)min(Kg - 1, kg0 + wave) * BLK, doff, lds_d + (ring + wave) * (STRIPS * 128));
+    };
+
+    if (st0 < st1) copy_stage(st0, 0);
+    v16f f[2];
+    v16i bias;
+#pragma unroll
+    for (int i = 0; i < 16; i++) f[0][i] = f[1][i] = 0.0f, bias[i] = PARTIALS ? 0 : kFoldBiasBits;
+    asm volatile("" : "+v"(bias));
+    constexpr int kVmcnt0 = 0x0F70;  // vmcnt(0), the other counters left alone
+    __builtin_amdgcn_s_waitcnt(kVmcnt0);
+    __syncthreads();
+
+    const int akey = (j + ((j >> 3) & 1)) & 7;
+    int a_rd[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ks++) a_rd[ks] = j * 128 + (((2 * ks + h) ^ akey) * 16);
+
+    for (int st = st0; st < st1; st++) {
+        const int buf = (st - st0) & 1, ring = ((st - st0) * GPS) & 15;
+        const bool more = st + 1 < st1;
+        v4i af[4];
+        float4 xf[2][4];
+        // lane half h holds the tile rows 8b + 4h + v (result register 4b + v)
+        auto load_x = [&](int kk) {
+            if (PARTIALS) return;
+#pragma unroll
+            for (int b = 0; b < 4; b++) xf[kk & 1][b] = *reinterpret_cast<const float4*>(&sx[buf][kk * BM + 8 * b + 4 * h]);
+        };
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) af[ks] = *reinterpret_cast<const v4i*>(&sa[buf][a_rd[ks]]);
+        load_x(0);
+        v4i bu[2][4];
+        float d[2][4];
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            const uint8_t* bs = &sbn[buf][(2 * wave + s) * 2048 + h * 128 + j * 4];
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+                const uint32_t w0 = *reinterpret_cast<const uint32_t*>(bs + ks * 512), w1 = *reinterpret_cast<const uint32_t*>(bs + ks * 512 + 256);
+                bu[s][ks] = v4i{(int)lo4(w0), (int)hi4(w0), (int)lo4(w1), (int)hi4(w1)};
+                // (k-groups past the end: d = 0 and nothing is added)
+                const uint16_t bits = sdm[(ring + ks) * (STRIPS * 64) + (2 * wave + s) * 64 + j];
+                d[s][ks] = f16_bits_to_f32(st * GPS + ks < kg1 ? bits : (uint16_t)0);
+                // converted once, not inside every fma of the fold (v_fma_mix runs at half the rate of v_fma)
+                asm volatile("" : "+v"(d[s][ks]));
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) copy_stage(st + 1, buf ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+
+        v16i acc[2];  // steps (k-group i >> 1, strip i & 1) alternate between the two
+        auto mma = [&](int i) { acc[i & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i >> 1], bu[i & 1][i >> 1], bias, 0, 0, 0); };
+        mma(0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int s = i & 1, kk = i >> 1;
+            if (s == 0 && kk + 1 < GPS) load_x(kk + 1);
+            if (i + 1 < 8) {
+                mma(i + 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (PARTIALS) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int row = row0 + 8 * (r >> 2) + 4 * h + (r & 3), kg = st * GPS + kk;
+                    if (strip0 + s < Ng && row < rows && kg < Kg)
+                        out_i[((int64_t)row * ((int64_t)Ng * kGroupN) + (strip0 + s) * kGroupN + j) * Kg + kg] = acc[s][r];
+                }
+            } else {
+                const float dd = d[s][kk], nbd = -kFoldBias * dd;
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    const float4 x = xf[kk & 1][b];
+                    f[s][4 * b + 0] = fmaf(fmaf(__int_as_float(acc[s][4 * b + 0]), dd, nbd), x.x, f[s][4 * b + 0]);
+                    f[s][4 * b + 1] = fmaf(fmaf(__int_as_float(acc[s][4 * b + 1]), dd, nbd), x.y, f[s][4 * b + 1]);
+                    f[s][4 * b + 2] = fmaf(fmaf(__int_as_float(acc[s][4 * b + 2]), dd, nbd), x.z, f[s][4 * b + 2]);
+                    f[s][4 * b + 3] = fmaf(fmaf(__int_as_float(acc[s][4 * b + 3]), dd, nbd), x.w, f[s][4 * b + 3]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // ---- min term of the eight k-groups of this stage and the one before (of this one alone where the run ends after
+        // an odd number of stages): lane half h has the groups 4h .. 4h+3, hi in the first four slots and lo in the others ----
+        if (!PARTIALS && (((st - st0) & 1) == 1 || !more)) {
+            const int rel = ((st - st0) & ~1) * GPS + 4 * h;  // first group of this lane, counted from the split's first
+            const int left = kg1 - st0 * GPS - rel;           // how many of its four count (the others: any value)
+            uint32_t mb[2][4];
+            float ga[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int slot = (rel + i) & 15;
+                const float v = sg[slot * BM + j];
+                ga[i] = i < left ? v : 0.0f;
+#pragma unroll
+                for (int s = 0; s < 2; s++) {
+                    const uint32_t m = sdm[slot * (STRIPS * 64) + (2 * wave + s) * 64 + 32 + j];
+                    mb[s][i] = i < left ? m : 0u;
+                }
+            }
+            // hi + lo in fp16 is good for a lane's four sums if the largest lies in [1/8, 60000]: below that lo falls into the
+            // subnormals, above it hi overflows.  Otherwise the wave takes fp32 MFMAs (exact products).
+            const float big = fmaxf(fmaxf(fabsf(ga[0]), fabsf(ga[1])), fmaxf(fabsf(ga[2]), fabsf(ga[3])));
+            const bool nan = ga[0] != ga[0] || ga[1] != ga[1] || ga[2] != ga[2] || ga[3] != ga[3];
+            if (__all(!nan && (big == 0.0f || (big >= 0.125f && big <= 60000.0f)))) {
+                Halves8 a;
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const v2h hh = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(ga[2 * i], ga[2 * i + 1]));
+                    a.u[i] = __builtin_bit_cast(uint32_t, hh);
+                    a.u[2 + i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(ga[2 * i] - (float)hh[0], ga[2 * i + 1] - (float)hh[1]));
+                }
+#pragma unroll
+                for (int s = 0; s < 2; s++) {
+                    Halves8 m;
+                    m.u[0] = m.u[2] = mb[s][0] | (mb[s][1] << 16);
+                    m.u[1] = m.u[3] = mb[s][2] | (mb[s][3] << 16);
+                    f[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.h, m.h, f[s], 0, 0, 0);
+                }
+            } else {
+                // slot i of lanes (h = 0, 1; j) is one 32x32x2 product: k = h
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int s = 0; s < 2; s++)
+                        f[s] = __builtin_amdgcn_mfma_f32_32x32x2f32(ga[i], f16_bits_to_f32((uint16_t)mb[s][i]), f[s], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(kVmcnt0);  // this wave's copies for the next stage have landed
+        __syncthreads();
+    }
+
+    if (PARTIALS) return;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+        const int64_t n = (int64_t)(strip0 + s) * kGroupN + j;
+        if (strip0 + s >= Ng || n >= N) continue;
+        float* o = out + (int64_t)blockIdx.z * split_stride + n;
+        // residual != nullptr only without split-K: then o is the result itself, row stride ldo
+        const float* res = residual ? residual + n : nullptr;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int row = row0 + 8 * (r >> 2) + 4 * h + (r & 3);
+            if (row < rows) o[(int64_t)row * ldo] = res ? f[s][r] + res[(int64_t)row * ldo] : f[s][r];
+        }
+    }
+}
+
+// Split-K factor.  Estimated time in us: a workgroup's run of stages plus half a stage, 1.43 us each, times how many
+// workgroups a compute unit has to run (two fit, and two together take 1.3 times what one does alone); the second launch
+// that adds the partial sums 2 us, 2 more per four splits (its loads in flight) and their traffic.  Measured against every
+// factor of 1, 2, 3, 4, 6, 8, 12, 16, 24 at 9 .. 2048 rows of five shapes: 0.9 % slower than the best on average, 9 % at worst.
+// Partial sums never take a workspace that fits the built-in scratch of llmops_fc_Q4A_noalloc beyond it.
+int plan_gemm_g32(int64_t rows, int64_t Ng, int64_t Kg, int force_split, int* st_per_split) {
+    const int64_t nst = (Kg + kG32Gps - 1) / kG32Gps;
+    const int64_t tiles = ((Ng + kG32Strips - 1) / kG32Strips) * ((rows + kG32Rows - 1) / kG32Rows);
+    // codes, scales, sums and pairs of a k-group: 48 bytes; the alignment of the five areas and the pairs' slack
+    const int64_t room = (int64_t)LLMOPS_FC_NOALLOC_SCRATCH_BYTES - LLMOPS_FC_COUNTER_BYTES - rows * Kg * 48 - 2048;
+    int64_t best_s = 1, best_per = nst;
+    double best = 0.0;
+    for (int64_t s = 1; s <= 24 && s <= nst; s++) {
+        if (force_split > 0 && s != (force_split < nst ? (force_split < 24 ? force_split : 24) : nst)) continue;
+        const int64_t per = (nst + s - 1) / s, S = (nst + per - 1) / per;
+        if (S > 1 && room >= 0 && S * rows * Ng * kGroupN * 4 > room && force_split <= 0) continue;
+        const int64_t full = tiles * S / 512, rest = tiles * S % 512;
+        double t = 1.43 * ((double)per + 0.5) * ((double)full * 1.3 + (rest == 0 ? 0.0 : rest <= 256 ? 1.0 : 1.3));
+        if (S > 1) t += 2.0 + 2.0 * (double)((S + 3) / 4) + 0.5e-6 * (double)S * (double)rows * (double)(Ng * kGroupN);
+        if (best == 0.0 || t < best) best = t, best_s = S, best_per = per;
+    }
+    *st_per_split = (int)best_per;
+    return (int)best_s;
+}
+
+int launch_gemm_g32(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, const float2* xsT, float* out, int64_t Ng,
+                    int64_t Kg, int64_t ldo, int64_t N, int64_t rows, int st_per_split, int S, int64_t split_stride,
+                    const float* residual, hipStream_t st) {
+    // (lane offsets of 32 bits: into a tile's strips, into its rows, into the pairs of one k-group)
+    if (Kg * kG32Blk * kG32Strips >= ((int64_t)1 << 32) || rows >= ((int64_t)1 << 28))
+        return fail(LLMOPS_EINVAL, "fc_Q4A group 32: Kg must be below 2^32 / 5120 and rows below 2^28");
+    const int64_t tiles = ((Ng + kG32Strips - 1) / kG32Strips) * ((rows + kG32Rows - 1) / kG32Rows);
+    const dim3 grid((unsigned)(8 * ((tiles + 7) / 8)), 1, (unsigned)S);  // one run of tiles per XCD
+    fc_gemm_g32_kernel<false><<<grid, 256, 0, st>>>(w, xq, xd, gs, xsT, out, nullptr, (int)Ng, (int)Kg, ldo, N, (int)rows, st_per_split,
+                                                    split_stride, residual);
+    LLMOPS_LAUNCH_CHECK();
+    return LLMOPS_OK;
+}
+
+int launch_gemm_g32_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg, hipStream_t st) {
+    const int64_t tiles = ((Ng + kG32Strips - 1) / kG32Strips) * ((rows + kG32Rows - 1) / kG32Rows);
+    fc_gemm_g32_kernel<true><<<(unsigned)(8 * ((tiles + 7) / 8)), 256, 0, st>>>(w, xq, nullptr, nullptr, nullptr, nullptr, acc, (int)Ng,
+                                                                                (int)Kg, 0, 0, (int)rows, (int)((Kg + kG32Gps - 1) / kG32Gps),
+                                                                                0, nullptr);
+    LLMOPS_LAUNCH_CHECK();
+    return LLMOPS_OK;
+}
+
+}  // namespace llmops

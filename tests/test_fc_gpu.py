@@ -633,6 +633,63 @@ def test_fc_prefill_min_term_at_any_activation_scale(ops, orc, K, split):
     assert np.all(err[:290] <= 1e-5 * scale[:290]), (err[:290] / scale[:290]).max()
 
 
+@pytest.mark.parametrize("rows,N,K", [(9, 30, 32), (31, 33, 96), (32, 256, 160), (33, 257, 544), (65, 1000, 4096), (40, 512, 1000), (130, 96, 2080)])
+@pytest.mark.parametrize("split", [0, 3])
+def test_fc_group32_tiles_vs_oracle(ops, orc, rows, N, K, split):
+    """The group-32 product of more than 8 rows (32-row x 8-strip tiles, stages of four k-groups): row and column edges,
+    one k-group, a last stage of one to four k-groups, an odd number of stages, a K that ends inside a k-group, K in one
+    piece and in three.  Rows of ordinary, tiny (group sums far below fp16's normal range), huge (beyond it) and zero
+    activations: every row to 1e-5 of its own largest output (the sums of Kg products carry at most Kg * 2^-24 < 1e-5),
+    with and without a residual, and through codes and scales that the caller quantized."""
+    from llmops import _lib
+    lib = _lib.load()
+    G = 32
+    rng = np.random.default_rng(rows * 31 + N + K)
+    x = rng.standard_normal((1, rows, K)).astype(np.float32)
+    x[0, 2:5] *= 1e-4
+    x[0, 5:8] *= 30000.0
+    x[0, 8] = 0.0
+    x[0, 1, :32] = 0.0
+    pw = orc.quant_w((rng.standard_normal((N, K)) * 0.02).astype(np.float32), G)
+    res = rng.standard_normal((1, rows, N)).astype(np.float32)
+    want = orc.fc(x, pw, N)
+    lib.llmops_test_gemm_set_split(split)
+    try:
+        got = host(ops.fc_Q4A(dev(x), dev(pw), N))
+        got_res = host(ops.fc_Q4A(dev(x), dev(pw), N, residual=dev(res)))
+        y = torch.empty(1, rows, N, device="cuda")
+        if K % G == 0:
+            Ng, Kg = pw.shape[0], pw.shape[1]
+            xq, xd, gs = ops.FC_dynamic_quantize_x(dev(x), G)
+            ws = ops._workspace(y.device, lib.llmops_fc_Q4A_workspace_bytes(rows, K, Ng, Kg, G))
+            wq = dev(pw)
+            assert lib.llmops_fc_Q4A_prequantized(ops._ptr(xq), ops._ptr(xd), ops._ptr(gs), rows, ops._ptr(wq), Ng, Kg, G, N, ops._ptr(y),
+                                                  ops._ptr(ws), ws.numel(), ops._stream(y)) == 0
+            pre = host(y)
+        else:
+            pre = got
+    finally:
+        lib.llmops_test_gemm_set_split(0)
+    scale = np.abs(want[0]).max(axis=1)
+    assert np.all(got[0, 8] == 0.0)
+    for r in (got, pre):
+        assert np.all(np.abs(r[0] - want[0]).max(axis=1) <= 1e-5 * scale)
+    assert np.all(np.abs(got_res[0] - (want + res)[0]).max(axis=1) <= 1e-5 * np.abs((want + res)[0]).max(axis=1) + 1e-5 * scale)
+
+
+def test_fc_group32_non_finite_rows_stay_theirs(ops, orc):
+    """An infinity or a NaN in one row of activations leaves the other rows of its tile as they are."""
+    rng = np.random.default_rng(5)
+    rows, N, K = 40, 288, 1024
+    pw = dev(orc.quant_w((rng.standard_normal((N, K)) * 0.02).astype(np.float32), 32))
+    x = rng.standard_normal((1, rows, K)).astype(np.float32)
+    clean = host(ops.fc_Q4A(dev(x), pw, N))
+    x[0, 3, 77], x[0, 35, 1000] = np.inf, np.nan
+    got = host(ops.fc_Q4A(dev(x), pw, N))
+    rest = [r for r in range(rows) if r not in (3, 35)]
+    assert max_rel_err(got[:, rest], clean[:, rest]) <= 1e-6 and not np.isfinite(got[0, 3]).any() and not np.isfinite(got[0, 35]).any()
+
+
 @pytest.mark.parametrize("rows", [9, 12, 16])
 @pytest.mark.parametrize("N,K", [(2070, 1024), (4096, 4096)])
 def test_fc_rows_9_to_16_streaming_mfma(ops, orc, rows, N, K):
