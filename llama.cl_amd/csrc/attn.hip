@@ -1,15 +1,13 @@
 // Rotary embedding, KV-cache update and attention over the cache
 // (attention_rope2 / attention_rope, /root/reference/ops/op_attn.hpp:721-1029 and :518-718).
 //
-// Three launches per call:
+// One query token: attn_decode_kernel (everything in one launch) and attn_merge_kernel.  More:
 //   1. attn_prep_kernel   rotate q and k in place (rope_embed, ops/op_attn.hpp:44-94), write the
 //                         rotated k and the v rows into the cache at slots[p] (:764-773), and
-//                         record which cache rows were written by which token of this call.
-//   2. attn_split_kernel  split-KV attention: one workgroup per (b, h, query, chunk of C cache
-//                         rows) streams its K and V rows exactly once with 16-byte loads (all
-//                         issued before the first use so a whole chunk is in flight), computes
-//                         the chunk's scores, their max, exp and sum, and the chunk's weighted
-//                         V sum.  Chunks make up for the low head count (B*H = 32 in decode).
+//                         from 32 tokens on record which cache rows were written by which token of this call.
+//   2. below 32 tokens    attn_split_kernel or attn_few_kernel: a workgroup takes a chunk of cache rows and leaves
+//                         per query the chunk's score maximum, its sum of exponentials and its weighted V sum.
+//      from 32 on         attn_prefill_kernel: 128 queries to a workgroup, the cache rows in one piece or in several.
 //   3. attn_merge_kernel  merges the chunks of a query with the usual max/sum rescaling and
 //                         overwrites q with the result (:1018-1025).
 // The cache element type is fp32 (reference layout) or fp16 (all arithmetic still fp32).
@@ -23,6 +21,8 @@
 #include "common.h"
 
 namespace llmops {
+
+typedef float v16f __attribute__((ext_vector_type(16)));
 
 // ---- rope ------------------------------------------------------------------------------------
 // theta = inv_freq[i] * (float)pos, cosf/sinf in fp32 (CosSin_cache::update, ops/op_attn.hpp:25-32)
@@ -73,7 +73,7 @@ __global__ void attn_prep_kernel(float* __restrict__ q, float* __restrict__ k, c
     const bool slot_ok = slot >= 0 && slot < maxlen;
     T* kdst = kc + ((b * H + h) * maxlen + (slot_ok ? slot : 0)) * S;
     T* vdst = vc + ((b * H + h) * maxlen + (slot_ok ? slot : 0)) * S;
-    if (blockIdx.x < qL && threadIdx.x == 0) {
+    if (row_token != nullptr && blockIdx.x < qL && threadIdx.x == 0) {
         const int s0 = slots[blockIdx.x];
         if (s0 >= 0 && s0 < maxlen) row_token[s0] = (int32_t)blockIdx.x;
     }
@@ -104,7 +104,6 @@ __global__ void fill_i32_kernel(int32_t* p, int64_t n, int32_t v) {
     if (i < n) p[i] = v;
 }
 
-// ---- split-KV attention ----------------------------------------------------------------------
 __device__ __forceinline__ float4 load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 __device__ __forceinline__ float4 load4(const __half* p) {
     const uint2 u = *reinterpret_cast<const uint2*>(p);
@@ -119,13 +118,14 @@ __device__ __forceinline__ float2 load2(const __half* p) {
     return __half22float2(*reinterpret_cast<const __half2*>(&u));
 }
 
+// ---- split-KV attention of few query tokens over a short cache ----
 // Per-chunk record in the workspace: [max, sum, out[S]]
 // Workgroup = 4 waves; wave w owns rows w*PW .. w*PW+PW-1 of the chunk (C = 4*PW rows);
 // lane = 32*hf + e: row parity hf, elements 4e..4e+3 (S == 128).
 template <typename T, int PW>
 __global__ __launch_bounds__(256) void attn_split_kernel(const float* __restrict__ q, const T* __restrict__ kc,
                                                           const T* __restrict__ vc, int64_t qL, int64_t H, int64_t maxlen,
-                                                          int64_t kvLen, const int32_t* __restrict__ row_token,
+                                                          int64_t kvLen, const int32_t* __restrict__ slots,
                                                           float* __restrict__ part, int nchunks) {
     constexpr int S = 128, C = 4 * PW, NL = PW / 2;
     __shared__ float sc[C];
@@ -151,6 +151,15 @@ __global__ __launch_bounds__(256) void attn_split_kernel(const float* __restrict
     }
     const float4 qv = load4(q + ((b * qL + pq) * H + h) * S + e * 4);
     const float d_scale = 1.0f / sqrtf((float)S);
+    // rows that a later token of this call has written
+    bool later[NL];
+#pragma unroll
+    for (int i = 0; i < NL; i++) later[i] = false;
+    for (int l = (int)pq + 1; l < (int)qL; l++) {
+        const int64_t rel = (int64_t)slots[l] - p0 - wave * PW - hf;
+#pragma unroll
+        for (int i = 0; i < NL; i++) later[i] = later[i] || rel == 2 * i;
+    }
 
 #pragma unroll
     for (int i = 0; i < NL; i++) {
@@ -162,9 +171,7 @@ __global__ __launch_bounds__(256) void attn_split_kernel(const float* __restrict
         for (int o = 16; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
         const int r = wave * PW + i * 2 + hf;
         const int64_t p = p0 + r;
-        bool live = p < kvLen;
-        if (live && qL > 1) live = !(row_token[p] > (int32_t)pq);  // written by a later token of this call
-        if (e == 0) sc[r] = live ? s * d_scale : -FLT_MAX;
+        if (e == 0) sc[r] = p < kvLen && !later[i] ? s * d_scale : -FLT_MAX;
     }
     __syncthreads();
     if (wave == 0) {
@@ -201,6 +208,181 @@ __global__ __launch_bounds__(256) void attn_split_kernel(const float* __restrict
     if (threadIdx.x == 0) {
         rec[0] = stat[0];
         rec[1] = stat[1];
+    }
+}
+
+// ---- split-KV attention of few query tokens (fewer than 32, or one that the decode kernel does not take) ----
+// Bound by reading the cache once: all query tokens of a head share every K and V row, through the matrix cores.  A
+// workgroup takes 128 cache rows of a head, each of its four waves 32 of them, every load asked for before the first use;
+// the waves' results meet in LDS and leave one record per query, [max, sum, out[S]], for attn_merge_kernel.  (One
+// workgroup per query and chunk, on the vector ALU, read and multiplied the rows once per token: 16 tokens behind 1500,
+// 32 heads, the whole call 68 us against 25; 31 behind 3500 239 against 44.)
+//
+// Arithmetic: fp32 operands are cut into three bf16 pieces, exactly (8 bits each, rounded to nearest; the exponent range
+// is fp32's own); a product a*b is a1b1 + a1b2 + a2b1 + a2b2 + a1b3 + a3b1, each exact in the fp32 accumulators; what is
+// dropped is below 2^-25 of the product.  Halves of an fp16 cache are two pieces.
+//   S^T = K * Q^T: A = the lane's cache row (lane % 32), dims 16i + 8*hf .. +7; B = the lane's query (lane % 32), same dims.
+//                  The result puts query lane % 32 into the lane, cache rows 8j + 4*hf + v.
+//   O^T = V^T * P^T: A = V[those rows][column 4 * (lane % 32) + c], one 16-byte load per row; B = the probabilities as
+//                  they sit in registers.  Result register 4j + v of product c: column 4 * (8j + 4*hf + v) + c.
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+union V8bfBits {
+    v8bf h;
+    uint32_t u[4];
+};
+struct Bf3 {
+    V8bfBits p[3];
+};
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef float v2f_a __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_bf(float a, float b) {  // rounded to nearest even (v_cvt_pk_bf16_f32)
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f_a{a, b}, v2bf));
+}
+// elements 2e, 2e+1 of the pieces
+template <int PIECES>
+__device__ __forceinline__ void split_bf(Bf3& d, int e, float a, float b) {
+#pragma unroll
+    for (int k = 0; k < PIECES; k++) {
+        const uint32_t u = pack_bf(a, b);
+        d.p[k].u[e] = u;
+        a -= __uint_as_float(u << 16), b -= __uint_as_float(u & 0xFFFF0000u);
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256, 2) void attn_few_kernel(const float* __restrict__ q, const T* __restrict__ kc,
+                                                           const T* __restrict__ vc, int qL, int64_t H, int64_t maxlen, int kvLen,
+                                                           const int32_t* __restrict__ slots, float* __restrict__ part, int nchunks) {
+    constexpr int S = 128, P = sizeof(T) == 4 ? 3 : 2;
+    __shared__ __align__(16) int tok[4][32];
+    __shared__ float wm[4][64], wl[4][64];
+    __shared__ __align__(16) float os[4][16][64][4];  // [wave][4j + v][lane][c]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int hf = lane >> 5, c32 = lane & 31;
+    const int chunk = blockIdx.x % nchunks;
+    const int64_t bh = blockIdx.x / nchunks, b = bh / H, h = bh % H;
+    const int p0 = chunk * 128 + wave * 32;  // this wave's first cache row
+    const T* kbase = kc + bh * maxlen * S;
+    const T* vbase = vc + bh * maxlen * S;
+    const T* krow = kbase + (int64_t)min(p0 + c32, kvLen - 1) * S + 8 * hf;
+    float4 kr[16], vr[16], qr[16];
+    const float* qrow = q + ((b * qL + min(c32, qL - 1)) * H + h) * S + 8 * hf;
+#pragma unroll
+    for (int i = 0; i < 8; i++) qr[2 * i] = load4(qrow + 16 * i), qr[2 * i + 1] = load4(qrow + 16 * i + 4);
+#pragma unroll
+    for (int i = 0; i < 8; i++) kr[2 * i] = load4(krow + 16 * i), kr[2 * i + 1] = load4(krow + 16 * i + 4);
+#pragma unroll
+    for (int r = 0; r < 16; r++) vr[r] = load4(vbase + (int64_t)min(p0 + 8 * (r >> 2) + 4 * hf + (r & 3), kvLen - 1) * S + 4 * c32);
+    __builtin_amdgcn_sched_barrier(0);
+    {
+        // which token of this call wrote the lane's cache row (-1: none); rows past the end belong to nobody
+        const int row = p0 + c32;
+        int t = -1;
+        for (int l = 0; l < qL; l++) t = slots[l] == row ? l : t;
+        tok[wave][c32] = row < kvLen ? t : INT_MAX;
+    }
+    // (two accumulators for the leading products and one for the small ones: fewer roundings at full size)
+    v16f s0[2], s1;
+#pragma unroll
+    for (int r = 0; r < 16; r++) s0[0][r] = s0[1][r] = s1[r] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        Bf3 a, w;
+        split_bf<P>(a, 0, kr[2 * i].x, kr[2 * i].y), split_bf<P>(a, 1, kr[2 * i].z, kr[2 * i].w);
+        split_bf<P>(a, 2, kr[2 * i + 1].x, kr[2 * i + 1].y), split_bf<P>(a, 3, kr[2 * i + 1].z, kr[2 * i + 1].w);
+        split_bf<3>(w, 0, qr[2 * i].x, qr[2 * i].y), split_bf<3>(w, 1, qr[2 * i].z, qr[2 * i].w);
+        split_bf<3>(w, 2, qr[2 * i + 1].x, qr[2 * i + 1].y), split_bf<3>(w, 3, qr[2 * i + 1].z, qr[2 * i + 1].w);
+        s0[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[0].h, w.p[0].h, s0[i & 1], 0, 0, 0);
+        if (P == 3) s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[2].h, w.p[0].h, s1, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[0].h, w.p[2].h, s1, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[1].h, w.p[1].h, s1, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[1].h, w.p[0].h, s1, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[0].h, w.p[1].h, s1, 0, 0, 0);
+    }
+    const float d_scale = 1.0f / sqrtf((float)S);
+    const int pq = c32 < qL ? c32 : INT_MIN;
+    __builtin_amdgcn_wave_barrier();
+    v16f pr;
+    float mx = -FLT_MAX;
+#pragma unroll
+    for (int jj = 0; jj < 4; jj++) {
+        const int4 t4 = *reinterpret_cast<const int4*>(&tok[wave][8 * jj + 4 * hf]);
+        const int tt[4] = {t4.x, t4.y, t4.z, t4.w};
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            pr[4 * jj + v] = tt[v] <= pq ? ((s0[0][4 * jj + v] + s0[1][4 * jj + v]) + s1[4 * jj + v]) * d_scale : -FLT_MAX;
+            mx = fmaxf(mx, pr[4 * jj + v]);
+        }
+    }
+    {  // the other half of the lane pair holds the other 16 rows
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+        mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    }
+    // the workgroup's maximum of every query, before the exponentials: all four waves use the same one
+    wm[wave][lane] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(wm[0][lane], wm[1][lane]), fmaxf(wm[2][lane], wm[3][lane]));
+    float sum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        pr[r] = pr[r] == -FLT_MAX ? 0.0f : expf(pr[r] - mx);
+        sum += pr[r];
+    }
+    wl[wave][lane] = sum;
+    v16f o[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[c][r] = 0.0f;
+    Bf3 w[2];
+#pragma unroll
+    for (int e = 0; e < 8; e++) split_bf<3>(w[e >> 2], e & 3, pr[2 * e], pr[2 * e + 1]);
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        Bf3 a[2];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float4 v0 = vr[2 * e], v1 = vr[2 * e + 1];
+            const float x0 = c == 0 ? v0.x : c == 1 ? v0.y : c == 2 ? v0.z : v0.w, x1 = c == 0 ? v1.x : c == 1 ? v1.y : c == 2 ? v1.z : v1.w;
+            split_bf<P>(a[e >> 2], e & 3, x0, x1);
+        }
+#pragma unroll
+        for (int bb = 0; bb < 2; bb++) {  // the small products first, while the sum is small
+            if (P == 3) o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[2].h, w[bb].p[0].h, o[c], 0, 0, 0);
+            o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[0].h, w[bb].p[2].h, o[c], 0, 0, 0);
+            o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[1].h, w[bb].p[1].h, o[c], 0, 0, 0);
+        }
+#pragma unroll
+        for (int bb = 0; bb < 2; bb++) {
+            o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[1].h, w[bb].p[0].h, o[c], 0, 0, 0);
+            o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[0].h, w[bb].p[1].h, o[c], 0, 0, 0);
+        }
+#pragma unroll
+        for (int bb = 0; bb < 2; bb++) o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[0].h, w[bb].p[0].h, o[c], 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r++) *reinterpret_cast<float4*>(&os[wave][r][lane][0]) = make_float4(o[0][r], o[1][r], o[2][r], o[3][r]);
+    __syncthreads();
+    // wave w finishes the result registers 4w .. 4w+3: columns 4 * (8w + 4*hf + v) + c of the lane's query
+    if (c32 >= qL) return;
+    float* rec = part + ((bh * qL + c32) * nchunks + chunk) * (S + 2);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const float4 x = *reinterpret_cast<const float4*>(&os[w][4 * wave + v][lane][0]);
+            a.x += x.x, a.y += x.y, a.z += x.z, a.w += x.w;
+        }
+        float2* dst = reinterpret_cast<float2*>(rec + 2 + 4 * (8 * wave + 4 * hf + v));
+        dst[0] = make_float2(a.x, a.y);
+        dst[1] = make_float2(a.z, a.w);
+    }
+    if (wave == 0 && hf == 0) {
+        float l = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) l += wl[w][lane] + wl[w][lane + 32];
+        *reinterpret_cast<float2*>(rec) = make_float2(mx, l);
     }
 }
 
@@ -687,7 +869,6 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const int32_t* __
 // no query of a wave may see (in-chunk causal mask, ops/op_attn.hpp:1007-1011) are skipped.  K rows
 // take 272 bytes per plane and V columns 80, so that the 16 lanes one phase of a 16-byte read serves
 // touch 16 different 16-byte slots of the 256-byte bank line (17 and 5 are odd).
-typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 
@@ -726,7 +907,8 @@ constexpr size_t prefill_smem_bytes() {
 template <typename T>
 __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __restrict__ kc, const T* __restrict__ vc,
                                                           int64_t qL, int64_t H, int64_t maxlen, int64_t kvLen,
-                                                          const int32_t* __restrict__ row_token, int qtiles) {
+                                                          const int32_t* __restrict__ row_token, int qtiles, int kv_span,
+                                                          float* __restrict__ part, int nsplit) {
     constexpr bool LO = sizeof(T) == 4;  // an fp16 cache holds no low halves
     constexpr int S = 128, BQ = 128, BK = 32, KSB = 272, VSB = 80;
     extern __shared__ __align__(16) uint8_t smem_raw[];
@@ -736,9 +918,11 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __
     PrefillSmem<LO>* const sm2 = reinterpret_cast<PrefillSmem<LO>*>(smem_raw) + 2 * set;
     const int hf = lane >> 5, c32 = lane & 31;
     // late query tiles see the most cache rows: they are dealt out first so that they do not form the tail
+    // (gridDim.y = nsplit workgroups share a query tile, each with kv_span cache rows; one: kv_span covers them all)
     const int64_t bhs = gridDim.x / qtiles;
     const int qt = qtiles - 1 - (int)(blockIdx.x / bhs);
     const int64_t bh = blockIdx.x % bhs, b = bh / H, h = bh % H;
+    const int kv_begin = (int)blockIdx.y * kv_span;
     // (32-bit arithmetic from here on: the launcher keeps qL and kvLen below 2^31 and a head's cache plane below 4 GiB)
     const int qLi = (int)qL, kvLeni = (int)kvLen;
     const int q_lo_wave = qt * BQ + wave * 32;
@@ -798,7 +982,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __
     {
         const int q_hi_wg = min((qt + 1) * BQ, qLi) - 1;
         int last = -1;
-        for (int r = tid; r < kvLeni; r += 256)
+        for (int r = kv_begin + tid; r < min(kvLeni, kv_begin + kv_span); r += 256)
             if (row_token[r] <= q_hi_wg) last = r;  // (r grows: the last hit is the largest; each set scans all rows)
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) last = max(last, __shfl_xor(last, off, 64));
@@ -807,7 +991,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __
         __syncthreads();
         kv_end = max(max(red[0], red[1]), max(red[2], red[3])) + 1;
     }
-    if (kv_end <= 0) kv_end = 1;  // no row is visible to anybody (cannot happen: a token sees its own row)
+    if (kv_end <= kv_begin) kv_end = kv_begin;  // no row of this range is visible to anybody: nothing to walk
     // Writing a staged tile: halves of K row-major, halves of V transposed, the tile's tokens and their range.
 #define LLMOPS_STAGE_STORE(SM)                                                                                  \
     do {                                                                                                        \
@@ -856,10 +1040,10 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __
     // Set 0 walks the tiles 0, 2, 4, ..., set 1 the tiles 1, 3, 5, ...: both make the same number of passes.  One
     // barrier per pass: behind it the pass's buffer is complete and nobody reads the other buffer any more, which
     // the pass then fills -- after its own products -- from the registers that the loads of the pass before filled.
-    LLMOPS_STAGE_LOAD(set * BK);
+    LLMOPS_STAGE_LOAD(kv_begin + set * BK);
     LLMOPS_STAGE_STORE(sm2[0]);
-    if (2 * BK < kv_end) LLMOPS_STAGE_LOAD(set * BK + 2 * BK);
-    for (int kv_pair = 0, pass = 0; kv_pair < kv_end; kv_pair += 2 * BK, pass++) {
+    if (kv_begin + 2 * BK < kv_end) LLMOPS_STAGE_LOAD(kv_begin + set * BK + 2 * BK);
+    for (int kv_pair = kv_begin, pass = 0; kv_pair < kv_end; kv_pair += 2 * BK, pass++) {
         PrefillSmem<LO>& sm = sm2[pass & 1];
         const uint8_t* kp_hi = &sm.k_hi[c32 * KSB + 16 * hf];  // + 32 i
         const uint8_t* kp_lo = &sm.k_lo[LO ? c32 * KSB + 16 * hf : 0];
@@ -1000,10 +1184,24 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __
         const float mm = fmaxf(m_run, m1);
         const float a0 = expf(m_run - mm), a1 = expf(m1 - mm);  // (a set that saw no row has sum 0 and outputs 0)
         l_run = l_run * a0 + l1 * a1;
+        m_run = mm;
 #pragma unroll
         for (int c = 0; c < 4; c++)
 #pragma unroll
             for (int r = 0; r < 16; r++) o[c][r] = o[c][r] * a0 + mrg[(2 + 16 * c + r) * 256] * a1;
+    }
+    if (nsplit > 1) {  // a record [max, sum, out[S]] for attn_merge_kernel
+        float* rec = part + ((bh * qL + pq) * nsplit + blockIdx.y) * (S + 2);
+        if (hf == 0) *reinterpret_cast<float2*>(rec) = make_float2(m_run, l_run);
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                float2* dst = reinterpret_cast<float2*>(rec + 2 + 32 * c + 8 * j + 4 * hf);
+                dst[0] = make_float2(o[c][4 * j], o[c][4 * j + 1]);
+                dst[1] = make_float2(o[c][4 * j + 2], o[c][4 * j + 3]);
+            }
+        return;
     }
     const float inv = 1.0f / l_run;
     // the lane holds columns 32c + 8j + 4*hf + v of its query's output row
@@ -1178,17 +1376,27 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
         return LLMOPS_OK;
     }
     if (pos_dev != nullptr) return fail(LLMOPS_EINVAL, "a position in device memory needs one query token and half %% 4 == 0");
+    // the tiled kernel finds the token of a cache row in row_token; with fewer tokens a wave compares the slots itself
+    const bool tiled = qL >= g_prefill_min_tokens;
+    // One workgroup per query and chunk while there is little to read and multiply again for every token: a wave of
+    // attn_few_kernel runs some 2500 instructions whatever the size.  Measured (us, per query / all tokens together, 32
+    // heads): 2 tokens behind 1000 14.8 / 17.1, behind 2000 21.0 / 23.3, behind 3500 47 / 33; 4 behind 500 14.2 / 16.8, behind
+    // 1000 19.4 / 17.5; 8 behind 100 12.6 / 15.8, behind 250 22.1 / 16.4; 16 behind 30 14.5 / 16.1, behind 100 18.2 / 16.9;
+    // 31 behind none 16.9 / 17.9, behind 30 19.6 / 18.2.
+    const bool per_query = bhq * kvLen < (qL <= 2 ? 192 << 10 : 56 << 10);
     const int pw = pick_pw(bhq, kvLen);
-    const int nchunks = (int)((kvLen + 4 * pw - 1) / (4 * pw));
-    const unsigned grid = (unsigned)(bhq * nchunks);
-    if (qL > 1) {
+    const int rows_chunk = per_query ? 4 * pw : 128;
+    const int nchunks = (int)((kvLen + rows_chunk - 1) / rows_chunk);
+    if (!tiled && (int64_t)bhq * nchunks > max_records)
+        return fail(LLMOPS_EWORKSPACE, "attention workspace too small for %lld chunk records", (long long)bhq * nchunks);
+    if (tiled) {
         fill_i32_kernel<<<(unsigned)((maxlen + 255) / 256), 256, 0, st>>>(row_token, maxlen, -1);
         LLMOPS_LAUNCH_CHECK();
     }
     attn_prep_kernel<T><<<(unsigned)(B * qL * H), 64, 0, st>>>(q, k, v, qL, H, S, inv_freq, half, kc, vc, maxlen, slots,
-                                                              position_id, row_token);
+                                                              position_id, tiled ? row_token : nullptr);
     LLMOPS_LAUNCH_CHECK();
-    if (qL >= g_prefill_min_tokens) {
+    if (tiled) {
         // enough query tokens to share K/V tiles: the MFMA kernel reads the cache once per 128 queries
         if (maxlen * S * (int64_t)sizeof(T) >= ((int64_t)1 << 32))
             return fail(LLMOPS_EINVAL, "attention over 32 or more query tokens: a head's cache plane must be below 4 GiB");
@@ -1200,17 +1408,34 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
             configured = true;
         }
-        attn_prefill_kernel<T><<<(unsigned)(B * H * qtiles), 512, smem, st>>>(q, kc, vc, qL, H, maxlen, kvLen, row_token, qtiles);
+        // A workgroup takes a compute unit: with fewer query tiles than those, ns workgroups share a tile's cache rows, at
+        // least 128 each.  A row costs a tile 0.041 us; the records and the launch that merges them cost 3 us and 1.6 us per
+        // 1000 queries (us, one / split, 32 heads: 32 tokens behind 500 35.8 / 22.9, behind 3500 158 / 40; 64 behind 100
+        // 22.3 / 24.9, behind 250 27.9 / 25.6; 128 behind 1500 91 / 44; 256 behind none 32 / 42, behind 500 56 / 47; 512 behind
+        // 500 72.6 / 74.4, behind 1500 119 / 98).
+        const int64_t wgs = B * H * qtiles;
+        int64_t ns = 256 / wgs;
+        if (ns > (kvLen + 127) / 128) ns = (kvLen + 127) / 128;
+        if (ns < 2 || bhq * ns > max_records || 0.041 * (double)(kvLen - kvLen / ns) < 3.0 + 1.6e-3 * (double)bhq) ns = 1;
+        const int64_t span = ((kvLen + ns - 1) / ns + 63) / 64 * 64;
+        ns = (kvLen + span - 1) / span;
+        attn_prefill_kernel<T><<<dim3((unsigned)wgs, (unsigned)ns), 512, smem, st>>>(q, kc, vc, qL, H, maxlen, kvLen, row_token, qtiles, (int)span,
+                                                                                     part, (int)ns);
         LLMOPS_LAUNCH_CHECK();
+        if (ns > 1) {
+            attn_merge_kernel<<<(unsigned)bhq, 128, 0, st>>>(q, part, qL, H, (int)ns);
+            LLMOPS_LAUNCH_CHECK();
+        }
         return LLMOPS_OK;
     }
-    if ((int64_t)bhq * nchunks > max_records) return fail(LLMOPS_EWORKSPACE, "attention workspace too small for %lld chunk records", (long long)bhq * nchunks);
-    if (pw == 16)
-        attn_split_kernel<T, 16><<<grid, 256, 0, st>>>(q, kc, vc, qL, H, maxlen, kvLen, row_token, part, nchunks);
+    if (!per_query)
+        attn_few_kernel<T><<<(unsigned)(B * H * nchunks), 256, 0, st>>>(q, kc, vc, (int)qL, H, maxlen, (int)kvLen, slots, part, nchunks);
+    else if (pw == 16)
+        attn_split_kernel<T, 16><<<(unsigned)(bhq * nchunks), 256, 0, st>>>(q, kc, vc, qL, H, maxlen, kvLen, slots, part, nchunks);
     else if (pw == 8)
-        attn_split_kernel<T, 8><<<grid, 256, 0, st>>>(q, kc, vc, qL, H, maxlen, kvLen, row_token, part, nchunks);
+        attn_split_kernel<T, 8><<<(unsigned)(bhq * nchunks), 256, 0, st>>>(q, kc, vc, qL, H, maxlen, kvLen, slots, part, nchunks);
     else
-        attn_split_kernel<T, 4><<<grid, 256, 0, st>>>(q, kc, vc, qL, H, maxlen, kvLen, row_token, part, nchunks);
+        attn_split_kernel<T, 4><<<(unsigned)(bhq * nchunks), 256, 0, st>>>(q, kc, vc, qL, H, maxlen, kvLen, slots, part, nchunks);
     LLMOPS_LAUNCH_CHECK();
     attn_merge_kernel<<<(unsigned)bhq, 128, 0, st>>>(q, part, qL, H, nchunks);
     LLMOPS_LAUNCH_CHECK();

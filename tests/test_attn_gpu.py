@@ -207,6 +207,48 @@ def _attend_cache(orc, q, inv_freq, cache, slots, past, maxlen):
     return o.transpose(0, 2, 1, 3).reshape(B, qL, HS)
 
 
+@pytest.mark.parametrize("B,qL,kv,H", [(1, 2, 6200, 32), (1, 3, 700, 32), (1, 31, 127, 32), (2, 17, 128, 32), (1, 16, 129, 32),
+                                       (1, 31, 60, 32), (1, 5, 385, 32), (1, 33, 700, 8), (2, 64, 449, 4), (1, 130, 1025, 4)])
+@pytest.mark.parametrize("cache_dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("order", ["in order", "shuffled", "one out of range"])
+def test_attention_tokens_behind_a_cache(ops, B, qL, kv, H, cache_dtype, order):
+    """Several query tokens behind a filled cache, on either side of every rule: one workgroup per query, all tokens of a
+    head in one workgroup (cache rows just below, at and above a workgroup's 128 and a wave's 32, longest and shortest
+    runs), and the tiled kernel with the cache rows in several pieces.  The new rows at the end of the cache in order, or
+    anywhere in any order (what a later token wrote is masked wherever it lies; a piece of the cache may hold nothing that
+    an early token may see), or with one slot outside the cache (dropped).  fp32: 1e-5 as in the other tests; an fp16
+    cache against fp32 math on its own rounded rows."""
+    S = 128
+    rng = np.random.default_rng(qL * 1000 + kv)
+    q, k, v = (rng.standard_normal((B, qL, H * S)).astype(np.float32) for _ in range(3))
+    cache = rng.standard_normal((2, B, H, kv, S)).astype(np.float32).astype(np.float16).astype(np.float32)
+    inv_freq = (1.0 / (10000.0 ** (np.arange(0, S, 2, dtype=np.float32) / np.float32(S)))).astype(np.float32)
+    slots = np.arange(kv - qL, kv, dtype=np.int32)
+    if order != "in order":
+        slots = rng.permutation(kv)[:qL].astype(np.int32)
+    tq, tk, tv, tc = dev(q), dev(k), dev(v), dev(cache).to(cache_dtype)
+    given = slots.copy()
+    if order == "one out of range":
+        given[qL // 2] = kv + 5
+    ops.attention_rope2(tq, tk, tv, dev(inv_freq), tc, dev(given), kv - qL, 0)
+    # the reference attends in 64 bits to what the call left in the cache, the in-chunk mask applied by hand
+    rows = host(tc.float())
+    tok = np.full(kv, -1)
+    for l, s in enumerate(given):
+        if s < kv:
+            tok[s] = l
+    rot = host(tk)
+    for l, s in enumerate(given):
+        if s < kv:
+            assert np.array_equal(rows[0, :, :, s].reshape(B, -1), rot[:, l].astype(np.float16).astype(np.float32) if cache_dtype == torch.float16 else rot[:, l])
+    qr = dev(q)
+    ops.rope_embed(q4 := qr.reshape(B, qL, H, S).transpose(1, 2).contiguous(), dev(inv_freq), kv - qL)
+    sc = torch.matmul(q4.double(), dev(rows[0]).double().transpose(-1, -2).contiguous()) / np.sqrt(np.float64(S))
+    sc = sc.masked_fill(dev(tok)[None, :] > torch.arange(qL, device="cuda")[:, None], float("-inf"))
+    want = torch.matmul(sc.softmax(-1), dev(rows[1]).double()).transpose(1, 2).reshape(B, qL, H * S)
+    assert max_rel_err(host(tq), want.cpu().numpy()) <= 1e-5
+
+
 def test_rope_and_softmax_golden(ops):
     g = load_golden("misc.npz")
     x = dev(g["rope_x"])
