@@ -57,6 +57,22 @@ def test_pack_row_stride(ops, orc):
     assert np.array_equal(host(ops.offline_FC_quant_Q4A(view, 128)), orc.quant_w(w[:, :512], 128))
 
 
+@pytest.mark.parametrize("G", [32, 128])
+@pytest.mark.parametrize("N,K,ld,shift", [(1, 1, 1, 0), (33, 129, 132, 0), (31, 127, 128, 0), (64, 256, 258, 0), (64, 256, 256, 1),
+                                          (40, 416, 420, 4), (32, 1001, 1004, 3), (96, 36, 36, 0)])
+def test_pack_and_unpack_edges(ops, orc, G, N, K, ld, shift):
+    """K that cuts a thread's eight values, a block or a workgroup's four blocks; rows that do not start on 16 bytes; values
+    half-way between two codes.  Bytes equal the oracle's, and so do the unpacked values."""
+    rng = np.random.default_rng(N * K + G + shift)
+    flat = (rng.standard_normal(N * ld + shift) * 0.02).astype(np.float32)
+    w = flat[shift:].reshape(N, ld)
+    w[::3] = rng.integers(0, 31, w[::3].shape) * np.float32(0.5)  # halves in a range of 15
+    got = ops.offline_FC_quant_Q4A(dev(flat)[shift:].view(N, ld)[:, :K], G)
+    want = orc.quant_w(np.ascontiguousarray(w[:, :K]), G)
+    assert np.array_equal(host(got), want)
+    assert np.array_equal(host(ops.offline_FC_dequant_Q4A(got)).view(np.uint32), orc.dequant_w(want).view(np.uint32))
+
+
 # ---- activation quantization --------------------------------------------------------------------
 @pytest.mark.parametrize("G", [32, 128])
 def test_quant_x_golden(ops, G):
