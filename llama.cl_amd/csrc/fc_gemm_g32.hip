@@ -100,14 +100,14 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int kg = min(Kg - 1, kg0 + (i & 1) * 2 + h);
-            copy16_to_lds(bbase, boff[i] + (uint32_t)kg * (uint32_t)BLK, lds_b + buf * (STRIPS * 2048) + (wave * 4 + i) * 1024);
+            copy16_to_lds(bbase, boff[i] + (uint32_t)kg * (uint32_t)BLK, uniform_u32(lds_b + buf * (STRIPS * 2048) + (wave * 4 + i) * 1024));
         }
-        copy16_to_lds(abase, arow + min((uint32_t)st * 128u + achunk, (uint32_t)Kp - 16u), lds_a + buf * (BM * 128) + wave * 1024);
+        copy16_to_lds(abase, arow + min((uint32_t)st * 128u + achunk, (uint32_t)Kp - 16u), uniform_u32(lds_a + buf * (BM * 128) + wave * 1024));
         if (PARTIALS) return;
         {
             const int c = wave & 1, kg = min(Kg - 1, kg0 + 2 * c + h);
             const bool sums = wave >= 2;  // uniform
-            const uint32_t dst = sums ? lds_g + (ring * BM + c * 64) * 4 : lds_x + (buf * GPS * BM + c * 64) * 4;
+            const uint32_t dst = uniform_u32(sums ? lds_g + (ring * BM + c * 64) * 4 : lds_x + (buf * GPS * BM + c * 64) * 4);
             if (xsT) {
                 const int kgb = min(Kg - 1, kg0 + 2 * c);
                 copy4_to_lds(uniform_ptr(reinterpret_cast<const float*>(xsT + (int64_t)kgb * rows) + (sums ? 1 : 0)),
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
                 copy4_to_lds(uniform_ptr((sums ? gs : xd) + (int64_t)row0 * Kg), (uint32_t)((xrow - row0) * Kg + kg) * 4u, dst);
             }
         }
-        copy16_to_lds(bbase + (int64_t)min(Kg - 1, kg0 + wave) * BLK, doff, lds_d + (ring + wave) * (STRIPS * 128));
+        copy16_to_lds(bbase + (int64_t)min(Kg - 1, kg0 + wave) * BLK, doff, uniform_u32(lds_d + (ring + wave) * (STRIPS * 128)));
     };
 
     if (st0 < st1) copy_stage(st0, 0);
