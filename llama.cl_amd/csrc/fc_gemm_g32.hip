@@ -7,22 +7,28 @@
 // and out of its way:
 //   * tile 32 rows x 256 columns, four waves side by side (each 32 x 64 = two strips): a strip's weights are unpacked by
 //     one wave only, and the rows' codes and scales are read from LDS by all four.  (Sixty-four rows x 128 columns, two
-//     waves either way: 0 to 3 % slower at almost every size, 512 x 11008 x 4096 116.4 against 113.8 us; 128 x 128 with
-//     64 x 64 per wave 122 us: its 256 registers leave two waves per SIMD.)
+//     waves either way: 0 to 3 % slower at almost every size, 512 x 11008 x 4096 by 2 %; 128 x 128 with 64 x 64 per wave by
+//     7 %: its 256 registers leave two waves per SIMD.)
 //   * a stage is four k-groups.  Codes, packed blocks, scales and sums are all copied to LDS asynchronously
 //     (global_load_lds) one stage ahead: no registers, no LDS store instructions, 16 bytes per lane where the layout has
 //     them.  (Weights taken straight from memory into operand registers, one dword per lane and load, cost more than
-//     all of the arithmetic: 203 against 124 us.)
+//     all of the arithmetic: 1.6 times the time of the call.)
 //   * the fold of one step runs while the next step's MFMA does: two accumulators, the order pinned.
 //   * f += d * dx * sum in two instructions: the sums start at the bit pattern of 1.5 * 2^23 (gemm_device.h), so the
 //     register read as a float X is bias + sum and fma(X, d, -bias * d) = sum * d, exact before its one rounding
 //     (|sum| <= 32 * 15 * 127 < 2^22; bias * d has 2 + 11 significant bits).
-//   * the min term, sum over k-groups of m[column] * gsum[row], is a product with K = number of k-groups: every eight
-//     k-groups one v_mfma_f32_32x32x16_f16 per strip on gsum = hi + lo (22 bits; fp32 MFMAs where the sums do not suit
-//     fp16), instead of a third vector instruction per element.
-// Measured (us for the whole call, before -- one wave per 64 rows x 64 columns, operands straight from memory, three
-// instructions per fold -- and now): 512 x 11008 x 4096 330 / 114, 512 x 4096 x 11008 230 / 103, 2048 x 4096^2 291 / 139,
-// 64 x 4096^2 40 / 21, 9 x 4096 x 11008 33 / 21, 300 x 1024 x 2048 35 / 19.
+//   * the min term, sum over k-groups of m[column] * gsum[row], is a product with K = number of k-groups, on the matrix
+//     cores instead of a third vector instruction per element: gsum = three and m = two bf16 pieces, exactly and at any
+//     scale, and the six products of two k-groups fill one v_mfma_f32_32x32x16_bf16 per strip.  It runs between the folds
+//     of its two groups: the weights' codes are positive, so what a fold adds is several times what the min term
+//     leaves of it, and the fewer groups a sum holds uncorrected the less it loses to rounding.  rms error of the outputs,
+//     64 x 1024, against 64 bits, in 1e-7 of their rms, two instructions per element and group as before / fp16 halves of
+//     gsum every eight groups / now: K = 512 1.16 / 2.91 / 1.16, 1024 1.36 / 3.04 / 1.30, 4096 2.22 / 3.54 / 1.58, 11008
+//     2.18 / 3.52 / 1.79.  (Four groups at a time, a bf16 and a half-length bf16 product: 1.20 / 1.25 / 1.51 / 1.72, and
+//     0 to 2 % faster.)
+// Measured (us for the whole call in a graph, before -- one wave per 64 rows x 64 columns, operands straight from memory,
+// three instructions per fold -- and now): 512 x 11008 x 4096 330 / 109, 512 x 4096 x 11008 230 / 97, 2048 x 4096^2
+// 291 / 133, 64 x 4096^2 40 / 20.5, 9 x 4096 x 11008 33 / 20.4, 300 x 1024 x 2048 35 / 18.5.
 #include "gemm_device.h"
 #include "gemv_device.h"
 
@@ -32,6 +38,17 @@ constexpr int kG32Blk = 640;       // bytes of a packed block: 512 of nibbles, 3
 constexpr int kG32Rows = 32;       // rows and strips of a tile
 constexpr int kG32Strips = 8;
 constexpr int kG32Gps = 4;         // k-groups per stage
+
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+union Bf16x8 {
+    v8bf h;
+    uint32_t u[4];
+};
+// the first 8 significant bits of a float (what its upper half is as a bf16), and the upper halves of two floats
+__device__ __forceinline__ float bf_piece(float v) { return __uint_as_float(__float_as_uint(v) & 0xFFFF0000u); }
+__device__ __forceinline__ uint32_t bf_pair(float lo, float hi) {
+    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
 
 // PARTIALS: test build that stores the int32 sums of every (row, column, k-group) into out_i ([rows][Ng*32][Kg])
 template <bool PARTIALS>
@@ -45,8 +62,8 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
     __shared__ __align__(16) uint8_t sa[2][BM * 128];           // codes, 128 bytes per row
     __shared__ __align__(16) uint8_t sbn[2][STRIPS * 2048];     // nibbles, 16 k8-rows of 128 bytes per strip
     __shared__ __align__(16) float sx[2][GPS * BM];             // activation scales [k-group][row]
-    __shared__ __align__(16) uint16_t sdm[16 * STRIPS * 64];    // ring of 16 k-groups: [strip][32 scales, 32 mins]
-    __shared__ __align__(16) float sg[16 * BM];                 // ring of 16 k-groups: activation sums [row]
+    __shared__ __align__(16) uint16_t sdm[2][GPS * STRIPS * 64];  // [k-group][strip][32 scales, 32 mins]
+    __shared__ __align__(16) float sg[2][GPS * BM];             // activation sums [k-group][row]
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -79,8 +96,8 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
     const uint8_t* abase = reinterpret_cast<const uint8_t*>(xq) + (int64_t)row0 * Kp;
     const uint32_t arow = (uint32_t)(min(rows - 1, row0 + wave * 8 + (lane >> 3)) - row0) * (uint32_t)Kp;
     const uint32_t achunk = (uint32_t)(((lane & 7) ^ (((lane >> 3) + (wave & 1)) & 7)) * 16);
-    const uint32_t lds_a = lds_off(&sa[0][0]), lds_b = lds_off(&sbn[0][0]), lds_x = lds_off(&sx[0][0]), lds_d = lds_off(&sdm[0]),
-                   lds_g = lds_off(&sg[0]);
+    const uint32_t lds_a = lds_off(&sa[0][0]), lds_b = lds_off(&sbn[0][0]), lds_x = lds_off(&sx[0][0]), lds_d = lds_off(&sdm[0][0]),
+                   lds_g = lds_off(&sg[0][0]);
     // nibbles: two strips, 8 k8-rows to a copy, the two low bits of the row number exchanged: the rows 4s+2h+p that the lane
     // halves h = 0, 1 read together lie side by side
     const uint32_t sb = (uint32_t)Kg * (uint32_t)BLK;  // bytes of a strip
@@ -96,7 +113,7 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
     // activation scales (waves 0, 1) and sums (waves 2, 3): two k-groups of 32 rows to a copy
     const int xrow = min(rows - 1, row0 + j);
     auto copy_stage = [&](int st, int buf) {
-        const int kg0 = st * GPS, ring = (kg0 - st0 * GPS) & 15;
+        const int kg0 = st * GPS;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int kg = min(Kg - 1, kg0 + (i & 1) * 2 + h);
@@ -107,7 +124,7 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
         {
             const int c = wave & 1, kg = min(Kg - 1, kg0 + 2 * c + h);
             const bool sums = wave >= 2;  // uniform
-            const uint32_t dst = uniform_u32(sums ? lds_g + (ring * BM + c * 64) * 4 : lds_x + (buf * GPS * BM + c * 64) * 4);
+            const uint32_t dst = uniform_u32((sums ? lds_g : lds_x) + (buf * GPS * BM + c * 64) * 4);
             if (xsT) {
                 const int kgb = min(Kg - 1, kg0 + 2 * c);
                 copy4_to_lds(uniform_ptr(reinterpret_cast<const float*>(xsT + (int64_t)kgb * rows) + (sums ? 1 : 0)),
@@ -116,7 +133,7 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
                 copy4_to_lds(uniform_ptr((sums ? gs : xd) + (int64_t)row0 * Kg), (uint32_t)((xrow - row0) * Kg + kg) * 4u, dst);
             }
         }
-        copy16_to_lds(bbase + (int64_t)min(Kg - 1, kg0 + wave) * BLK, doff, uniform_u32(lds_d + (ring + wave) * (STRIPS * 128)));
+        copy16_to_lds(bbase + (int64_t)min(Kg - 1, kg0 + wave) * BLK, doff, uniform_u32(lds_d + (buf * GPS + wave) * (STRIPS * 128)));
     };
 
     if (st0 < st1) copy_stage(st0, 0);
@@ -135,7 +152,7 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
     for (int ks = 0; ks < 4; ks++) a_rd[ks] = j * 128 + (((2 * ks + h) ^ akey) * 16);
 
     for (int st = st0; st < st1; st++) {
-        const int buf = (st - st0) & 1, ring = ((st - st0) * GPS) & 15;
+        const int buf = (st - st0) & 1;
         const bool more = st + 1 < st1;
         v4i af[4];
         float4 xf[2][4];
@@ -158,10 +175,29 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
                 const uint32_t w0 = *reinterpret_cast<const uint32_t*>(bs + ks * 512), w1 = *reinterpret_cast<const uint32_t*>(bs + ks * 512 + 256);
                 bu[s][ks] = v4i{(int)lo4(w0), (int)hi4(w0), (int)lo4(w1), (int)hi4(w1)};
                 // (k-groups past the end: d = 0 and nothing is added)
-                const uint16_t bits = sdm[(ring + ks) * (STRIPS * 64) + (2 * wave + s) * 64 + j];
+                const uint16_t bits = sdm[buf][ks * (STRIPS * 64) + (2 * wave + s) * 64 + j];
                 d[s][ks] = f16_bits_to_f32(st * GPS + ks < kg1 ? bits : (uint16_t)0);
                 // converted once, not inside every fma of the fold (v_fma_mix runs at half the rate of v_fma)
                 asm volatile("" : "+v"(d[s][ks]));
+            }
+        }
+        // Min term operands: lane half h has the stage's k-groups h and 2 + h.  The row's sum g = g1 + g2 + g3 and the
+        // column's min m = m1 + m2 in bf16 pieces (g3 and m2 have at most 8 bits left, so their low halves are zero; the low
+        // half of m meets that of g3).
+        Bf16x8 ga[2], ma[2][2];  // [pair of k-groups], [strip][pair]
+        if (!PARTIALS) {
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                const float sum = sg[buf][(2 * p + h) * BM + j];
+                const float g1 = st * GPS + 2 * p + h < kg1 ? sum : 0.0f;  // (k-groups past the end add nothing)
+                const float g2 = g1 - bf_piece(g1), g3 = g2 - bf_piece(g2);
+                ga[p].u[0] = ga[p].u[2] = bf_pair(g1, g2), ga[p].u[1] = ga[p].u[3] = __float_as_uint(g3);
+#pragma unroll
+                for (int s = 0; s < 2; s++) {
+                    const float m = f16_bits_to_f32(sdm[buf][(2 * p + h) * (STRIPS * 64) + (2 * wave + s) * 64 + 32 + j]), m2 = m - bf_piece(m);
+                    ma[s][p].u[0] = bf_pair(m, m), ma[s][p].u[1] = __float_as_uint(m);
+                    ma[s][p].u[2] = bf_pair(m2, m2), ma[s][p].u[3] = __float_as_uint(m2);
+                }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -197,54 +233,10 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
                     f[s][4 * b + 2] = fmaf(fmaf(__int_as_float(acc[s][4 * b + 2]), dd, nbd), x.z, f[s][4 * b + 2]);
                     f[s][4 * b + 3] = fmaf(fmaf(__int_as_float(acc[s][4 * b + 3]), dd, nbd), x.w, f[s][4 * b + 3]);
                 }
+                // (the strip's next fold is two steps away: nothing waits for the product)
+                if ((kk & 1) == 0) f[s] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ga[kk >> 1].h, ma[s][kk >> 1].h, f[s], 0, 0, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
-        }
-        // ---- min term of the eight k-groups of this stage and the one before (of this one alone where the run ends after
-        // an odd number of stages): lane half h has the groups 4h .. 4h+3, hi in the first four slots and lo in the others ----
-        if (!PARTIALS && (((st - st0) & 1) == 1 || !more)) {
-            const int rel = ((st - st0) & ~1) * GPS + 4 * h;  // first group of this lane, counted from the split's first
-            const int left = kg1 - st0 * GPS - rel;           // how many of its four count (the others: any value)
-            uint32_t mb[2][4];
-            float ga[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int slot = (rel + i) & 15;
-                const float v = sg[slot * BM + j];
-                ga[i] = i < left ? v : 0.0f;
-#pragma unroll
-                for (int s = 0; s < 2; s++) {
-                    const uint32_t m = sdm[slot * (STRIPS * 64) + (2 * wave + s) * 64 + 32 + j];
-                    mb[s][i] = i < left ? m : 0u;
-                }
-            }
-            // hi + lo in fp16 is good for a lane's four sums if the largest lies in [1/8, 60000]: below that lo falls into the
-            // subnormals, above it hi overflows.  Otherwise the wave takes fp32 MFMAs (exact products).
-            const float big = fmaxf(fmaxf(fabsf(ga[0]), fabsf(ga[1])), fmaxf(fabsf(ga[2]), fabsf(ga[3])));
-            const bool nan = ga[0] != ga[0] || ga[1] != ga[1] || ga[2] != ga[2] || ga[3] != ga[3];
-            if (__all(!nan && (big == 0.0f || (big >= 0.125f && big <= 60000.0f)))) {
-                Halves8 a;
-#pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    const v2h hh = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(ga[2 * i], ga[2 * i + 1]));
-                    a.u[i] = __builtin_bit_cast(uint32_t, hh);
-                    a.u[2 + i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(ga[2 * i] - (float)hh[0], ga[2 * i + 1] - (float)hh[1]));
-                }
-#pragma unroll
-                for (int s = 0; s < 2; s++) {
-                    Halves8 m;
-                    m.u[0] = m.u[2] = mb[s][0] | (mb[s][1] << 16);
-                    m.u[1] = m.u[3] = mb[s][2] | (mb[s][3] << 16);
-                    f[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.h, m.h, f[s], 0, 0, 0);
-                }
-            } else {
-                // slot i of lanes (h = 0, 1; j) is one 32x32x2 product: k = h
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-#pragma unroll
-                    for (int s = 0; s < 2; s++)
-                        f[s] = __builtin_amdgcn_mfma_f32_32x32x2f32(ga[i], f16_bits_to_f32((uint16_t)mb[s][i]), f[s], 0, 0, 0);
-            }
         }
         __builtin_amdgcn_s_waitcnt(kVmcnt0);  // this wave's copies for the next stage have landed
         __syncthreads();
