@@ -249,6 +249,64 @@ __device__ __forceinline__ void split_bf(Bf3& d, int e, float a, float b) {
     }
 }
 
+// What does not go through the pieces: infinities (and what rounds to one, or whose products of pieces overflow where
+// the sum would not) and values whose later pieces are subnormal, which the matrix cores take as zero.  A wave that meets
+// such rows or queries forms its sums in fp32, as the per-query kernel does.  Scores: the former leave a score that is
+// not finite; of the latter less than 2^-126 of the other factor is lost, which an exponent does not notice while |q| and
+// |k| stay below 2^90.  Outputs: the lane's values are all below 2^56 and, unless all are zero, one of them reaches 2^-90.
+constexpr float kFewMax = 0x1p56f, kFewMin = 0x1p-90f;
+__device__ __forceinline__ float max_abs(float m, float4 v) {
+    return fmaxf(fmaxf(fmaxf(fmaxf(m, fabsf(v.x)), fabsf(v.y)), fabsf(v.z)), fabsf(v.w));  // (in this order: two v_max3_f32)
+}
+// the wave's 32 x qL scores before scaling, into the layout of the MFMA's result; krow, q0: the lane's row and the first
+// query from dim 8 * hf on; buf: 32 * 32 floats of the wave's own
+template <typename T>
+__device__ __forceinline__ void few_scores_fp32(const T* krow, const float* q0, int qL, int64_t q_stride, float* buf, int c32,
+                                                          int hf, v16f& pr) {
+    for (int l = 0; l < qL; l++) {
+        float s = 0.0f;
+#pragma unroll 1
+        for (int i = 0; i < 8; i++) {
+#pragma unroll
+            for (int e = 0; e < 8; e += 4) {
+                const float4 a = load4(krow + 16 * i + e), w = load4(q0 + l * q_stride + 16 * i + e);
+                s = fmaf(a.x, w.x, s), s = fmaf(a.y, w.y, s), s = fmaf(a.z, w.z, s), s = fmaf(a.w, w.w, s);
+            }
+        }
+        s += __shfl_xor(s, 32, 64);
+        if (hf == 0) buf[l * 32 + c32] = s;
+    }
+    __builtin_amdgcn_wave_barrier();
+    const float* mine = buf + min(c32, qL - 1) * 32 + 4 * hf;
+#pragma unroll
+    for (int jj = 0; jj < 4; jj++) {
+        const float4 x = *reinterpret_cast<const float4*>(mine + 8 * jj);
+        pr[4 * jj] = x.x, pr[4 * jj + 1] = x.y, pr[4 * jj + 2] = x.z, pr[4 * jj + 3] = x.w;
+    }
+}
+// the wave's 64 output elements of the lane's query; dst: the lane's place in the first of the 16 result registers
+template <typename T>
+__device__ __forceinline__ void few_outputs_fp32(const T* vbase, int p0, int kvLen, int c32, int hf, const v16f& pr, float* dst) {
+    float w[2][16];  // [half that holds the row][register]
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(pr[r]), __float_as_uint(pr[r]), false, false);
+        w[0][r] = __uint_as_float(sw[0]), w[1][r] = __uint_as_float(sw[1]);
+    }
+#pragma unroll 1
+    for (int r = 0; r < 16; r++) {
+        const int col = 4 * (8 * (r >> 2) + 4 * hf + (r & 3));
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int row = 0; row < 32; row++) {
+            const float4 v = load4(vbase + (int64_t)min(p0 + row, kvLen - 1) * 128 + col);
+            const float p = w[(row >> 2) & 1][4 * (row >> 3) + (row & 3)];
+            a.x = fmaf(p, v.x, a.x), a.y = fmaf(p, v.y, a.y), a.z = fmaf(p, v.z, a.z), a.w = fmaf(p, v.w, a.w);
+        }
+        *reinterpret_cast<float4*>(dst + r * 256) = a;
+    }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256, 2) void attn_few_kernel(const float* __restrict__ q, const T* __restrict__ kc,
                                                            const T* __restrict__ vc, int qL, int64_t H, int64_t maxlen, int kvLen,
@@ -302,7 +360,12 @@ __global__ __launch_bounds__(256, 2) void attn_few_kernel(const float* __restric
     const float d_scale = 1.0f / sqrtf((float)S);
     const int pq = c32 < qL ? c32 : INT_MIN;
     __builtin_amdgcn_wave_barrier();
-    v16f pr;
+    v16f pr = (s0[0] + s0[1]) + s1;
+    float z = 0.0f;  // NaN if a score is not finite
+#pragma unroll
+    for (int r = 0; r < 16; r++) z = fmaf(pr[r], 0.0f, z);
+    if (__builtin_expect(__any(z != 0.0f), 0))
+        few_scores_fp32<T>(krow, q + (b * qL * H + h) * S + 8 * hf, qL, H * S, &os[wave][0][0][0], c32, hf, pr);
     float mx = -FLT_MAX;
 #pragma unroll
     for (int jj = 0; jj < 4; jj++) {
@@ -310,7 +373,7 @@ __global__ __launch_bounds__(256, 2) void attn_few_kernel(const float* __restric
         const int tt[4] = {t4.x, t4.y, t4.z, t4.w};
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            pr[4 * jj + v] = tt[v] <= pq ? ((s0[0][4 * jj + v] + s0[1][4 * jj + v]) + s1[4 * jj + v]) * d_scale : -FLT_MAX;
+            pr[4 * jj + v] = tt[v] <= pq ? pr[4 * jj + v] * d_scale : -FLT_MAX;
             mx = fmaxf(mx, pr[4 * jj + v]);
         }
     }
@@ -322,46 +385,55 @@ __global__ __launch_bounds__(256, 2) void attn_few_kernel(const float* __restric
     wm[wave][lane] = mx;
     __syncthreads();
     mx = fmaxf(fmaxf(wm[0][lane], wm[1][lane]), fmaxf(wm[2][lane], wm[3][lane]));
+    const float m0 = mx == -FLT_MAX ? 0.0f : mx;  // (a query that sees no row of the workgroup: all weights 0, sum 0)
     float sum = 0.0f;
 #pragma unroll
     for (int r = 0; r < 16; r++) {
-        pr[r] = pr[r] == -FLT_MAX ? 0.0f : expf(pr[r] - mx);
+        pr[r] = expf(pr[r] - m0);
         sum += pr[r];
     }
     wl[wave][lane] = sum;
-    v16f o[4];
+    float big[2] = {0.0f, 0.0f};
 #pragma unroll
-    for (int c = 0; c < 4; c++)
+    for (int r = 0; r < 16; r++) big[r & 1] = max_abs(big[r & 1], vr[r]);
+    big[0] = fmaxf(big[0], big[1]);
+    if (__builtin_expect(__any(big[0] > kFewMax || (big[0] < kFewMin && big[0] > 0.0f)), 0)) {
+        few_outputs_fp32<T>(vbase, p0, kvLen, c32, hf, pr, &os[wave][0][lane][0]);
+    } else {
+        v16f o[4];
 #pragma unroll
-        for (int r = 0; r < 16; r++) o[c][r] = 0.0f;
-    Bf3 w[2];
+        for (int c = 0; c < 4; c++)
 #pragma unroll
-    for (int e = 0; e < 8; e++) split_bf<3>(w[e >> 2], e & 3, pr[2 * e], pr[2 * e + 1]);
+            for (int r = 0; r < 16; r++) o[c][r] = 0.0f;
+        Bf3 w[2];
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-        Bf3 a[2];
+        for (int e = 0; e < 8; e++) split_bf<3>(w[e >> 2], e & 3, pr[2 * e], pr[2 * e + 1]);
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const float4 v0 = vr[2 * e], v1 = vr[2 * e + 1];
-            const float x0 = c == 0 ? v0.x : c == 1 ? v0.y : c == 2 ? v0.z : v0.w, x1 = c == 0 ? v1.x : c == 1 ? v1.y : c == 2 ? v1.z : v1.w;
-            split_bf<P>(a[e >> 2], e & 3, x0, x1);
+        for (int c = 0; c < 4; c++) {
+            Bf3 a[2];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float4 v0 = vr[2 * e], v1 = vr[2 * e + 1];
+                const float x0 = c == 0 ? v0.x : c == 1 ? v0.y : c == 2 ? v0.z : v0.w, x1 = c == 0 ? v1.x : c == 1 ? v1.y : c == 2 ? v1.z : v1.w;
+                split_bf<P>(a[e >> 2], e & 3, x0, x1);
+            }
+#pragma unroll
+            for (int bb = 0; bb < 2; bb++) {  // the small products first, while the sum is small
+                if (P == 3) o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[2].h, w[bb].p[0].h, o[c], 0, 0, 0);
+                o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[0].h, w[bb].p[2].h, o[c], 0, 0, 0);
+                o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[1].h, w[bb].p[1].h, o[c], 0, 0, 0);
+            }
+#pragma unroll
+            for (int bb = 0; bb < 2; bb++) {
+                o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[1].h, w[bb].p[0].h, o[c], 0, 0, 0);
+                o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[0].h, w[bb].p[1].h, o[c], 0, 0, 0);
+            }
+#pragma unroll
+            for (int bb = 0; bb < 2; bb++) o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[0].h, w[bb].p[0].h, o[c], 0, 0, 0);
         }
 #pragma unroll
-        for (int bb = 0; bb < 2; bb++) {  // the small products first, while the sum is small
-            if (P == 3) o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[2].h, w[bb].p[0].h, o[c], 0, 0, 0);
-            o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[0].h, w[bb].p[2].h, o[c], 0, 0, 0);
-            o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[1].h, w[bb].p[1].h, o[c], 0, 0, 0);
-        }
-#pragma unroll
-        for (int bb = 0; bb < 2; bb++) {
-            o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[1].h, w[bb].p[0].h, o[c], 0, 0, 0);
-            o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[0].h, w[bb].p[1].h, o[c], 0, 0, 0);
-        }
-#pragma unroll
-        for (int bb = 0; bb < 2; bb++) o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bb].p[0].h, w[bb].p[0].h, o[c], 0, 0, 0);
+        for (int r = 0; r < 16; r++) *reinterpret_cast<float4*>(&os[wave][r][lane][0]) = make_float4(o[0][r], o[1][r], o[2][r], o[3][r]);
     }
-#pragma unroll
-    for (int r = 0; r < 16; r++) *reinterpret_cast<float4*>(&os[wave][r][lane][0]) = make_float4(o[0][r], o[1][r], o[2][r], o[3][r]);
     __syncthreads();
     // wave w finishes the result registers 4w .. 4w+3: columns 4 * (8w + 4*hf + v) + c of the lane's query
     if (c32 >= qL) return;

@@ -249,6 +249,64 @@ def test_attention_tokens_behind_a_cache(ops, B, qL, kv, H, cache_dtype, order):
     assert max_rel_err(host(tq), want.cpu().numpy()) <= 1e-5
 
 
+@pytest.mark.parametrize("B,qL,kv", [(1, 4, 100), (1, 2, 2500), (1, 4, 2000), (2, 16, 700), (1, 31, 130)])
+@pytest.mark.parametrize("cache_dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("case", ["k -inf", "k +inf", "k huge", "v +inf", "v huge", "q inf", "new k inf", "tiny k", "tiny v"])
+def test_attention_few_tokens_extreme_values(ops, B, qL, kv, cache_dtype, case):
+    """2..31 tokens with one cache row (or one token's q, or the last token's k) that holds infinities or the largest finite
+    values, and with a whole cache of tiny ones: what 64-bit attention gives, NaN for NaN, infinity for
+    infinity.  A score of -inf is a row that drops out; a row that a token may not see does not reach it, whatever is in its
+    k; other heads and batch entries are untouched.  Finite outputs to 1e-5 of the sum of |weight * value|."""
+    H, S, half, tol = 8, 128, cache_dtype == torch.float16, 1e-5
+    rng = np.random.default_rng(qL + kv)
+    q, k, v = (rng.standard_normal((B, qL, H * S)).astype(np.float32) for _ in range(3))
+    cache = torch.from_numpy(rng.standard_normal((2, B, H, kv, S)).astype(np.float32))
+    top = 65504.0 if half else 3.395e38  # (above the largest bf16)
+    q *= 0.01  # (scores of the largest values stay finite)
+    row = (0, 0, slice(1, H), 7, 3)
+    vrow = (1,) + row[1:]
+    if case == "k -inf":
+        cache[row] = -np.inf
+    elif case == "k +inf":
+        cache[row] = np.inf
+    elif case == "k huge":
+        cache[row] = -top
+    elif case == "v +inf":
+        cache[vrow] = np.inf
+    elif case == "v huge":
+        cache[vrow] = top
+    elif case == "q inf":
+        q[0, 1, S + 3] = np.inf
+    elif case == "new k inf":
+        k[0, qL - 1, S + 3] = np.inf
+    elif case == "tiny k" and not half:
+        cache[0] *= 1e-25
+        q *= 1e27
+        k *= 1e-25
+    elif case == "tiny v" and not half:
+        cache[1] *= 1e-37
+        v *= 1e-37
+    inv_freq = (1.0 / (10000.0 ** (np.arange(0, S, 2, dtype=np.float32) / np.float32(S)))).astype(np.float32)
+    slots = np.arange(kv - qL, kv, dtype=np.int32)
+    tq, tk, tv, tc = dev(q), dev(k), dev(v), cache.cuda().to(cache_dtype)
+    ops.attention_rope2(tq, tk, tv, dev(inv_freq), tc, dev(slots), kv - qL, 0)
+    ops.rope_embed(q4 := dev(q).reshape(B, qL, H, S).transpose(1, 2).contiguous(), dev(inv_freq), kv - qL)
+    rows = tc.double().cpu()
+    sc = (q4.double().cpu().unsqueeze(3) * rows[0].unsqueeze(2)).sum(-1) / np.sqrt(np.float64(S))
+    later = torch.arange(kv)[None, :] - (kv - qL) > torch.arange(qL)[:, None]
+    w = sc.masked_fill(later, -np.inf).softmax(-1)
+    # (summed column by column, zero weights included: 0 * inf is NaN, as in fp32)
+    want = torch.stack([(w[..., None, :] * rows[1][:, :, None, :, c:c + 1].transpose(-1, -2)).sum(-1)[..., 0] for c in range(S)], -1)
+    want = want.transpose(1, 2).reshape(B, qL, H * S).numpy()
+    got = host(tq)
+    assert np.array_equal(np.isnan(got), np.isnan(want)), (np.isnan(got).sum(), np.isnan(want).sum())
+    fin = np.isfinite(want)
+    assert np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)])
+    scale = torch.matmul(w, rows[1].abs()).transpose(1, 2).reshape(B, qL, H * S).numpy()
+    err = np.where(fin, np.abs(got - np.where(fin, want, 0.0)), 0.0)[fin] / scale[fin]
+    assert err.max() <= tol, err.max()
+
+
 def test_rope_and_softmax_golden(ops):
     g = load_golden("misc.npz")
     x = dev(g["rope_x"])
