@@ -29,6 +29,8 @@
 // Measured (us for the whole call in a graph, before -- one wave per 64 rows x 64 columns, operands straight from memory,
 // three instructions per fold -- and now): 512 x 11008 x 4096 330 / 109, 512 x 4096 x 11008 230 / 97, 2048 x 4096^2
 // 291 / 133, 64 x 4096^2 40 / 20.5, 9 x 4096 x 11008 33 / 20.4, 300 x 1024 x 2048 35 / 18.5.
+#include <type_traits>
+
 #include "gemm_device.h"
 #include "gemv_device.h"
 
@@ -51,7 +53,8 @@ __device__ __forceinline__ uint32_t bf_pair(float lo, float hi) {
 }
 
 // PARTIALS: test build that stores the int32 sums of every (row, column, k-group) into out_i ([rows][Ng*32][Kg])
-template <bool PARTIALS>
+// WIDE: lane offsets of 64 bits, for a K whose eight strips are 4 GiB and more (K above 26.8 million)
+template <bool PARTIALS, bool WIDE>
 __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __restrict__ weiq, const int8_t* __restrict__ xq,
                                                               const float* __restrict__ xd, const float* __restrict__ gs,
                                                               const float2* __restrict__ xsT, float* __restrict__ out,
@@ -59,6 +62,7 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
                                                               int rows, int st_per_split, int64_t split_stride,
                                                               const float* __restrict__ residual) {
     constexpr int BM = kG32Rows, STRIPS = kG32Strips, GPS = kG32Gps, BLK = kG32Blk;
+    using offset_t = typename std::conditional<WIDE, uint64_t, uint32_t>::type;
     __shared__ __align__(16) uint8_t sa[2][BM * 128];           // codes, 128 bytes per row
     __shared__ __align__(16) uint8_t sbn[2][STRIPS * 2048];     // nibbles, 16 k8-rows of 128 bytes per strip
     __shared__ __align__(16) float sx[2][GPS * BM];             // activation scales [k-group][row]
@@ -87,29 +91,29 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
     const int nst = (Kg + GPS - 1) / GPS;
     const int st0 = blockIdx.z * st_per_split, st1 = min(nst, st0 + st_per_split);
     const int kg1 = min(Kg, st1 * GPS);
-    const int Kp = Kg * 32;
+    const offset_t Kp = (offset_t)Kg * 32;
 
     // ---- what this wave copies per stage.  Sources past the end (rows, strips, the last stage's k-groups) re-read the
     // last one that exists. ----
     // codes: rows 8*wave .. +7.  16-byte chunk c of row r lies at position c ^ key(r), key(r) = (r + ((r >> 3) & 1)) & 7: the
     // 16 rows that one phase of a ds_read_b128 touches fall on 16 different bank groups
-    const uint8_t* abase = reinterpret_cast<const uint8_t*>(xq) + (int64_t)row0 * Kp;
-    const uint32_t arow = (uint32_t)(min(rows - 1, row0 + wave * 8 + (lane >> 3)) - row0) * (uint32_t)Kp;
+    const uint8_t* abase = reinterpret_cast<const uint8_t*>(xq) + (int64_t)row0 * (int64_t)Kp;
+    const offset_t arow = (offset_t)(min(rows - 1, row0 + wave * 8 + (lane >> 3)) - row0) * Kp;
     const uint32_t achunk = (uint32_t)(((lane & 7) ^ (((lane >> 3) + (wave & 1)) & 7)) * 16);
     const uint32_t lds_a = lds_off(&sa[0][0]), lds_b = lds_off(&sbn[0][0]), lds_x = lds_off(&sx[0][0]), lds_d = lds_off(&sdm[0][0]),
                    lds_g = lds_off(&sg[0][0]);
     // nibbles: two strips, 8 k8-rows to a copy, the two low bits of the row number exchanged: the rows 4s+2h+p that the lane
     // halves h = 0, 1 read together lie side by side
-    const uint32_t sb = (uint32_t)Kg * (uint32_t)BLK;  // bytes of a strip
-    const uint8_t* bbase = weiq + (int64_t)tstrip * sb;
-    uint32_t boff[4];
+    const offset_t sb = (offset_t)Kg * BLK;  // bytes of a strip
+    const uint8_t* bbase = weiq + (int64_t)tstrip * (int64_t)sb;
+    offset_t boff[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int slot = (i & 1) * 8 + (lane >> 3), r = (slot & 12) | ((slot & 1) << 1) | ((slot >> 1) & 1);
-        boff[i] = (uint32_t)(min(Ng - 1, strip0 + (i >> 1)) - tstrip) * sb + (uint32_t)((r & 3) * kRowBytes + (lane & 7) * 16);
+        boff[i] = (offset_t)(min(Ng - 1, strip0 + (i >> 1)) - tstrip) * sb + (uint32_t)((r & 3) * kRowBytes + (lane & 7) * 16);
     }
     // scales and mins: k-group `wave` of the stage, 128 bytes per block, eight strips
-    const uint32_t doff = (uint32_t)(min(Ng - 1, tstrip + (lane >> 3)) - tstrip) * sb + (uint32_t)(512 + (lane & 7) * 16);
+    const offset_t doff = (offset_t)(min(Ng - 1, tstrip + (lane >> 3)) - tstrip) * sb + (uint32_t)(512 + (lane & 7) * 16);
     // activation scales (waves 0, 1) and sums (waves 2, 3): two k-groups of 32 rows to a copy
     const int xrow = min(rows - 1, row0 + j);
     auto copy_stage = [&](int st, int buf) {
@@ -117,9 +121,9 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int kg = min(Kg - 1, kg0 + (i & 1) * 2 + h);
-            copy16_to_lds(bbase, boff[i] + (uint32_t)kg * (uint32_t)BLK, uniform_u32(lds_b + buf * (STRIPS * 2048) + (wave * 4 + i) * 1024));
+            copy16_to_lds(bbase, boff[i] + (offset_t)kg * BLK, uniform_u32(lds_b + buf * (STRIPS * 2048) + (wave * 4 + i) * 1024));
         }
-        copy16_to_lds(abase, arow + min((uint32_t)st * 128u + achunk, (uint32_t)Kp - 16u), uniform_u32(lds_a + buf * (BM * 128) + wave * 1024));
+        copy16_to_lds(abase, arow + min((offset_t)st * 128u + achunk, Kp - 16u), uniform_u32(lds_a + buf * (BM * 128) + wave * 1024));
         if (PARTIALS) return;
         {
             const int c = wave & 1, kg = min(Kg - 1, kg0 + 2 * c + h);
@@ -128,9 +132,9 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
             if (xsT) {
                 const int kgb = min(Kg - 1, kg0 + 2 * c);
                 copy4_to_lds(uniform_ptr(reinterpret_cast<const float*>(xsT + (int64_t)kgb * rows) + (sums ? 1 : 0)),
-                             (uint32_t)((kg - kgb) * rows + xrow) * 8u, dst);
+                             (offset_t)((kg - kgb) * rows + xrow) * 8u, dst);
             } else {
-                copy4_to_lds(uniform_ptr((sums ? gs : xd) + (int64_t)row0 * Kg), (uint32_t)((xrow - row0) * Kg + kg) * 4u, dst);
+                copy4_to_lds(uniform_ptr((sums ? gs : xd) + (int64_t)row0 * Kg), ((offset_t)(xrow - row0) * Kg + kg) * 4u, dst);
             }
         }
         copy16_to_lds(bbase + (int64_t)min(Kg - 1, kg0 + wave) * BLK, doff, uniform_u32(lds_d + (buf * GPS + wave) * (STRIPS * 128)));
@@ -283,25 +287,36 @@ int plan_gemm_g32(int64_t rows, int64_t Ng, int64_t Kg, int force_split, int* st
     return (int)best_s;
 }
 
+// 32-bit lane offsets reach into a tile's strips (5120 bytes per k-group) and, of fewer bytes, its rows' codes and scales
+static bool g32_wide(int64_t Kg) { return Kg * kG32Blk * kG32Strips >= ((int64_t)1 << 32); }
+
 int launch_gemm_g32(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, const float2* xsT, float* out, int64_t Ng,
                     int64_t Kg, int64_t ldo, int64_t N, int64_t rows, int st_per_split, int S, int64_t split_stride,
                     const float* residual, hipStream_t st) {
-    // (lane offsets of 32 bits: into a tile's strips, into its rows, into the pairs of one k-group)
-    if (Kg * kG32Blk * kG32Strips >= ((int64_t)1 << 32) || rows >= ((int64_t)1 << 28))
-        return fail(LLMOPS_EINVAL, "fc_Q4A group 32: Kg must be below 2^32 / 5120 and rows below 2^28");
+    if (rows >= ((int64_t)1 << 28)) return fail(LLMOPS_EINVAL, "fc_Q4A group 32: rows must be below 2^28");  // (pairs of two k-groups)
     const int64_t tiles = ((Ng + kG32Strips - 1) / kG32Strips) * ((rows + kG32Rows - 1) / kG32Rows);
     const dim3 grid((unsigned)(8 * ((tiles + 7) / 8)), 1, (unsigned)S);  // one run of tiles per XCD
-    fc_gemm_g32_kernel<false><<<grid, 256, 0, st>>>(w, xq, xd, gs, xsT, out, nullptr, (int)Ng, (int)Kg, ldo, N, (int)rows, st_per_split,
-                                                    split_stride, residual);
+    if (g32_wide(Kg))
+        fc_gemm_g32_kernel<false, true><<<grid, 256, 0, st>>>(w, xq, xd, gs, xsT, out, nullptr, (int)Ng, (int)Kg, ldo, N, (int)rows,
+                                                              st_per_split, split_stride, residual);
+    else
+        fc_gemm_g32_kernel<false, false><<<grid, 256, 0, st>>>(w, xq, xd, gs, xsT, out, nullptr, (int)Ng, (int)Kg, ldo, N, (int)rows,
+                                                               st_per_split, split_stride, residual);
     LLMOPS_LAUNCH_CHECK();
     return LLMOPS_OK;
 }
 
 int launch_gemm_g32_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg, hipStream_t st) {
+    if (rows >= ((int64_t)1 << 28)) return fail(LLMOPS_EINVAL, "fc_Q4A group 32: rows must be below 2^28");
     const int64_t tiles = ((Ng + kG32Strips - 1) / kG32Strips) * ((rows + kG32Rows - 1) / kG32Rows);
-    fc_gemm_g32_kernel<true><<<(unsigned)(8 * ((tiles + 7) / 8)), 256, 0, st>>>(w, xq, nullptr, nullptr, nullptr, nullptr, acc, (int)Ng,
-                                                                                (int)Kg, 0, 0, (int)rows, (int)((Kg + kG32Gps - 1) / kG32Gps),
-                                                                                0, nullptr);
+    const unsigned grid = (unsigned)(8 * ((tiles + 7) / 8));
+    const int nst = (int)((Kg + kG32Gps - 1) / kG32Gps);
+    if (g32_wide(Kg))
+        fc_gemm_g32_kernel<true, true><<<grid, 256, 0, st>>>(w, xq, nullptr, nullptr, nullptr, nullptr, acc, (int)Ng, (int)Kg, 0, 0, (int)rows,
+                                                             nst, 0, nullptr);
+    else
+        fc_gemm_g32_kernel<true, false><<<grid, 256, 0, st>>>(w, xq, nullptr, nullptr, nullptr, nullptr, acc, (int)Ng, (int)Kg, 0, 0, (int)rows,
+                                                              nst, 0, nullptr);
     LLMOPS_LAUNCH_CHECK();
     return LLMOPS_OK;
 }

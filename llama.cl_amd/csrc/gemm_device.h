@@ -43,6 +43,13 @@ __device__ __forceinline__ void copy16_to_lds(const void* base, uint32_t off, ui
 __device__ __forceinline__ void copy4_to_lds(const void* base, uint32_t off, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(lds_base) : "memory", "m0");
 }
+// the same with byte offsets of 64 bits
+__device__ __forceinline__ void copy16_to_lds(const void* base, uint64_t off, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(reinterpret_cast<uint64_t>(base) + off), "s"(lds_base) : "memory", "m0");
+}
+__device__ __forceinline__ void copy4_to_lds(const void* base, uint64_t off, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(reinterpret_cast<uint64_t>(base) + off), "s"(lds_base) : "memory", "m0");
+}
 
 // 16 bytes from a 4-byte boundary
 struct __attribute__((packed, aligned(4))) Float4U {

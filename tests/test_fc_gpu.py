@@ -726,6 +726,32 @@ def test_fc_group32_is_as_precise_as_fp32_in_order(ops, orc, K, scale):
     assert rms(host(y)[0] - exact) <= rms(plain - exact), (rms(host(y)[0] - exact) / rms(exact), rms(plain - exact) / rms(exact))
 
 
+def test_fc_group32_tile_of_more_than_4_gib(ops):
+    """K so long that a tile's eight strips pass 4 GiB: offsets of 64 bits.  Activations are whole numbers with 127 in every
+    k-group (their own codes, scale 1) and the packed blocks random, so y = x W^T with the unpacked weights, in 64 bits.
+    1e-4: about the square root of 900001 fp32 roundings, each 6e-8 of a sum of the outputs' size."""
+    lib = ops._lib.load()
+    rows, Ng, Kg, G = 9, 8, 900001, 32
+    N, K = Ng * 32, Kg * G
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    wq = torch.randint(-128, 128, (Ng, Kg, 640), dtype=torch.int8, generator=gen, device="cuda")
+    wq[..., 512:576] = torch.full((32,), 0.01, dtype=torch.float16, device="cuda").view(torch.int8)
+    wq[..., 576:640] = torch.full((32,), -0.07, dtype=torch.float16, device="cuda").view(torch.int8)
+    x = torch.randint(-126, 127, (rows, K), dtype=torch.int8, generator=gen, device="cuda").float()
+    x.view(rows, Kg, G)[:, :, 0] = 127.0
+    ws = torch.zeros(lib.llmops_fc_Q4A_workspace_bytes(rows, K, Ng, Kg, G), dtype=torch.uint8, device="cuda")
+    y = torch.empty(rows, N, device="cuda")
+    ops._lib.check(lib.llmops_fc_Q4A(ops._ptr(x), rows, K, ops._ptr(wq), Ng, Kg, G, N, ops._ptr(y), ops._ptr(ws), ws.numel(),
+                                     ops._stream(y)))
+    want, step = torch.zeros(rows, N, dtype=torch.float64, device="cuda"), 30000
+    for k in range(0, Kg, step):
+        w = ops.offline_FC_dequant_Q4A(wq[:, k:k + step].contiguous())
+        want += x[:, k * G:(k + step) * G].double() @ w.double().t()
+    assert max_rel_err(host(y), host(want)) <= 1e-4
+    codes = x[:2].to(torch.int8)
+    assert torch.equal(ops.fc_Q4A_partials(codes, wq, use_mfma=True), ops.fc_Q4A_partials(codes, wq))
+
+
 def test_fc_group32_non_finite_rows_stay_theirs(ops, orc):
     """An infinity or a NaN in one row of activations leaves the other rows of its tile as they are."""
     rng = np.random.default_rng(5)
