@@ -150,16 +150,8 @@ __global__ __launch_bounds__(256) void attn_split_kernel(const float* __restrict
         vv[i] = load4(vbase + pc * S + e * 4);
     }
     const float4 qv = load4(q + ((b * qL + pq) * H + h) * S + e * 4);
+    const int my_slot = slots[lane < qL ? lane : 0];  // (fewer than 32 tokens: a lane per slot)
     const float d_scale = 1.0f / sqrtf((float)S);
-    // rows that a later token of this call has written
-    bool later[NL];
-#pragma unroll
-    for (int i = 0; i < NL; i++) later[i] = false;
-    for (int l = (int)pq + 1; l < (int)qL; l++) {
-        const int64_t rel = (int64_t)slots[l] - p0 - wave * PW - hf;
-#pragma unroll
-        for (int i = 0; i < NL; i++) later[i] = later[i] || rel == 2 * i;
-    }
 
 #pragma unroll
     for (int i = 0; i < NL; i++) {
@@ -171,11 +163,15 @@ __global__ __launch_bounds__(256) void attn_split_kernel(const float* __restrict
         for (int o = 16; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
         const int r = wave * PW + i * 2 + hf;
         const int64_t p = p0 + r;
-        if (e == 0) sc[r] = p < kvLen && !later[i] ? s * d_scale : -FLT_MAX;
+        if (e == 0) sc[r] = p < kvLen ? s * d_scale : -FLT_MAX;
     }
     __syncthreads();
     if (wave == 0) {
         float v = lane < C ? sc[lane] : -FLT_MAX;
+        // rows that a later token of this call has written (slots from registers: with a scalar load for each, in every
+        // wave, 31 tokens behind 97 of 8 heads took 15.6 us instead of 12.6)
+        for (int l = (int)pq + 1; l < (int)qL; l++)
+            if ((int64_t)__builtin_amdgcn_readlane(my_slot, l) == p0 + lane) v = -FLT_MAX;
         const float mx = wave_max(v);
         // a row counts only if it is live; a chunk with no live row reports sum 0
         float ex = (lane < C && v != -FLT_MAX) ? expf(v - mx) : 0.0f;
