@@ -66,6 +66,13 @@ void llmops_test_fc_set_row_routing(int rows_from_small, int rows_from_large);
  * 32; a chunk is 4 times that); 0 = choose */
 void llmops_test_attn_set_decode_plan(int rows_per_wave);
 
+/* attention of several query tokens, or of one that the decode kernel does not take (host arithmetic only, no launch):
+ * the kernel chosen -- 1: one workgroup per query and chunk of cache rows, 2: all tokens of a head in one workgroup
+ * per 128 cache rows, 3: 128 queries to a workgroup --, the cache rows a workgroup has, and how many workgroups share
+ * a query's rows.  For a workspace of llmops_attention_workspace_bytes. */
+int llmops_test_attn_plan(int64_t B, int64_t qL, int64_t H, int64_t maxlen, int position_id, int cache_dtype, int* kernel,
+                          int* rows, int* pieces);
+
 /* The decode kernel of llmops_fc_Q4A (rows <= 8, the one that quantizes the activations on the fly) in its
  * dump build: y as llmops_fc_Q4A computes it, plus what the kernel itself quantized -- xq int8 [rows,Kg*G],
  * xd and gsum fp32 [rows,Kg] (FC_dynamic_quantize_x, ops/op_fc.hpp:221-272; gsum is a tree sum here) -- and

@@ -1320,6 +1320,56 @@ static int pick_pw(int64_t bhq, int64_t kvLen) {
     return 4;
 }
 
+// Calls that the decode kernel does not take: which kernel, and how many cache rows a workgroup of it has.
+struct TokensPlan {
+    int kernel;  // 1 attn_split_kernel (a workgroup per query and chunk), 2 attn_few_kernel (all tokens of a head), 3 attn_prefill_kernel
+    int pw;      // split kernel: cache rows per wavefront
+    int rows;    // cache rows per workgroup
+    int pieces;  // workgroups that share a query's cache rows
+};
+static TokensPlan plan_tokens(int64_t bh, int64_t qL, int64_t kvLen, bool half_cache, int64_t max_records) {
+    const int64_t bhq = bh * qL;
+    TokensPlan p{};
+    if (qL >= g_prefill_min_tokens) {
+        // A workgroup takes a compute unit: with fewer query tiles than those, ns workgroups share a tile's cache rows, at
+        // least 128 each.  A row costs a tile 0.041 us; the records and the launch that merges them cost 3 us and 1.6 us per
+        // 1000 queries (us, one / split, 32 heads: 32 tokens behind 500 35.8 / 22.9, behind 3500 158 / 40; 64 behind 100
+        // 22.3 / 24.9, behind 250 27.9 / 25.6; 128 behind 1500 91 / 44; 256 behind none 32 / 42, behind 500 56 / 47; 512 behind
+        // 500 72.6 / 74.4, behind 1500 119 / 98).
+        p.kernel = 3;
+        int64_t ns = 256 / (bh * ((qL + 127) / 128));
+        if (ns > (kvLen + 127) / 128) ns = (kvLen + 127) / 128;
+        if (ns < 2 || bhq * ns > max_records || 0.041 * (double)(kvLen - kvLen / ns) < 3.0 + 1.6e-3 * (double)bhq) ns = 1;
+        p.rows = (int)(((kvLen + ns - 1) / ns + 63) / 64 * 64);
+        p.pieces = (int)((kvLen + p.rows - 1) / p.rows);
+        return p;
+    }
+    // One workgroup per query and chunk while there is little to read and multiply again for every token: a wave of
+    // attn_few_kernel runs some 2500 instructions however few of its 32 columns and 128 rows are in use.  Estimates in us, up
+    // to what both have in common; per query: rounds of the 1024 workgroups with chunks of 64 rows that the chip holds, rows
+    // multiplied, rows read, queries, chunks beyond the merge's 64 lanes; together: workgroups, up to one and up to two on
+    // a compute unit and more.  Measured with both kernels at 2620 sizes (1 to 31 tokens, 4 to 4096 heads in all, 1 to 8192
+    // cache rows of both types, in memory and not in a cache): the choice is 0.08 % slower than the better one on average,
+    // 13 % at worst.  (us, per query / together, fp32: 32 heads, 2 tokens behind 1000 17.4 / 18.3, behind 4000 35.9 / 36.8;
+    // 4 behind 500 15.0 / 17.2, behind 1000 21.0 / 18.6; 8 behind 120 11.7 / 16.0, behind 250 15.0 / 16.5; 31 behind 33
+    // 15.3 / 18.2, behind 97 19.9 / 18.9; 512 heads, 4 tokens, 32 rows 23.7 / 22.1; 4096 heads, 1 token, 48 rows 53 / 87,
+    // fp16 37 / 73; 4 heads, 1 token, 8192 rows 41 / 20.)
+    p.pw = pick_pw(bhq, kvLen);
+    const int64_t chunk = 4 * p.pw, chunks = (kvLen + chunk - 1) / chunk, few_chunks = (kvLen + 127) / 128, wgs = bh * few_chunks;
+    struct Cost {
+        double round, query_row, row, query, chunk, few, few_two, few_wg, few_wg_more;
+    };
+    const Cost c = half_cache ? Cost{0.273, 16.6e-6, 14.1e-6, 0.844e-3, 0.0568, 2.01, 1.9, 0.0, 7.56e-3}
+                              : Cost{0.5, 7.84e-6, 38.8e-6, 1.225e-3, 0.0347, 2.025, 2.0, 1.71e-3, 5.09e-3};
+    const double per_query = c.round * (double)(chunk == 64 ? (bhq * chunks + 1023) / 1024 : 0) + c.query_row * (double)(bhq * kvLen) +
+                             c.row * (double)(bh * kvLen) + c.query * (double)bhq + c.chunk * (double)(chunks > 64 ? chunks - 64 : 0);
+    const double together = c.few + (wgs > 256 ? c.few_two : 0.0) + c.few_wg * (double)wgs + c.few_wg_more * (double)(wgs > 512 ? wgs - 512 : 0);
+    p.kernel = per_query < together ? 1 : 2;
+    p.rows = p.kernel == 1 ? (int)chunk : 128;
+    p.pieces = (int)(p.kernel == 1 ? chunks : few_chunks);
+    return p;
+}
+
 // cache rows per chunk when the chunk records go to the consumer FC (at most kAttnRecChunks chunks per head): 0 = the
 // cache is too long for that
 static int records_chunk_rows(int64_t maxlen, bool half_cache) {
@@ -1444,17 +1494,10 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
         return LLMOPS_OK;
     }
     if (pos_dev != nullptr) return fail(LLMOPS_EINVAL, "a position in device memory needs one query token and half %% 4 == 0");
-    // the tiled kernel finds the token of a cache row in row_token; with fewer tokens a wave compares the slots itself
-    const bool tiled = qL >= g_prefill_min_tokens;
-    // One workgroup per query and chunk while there is little to read and multiply again for every token: a wave of
-    // attn_few_kernel runs some 2500 instructions whatever the size.  Measured (us, per query / all tokens together, 32
-    // heads): 2 tokens behind 1000 14.8 / 17.1, behind 2000 21.0 / 23.3, behind 3500 47 / 33; 4 behind 500 14.2 / 16.8, behind
-    // 1000 19.4 / 17.5; 8 behind 100 12.6 / 15.8, behind 250 22.1 / 16.4; 16 behind 30 14.5 / 16.1, behind 100 18.2 / 16.9;
-    // 31 behind none 16.9 / 17.9, behind 30 19.6 / 18.2.
-    const bool per_query = bhq * kvLen < (qL <= 2 ? 192 << 10 : 56 << 10);
-    const int pw = pick_pw(bhq, kvLen);
-    const int rows_chunk = per_query ? 4 * pw : 128;
-    const int nchunks = (int)((kvLen + rows_chunk - 1) / rows_chunk);
+    const TokensPlan plan = plan_tokens(B * H, qL, kvLen, kHalfCache, max_records);
+    const int nchunks = plan.pieces;
+    // the tiled kernel finds the token of a cache row in row_token; the others compare the slots themselves
+    const bool tiled = plan.kernel == 3;
     if (!tiled && (int64_t)bhq * nchunks > max_records)
         return fail(LLMOPS_EWORKSPACE, "attention workspace too small for %lld chunk records", (long long)bhq * nchunks);
     if (tiled) {
@@ -1476,31 +1519,20 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
             configured = true;
         }
-        // A workgroup takes a compute unit: with fewer query tiles than those, ns workgroups share a tile's cache rows, at
-        // least 128 each.  A row costs a tile 0.041 us; the records and the launch that merges them cost 3 us and 1.6 us per
-        // 1000 queries (us, one / split, 32 heads: 32 tokens behind 500 35.8 / 22.9, behind 3500 158 / 40; 64 behind 100
-        // 22.3 / 24.9, behind 250 27.9 / 25.6; 128 behind 1500 91 / 44; 256 behind none 32 / 42, behind 500 56 / 47; 512 behind
-        // 500 72.6 / 74.4, behind 1500 119 / 98).
-        const int64_t wgs = B * H * qtiles;
-        int64_t ns = 256 / wgs;
-        if (ns > (kvLen + 127) / 128) ns = (kvLen + 127) / 128;
-        if (ns < 2 || bhq * ns > max_records || 0.041 * (double)(kvLen - kvLen / ns) < 3.0 + 1.6e-3 * (double)bhq) ns = 1;
-        const int64_t span = ((kvLen + ns - 1) / ns + 63) / 64 * 64;
-        ns = (kvLen + span - 1) / span;
-        attn_prefill_kernel<T><<<dim3((unsigned)wgs, (unsigned)ns), 512, smem, st>>>(q, kc, vc, qL, H, maxlen, kvLen, row_token, qtiles, (int)span,
-                                                                                     part, (int)ns);
+        attn_prefill_kernel<T><<<dim3((unsigned)(B * H * qtiles), (unsigned)nchunks), 512, smem, st>>>(q, kc, vc, qL, H, maxlen, kvLen, row_token,
+                                                                                                       qtiles, plan.rows, part, nchunks);
         LLMOPS_LAUNCH_CHECK();
-        if (ns > 1) {
-            attn_merge_kernel<<<(unsigned)bhq, 128, 0, st>>>(q, part, qL, H, (int)ns);
+        if (nchunks > 1) {
+            attn_merge_kernel<<<(unsigned)bhq, 128, 0, st>>>(q, part, qL, H, nchunks);
             LLMOPS_LAUNCH_CHECK();
         }
         return LLMOPS_OK;
     }
-    if (!per_query)
+    if (plan.kernel == 2)
         attn_few_kernel<T><<<(unsigned)(B * H * nchunks), 256, 0, st>>>(q, kc, vc, (int)qL, H, maxlen, (int)kvLen, slots, part, nchunks);
-    else if (pw == 16)
+    else if (plan.pw == 16)
         attn_split_kernel<T, 16><<<(unsigned)(bhq * nchunks), 256, 0, st>>>(q, kc, vc, qL, H, maxlen, kvLen, slots, part, nchunks);
-    else if (pw == 8)
+    else if (plan.pw == 8)
         attn_split_kernel<T, 8><<<(unsigned)(bhq * nchunks), 256, 0, st>>>(q, kc, vc, qL, H, maxlen, kvLen, slots, part, nchunks);
     else
         attn_split_kernel<T, 4><<<(unsigned)(bhq * nchunks), 256, 0, st>>>(q, kc, vc, qL, H, maxlen, kvLen, slots, part, nchunks);
@@ -1571,6 +1603,18 @@ extern "C" int llmops_attention_rope_decode_records(float* q, float* k, const fl
     LLMOPS_REQUIRE(rec_stats != nullptr && rec_outs != nullptr && aligned(rec_stats, 16) && aligned(rec_outs, 16));
     return attention_entry(q, k, v, B, 1, H, S, inv_freq, half, kv_cache, cache_dtype, planes, maxlen, slot, position_id,
                            position_id_dev, layer_id, workspace, workspace_bytes, stream, rec_stats, rec_outs);
+}
+
+extern "C" int llmops_test_attn_plan(int64_t B, int64_t qL, int64_t H, int64_t maxlen, int position_id, int cache_dtype, int* kernel,
+                                     int* rows, int* pieces) {
+    LLMOPS_TEST_HOOK();
+    LLMOPS_REQUIRE(B > 0 && qL > 0 && H > 0 && maxlen > 0 && position_id >= 0 && kernel != nullptr && rows != nullptr && pieces != nullptr);
+    const size_t head = LLMOPS_ATTN_COUNTER_BYTES + align_up((size_t)maxlen * 4, 256);
+    const int64_t max_records = (int64_t)((llmops_attention_workspace_bytes(B, qL, H, 128, maxlen) - head) / (130 * sizeof(float)));
+    const int64_t kv = position_id + qL < maxlen ? position_id + qL : maxlen;
+    const TokensPlan p = plan_tokens(B * H, qL, kv, cache_dtype == LLMOPS_CACHE_F16, max_records);
+    *kernel = p.kernel, *rows = p.rows, *pieces = p.pieces;
+    return LLMOPS_OK;
 }
 
 extern "C" void llmops_test_attn_set_decode_plan(int rows_per_wave) {

@@ -167,3 +167,20 @@ def test_tensor_attributes_the_reference_callers_use():
     t = torch.zeros(3, 5, dtype=torch.int8)
     assert t.item_size == 1 and torch.zeros(2, dtype=torch.float32).item_size == 4
     assert t.numel() * t.item_size == 15 and tuple(t.shape) == (3, 5) and t.clone().numpy().shape == (3, 5)
+
+
+@pytest.mark.parametrize("half", [0, 1])
+def test_attention_planner_measured_sizes(half):
+    """Calls below 32 query tokens, and one token where the decode kernel is not taken: sizes at which one of the two
+    kernels measured at least 15 % faster than the other (heads in all, tokens, cache rows; 1: a workgroup per query and
+    chunk, 2: all tokens of a head together)."""
+    from llmops import _lib
+    lib = _lib.load()
+    want = {1: [(4096, 1, 48), (4096, 1, 16), (512, 1, 16), (1024, 2, 16), (32, 8, 128), (32, 16, 32), (8, 2, 100), (4, 31, 48), (70000, 1, 16),
+                (70000, 1, 64)],
+            2: [(4, 1, 8192), (32, 16, 1516), (32, 31, 512), (256, 8, 500), (512, 8, 64), (1024, 6, 64), (4096, 8, 16), (4, 3, 8192)]}
+    k, r, n = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    for kernel, sizes in want.items():
+        for heads, tokens, kv in sizes:
+            assert lib.llmops_test_attn_plan(1, tokens, heads, kv, kv - tokens, half, ctypes.byref(k), ctypes.byref(r), ctypes.byref(n)) == 0
+            assert k.value == kernel and n.value == -(-kv // r.value), (heads, tokens, kv)

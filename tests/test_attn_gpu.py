@@ -1,5 +1,7 @@
 """GPU parity of rope / KV-cache update / attention and of the small neighbour ops.
 fp32 outputs: max|err|/max|ref| <= 1e-3 against the reference-made golden vectors and the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -207,17 +209,16 @@ def _attend_cache(orc, q, inv_freq, cache, slots, past, maxlen):
     return o.transpose(0, 2, 1, 3).reshape(B, qL, HS)
 
 
-@pytest.mark.parametrize("B,qL,kv,H", [(1, 2, 6200, 32), (1, 3, 700, 32), (1, 31, 127, 32), (2, 17, 128, 32), (1, 16, 129, 32),
-                                       (1, 31, 60, 32), (1, 5, 385, 32), (1, 33, 700, 8), (2, 64, 449, 4), (1, 130, 1025, 4)])
-@pytest.mark.parametrize("cache_dtype", [torch.float32, torch.float16])
-@pytest.mark.parametrize("order", ["in order", "shuffled", "one out of range"])
-def test_attention_tokens_behind_a_cache(ops, B, qL, kv, H, cache_dtype, order):
-    """Several query tokens behind a filled cache, on either side of every rule: one workgroup per query, all tokens of a
-    head in one workgroup (cache rows just below, at and above a workgroup's 128 and a wave's 32, longest and shortest
-    runs), and the tiled kernel with the cache rows in several pieces.  The new rows at the end of the cache in order, or
-    anywhere in any order (what a later token wrote is masked wherever it lies; a piece of the cache may hold nothing that
-    an early token may see), or with one slot outside the cache (dropped).  fp32: 1e-5 as in the other tests; an fp16
-    cache against fp32 math on its own rounded rows."""
+def _plan(ops, B, qL, H, maxlen, position_id, cache_dtype):
+    """(kernel, cache rows of a workgroup) as the planner chooses: 1 a workgroup per query and chunk, 2 all tokens of a head,
+    3 tiles of 128 queries"""
+    k, r, n = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    assert ops._lib.load().llmops_test_attn_plan(B, qL, H, maxlen, position_id, int(cache_dtype == torch.float16), ctypes.byref(k), ctypes.byref(r),
+                                                 ctypes.byref(n)) == 0
+    return k.value, r.value
+
+
+def _tokens_behind_a_cache(ops, B, qL, kv, H, cache_dtype, order):
     S = 128
     rng = np.random.default_rng(qL * 1000 + kv)
     q, k, v = (rng.standard_normal((B, qL, H * S)).astype(np.float32) for _ in range(3))
@@ -249,15 +250,45 @@ def test_attention_tokens_behind_a_cache(ops, B, qL, kv, H, cache_dtype, order):
     assert max_rel_err(host(tq), want.cpu().numpy()) <= 1e-5
 
 
-@pytest.mark.parametrize("B,qL,kv", [(1, 4, 100), (1, 2, 2500), (1, 4, 2000), (2, 16, 700), (1, 31, 130)])
+@pytest.mark.parametrize("B,qL,kv,H,kernel", [
+    (1, 2, 6200, 32, 2), (1, 3, 700, 32, 2), (1, 31, 127, 32, 2), (2, 17, 128, 32, 2), (1, 16, 129, 32, 2), (1, 31, 60, 32, 1),
+    (4, 31, 60, 32, 2), (1, 5, 385, 32, 1), (1, 9, 385, 32, 2), (1, 33, 700, 8, 3), (2, 64, 449, 4, 3), (1, 130, 1025, 4, 3)])
+@pytest.mark.parametrize("cache_dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("order", ["in order", "shuffled", "one out of range"])
+def test_attention_tokens_behind_a_cache(ops, B, qL, kv, H, kernel, cache_dtype, order):
+    """Several query tokens behind a filled cache, on either side of every rule: one workgroup per query, all tokens of a
+    head in one workgroup (cache rows just below, at and above a workgroup's 128 and a wave's 32, longest and shortest runs),
+    and from 32 tokens the tiled kernel with the cache rows in several pieces.  The new rows at the end of the cache in order, or anywhere in any order (what a later token wrote is
+    masked wherever it lies; a piece of the cache may hold nothing that an early token may see), or with one slot outside
+    the cache (dropped).  fp32: 1e-5 as in the other tests; an fp16 cache against fp32 math on its own rounded rows."""
+    assert _plan(ops, B, qL, H, kv, kv - qL, cache_dtype)[0] == kernel
+    _tokens_behind_a_cache(ops, B, qL, kv, H, cache_dtype, order)
+
+
+@pytest.mark.parametrize("B,qL,kv,H,plan", [
+    (1, 3, 100, 4, (1, 16)), (1, 31, 40, 8, (1, 16)),                             # chunks of 16 rows
+    (1, 8, 131, 32, (1, 32)), (4, 3, 100, 32, (1, 32)), (4, 3, 140, 32, (2, 128)),  # of 32, and just beyond the rule
+    (32, 2, 48, 32, (1, 64)), (16, 2, 65, 32, (1, 64)), (16, 3, 65, 32, (2, 128)),  # of 64
+    (1, 2, 2000, 32, (1, 64)), (1, 8, 200, 32, (1, 64)), (1, 8, 300, 32, (2, 128))])
+@pytest.mark.parametrize("cache_dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("order", ["in order", "shuffled", "one out of range"])
+def test_attention_tokens_one_workgroup_per_query(ops, B, qL, kv, H, plan, cache_dtype, order):
+    """The same with a workgroup per query and chunk, in each of its chunk sizes, whose rows are compared with the slots of
+    the later tokens, and sizes just beyond the rule."""
+    assert _plan(ops, B, qL, H, kv, kv - qL, cache_dtype) == plan
+    _tokens_behind_a_cache(ops, B, qL, kv, H, cache_dtype, order)
+
+
+@pytest.mark.parametrize("B,qL,kv,kernel", [(1, 4, 100, 1), (1, 2, 1000, 1), (4, 4, 2000, 2), (2, 16, 700, 2), (1, 31, 130, 1)])
 @pytest.mark.parametrize("cache_dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("case", ["k -inf", "k +inf", "k huge", "v +inf", "v huge", "q inf", "new k inf", "tiny k", "tiny v"])
-def test_attention_few_tokens_extreme_values(ops, B, qL, kv, cache_dtype, case):
+def test_attention_few_tokens_extreme_values(ops, B, qL, kv, kernel, cache_dtype, case):
     """2..31 tokens with one cache row (or one token's q, or the last token's k) that holds infinities or the largest finite
     values, and with a whole cache of tiny ones: what 64-bit attention gives, NaN for NaN, infinity for
     infinity.  A score of -inf is a row that drops out; a row that a token may not see does not reach it, whatever is in its
     k; other heads and batch entries are untouched.  Finite outputs to 1e-5 of the sum of |weight * value|."""
     H, S, half, tol = 8, 128, cache_dtype == torch.float16, 1e-5
+    assert _plan(ops, B, qL, H, kv, kv - qL, cache_dtype)[0] == kernel
     rng = np.random.default_rng(qL + kv)
     q, k, v = (rng.standard_normal((B, qL, H * S)).astype(np.float32) for _ in range(3))
     cache = torch.from_numpy(rng.standard_normal((2, B, H, kv, S)).astype(np.float32))
