@@ -35,15 +35,19 @@ __device__ __forceinline__ void column_min_max(float& vmin, float& vmax) {
     }
 }
 
+typedef float float4_4 __attribute__((ext_vector_type(4), aligned(4)));  // 16 bytes from any 4
+
 // Bound by reading the fp32 matrix.  A workgroup takes 128 k-values of 32 columns (one block of group 128, four of group
 // 32); a thread loads 8 values of each of two columns, 16 bytes a load, before it uses any (128 KB in flight per compute
 // unit), and the packed dwords go through LDS so that a wave writes 256 consecutive bytes instead of 16 bytes in each of
 // 16 rows.  11008 x 4096, before (4-byte loads, one block of 512 threads per column set) / now: group 128 99 / 36.4 us
-// (5.6 TB/s), group 32 117 / 36.5 us; 1000 x 4096 11.6 / 5.7 us; 512 x 512, too little to fill the chip, 4.0 / 4.6 us.
-// `vec`: rows start on 16 bytes (scalar loads otherwise, and for a thread that K cuts).
+// (5.6 TB/s), group 32 117 / 36.5 us; in a graph 1000 x 4096 12.0 / 5.8 us, 512 x 512, too little to fill the chip, 4.3 / 3.2
+// and 3.4 / 3.0 us.  Rows may start on any 4 bytes: the loads do not ask for more (2048 x 4098 21.7 / 9.4 us; four bytes a
+// load 20.4).  A thread that K cuts loads the last value again instead of branching around each (513 x 513 4.4 / 3.4 and, group
+// 32, 3.5 / 3.1 us; with the branches 4.7 and 4.4).
 template <int G>
 __global__ __launch_bounds__(256) void quant_w_kernel(const float* __restrict__ wei, int64_t N, int64_t K, int64_t ld,
-                                                      uint8_t* __restrict__ out, int64_t Kg, bool vec) {
+                                                      uint8_t* __restrict__ out, int64_t Kg) {
     constexpr int R = G / 8;         // packed rows (and lanes of a column) per block
     constexpr int kSub = 128 / G;    // blocks per workgroup
     constexpr int kPitch = 33;       // dwords; lanes of a column write consecutive rows: an odd pitch spreads the banks
@@ -56,23 +60,23 @@ __global__ __launch_bounds__(256) void quant_w_kernel(const float* __restrict__ 
     const int cnt = (int)(K - k0 >= 8 ? 8 : K > k0 ? K - k0 : 0);
 
     float v[2][8];
-    if (vec && cnt == 8) {
+    if (cnt == 8) {
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             const int64_t n = (int64_t)nb * kGroupN + c0 + 16 * c;
-            const float4* src = reinterpret_cast<const float4*>(wei + (n < N ? n : N - 1) * ld + k0);
-            const float4 lo = src[0], hi = src[1];
-            v[c][0] = lo.x, v[c][1] = lo.y, v[c][2] = lo.z, v[c][3] = lo.w;
-            v[c][4] = hi.x, v[c][5] = hi.y, v[c][6] = hi.z, v[c][7] = hi.w;
+            const float4_4* src = reinterpret_cast<const float4_4*>(wei + (n < N ? n : N - 1) * ld + k0);
+            const float4_4 lo = src[0], hi = src[1];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[c][j] = lo[j], v[c][4 + j] = hi[j];
         }
     } else {
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             const int64_t n = (int64_t)nb * kGroupN + c0 + 16 * c;
-            const float* src = wei + (n < N ? n : N - 1) * ld + k0;
-            // (values past K repeat the first one: no effect on strict comparisons; their codes are cleared below)
+            const float* src = wei + (n < N ? n : N - 1) * ld;
+            // (values past K repeat the last one: no effect on strict comparisons; their codes are cleared below)
 #pragma unroll
-            for (int j = 0; j < 8; j++) v[c][j] = j < cnt ? src[j] : j > 0 ? v[c][0] : 0.0f;
+            for (int j = 0; j < 8; j++) v[c][j] = src[k0 + j < K ? k0 + j : K - 1];
         }
     }
 #pragma unroll
@@ -124,7 +128,8 @@ __global__ __launch_bounds__(256) void quant_w_kernel(const float* __restrict__ 
 // bits and q 4, so the product is exact and contraction cannot change the result.
 // Bound by writing the fp32 matrix.  A workgroup takes 128 k-values of 32 columns, as above: the blocks come through LDS
 // with consecutive reads, and 32 lanes write 512 consecutive bytes of a row, 16 bytes a lane.
-// 11008 x 4096, before / now: group 128 46.1 / 40.7 us (5.0 TB/s), group 32 42.7 / 41.1 us; 1000 x 4096 6.3 / 5.1, 5.7 / 5.1 us.
+// 11008 x 4096, before / now: group 128 46.1 / 40.7 us (5.0 TB/s), group 32 42.7 / 41.1 us; 1000 x 4096 6.3 / 5.1, 5.7 / 5.1 us;
+// 512 x 512, all latency, 2.5 / 2.6 us.
 template <int G>
 __global__ __launch_bounds__(256) void dequant_w_kernel(const uint8_t* __restrict__ weiq, int64_t Kg, float* __restrict__ out) {
     constexpr int R = G / 8, kSub = 128 / G, kPitch = 33;  // (33: the rows of a column fall into different banks)
@@ -167,11 +172,10 @@ extern "C" int llmops_offline_FC_quant_Q4A(const float* wei, int64_t N, int64_t 
     const int64_t Ng = (N + kGroupN - 1) / kGroupN, Kg = (K + group_k - 1) / group_k;
     LLMOPS_REQUIRE(Ng <= 65535 && Kg <= 0x7fffffff);
     uint8_t* out = reinterpret_cast<uint8_t*>(weiq);
-    const bool vec = aligned(wei, 16) && (ld % 4) == 0;
     if (group_k == 32)
-        quant_w_kernel<32><<<dim3((unsigned)((Kg + 3) / 4), (unsigned)Ng), 256, 0, as_stream(stream)>>>(wei, N, K, ld, out, Kg, vec);
+        quant_w_kernel<32><<<dim3((unsigned)((Kg + 3) / 4), (unsigned)Ng), 256, 0, as_stream(stream)>>>(wei, N, K, ld, out, Kg);
     else
-        quant_w_kernel<128><<<dim3((unsigned)Kg, (unsigned)Ng), 256, 0, as_stream(stream)>>>(wei, N, K, ld, out, Kg, vec);
+        quant_w_kernel<128><<<dim3((unsigned)Kg, (unsigned)Ng), 256, 0, as_stream(stream)>>>(wei, N, K, ld, out, Kg);
     LLMOPS_LAUNCH_CHECK();
     return LLMOPS_OK;
 }
