@@ -1332,14 +1332,17 @@ static TokensPlan plan_tokens(int64_t bh, int64_t qL, int64_t kvLen, bool half_c
     TokensPlan p{};
     if (qL >= g_prefill_min_tokens) {
         // A workgroup takes a compute unit: with fewer query tiles than those, ns workgroups share a tile's cache rows, at
-        // least 128 each.  A row costs a tile 0.041 us; the records and the launch that merges them cost 3 us and 1.6 us per
-        // 1000 queries (us, one / split, 32 heads: 32 tokens behind 500 35.8 / 22.9, behind 3500 158 / 40; 64 behind 100
-        // 22.3 / 24.9, behind 250 27.9 / 25.6; 128 behind 1500 91 / 44; 256 behind none 32 / 42, behind 500 56 / 47; 512 behind
-        // 500 72.6 / 74.4, behind 1500 119 / 98).
+        // least 128 each.  A row costs a tile 0.041 us (halves 0.0365: two products instead of three); the launch that merges
+        // the records costs 3.5 us, 0.55 us per 1000 queries and 0.25 us per 1000 records (0.3 beside halves).  Against one
+        // piece and all pieces at 2016 sizes (1 to 128 heads in all, 32 to 2048 tokens behind 0 to 6000, both cache types, not
+        // from a cache): 0.06 % slower than the better one on average, 8 % at worst.  (us, one / split, 32 heads: 32 tokens
+        // behind 500 35.1 / 23.4; 64 behind 100 22.6 / 25.4, behind 300 30.1 / 26.8; 256 behind none 32.2 / 41.1, behind 300
+        // 46.3 / 43.1, halves 40.6 / 43.6; 200 behind 300, halves 35.8 / 38.9; 512 behind 500 71.4 / 70.9, behind 1500 116 / 94.)
         p.kernel = 3;
+        const double row = half_cache ? 0.0365 : 0.041, record = half_cache ? 0.3e-3 : 0.25e-3;
         int64_t ns = 256 / (bh * ((qL + 127) / 128));
         if (ns > (kvLen + 127) / 128) ns = (kvLen + 127) / 128;
-        if (ns < 2 || bhq * ns > max_records || 0.041 * (double)(kvLen - kvLen / ns) < 3.0 + 1.6e-3 * (double)bhq) ns = 1;
+        if (ns < 2 || bhq * ns > max_records || row * (double)(kvLen - kvLen / ns) < 3.5 + 0.55e-3 * (double)bhq + record * (double)(bhq * ns)) ns = 1;
         p.rows = (int)(((kvLen + ns - 1) / ns + 63) / 64 * 64);
         p.pieces = (int)((kvLen + p.rows - 1) / p.rows);
         return p;
