@@ -188,15 +188,15 @@ def test_attention_planner_measured_sizes(half):
 
 @pytest.mark.parametrize("heads,tokens,past,pieces32,pieces16", [
     (32, 32, 500, True, True), (32, 64, 100, False, False), (32, 256, 0, False, False), (32, 256, 300, True, False),
-    (32, 200, 300, False, False), (16, 384, 64, False, False), (16, 1024, 400, True, True), (32, 512, 1500, True, True),
+    (32, 200, 300, True, False), (16, 384, 64, None, False), (16, 1024, 400, True, True), (32, 512, 1500, True, True),
     (32, 2048, 0, False, False), (128, 512, 3500, False, False)])
 def test_attention_planner_pieces_of_the_tiled_kernel(heads, tokens, past, pieces32, pieces16):
     """From 32 query tokens: the cache rows of a tile in several workgroups or in one, at sizes where one of the two measured
-    faster (or where the tiles fill the chip)."""
+    faster (or where the tiles fill the chip); None: the same within 3 %."""
     from llmops import _lib
     lib = _lib.load()
     k, r, n = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     for half, several in ((0, pieces32), (1, pieces16)):
         kv = past + tokens
         assert lib.llmops_test_attn_plan(1, tokens, heads, kv, past, half, ctypes.byref(k), ctypes.byref(r), ctypes.byref(n)) == 0
-        assert k.value == 3 and (n.value > 1) == several and r.value % 64 == 0 and (n.value - 1) * r.value < kv <= n.value * r.value
+        assert k.value == 3 and several in (None, n.value > 1) and r.value % 64 == 0 and (n.value - 1) * r.value < kv <= n.value * r.value
