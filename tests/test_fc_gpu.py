@@ -404,29 +404,35 @@ def test_fc_decode_many_rows_producer_inside_the_quantization(ops, orc, G, rows,
 @pytest.mark.parametrize("G", [32, 128])
 def test_fc_decode_parts_stay_inside_the_workspace(ops, G):
     """Three parts of 4096 columns and 512 rows: a part is split over K where the whole is not, and its partial sums
-    took more room than the whole's workspace has.  A workspace of exactly the size the whole needs, in front of a guard:
-    the call either says that it needs more or leaves the guard alone; through the module (a workspace of its own on a
-    fresh stream) the first result equals the next ones."""
+    took more room than the whole's workspace has.  A workspace of the size the whole needs is refused if a part needs more;
+    one of exactly the larger size, in front of a guard, is enough and the guard is left alone; through the module (a
+    workspace of its own on a fresh stream) the first result equals the next ones."""
     lib = ops._lib.load()
     rows, N, K, parts = 512, 12288, 4096, 3
     Ng, Kg = N // 32, K // G
     wq = ops.offline_FC_quant_Q4A(torch.randn(N, K, generator=torch.Generator(device="cuda").manual_seed(1), device="cuda") * 0.02, G)
     x = torch.randn(1, rows, K, generator=torch.Generator(device="cuda").manual_seed(2), device="cuda")
-    need = lib.llmops_fc_Q4A_workspace_bytes(rows, K, Ng, Kg, G)
-    ws = torch.zeros(need + (192 << 20), dtype=torch.uint8, device="cuda")
+    whole_need, part_need = (lib.llmops_fc_Q4A_workspace_bytes(rows, K, n, Kg, G) for n in (Ng, Ng // parts))
+    need = max(whole_need, part_need)
+    assert part_need > whole_need                                         # (what the shape was chosen for)
+    ws = torch.zeros(need + (64 << 20), dtype=torch.uint8, device="cuda")
     ws[need:] = 0x5A
     y = torch.empty(parts, rows, N // parts, device="cuda")
-    rc = lib.llmops_fc_Q4A_decode_parts(ops._ptr(x), rows, K, ops._ptr(wq), Ng, Kg, G, N, None, 0.0, 0, parts, ops._ptr(y), ops._ptr(ws),
-                                        need, ops._stream(x))
-    torch.cuda.synchronize()
-    assert rc in (0, 2)                                                   # LLMOPS_OK or LLMOPS_EWORKSPACE
-    touched = int((ws[need:] != 0x5A).sum())
-    assert touched == 0
+
+    def call(nbytes):
+        rc = lib.llmops_fc_Q4A_decode_parts(ops._ptr(x), rows, K, ops._ptr(wq), Ng, Kg, G, N, None, 0.0, 0, parts, ops._ptr(y),
+                                            ops._ptr(ws), nbytes, ops._stream(x))
+        torch.cuda.synchronize()
+        return rc
+    assert call(need - 1) == 2 and call(whole_need) == 2                  # LLMOPS_EWORKSPACE
+    assert call(need) == 0
+    assert int((ws[need:] != 0x5A).sum()) == 0
     with torch.cuda.stream(torch.cuda.Stream()):
         first = ops.fc_Q4A_decode(x, wq, N, out_parts=parts)
         for _ in range(2):
             assert torch.equal(ops.fc_Q4A_decode(x, wq, N, out_parts=parts), first)
     whole = ops.fc_Q4A(x, wq, N)
+    assert torch.equal(y, first.reshape(y.shape))
     for p in range(parts):
         assert max_rel_err(host(first[p]), host(whole[..., p * (N // parts):(p + 1) * (N // parts)])) <= 1e-5
 
