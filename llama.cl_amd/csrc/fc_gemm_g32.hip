@@ -4,7 +4,8 @@
 // What bounds it: with a group of 32 every v_mfma_i32_32x32x32_i8 (32 cycles) is a whole k-group of its tile, and its 16
 // results per lane are folded into the fp32 accumulators with 32 vector instructions: the vector ALU (about 60 ns per
 // step and SIMD in a loop of nothing else, against 14 ns of matrix core) is the limit, so everything else is kept off it
-// and out of its way:
+// and out of its way (counters at 512 x 11008 x 4096: the vector ALU issues 66 % of the time, 64 of a wave's 108 vector
+// instructions per k-group are the fold; the matrix cores are busy 15 %; waves wait 24 %):
 //   * tile 32 rows x 256 columns, four waves side by side (each 32 x 64 = two strips): a strip's weights are unpacked by
 //     one wave only, and the rows' codes and scales are read from LDS by all four.  (Sixty-four rows x 128 columns, two
 //     waves either way: 0 to 3 % slower at almost every size, 512 x 11008 x 4096 by 2 %; 128 x 128 with 64 x 64 per wave by
