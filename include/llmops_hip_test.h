@@ -33,8 +33,7 @@ int llmops_test_calib_copy(const void* src, void* dst, int64_t bytes, int workgr
 void llmops_test_fc_set_tuning(int target_workgroups, int waves_per_workgroup);
 
 /* prefill GEMM planner knob: force the row-tile factor of the LDS-tiled MFMA kernel (1, 2 or 4:
- * 32, 64 or 128 rows per workgroup; 8: the 256-row kernel whose two wave groups alternate between
- * MFMA and fold phases, which the planner takes from 512 rows on); 0 = choose per shape; -1 = choose
+ * 32, 64 or 128 rows per workgroup; 8: as 4); 0 = choose per shape; -1 = choose
  * per shape and send 9..16 rows to the tiled kernel too instead of the weight-streaming MFMA kernel */
 void llmops_test_gemm_set_tuning(int row_tile_factor);
 
@@ -49,8 +48,8 @@ void llmops_test_gemm_set_reduce(int in_kernel);
 void llmops_test_gemm_set_split(int splits);
 
 /* prefill GEMM: what the planner chooses for a product of `rows` rows with a packed tensor of Ng strips x Kg
- * k-groups (host arithmetic only, no launch): the row-tile factor (1, 2, 4: 32, 64, 128 rows per workgroup of
- * the four-wave kernel; 8: the 256-row kernel) and the split-K factor.  Reads the knobs above. */
+ * k-groups (host arithmetic only, no launch): the row-tile factor (1, 2, 4: 32, 64, 128 rows per workgroup; 8: 128
+ * rows, unsplit, two workgroups to a compute unit) and the split-K factor.  Reads the knobs above. */
 int llmops_test_gemm_plan(int64_t rows, int64_t Ng, int64_t Kg, int group_k, int* row_tile_factor, int* splits);
 
 /* weight-streaming MFMA kernel (3..16 rows, 17..32 for tensors of fewer than 256 strips): two workgroups per strip with half of K each for tensors of

@@ -23,12 +23,12 @@ int launch_gemv_fused(const uint8_t* w, const float* x, float* y, float* part, u
 int launch_add(float* a, const float* b, int64_t total, hipStream_t st);
 int launch_gemv_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg, int G,
                          hipStream_t st);
-size_t gemm_workspace_bytes(int64_t rows, int64_t Ng, int64_t Kg, int G);
+size_t gemm_workspace_bytes(int64_t rows, int64_t Ng, int64_t Kg, int G, int64_t room);
 int launch_gemm(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, const float2* xsT, float* y,
                 float* part, unsigned* counters, int64_t rows, int64_t Ng, int64_t Kg, int G, int64_t N, const float* residual,
-                hipStream_t st);
+                int64_t room, hipStream_t st);
 int launch_gemm_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg, int G,
-                         bool two_groups, hipStream_t st);
+                         bool rows128, hipStream_t st);
 int launch_fc_rows(const uint8_t* w, const int8_t* xq, const float2* xsT, float* y, int64_t rows, int64_t Ng, int64_t Kg,
                    int64_t N, const float* residual, unsigned long long* slots, size_t slot_bytes, hipStream_t st);
 int launch_fc_rows_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg,
@@ -39,9 +39,11 @@ static inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; 
 
 struct FcWorkspace {
     size_t off_xq, off_xd, off_gs, off_xst, off_part, total;
+    int64_t room;  // what partial sums may take
 };
 
-static FcWorkspace fc_layout(int64_t rows, int64_t Ng, int64_t Kg, int G) {
+// limit: bytes that the workspace has, where that is fixed (the tiled product then splits K no further than they allow)
+static FcWorkspace fc_layout(int64_t rows, int64_t Ng, int64_t Kg, int G, size_t limit = 0) {
     FcWorkspace w;
     size_t o = LLMOPS_FC_COUNTER_BYTES;
     w.off_xq = o;
@@ -54,7 +56,8 @@ static FcWorkspace fc_layout(int64_t rows, int64_t Ng, int64_t Kg, int G) {
     // (+256: the weight-streaming MFMA kernel fetches the pairs of whole 16-row tiles, up to 31 pairs past the last row)
     o = align_up(o + (size_t)rows * Kg * 2 * sizeof(float) + 256, 256);
     w.off_part = o;
-    o = align_up(o + (rows <= kMaxGemvRows ? gemv_workspace_bytes(rows, Ng, Kg, G) : gemm_workspace_bytes(rows, Ng, Kg, G)), 256);
+    w.room = limit == 0 ? INT64_MAX : (int64_t)limit - (int64_t)o - 256;
+    o = align_up(o + (rows <= kMaxGemvRows ? gemv_workspace_bytes(rows, Ng, Kg, G) : gemm_workspace_bytes(rows, Ng, Kg, G, w.room)), 256);
     w.total = o;
     return w;
 }
@@ -105,17 +108,17 @@ static int fc_product_many_rows(const uint8_t* w, uint8_t* ws, const FcWorkspace
         return launch_fc_rows(w, xq, xst, y, rows, Ng, Kg, N, residual, reinterpret_cast<unsigned long long*>(ws + kTicketBytes),
                               LLMOPS_FC_COUNTER_BYTES - kTicketBytes, st);
     return launch_gemm(w, xq, xd, gs, xst, y, reinterpret_cast<float*>(ws + lay.off_part), reinterpret_cast<unsigned*>(ws), rows, Ng,
-                       Kg, group_k, N, residual, st);
+                       Kg, group_k, N, residual, lay.room, st);
 }
 
 static int fc_impl(const float* x, int64_t rows, int64_t K, const int8_t* weiq, int64_t Ng, int64_t Kg, int group_k,
                    int64_t N, const float* residual, float* y, void* workspace, size_t workspace_bytes,
-                   llmops_stream_t stream) {
+                   llmops_stream_t stream, size_t limit = 0) {
     const int bad = fc_check_args(x, rows, K, weiq, Ng, Kg, group_k, N, y);
     if (bad) return bad;
     LLMOPS_REQUIRE(workspace != nullptr && aligned(workspace, 256));
     const bool k_tail = K != Kg * group_k;
-    const FcWorkspace lay = fc_layout(rows, Ng, Kg, group_k);
+    const FcWorkspace lay = fc_layout(rows, Ng, Kg, group_k, limit);
     if (workspace_bytes < lay.total)
         return fail(LLMOPS_EWORKSPACE, "fc_Q4A needs %zu workspace bytes, got %zu", lay.total, workspace_bytes);
     uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
@@ -141,7 +144,7 @@ static int fc_impl(const float* x, int64_t rows, int64_t K, const int8_t* weiq, 
         float2* xst_t = reinterpret_cast<float2*>(ws + lay.off_xst);
         int rc_t = launch_quant_x(x, rows, K, group_k, xq, xd, gs, xst_t, false, st);
         if (rc_t) return rc_t;
-        if (rows > kMaxGemvRows) return launch_gemm(w, xq, xd, gs, xst_t, y, part, counters, rows, Ng, Kg, group_k, N, residual, st);
+        if (rows > kMaxGemvRows) return launch_gemm(w, xq, xd, gs, xst_t, y, part, counters, rows, Ng, Kg, group_k, N, residual, lay.room, st);
         if (residual == y) return fail(LLMOPS_EINVAL, "fc_Q4A with a short last k-group and up to 8 rows: residual must not be y");
         rc_t = launch_gemv(w, xq, xd, gs, y, part, counters, rows, Ng, Kg, group_k, N, st);
         if (rc_t == 0 && residual != nullptr) rc_t = launch_add(y, residual, rows * N, st);
@@ -313,7 +316,7 @@ extern "C" int llmops_fc_Q4A_prequantized(const int8_t* xq, const float* xd, con
     hipStream_t st = as_stream(stream);
     if (rows <= kMaxGemvRows)
         return launch_gemv(w, xq, xd, gsum, y, part, reinterpret_cast<unsigned*>(ws), rows, Ng, Kg, group_k, N, st);
-    return launch_gemm(w, xq, xd, gsum, nullptr, y, part, reinterpret_cast<unsigned*>(ws), rows, Ng, Kg, group_k, N, nullptr, st);
+    return launch_gemm(w, xq, xd, gsum, nullptr, y, part, reinterpret_cast<unsigned*>(ws), rows, Ng, Kg, group_k, N, nullptr, lay.room, st);
 }
 
 extern "C" int llmops_fc_Q4A_partials(const int8_t* xq, int64_t rows, const int8_t* weiq, int64_t Ng, int64_t Kg,
@@ -393,7 +396,7 @@ extern "C" int llmops_fc_Q4A_noalloc(const float* x, int64_t rows, int64_t K, co
     // everything fc_impl will check is checked here first: a refused call must not enqueue the zero fill either
     const int bad = fc_check_args(x, rows, K, weiq, Ng, Kg, group_k, N, y);
     if (bad) return bad;
-    const size_t need = fc_layout(rows, Ng, Kg, group_k).total;
+    const size_t need = fc_layout(rows, Ng, Kg, group_k, LLMOPS_FC_NOALLOC_SCRATCH_BYTES).total;
     if (need > (size_t)LLMOPS_FC_NOALLOC_SCRATCH_BYTES)
         return fail(LLMOPS_EWORKSPACE,
                     "llmops_fc_Q4A_noalloc: rows=%lld, strips=%lld, k-groups=%lld need %zu scratch bytes, the built-in "
@@ -407,7 +410,7 @@ extern "C" int llmops_fc_Q4A_noalloc(const float* x, int64_t rows, int64_t K, co
     const int64_t n16 = LLMOPS_FC_COUNTER_BYTES / 16;
     zero16_kernel<<<(unsigned)((n16 + 255) / 256), 256, 0, as_stream(stream)>>>(reinterpret_cast<uint4*>(ws), n16);
     LLMOPS_LAUNCH_CHECK();
-    return fc_impl(x, rows, K, weiq, Ng, Kg, group_k, N, nullptr, y, ws, LLMOPS_FC_NOALLOC_SCRATCH_BYTES, stream);
+    return fc_impl(x, rows, K, weiq, Ng, Kg, group_k, N, nullptr, y, ws, LLMOPS_FC_NOALLOC_SCRATCH_BYTES, stream, LLMOPS_FC_NOALLOC_SCRATCH_BYTES);
 }
 
 // The production decode kernel in its dump build: y as llmops_fc_Q4A computes it for rows <= 8 with the kernel

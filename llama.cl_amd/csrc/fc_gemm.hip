@@ -2,11 +2,10 @@
 // launching of the product for both group sizes (group 32: fc_gemm_g32.hip).
 //
 // Operand layout of v_mfma_i32_16x16x64_i8: lane = 16*g + jj; the A lane holds row jj, the B lane holds column jj, both
-// for the same set of k-values chosen by g.  The packed format gives, per 16-byte load, 4 adjacent columns x 8 k-values
-// of one k8-row.  So lane (g, jj) takes the k8-rows that belong to g for columns 4*(jj&7)..+3 of strip (jj>>3); dword c
-// of that load is the lane's B operand for MFMA number c, whose 16 tile columns are
-// { strip (jj>>3), column 4*(jj&7)+c }.  Unpacking is two ANDs and a shift per dword; nothing is shuffled between lanes.
-// One MFMA covers 8 k8-rows (g owns rows 2g,2g+1 = 16 consecutive k); two of them make one k-group.
+// for the same set of k-values chosen by g.  A packed block has 8 k-values of a column in a dword, k8-row after k8-row; lane
+// (g, jj) takes the k8-rows 2g and 2g + 1 of columns 2*jj and 2*jj + 1 (one 8-byte read per k8-row), column 2*jj + c is its
+// operand for MFMA number c.  Unpacking is two ANDs and a shift per dword; nothing is shuffled between lanes.
+// One MFMA covers 8 k8-rows; two of them make one k-group.  Result register v of MFMA c: row 4*g + v, column 2*jj + c.
 // After every k-group the int32 tile is folded into fp32 accumulators:
 //   f += (d[n]*dx[row]) * float(acc) ; f += m[n]*gsum[row]        (fc_Q4A,
 //   /root/reference/ops/op_fc.hpp:381-412; min term is m * raw group sum).
@@ -15,253 +14,175 @@
 // float X, IS B + sum (|sum| <= 128*15*127 < 2^22), and X*d - B*d = sum*d is exact before the fma's
 // one rounding because B*d (2 significant bits times the 11 of an fp16) is itself a float.  Two
 // vector instructions per output element and k-group instead of three (convert, multiply, fma).
-// Result tile layout of the 16x16 MFMAs: lane holds column jj, rows 4*g+v in register v.
 #include "gemm_device.h"
 #include "gemv_device.h"
 
 namespace llmops {
 
+// two adjacent results, columns n0 and n0 + 1 of n, (+ residual) to a row of stride ld
+__device__ __forceinline__ void store_pair(float* dst, const float* res, float a, float b, int64_t n0, int64_t n, int64_t ld) {
+    if (n0 + 1 < n && (ld & 3) == 0) {
+        if (res) {
+            const float2 r = *reinterpret_cast<const float2*>(res);
+            a += r.x, b += r.y;
+        }
+        *reinterpret_cast<float2*>(dst) = make_float2(a, b);
+    } else {
+        if (n0 < n) dst[0] = res ? a + res[0] : a;
+        if (n0 + 1 < n) dst[1] = res ? b + res[1] : b;
+    }
+}
+
 // ---- split-K without a second launch -------------------------------------------------------------------
 // Every split stores its tile of partial sums with device-scope (write-through) stores, waits for them and
 // takes a ticket on the tile's counter; the split that draws the last ticket adds all splits' tiles in
 // index order (so the sum does not depend on who arrives when), adds the residual and writes the result.
-// Nobody waits for anybody.  The partial sums' row stride is a multiple of 32 floats; strips beyond Ng and
-// rows beyond `rows` fall outside the buffer descriptor (loads return 0, stores are dropped).
-// Called by every thread of the workgroup.  row0 / tile_rows: first row and row count of the rows this
-// thread's wave group owns; wave_row: the wave's first row inside them; a thread holds rows
-// wave_row + 16t + 4g + v, columns 32*strip + 4q .. + 3 in f[t][c][v].
-// The last arrival works one row tile at a time with all of its loads (up to SU splits x 4 rows) in flight
-// together: the reduction then costs about RT round trips to memory whatever the split count.  A split past
+// Nobody waits for anybody.  Called by every thread of the workgroup, with LDS no longer in use once all have arrived.
+// row0 / tile_rows: first row and row count of the tile; a thread holds rows 16t + 4g + v of it, columns
+// 32*strip + 2*jj + c in f[t][c][v].
+// Where the sums of a tile lie: a row block's rows * Np floats strip by strip, a strip's rows in pairs, a pair as
+// [jj][row of the pair][c]: 16 bytes per lane, 256 of them consecutive (and the last of an odd number of rows by itself, 8 bytes
+// per lane).  Accesses of rows beyond `rows` fall outside the buffer descriptor (loads return 0, stores are dropped), as do
+// those of strips beyond Ng.
+// The last arrival works two row tiles at a time with all of its loads (up to SU splits x 8 rows) in flight
+// together: the reduction then costs about T / 2 round trips to memory whatever the split count.  A split past
 // the last is asked for through an empty descriptor: it returns 0 without touching memory.
-template <int RT, int SU>
-__device__ __forceinline__ void splitk_finish(const v4f (&f)[RT][4], float* __restrict__ out, int64_t split_stride, int64_t ldo,
-                                              int row0, int tile_rows, int wave_row, int strip, int Ng, int q, int g, int rows,
+template <int T, int SU>
+__device__ __forceinline__ void splitk_finish(const v4f (&f)[T][2], float* __restrict__ out, int64_t split_stride, int64_t Np,
+                                              int row0, int tile_rows, int strip, int Ng, int jj, int g, int rows,
                                               float* __restrict__ y_final, int64_t Ny, const float* __restrict__ residual,
-                                              unsigned* counter, int tid) {
+                                              unsigned* counter, int tid, unsigned* ticket_sh) {
     constexpr int kAgent = 16;  // sc1: coherent at device scope, as a relaxed atomic store / load would be
     const int S = (int)gridDim.z;
-    const uint32_t tile_bytes = tile_rows > 0 ? (uint32_t)tile_rows * (uint32_t)ldo * 4u : 0u;
-    const uint32_t col_off = (uint32_t)(strip * kGroupN + q * 4) * 4u;
-    const bool strip_ok = strip < Ng;
+    const bool strip_ok = strip < Ng, odd = (tile_rows & 1) != 0;
+    const uint32_t strip_bytes = strip_ok ? (uint32_t)tile_rows * (kGroupN * 4u) : 0u;
+    float* base = out + (int64_t)row0 * Np + (int64_t)strip * kGroupN * tile_rows;
+    // rows r = 16t + 4g + 2e and r + 1, or (last) r alone
+    const auto place = [&](int t, int e) {
+        const int r = t * 16 + 4 * g + 2 * e;
+        return r + 1 < tile_rows ? (uint32_t)(r * (kGroupN * 4) + jj * 16) : 0xFFFFFF00u;
+    };
+    const auto place_last = [&](int t, int e) {
+        const int r = t * 16 + 4 * g + 2 * e;
+        return r + 1 == tile_rows ? (uint32_t)(r * (kGroupN * 4) + jj * 8) : 0xFFFFFF00u;
+    };
     {
-        const buffer_rsrc rs = make_rsrc(out + (int64_t)blockIdx.z * split_stride + (int64_t)row0 * ldo, strip_ok ? tile_bytes : 0u);
+        const buffer_rsrc rs = make_rsrc(base + (int64_t)blockIdx.z * split_stride, strip_bytes);
 #pragma unroll
-        for (int t = 0; t < RT; t++)
+        for (int t = 0; t < T; t++)
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int r = wave_row + t * 16 + g * 4 + v;
-                const u32x4 val = {__float_as_uint(f[t][0][v]), __float_as_uint(f[t][1][v]), __float_as_uint(f[t][2][v]),
-                                   __float_as_uint(f[t][3][v])};
-                __builtin_amdgcn_raw_buffer_store_b128(val, rs, (uint32_t)r * (uint32_t)ldo * 4u + col_off, 0, kAgent);
+            for (int e = 0; e < 2; e++) {
+                const u32x4 val = {__float_as_uint(f[t][0][2 * e]), __float_as_uint(f[t][1][2 * e]), __float_as_uint(f[t][0][2 * e + 1]),
+                                   __float_as_uint(f[t][1][2 * e + 1])};
+                __builtin_amdgcn_raw_buffer_store_b128(val, rs, place(t, e), 0, kAgent);
+                if (odd) __builtin_amdgcn_raw_buffer_store_b64(v2u{val[0], val[1]}, rs, place_last(t, e), 0, kAgent);
             }
     }
-    __shared__ unsigned ticket_sh;
     __builtin_amdgcn_s_waitcnt(0);  // this wave's stores have been acknowledged
     __syncthreads();
-    if (tid == 0) ticket_sh = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) *ticket_sh = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    if (ticket_sh != (unsigned)(S - 1)) return;
+    if (*ticket_sh != (unsigned)(S - 1)) return;
     if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // next launch
     if (!strip_ok) return;
-    const int64_t n0 = (int64_t)strip * kGroupN + q * 4;
+    const int64_t n0 = (int64_t)strip * kGroupN + 2 * jj;
 #pragma unroll
-    for (int t = 0; t < RT; t++) {
-        float4 a[4];
+    for (int t = 0; t < T; t += 2) {
+        float a[4][4];
 #pragma unroll
-        for (int v = 0; v < 4; v++) a[v] = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int p = 0; p < 4; p++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) a[p][v] = 0.0f;
         for (int s0 = 0; s0 < S; s0 += SU) {
             u32x4 pv[SU][4];
 #pragma unroll
             for (int u = 0; u < SU; u++) {
-                const int sidx = min(s0 + u, S - 1);
-                const buffer_rsrc rs =
-                    make_rsrc(out + (int64_t)sidx * split_stride + (int64_t)row0 * ldo, s0 + u < S ? tile_bytes : 0u);
+                const buffer_rsrc rs = make_rsrc(base + (int64_t)min(s0 + u, S - 1) * split_stride, s0 + u < S ? strip_bytes : 0u);
 #pragma unroll
-                for (int v = 0; v < 4; v++)
-                    pv[u][v] = __builtin_amdgcn_raw_buffer_load_b128(
-                        rs, (uint32_t)(wave_row + t * 16 + g * 4 + v) * (uint32_t)ldo * 4u + col_off, 0, kAgent);
+                for (int p = 0; p < 4; p++) pv[u][p] = __builtin_amdgcn_raw_buffer_load_b128(rs, place(t + (p >> 1), p & 1), 0, kAgent);
             }
 #pragma unroll
             for (int u = 0; u < SU; u++)
 #pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    a[v].x += __uint_as_float(pv[u][v][0]), a[v].y += __uint_as_float(pv[u][v][1]);
-                    a[v].z += __uint_as_float(pv[u][v][2]), a[v].w += __uint_as_float(pv[u][v][3]);
-                }
+                for (int p = 0; p < 4; p++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) a[p][v] += __uint_as_float(pv[u][p][v]);
         }
+        if (odd && t * 16 + 32 >= tile_rows && t * 16 < tile_rows) {
+            for (int sp = 0; sp < S; sp++) {
+                const buffer_rsrc rs = make_rsrc(base + (int64_t)sp * split_stride, strip_bytes);
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int row = row0 + wave_row + t * 16 + g * 4 + v;
-            if (row >= rows) continue;
-            float* dst = y_final + (int64_t)row * Ny + n0;
-            const float* res = residual ? residual + (int64_t)row * Ny + n0 : nullptr;
-            if (n0 + 3 < Ny && (Ny & 3) == 0) {
-                float4 val = a[v];
-                if (res) {
-                    const float4 r4 = *reinterpret_cast<const float4*>(res);
-                    val.x += r4.x, val.y += r4.y, val.z += r4.z, val.w += r4.w;
+                for (int p = 0; p < 4; p++) {
+                    const v2u last = __builtin_amdgcn_raw_buffer_load_b64(rs, place_last(t + (p >> 1), p & 1), 0, kAgent);
+                    a[p][0] += __uint_as_float(last[0]), a[p][1] += __uint_as_float(last[1]);
                 }
-                *reinterpret_cast<float4*>(dst) = val;
-            } else {
-                const float av[4] = {a[v].x, a[v].y, a[v].z, a[v].w};
-#pragma unroll
-                for (int c = 0; c < 4; c++)
-                    if (n0 + c < Ny) dst[c] = res ? av[c] + res[c] : av[c];
             }
         }
+#pragma unroll
+        for (int p = 0; p < 4; p++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int row = row0 + (t + (p >> 1)) * 16 + 4 * g + 2 * (p & 1) + i;
+                if (row < rows)
+                    store_pair(y_final + (int64_t)row * Ny + n0, residual ? residual + (int64_t)row * Ny + n0 : nullptr, a[p][2 * i], a[p][2 * i + 1], n0, Ny, Ny);
+            }
     }
 }
 
-// ---- LDS-tiled kernel for group 128 ---------------------------------------------------------------
-// Workgroup = 4 wavefronts (2 x 2), tile = BM rows x 128 columns (4 strips), one k-group per
-// iteration.  Per iteration the workgroup stages into LDS, through registers and double buffered:
-//   A : BM rows x 128 activation codes (row stride 144 B so that the 16 rows a ds_read_b128 wave
-//       access touches fall into different banks)
-//   B : the 4 packed blocks as they are in memory (nibbles + fp16 d + fp16 m, 2176 B each)
-//   XS: (dx, gsum) of the BM rows for this k-group
-// The global loads of iteration kb+1 are issued before the MFMAs of iteration kb and written to the
-// other LDS buffer after them; one barrier per iteration.  Each wave owns 64 rows x 64 columns
-// (RT = BM/32 row tiles x 4 column sets); operand mapping as at the top of this file.
-constexpr int kAStride = 144;
+// ---- the tiled kernel -------------------------------------------------------------------------------
+// What bounds it: everything at once.  Per k-group and 128 x 128 tile a wave has 32 int8 MFMAs (512 cycles), 128 fold
+// instructions and about 40 others (600 cycles and more of vector issue, which the int8 MFMA shares only in part: 395 cycles
+// for two waves' 4 x 32x32x32 and 32 fold instructions each, against 263 and 193 alone), 26 KB of LDS reads and 6.4 KB
+// of copies.  With parts left out (2048 x 11008 x 4096, 163 us at that point): no copies 141, no code reads 151, no fold 133,
+// no MFMA 133, neither 114, copies alone 107.  So each is kept small, and two to four workgroups share a compute unit so that
+// one's waits are another's work:
+//   * tile 32*RT rows x 128 columns, four waves side by side, a strip each: a strip's weights are unpacked by one wave only
+//     (2 x 2 waves of 64 x 64 unpack twice as much: 32-row tiles 2 to 7 % slower, 128 rows even), codes are read by all four.
+//     (The weights as the A operand, a row and eight adjacent columns in a lane: 2 % faster with 128 rows, but eight scales to
+//     convert instead of two, 2 to 6 % slower with 32 and 64.)
+//   * codes, nibbles, scales, sums and mins are copied to LDS asynchronously (global_load_lds) two k-groups ahead: no
+//     registers, no LDS store instructions.  (Through registers one k-group ahead: 5 to 13 % slower, 512 x 22016 x 4096 103 us
+//     against 90.)  Codes, scales and nibbles have three slots; sums and mins six, since the min term is formed for four
+//     k-groups together.
+//   * the first operands of a k-group are read from LDS while the last row tiles of the one before are multiplied, and the
+//     fold of one pair of row tiles runs beside the products of the next: the order is pinned.
+// A 256 x 128 tile with two wave groups (one workgroup per compute unit, 20 % less to copy) takes 165 to 170 us at
+// 2048 x 11008 x 4096 where 128 rows take 156: nothing covers its barriers, its first fetch and its stores.
+// Measured, us for the whole call in a graph, kernels before (weights and codes through registers below 512 rows, two wave
+// groups in alternating phases from there on) and now: 128 x 4096 x 11008 27.5 / 24.4, 300 x 4090 x 11008 46 / 39, 512 x 4096^2
+// 33.8 / 27.7, 512 x 22016 x 4096 102.5 / 88, 512 x 4096 x 11008 57 / 53, 2048 x 11008 x 4096 164 / 157, 2048 x 4096 x 11008 153 / 150.
 constexpr int kBlk128 = 2176;
-
-__device__ __forceinline__ v2f buf_ld_pair(buffer_rsrc r, uint32_t voff, uint32_t soff) {
-    typedef unsigned int u32x2_g __attribute__((ext_vector_type(2)));
-    const u32x2_g t = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
-    return v2f{__uint_as_float(t.x), __uint_as_float(t.y)};
-}
-
-// ---- the min term of a tile on the fp16 matrix cores -------------------------------------------------
-// sum over k-groups of m[column][kg] * gsum[row][kg] is a product with K = number of k-groups.  It is
-// taken out of the k-group loop and computed once per tile, 32 k-groups per MFMA, with fp32 accumulation:
-// gsum = hi + lo (hi = gsum rounded toward zero to fp16, lo = the rest: 22 significant bits in all), m as
-// it is stored (fp16), two MFMAs per 16x16 tile.  (The fp32 MFMA that did this inside the loop stalls the
-// vector ALU for its whole duration; the fp16 one runs beside vector work.)  That is good for a row's eight
-// k-groups in one lane if the largest |gsum| among them lies in [1/8, 60000]: below that lo falls into fp16's
-// subnormals and the row could lose bits relative to its own size, above it hi overflows.  Zeros are exact.
-// When a lane of the wave does not qualify, the wave takes the round with fp32 MFMAs instead (four k-groups
-// each, exact products): the slow path, there for correctness on any input.
-// What a lane fetches for one round of 32 k-groups (k32 .. k32+31, those below kb1): for its eight k-groups
-// kgs .. kgs+7 the group sums of its row in each of RT row tiles (32 contiguous bytes of the [row][kg] matrix, which
-// start on a 4-byte boundary only) and the mins of its four columns.  kgs is k32 + 8g unless that would read past
-// the end of a row: then it is Kg - 8, and the slots below k32 + 8g do not count (min_term_add).
+constexpr int kStages = 3;    // LDS slots of a k-group: one is multiplied, one has landed, one is on its way
+constexpr int kMinRing = 6;   // LDS slots of sums and mins: the last four k-groups and the two ahead
 template <int RT>
-struct MinTermRound {
-    Float4U ga[RT][2];
-    uint2 mb[8];
-};
-// roff[t] = Kg * the lane's row of row tile t (clamped to the matrix); strip: its strip (clamped); q: its column
-// quad.  Rows and strip count from wherever gs and weiq point (the matrix, or the workgroup's tile of it): offsets
-// from there must fit 32 bits.
-template <int RT>
-__device__ __forceinline__ void min_term_fetch(MinTermRound<RT>& r, const float* __restrict__ gs, const int (&roff)[RT],
-                                               const uint8_t* __restrict__ weiq, int Kg, int kgs, int strip, int q) {
-    // (a uniform base and a 32-bit byte offset per lane: one address register per load, not two)
-    const uint8_t* gb = reinterpret_cast<const uint8_t*>(gs);
-#pragma unroll
-    for (int t = 0; t < RT; t++) {
-        const uint32_t off = (uint32_t)(roff[t] + kgs) * 4u;
-        r.ga[t][0] = *reinterpret_cast<const Float4U*>(gb + off);
-        r.ga[t][1] = *reinterpret_cast<const Float4U*>(gb + off + 16u);
-    }
-    const uint32_t moff = (uint32_t)((strip * Kg + kgs) * kBlk128 + 2112 + q * 8);
-#pragma unroll
-    for (int i = 0; i < 8; i++) r.mb[i] = *reinterpret_cast<const uint2*>(weiq + (moff + (uint32_t)(i * kBlk128)));
-}
-// f[t][c] += the round's part of the min term; operand layout of the 16x16x32 MFMA: A lane (row = lane & 15,
-// k = 8 * (lane >> 4) + i), B lane (column = lane & 15, same k), D as the int8 MFMAs' (row 4g+v, column = lane & 15).
-// Slot i of the lane is k-group kgs + i and counts if it lies in [lo, kb1).  FIRST: f = instead of f += (the
-// accumulators then do not exist yet while the operands are fetched and examined).
-template <int RT, bool FIRST>
-__device__ __forceinline__ void min_term_add(v4f (&f)[RT][4], const MinTermRound<RT>& r, int kgs, int lo, int kb1) {
-    const v4f zero = {0.f, 0.f, 0.f, 0.f};
-    // (the slot tests are repeated where the values are used -- behind an empty asm statement, or the compiler
-    // keeps the 8 * RT masked values of the first pass in registers, which do not fit beside the accumulators,
-    // the operands and what the k-group loop keeps across this prologue)
-#define LLMOPS_GSUM(T, I) ((kgs + (I) >= lo && kgs + (I) < kb1) ? r.ga[T][(I) >> 2].v[(I) & 3] : 0.0f)
-    // (tested per lane, i.e. per row and eight k-groups, which is stricter than per row and needs no exchange)
-    bool rows_fit = true;
-#pragma unroll
-    for (int t = 0; t < RT; t++) {
-        float big = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; i++) big = fmaxf(big, fabsf(LLMOPS_GSUM(t, i)));
-        rows_fit = rows_fit && (big == 0.0f || (big >= 0.125f && big <= 60000.0f));
-    }
-    asm volatile("" : "+v"(lo));
-    if (__all(rows_fit)) {
-        Halves8 m[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint2 e = r.mb[2 * j], o = r.mb[2 * j + 1];
-            m[0].u[j] = __builtin_amdgcn_perm(o.x, e.x, 0x05040100u);
-            m[1].u[j] = __builtin_amdgcn_perm(o.x, e.x, 0x07060302u);
-            m[2].u[j] = __builtin_amdgcn_perm(o.y, e.y, 0x05040100u);
-            m[3].u[j] = __builtin_amdgcn_perm(o.y, e.y, 0x07060302u);
-        }
-#pragma unroll
-        for (int t = 0; t < RT; t++) {
-            Halves8 ah, al;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float e = LLMOPS_GSUM(t, 2 * j), o = LLMOPS_GSUM(t, 2 * j + 1);
-                const v2h h = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(e, o));
-                ah.u[j] = __builtin_bit_cast(uint32_t, h);
-                al.u[j] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(e - (float)h[0], o - (float)h[1]));
-            }
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-                f[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al.h, m[c].h, FIRST ? zero : f[t][c], 0, 0, 0);
-#pragma unroll
-            for (int c = 0; c < 4; c++) f[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah.h, m[c].h, f[t][c], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);  // one row tile's halves at a time: registers
-        }
-    } else {
-        // slot i of the four lanes (row or column, g = 0..3) is one 16x16x4 product: k = g
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float mc[4] = {f16_bits_to_f32((uint16_t)(r.mb[i].x & 0xFFFFu)), f16_bits_to_f32((uint16_t)(r.mb[i].x >> 16)),
-                                 f16_bits_to_f32((uint16_t)(r.mb[i].y & 0xFFFFu)), f16_bits_to_f32((uint16_t)(r.mb[i].y >> 16))};
-#pragma unroll
-            for (int t = 0; t < RT; t++) {
-                const float a = LLMOPS_GSUM(t, i);
-#pragma unroll
-                for (int c = 0; c < 4; c++)
-                    f[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, mc[c], (FIRST && i == 0) ? zero : f[t][c], 0, 0, 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);  // one slot's operands at a time: registers, not speed, matter here
-        }
-    }
-#undef LLMOPS_GSUM
-}
-
-template <int RT>
-struct GemmSmem {
+struct GemmTile {
     static constexpr int BM = RT * 32;
-    uint8_t a[2][BM * kAStride];
-    uint8_t b[2][4 * kBlk128];
-    float2 xs[2][BM];
+    static constexpr int T = BM / 16;  // row tiles of a wave: all of them
+    struct Stage {
+        uint8_t a[BM * 128];     // codes
+        uint8_t b[4 * 2048];     // nibbles of the four strips
+        uint16_t d[4 * 32];      // their scales
+        float dx[BM];            // the rows' scales
+    };
+    Stage st[kStages];
+    float gs[kMinRing][BM];      // the rows' sums
+    uint16_t m[kMinRing][4 * 32];  // the strips' mins
 };
 
 template <int RT, bool PARTIALS>
-__global__ __launch_bounds__(256, (RT == 4 ? 2 : (RT == 2 ? 3 : 4))) void fc_gemm_lds_kernel(const uint8_t* __restrict__ weiq, const int8_t* __restrict__ xq,
-                                                           const float* __restrict__ xd, const float* __restrict__ gs,
-                                                           const float2* __restrict__ xsT, float* __restrict__ out,
-                                                           int32_t* __restrict__ out_i, int Ng, int Kg, int64_t ldo,
-                                                           int64_t N, int rows, int kb_per_split, int64_t split_stride,
-                                                           const float* __restrict__ residual, float* __restrict__ y_final,
-                                                           int64_t Ny, unsigned* __restrict__ counters) {
-    constexpr int BM = RT * 32;
-    constexpr int A_CHUNKS = BM * 8;                     // 16-byte chunks of the A tile
-    constexpr int A_PER_THREAD = A_CHUNKS / 256;         // RT
-    constexpr int B_CHUNKS = 4 * (kBlk128 / 16);         // 544
-    constexpr int B_PER_THREAD = (B_CHUNKS + 255) / 256; // 3
+__global__ __launch_bounds__(256, (RT == 4 ? 2 : (RT == 2 ? 3 : 4))) void fc_gemm_tile_kernel(
+    const uint8_t* __restrict__ weiq, const int8_t* __restrict__ xq, const float* __restrict__ xd, const float* __restrict__ gs,
+    const float2* __restrict__ xsT, float* __restrict__ out, int32_t* __restrict__ out_i, int Ng, int Kg, int64_t ldo, int64_t N,
+    int rows, int kb_per_split, int64_t split_stride, const float* __restrict__ residual, float* __restrict__ y_final, int64_t Ny,
+    unsigned* __restrict__ counters) {
+    using Tile = GemmTile<RT>;
+    constexpr int BM = Tile::BM, T = Tile::T;
     extern __shared__ __align__(16) uint8_t smem_raw[];
-    GemmSmem<RT>& sm = *reinterpret_cast<GemmSmem<RT>*>(smem_raw);
+    Tile& sm = *reinterpret_cast<Tile*>(smem_raw);
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = wave >> 1, wc = wave & 1;  // wave's row half / column half
-    const int g = lane >> 4, jj = lane & 15, q = jj & 7, sp = jj >> 3;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, jj = lane & 15;
     // Which tile: workgroups go to the 8 XCDs round robin, each XCD has its own L2, and an XCD runs
     // about 32 CUs x (workgroups per CU) workgroups at a time.  The tiles are therefore numbered so that
     // each XCD gets one contiguous run of them and a run walks the tile grid in bands of 8 row blocks,
@@ -286,597 +207,256 @@ __global__ __launch_bounds__(256, (RT == 4 ? 2 : (RT == 2 ? 3 : 4))) void fc_gem
     const int kb0 = blockIdx.z * kb_per_split, kb1 = min(Kg, kb0 + kb_per_split);
     const int64_t Kp = (int64_t)Kg * 128;
 
-    // ---- global -> register staging of one k-group (macros: the arrays must stay in registers) ----
-    v4u ra[A_PER_THREAD], rb[B_PER_THREAD];  // native vector types: these must live in registers
-    v2f rxs = {0.f, 0.f};
-    // Source addresses: buffer descriptors whose base is the same for the whole workgroup, a scalar offset that advances
-    // with kb, and a 32-bit offset per thread that does not depend on kb: no 64-bit address arithmetic in the loop,
-    // which is bound by instruction issue (128 rows, 4096 -> 11008: 26.65 -> 26.2 us).
-    const buffer_rsrc a_rs = make_rsrc(xq + (int64_t)row0 * Kp, (uint32_t)min(BM, rows - row0) * (uint32_t)Kp);
-    const buffer_rsrc b_rs = make_rsrc(weiq + (int64_t)strip0 * Kg * kBlk128, (uint32_t)min(4, Ng - strip0) * (uint32_t)Kg * (uint32_t)kBlk128);
-    const buffer_rsrc x_rs = make_rsrc(xsT != nullptr ? xsT : reinterpret_cast<const float2*>(xq), xsT != nullptr ? (uint32_t)Kg * (uint32_t)rows * 8u : 0u);
-    uint32_t aoff[A_PER_THREAD];
-    int adst[A_PER_THREAD];
+    // ---- what this wave copies per k-group (rows and strips past the end re-read the last one that exists) ----
+    // codes: BM / 4 rows, 8 rows of 128 bytes to a copy.  16-byte chunk c of row r lies at position c ^ key(r), key(r) =
+    // (r + ((r >> 3) & 1)) & 7: the 16 rows that one phase of a ds_read_b128 touches fall on 16 different bank groups
+    constexpr int AC = RT;
+    const uint8_t* abase = reinterpret_cast<const uint8_t*>(xq) + (int64_t)row0 * Kp;
+    uint32_t aoff[AC];
 #pragma unroll
-    for (int i = 0; i < A_PER_THREAD; i++) {
-        const int c = tid + i * 256, r = c >> 3, part = c & 7;
-        aoff[i] = (uint32_t)(min(rows - 1, row0 + r) - row0) * (uint32_t)Kp + (uint32_t)(part * 16);
-        adst[i] = r * kAStride + part * 16;
+    for (int i = 0; i < AC; i++) {
+        const int r = (wave * AC + i) * 8 + (lane >> 3), key = (r + ((r >> 3) & 1)) & 7;
+        aoff[i] = (uint32_t)(min(rows - 1, row0 + r) - row0) * (uint32_t)Kp + (uint32_t)(((lane & 7) ^ key) * 16);
     }
-    uint32_t boff[B_PER_THREAD];
+    // nibbles: 8 k8-rows of 128 bytes to a copy, row 2g + p of the eight at place 4p + g: the rows that the lane groups
+    // g = 0..3 read together lie side by side
+    constexpr int BC = 2;
+    const uint8_t* tbase = weiq + (int64_t)strip0 * Kg * kBlk128;
+    const auto strip_off = [&](int s) { return (uint32_t)(min(Ng - 1, strip0 + s) - strip0) * (uint32_t)Kg * (uint32_t)kBlk128; };
+    uint32_t boff[BC];
 #pragma unroll
-    for (int i = 0; i < B_PER_THREAD; i++) {
-        const int c = min(B_CHUNKS - 1, tid + i * 256);
-        const int st = c / (kBlk128 / 16), off = c % (kBlk128 / 16);
-        boff[i] = (uint32_t)(min(Ng - 1, strip0 + st) - strip0) * (uint32_t)Kg * (uint32_t)kBlk128 + (uint32_t)(off * 16);
+    for (int i = 0; i < BC; i++) {
+        const int c = wave * BC + i, place = lane >> 3;
+        boff[i] = strip_off(c >> 1) + (uint32_t)((c & 1) * 1024 + (2 * (place & 3) + (place >> 2)) * 128 + (lane & 7) * 16);
     }
-    const int64_t xrow = min(rows - 1, row0 + (tid < BM ? tid : 0));
-#define LLMOPS_FETCH(KB)                                                                                              \
-    do {                                                                                                              \
-        _Pragma("unroll") for (int i = 0; i < A_PER_THREAD; i++) {                                                    \
-            const u32x4 t_ = __builtin_amdgcn_raw_buffer_load_b128(a_rs, aoff[i], (uint32_t)(KB) * 128u, 0);          \
-            ra[i] = v4u{t_.x, t_.y, t_.z, t_.w};                                                                      \
-        }                                                                                                             \
-        _Pragma("unroll") for (int i = 0; i < B_PER_THREAD; i++) { /* clamped offset */                               \
-            const u32x4 t_ = __builtin_amdgcn_raw_buffer_load_b128(b_rs, boff[i], (uint32_t)(KB) * (uint32_t)kBlk128, 0); \
-            rb[i] = v4u{t_.x, t_.y, t_.z, t_.w};                                                                      \
-        }                                                                                                             \
-        if (!PARTIALS)                                                                                                \
-            rxs = xsT ? buf_ld_pair(x_rs, (uint32_t)xrow * 8u, (uint32_t)(KB) * (uint32_t)rows * 8u)                  \
-                      : v2f{xd[xrow * Kg + (KB)], gs[xrow * Kg + (KB)]};                                            \
-    } while (0)
-#define LLMOPS_STASH(BUF)                                                                                  \
-    do {                                                                                                   \
-        _Pragma("unroll") for (int i = 0; i < A_PER_THREAD; i++)                                           \
-            *reinterpret_cast<v4u*>(&sm.a[BUF][adst[i]]) = ra[i];                                          \
-        _Pragma("unroll") for (int i = 0; i < B_PER_THREAD; i++)                                           \
-            if (tid + i * 256 < B_CHUNKS) *reinterpret_cast<v4u*>(&sm.b[BUF][(tid + i * 256) * 16]) = rb[i]; \
-        if (tid < BM) *reinterpret_cast<v2f*>(&sm.xs[BUF][tid]) = rxs;                                                            \
-    } while (0)
-
-    v4f f[RT][4];
+    // the rows' scales and sums, 64 rows to a copy, then the strips' scales and mins: copies 0 .. 2*XC+1, one or two per wave
+    constexpr int XC = BM > 64 ? BM / 64 : 1;
+    const uint8_t* sbase[2] = {nullptr, nullptr};
+    uint32_t soff[2] = {0, 0}, sdst[2] = {0, 0}, sring[2] = {0, 0};
+    int64_t sstep[2] = {0, 0};
+    bool slive[2];
+    const uint32_t lds0 = lds_off(smem_raw);
 #pragma unroll
-    for (int t = 0; t < RT; t++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) f[t][c] = v4f{0.f, 0.f, 0.f, 0.f};
-    // Min term sum_kb m[n,kb]*gsum[row,kb]: a rank-Kg product, done four k-groups at a time by
-    // v_mfma_f32_16x16x4_f32 straight into the fp32 accumulators (same tile layout as the int8
-    // MFMAs).  Lane (jj, g) keeps gsum of row jj and m of its columns for the group with index g
-    // of the current four.
-    float gk[RT], mk[4];
-#pragma unroll
-    for (int t = 0; t < RT; t++) gk[t] = 0.0f;
-#pragma unroll
-    for (int c = 0; c < 4; c++) mk[c] = 0.0f;
-
-    if (kb0 < kb1) {
-        LLMOPS_FETCH(kb0);
-        LLMOPS_STASH(0);
+    for (int u = 0; u < 2; u++) {
+        const int s = wave + u * 4;
+        slive[u] = s < 2 * XC + 2;
+        if (s < 2 * XC) {
+            const bool sums = s >= XC;
+            const int part = sums ? s - XC : s, row = min(rows - 1, row0 + part * 64 + min(lane, BM - 1));
+            if (PARTIALS) slive[u] = false;
+            if (xsT != nullptr) {
+                sbase[u] = reinterpret_cast<const uint8_t*>(xsT) + (sums ? 4 : 0);
+                soff[u] = (uint32_t)row * 8u, sstep[u] = (int64_t)rows * 8;
+            } else {
+                sbase[u] = reinterpret_cast<const uint8_t*>((sums ? gs : xd) + (int64_t)row0 * Kg);
+                soff[u] = (uint32_t)(row - row0) * (uint32_t)Kg * 4u, sstep[u] = 4;
+            }
+            sring[u] = sums ? BM * 4 : 0;
+            sdst[u] = (sums ? lds_off(&sm.gs[0][0]) : lds_off(&sm.st[0].dx[0])) + part * 256;
+        } else {
+            const bool mins = s == 2 * XC + 1;
+            sbase[u] = tbase + 2048 + (mins ? 64 : 0);
+            soff[u] = strip_off(lane >> 4) + (uint32_t)(lane & 15) * 4u, sstep[u] = kBlk128;
+            sring[u] = mins ? 256 : 0;
+            sdst[u] = mins ? lds_off(&sm.m[0][0]) : lds_off(&sm.st[0].d[0]);
+        }
     }
-    __syncthreads();
+    auto copy_stage = [&](int kb, int slot, int ring) {
+        const uint32_t base = uniform_u32(lds0 + slot * (int)sizeof(typename Tile::Stage));
+        const uint8_t* as = abase + (int64_t)kb * 128;
+#pragma unroll
+        for (int i = 0; i < AC; i++) copy16_to_lds(as, aoff[i], base + (wave * AC + i) * 1024);
+        const uint8_t* bs = tbase + (int64_t)kb * kBlk128;
+#pragma unroll
+        for (int i = 0; i < BC; i++) copy16_to_lds(bs, boff[i], base + BM * 128 + (wave * BC + i) * 1024);
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+            if (slive[u]) {  // (uniform)
+                const uint32_t dst = uniform_u32(sdst[u] + (sring[u] != 0 ? ring * sring[u] : slot * (uint32_t)sizeof(typename Tile::Stage)));
+                const void* from = uniform_ptr(sbase[u] + (int64_t)kb * sstep[u]);
+                if (RT > 1) copy4_to_lds(from, soff[u], dst);
+                else if (lane < 32 || wave >= 2) copy4_to_lds(from, soff[u], dst);  // (32 rows; the strips' copies are whole)
+            }
+    };
 
-    const int strip_l = wc * 2 + sp;  // strip (0..3) of the tile this lane's B operands come from
+    v4f f[T][2];
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) f[t][c] = v4f{0.f, 0.f, 0.f, 0.f};
+    // the sums start at the bit pattern of 1.5 * 2^23, so that the fold needs no convert instruction
+    constexpr int kInit = PARTIALS ? 0 : kFoldBiasBits;
+    v4i bias = {kInit, kInit, kInit, kInit};
+    asm volatile("" : "+v"(bias));  // (in registers once, not set up for every product)
+
+#pragma unroll
+    for (int i = 0; i < kStages - 1; i++)
+        if (kb0 + i < kb1) copy_stage(kb0 + i, i, i);
+
+    const int akey = (jj + (jj >> 3)) & 7;
+    const int a_rd[2] = {jj * 128 + ((g ^ akey) * 16), jj * 128 + (((4 + g) ^ akey) * 16)};
+    const int b_rd = wave * 2048 + g * 128 + jj * 8;
+    // what the next k-group starts with is read while the last row tiles of this one are multiplied
+    v4i a[2][2][2];  // [pair of row tiles, odd or even][tile][k half]
+    uint2 wraw[2][2];
+    uint32_t dh;
+    constexpr int P = T / 2;
+    auto load_a = [&](const typename Tile::Stage& st, int p) {
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) a[p & 1][i][h] = *reinterpret_cast<const v4i*>(&st.a[a_rd[h] + (2 * p + i) * 2048]);
+    };
+    auto load_first = [&](const typename Tile::Stage& st) {
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) a[P & 1][i][h] = *reinterpret_cast<const v4i*>(&st.a[a_rd[h] + i * 2048]);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int p = 0; p < 2; p++) wraw[h][p] = *reinterpret_cast<const uint2*>(&st.b[b_rd + h * 1024 + p * 512]);
+        dh = *reinterpret_cast<const uint32_t*>(&st.d[wave * 32 + jj * 2]);
+    };
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
+    load_first(sm.st[0]);
+    int slot = 0, ring = 0, since = 0;  // since: k-groups whose min term is not in yet
     for (int kb = kb0; kb < kb1; kb++) {
-        const int buf = (kb - kb0) & 1;
-        if (kb + 1 < kb1) LLMOPS_FETCH(kb + 1);
+        // this wave's copies for k-group kb + 1 have landed, then everyone's; the slot of kb - 1 is free
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
+        if (kb + 2 < kb1) copy_stage(kb + 2, slot == 0 ? 2 : slot - 1, ring >= kMinRing - 2 ? ring + 2 - kMinRing : ring + 2);
+        const typename Tile::Stage& st = sm.st[slot];
+        slot = slot == kStages - 1 ? 0 : slot + 1;
 
-        const uint8_t* bblk = &sm.b[buf][strip_l * kBlk128];
-        const uint8_t* abase = &sm.a[buf][(wr * (BM / 2) + jj) * kAStride + g * 16];
-        v4i acc[RT][4];
-        // the sums start at the bit pattern of 1.5 * 2^23, so that the fold needs no convert instruction
-        // (see fc_gemm_pp_kernel)
-        constexpr int kInit = PARTIALS ? 0 : kFoldBiasBits;
-#pragma unroll
-        for (int t = 0; t < RT; t++)
-#pragma unroll
-            for (int c = 0; c < 4; c++) acc[t][c] = v4i{kInit, kInit, kInit, kInit};
+        v4i b[2][2];
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            const uint4 wa = *reinterpret_cast<const uint4*>(bblk + h * 1024 + (2 * g) * kRowBytes + q * 16);
-            const uint4 wb = *reinterpret_cast<const uint4*>(bblk + h * 1024 + (2 * g + 1) * kRowBytes + q * 16);
-            const uint32_t* pa = reinterpret_cast<const uint32_t*>(&wa);
-            const uint32_t* pb = reinterpret_cast<const uint32_t*>(&wb);
-            v4i b[4];
+            b[h][0] = v4i{(int)lo4(wraw[h][0].x), (int)hi4(wraw[h][0].x), (int)lo4(wraw[h][1].x), (int)hi4(wraw[h][1].x)};
+            b[h][1] = v4i{(int)lo4(wraw[h][0].y), (int)hi4(wraw[h][0].y), (int)lo4(wraw[h][1].y), (int)hi4(wraw[h][1].y)};
+        }
+        if (P & 1) {
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-                b[c][0] = (int)lo4(pa[c]);
-                b[c][1] = (int)hi4(pa[c]);
-                b[c][2] = (int)lo4(pb[c]);
-                b[c][3] = (int)hi4(pb[c]);
-            }
+            for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int t = 0; t < RT; t++) {
-                const v4i a = *reinterpret_cast<const v4i*>(abase + t * 16 * kAStride + h * 64);
+                for (int h = 0; h < 2; h++) a[0][i][h] = a[1][i][h];
+        }
+        float d[2] = {f16_bits_to_f32((uint16_t)(dh & 0xFFFFu)), f16_bits_to_f32((uint16_t)(dh >> 16))}, nbd[2];
 #pragma unroll
-                for (int c = 0; c < 4; c++) acc[t][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b[c], acc[t][c], 0, 0, 0);
-            }
+        for (int c = 0; c < 2; c++) {
+            asm volatile("" : "+v"(d[c]));  // (converted once: v_fma_mix runs at half the rate of v_fma)
+            nbd[c] = -kFoldBias * d[c];
         }
 
-        if (PARTIALS) {
-            const int strip = strip0 + strip_l;
-            if (strip < Ng) {
+        v4i acc[2][2][2];  // [pair][tile][c]
+        float4 x[2][2];
+        auto mma = [&](int p) {
 #pragma unroll
-                for (int t = 0; t < RT; t++)
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int c = 0; c < 2; c++)
+                        acc[p & 1][i][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[p & 1][i][h], b[h][c], h == 0 ? bias : acc[p & 1][i][c], 0, 0, 0);
+        };
+        auto fold = [&](int p) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int t = 2 * p + i;
+                if (PARTIALS) {
+                    const int strip = strip0 + wave;
 #pragma unroll
                     for (int v = 0; v < 4; v++) {
-                        const int row = row0 + wr * (BM / 2) + t * 16 + g * 4 + v;
-                        if (row < rows) {
+                        const int row = row0 + t * 16 + g * 4 + v;
+                        if (strip >= Ng || row >= rows) continue;
 #pragma unroll
-                            for (int c = 0; c < 4; c++)
-                                out_i[((int64_t)row * ((int64_t)Ng * kGroupN) + strip * kGroupN + q * 4 + c) * Kg + kb] =
-                                    acc[t][c][v];
-                        }
+                        for (int c = 0; c < 2; c++)
+                            out_i[((int64_t)row * ((int64_t)Ng * kGroupN) + strip * kGroupN + 2 * jj + c) * Kg + kb] = acc[p & 1][i][c][v];
                     }
-            }
-        } else {
-            const uint2 dh = *reinterpret_cast<const uint2*>(bblk + 2048 + q * 8);
-            const uint2 mh = *reinterpret_cast<const uint2*>(bblk + 2048 + 64 + q * 8);
-            float d[4], m[4];
-            d[0] = f16_bits_to_f32((uint16_t)(dh.x & 0xFFFFu));
-            d[1] = f16_bits_to_f32((uint16_t)(dh.x >> 16));
-            d[2] = f16_bits_to_f32((uint16_t)(dh.y & 0xFFFFu));
-            d[3] = f16_bits_to_f32((uint16_t)(dh.y >> 16));
-            m[0] = f16_bits_to_f32((uint16_t)(mh.x & 0xFFFFu));
-            m[1] = f16_bits_to_f32((uint16_t)(mh.x >> 16));
-            m[2] = f16_bits_to_f32((uint16_t)(mh.y & 0xFFFFu));
-            m[3] = f16_bits_to_f32((uint16_t)(mh.y >> 16));
-            const float nbd[4] = {-kFoldBias * d[0], -kFoldBias * d[1], -kFoldBias * d[2], -kFoldBias * d[3]};
-            const int slot4 = (kb - kb0) & 3;
-            const bool mine4 = slot4 == g;
-#pragma unroll
-            for (int c = 0; c < 4; c++) mk[c] = mine4 ? m[c] : mk[c];
-#pragma unroll
-            for (int t = 0; t < RT; t++) {
-                const float gsr = sm.xs[buf][wr * (BM / 2) + t * 16 + jj].y;
-                gk[t] = mine4 ? gsr : gk[t];
-                // dx of the 4 rows this lane holds results for: rows wr*BM/2 + t*16 + 4g + v
-                const float4* xp = reinterpret_cast<const float4*>(&sm.xs[buf][wr * (BM / 2) + t * 16 + g * 4]);
-                const float4 x01 = xp[0], x23 = xp[1];
-                const float dxv[4] = {x01.x, x01.z, x23.x, x23.z};
+                    continue;
+                }
+                const float dxv[4] = {x[p & 1][i].x, x[p & 1][i].y, x[p & 1][i].z, x[p & 1][i].w};
 #pragma unroll
                 for (int v = 0; v < 4; v++)
 #pragma unroll
-                    for (int c = 0; c < 4; c++)
-                        f[t][c][v] = fmaf(fmaf(__int_as_float(acc[t][c][v]), d[c], nbd[c]), dxv[v], f[t][c][v]);
+                    for (int c = 0; c < 2; c++)
+                        f[t][c][v] = fmaf(fmaf(__int_as_float(acc[p & 1][i][c][v]), d[c], nbd[c]), dxv[v], f[t][c][v]);
+                // (register arithmetic, which the compiler would gather behind the last product)
+                asm volatile("" : "+v"(f[t][0]), "+v"(f[t][1]));
             }
-            if (slot4 == 3 || kb + 1 == kb1) {
+        };
 #pragma unroll
-                for (int t = 0; t < RT; t++) {
+        for (int p = 0; p < P; p++) {
+            if (p + 1 < P) load_a(st, p + 1);
+            if (!PARTIALS) {
+                // dx of the 4 rows this lane holds results for: rows 16t + 4g + v
 #pragma unroll
-                    for (int c = 0; c < 4; c++) f[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(gk[t], mk[c], f[t][c], 0, 0, 0);
-                    gk[t] = 0.0f;
-                }
-#pragma unroll
-                for (int c = 0; c < 4; c++) mk[c] = 0.0f;
+                for (int i = 0; i < 2; i++) x[p & 1][i] = *reinterpret_cast<const float4*>(&st.dx[(2 * p + i) * 16 + g * 4]);
+            }
+            mma(p);
+            __builtin_amdgcn_sched_barrier(0);
+            if (p == P - 1) load_first(sm.st[slot]);  // (past the last k-group: what the slot still holds, unused)
+            if (p > 0) {
+                fold(p - 1);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-
-        if (kb + 1 < kb1) LLMOPS_STASH(buf ^ 1);
-        __syncthreads();
+        fold(P - 1);
+        if (!PARTIALS && (since == 3 || kb + 1 == kb1)) {
+            // Min term sum_kb m[n,kb]*gsum[row,kb]: a rank-Kg product, done four k-groups at a time straight into the fp32
+            // accumulators; lane (jj, g) has gsum of row jj and m of its columns for the group with index g of the four.
+            // gsum = three and m = two bf16 pieces, exactly and at any scale (as in fc_gemm_g32_kernel); the six products of a
+            // k-group fit into the eight slots that a lane has in v_mfma_f32_16x16x32_bf16.  An infinity has no pieces: it is
+            // in the first product alone, zeros stand for it in the others.
+            int mine = ring - since + g;
+            mine += mine < 0 ? kMinRing : 0;
+            const bool live = g <= since;
+            const uint32_t mh = *reinterpret_cast<const uint32_t*>(&sm.m[live ? mine : 0][wave * 32 + jj * 2]);
+            const float* gsr = &sm.gs[live ? mine : 0][jj];
+            float gv[T];
+#pragma unroll
+            for (int t = 0; t < T; t++) gv[t] = gsr[t * 16];
+            __builtin_amdgcn_sched_barrier(0);
+            Bf16x8 mb[2];
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const float mv = live ? f16_bits_to_f32((uint16_t)(c == 0 ? mh & 0xFFFFu : mh >> 16)) : 0.0f;
+                const float mf = __builtin_isinf(mv) ? 0.0f : mv, m2 = mf - bf_piece(mf);
+                mb[c].u[0] = bf_pair(mv, mf), mb[c].u[1] = __float_as_uint(mf);
+                mb[c].u[2] = bf_pair(m2, m2), mb[c].u[3] = __float_as_uint(m2);
+            }
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                gv[t] = live ? gv[t] : 0.0f;
+                const float gf = __builtin_isinf(gv[t]) ? 0.0f : gv[t], g2 = gf - bf_piece(gf), g3 = g2 - bf_piece(g2);
+                Bf16x8 ga;
+                ga.u[0] = bf_pair(gv[t], g2), ga.u[2] = bf_pair(gf, g2), ga.u[1] = ga.u[3] = __float_as_uint(g3);
+#pragma unroll
+                for (int c = 0; c < 2; c++) f[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga.h, mb[c].h, f[t][c], 0, 0, 0);
+            }
+        }
+        since = since == 3 ? 0 : since + 1;
+        ring = ring == kMinRing - 1 ? 0 : ring + 1;
     }
-#undef LLMOPS_FETCH
-#undef LLMOPS_STASH
 
     if (PARTIALS) return;
-    const int strip = strip0 + strip_l;
+    const int strip = strip0 + wave;
     if (counters != nullptr) {
-        splitk_finish<RT, (RT == 4 ? 12 : (RT == 2 ? 6 : 4))>(f, out, split_stride, ldo, row0, min(BM, rows - row0), wr * (BM / 2), strip,
-                                                             Ng, q, g, rows, y_final, Ny, residual, &counters[by * nbx + bx], tid);
+        splitk_finish<T, (RT == 4 ? 12 : (RT == 2 ? 6 : 4))>(f, out, split_stride, ldo, row0, min(BM, rows - row0), strip, Ng, jj, g,
+                                                            rows, y_final, Ny, residual, &counters[by * nbx + bx], tid,
+                                                            reinterpret_cast<unsigned*>(smem_raw));
         return;
     }
     if (strip >= Ng) return;
     float* o = out + (int64_t)blockIdx.z * split_stride;
-    const int64_t n0 = (int64_t)strip * kGroupN + q * 4;
+    const int64_t n0 = (int64_t)strip * kGroupN + 2 * jj;
 #pragma unroll
-    for (int t = 0; t < RT; t++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int row = row0 + wr * (BM / 2) + t * 16 + g * 4 + v;
-            if (row >= rows) continue;
-            float* dst = o + (int64_t)row * ldo + n0;
-            // residual != nullptr only without split-K: then o is the result itself, row stride ldo
-            const float* res = residual ? residual + (int64_t)row * ldo + n0 : nullptr;
-            if (n0 + 3 < N && (ldo & 3) == 0) {
-                float4 val = make_float4(f[t][0][v], f[t][1][v], f[t][2][v], f[t][3][v]);
-                if (res) {
-                    const float4 r4 = *reinterpret_cast<const float4*>(res);
-                    val.x += r4.x, val.y += r4.y, val.z += r4.z, val.w += r4.w;
-                }
-                *reinterpret_cast<float4*>(dst) = val;
-            } else {
-#pragma unroll
-                for (int c = 0; c < 4; c++)
-                    if (n0 + c < N) dst[c] = res ? f[t][c][v] + res[c] : f[t][c][v];
-            }
-        }
-}
-
-// ---- two groups of wavefronts in alternating phases (group 128, many rows) -------------------------
-// Per k-group a wavefront has a matrix-core phase (operand reads, 32 int8 MFMAs) and a vector-ALU
-// phase (the fp32 fold: convert, scale product, fma per output element).  Two independent wavefronts
-// on one SIMD drift into the same phase and then simply take turns on the same pipe, so nothing
-// overlaps.  Here a workgroup has 8 wavefronts = two groups of 4, one of each per SIMD, and the phases
-// are separated by workgroup barriers with the second group started one phase late: while one group's
-// MFMAs run, the other group's fold has the vector ALU, by construction.  The vector ALU is the
-// scarcer unit (3 instructions per output element and k-group against 2 MFMAs per 256 elements), so
-// everything else is kept off it:
-//   tile: 256 rows x 128 columns; group p owns rows 128p..128p+127 (wave = 64 x 64, as in the kernel
-//   above); the weights of the tile are staged once and used by both groups.
-//   weights: fetched by group 0 (the one ahead in time) into registers one k-group ahead, unpacked
-//   ONCE per workgroup to int8 and stored to LDS in MFMA operand order ([strip][k half][column
-//   set c][g][q] -> 16 bytes), fp16 scales converted to fp32 on the way; a wave's B operands are
-//   then plain 16-byte LDS reads, no unpacking per wave.
-//   activations and their scales: asynchronous global->LDS copies (no registers, no LDS store
-//   instructions) for the next k-group, issued one at a time between the MFMAs of the matrix-core
-//   phase and waited for before the iteration's last barrier; each group copies its own rows.
-//   (All copies at the top of the phase measured ~500 cycles before the first MFMA: the four waves'
-//   copies queue up in the CU's address unit.)  Tile rows are 128 bytes with the
-//   16-byte chunk c of row r at chunk position c ^ key(r), key(r) = (r + ((r >> 3) & 1)) & 7: the 16
-//   rows that one ds_read_b128 touches then fall on 16 different 16-byte bank groups of the 256-byte
-//   bank line (and any aligned 8 of them on 8 different ones).  The copies land lane by lane, so the
-//   spreading is done by choosing what each lane fetches.  The unpacked weights of a strip take
-//   4096 + 128 bytes for the same reason (a read touches two strips).
-//   Group 1 still folds k-group kb-1 while group 0 overwrites that k-group's weight buffer, which is
-//   why the weight scales are taken into registers in the matrix-core phase.
-//   The A operands are read by hand-placed ds_read_b128 (four row tiles ahead of the MFMAs that use
-//   them) with hand-placed waits: the compiler would issue each read right before its use and leave
-//   the matrix cores waiting for LDS eight times per k-group.
-//   The fold is register arithmetic and the MFMAs have no side effects, so the compiler is free to
-//   move either across a barrier into the other phase (it did: the fold ended up next to the same
-//   group's MFMAs).  Empty asm statements that name the accumulators as operands pin them.
-//   The min term is not in the loop: the accumulators start at it (min_term_add above), formed from
-//   the [row][kg] group sums and the blocks' mins before the first k-group -- by group 0 while group 1
-//   unpacks the first k-group's weights, by group 1 in the phase it has to wait anyway.  In the loop
-//   it was 16 fp32 MFMAs per four k-groups and wave, each of which holds up the vector ALU of its SIMD
-//   for its 32 cycles (2048 rows: 11008 x 4096 187 -> 181 us, 4096 x 11008 164 -> 159 us).
-// Measured per k-group with the min term still in the loop (2048 x 11008 x 4096, cycles of the shader clock): matrix-core side ~1500
-// (operand reads 450, 32 MFMAs with the copies between them 1000), fold side ~1350-1900 (the fold
-// itself 1350: the vector ALU is shared with the other group's MFMA issue; unpacking the weights on
-// group 0 adds the wait for their fetch), barriers ~400; 4000 per k-group against ~4700 for the
-// four-wave kernel above.
-constexpr int kBuStrip = 2 * 4 * 4 * 8 * 16 + 128;
-struct GemmPPSmem {
-    static constexpr int BM = 256;
-    uint8_t a[2][BM * 128];
-    uint8_t bu[2][4 * kBuStrip];            // unpacked weights: [strip][h][c][g][q][16], strips padded
-    float d[2][4 * 32];                     // weight scale per strip column
-    float dx[2][BM];
-};
-
-// 16-byte LDS read whose result may only be used after lds_ready<N>() on it, N = number of LDS
-// operations issued after this one that may still be pending (LDS operations complete in order).
-// Between the two calls the variable must not be touched.
-// Between the two calls the variable must not be touched -- which the compiler cannot know, so this
-// pair is only for code that is known not to spill registers (the build of the kernel below that
-// writes int32 tiles does spill, and passes PLAIN = true to get an ordinary load instead).
-template <int OFF, bool PLAIN>
-__device__ __forceinline__ void lds_read16_issue(v4i& r, uint32_t addr) {
-    if (PLAIN) {
-        r = *reinterpret_cast<const __attribute__((address_space(3))) v4i*>((uintptr_t)(addr + OFF));
-    } else {
-        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(r) : "v"(addr), "n"(OFF) : "memory");
-    }
-}
-template <int N, bool PLAIN>
-__device__ __forceinline__ void lds_ready(v4i& r) {
-    if (!PLAIN) asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(r) : "n"(N) : "memory");
-}
-
-template <bool PARTIALS>
-__global__ __launch_bounds__(512, 2) void fc_gemm_pp_kernel(const uint8_t* __restrict__ weiq, const int8_t* __restrict__ xq,
-                                                             const float* __restrict__ xd, const float* __restrict__ gs,
-                                                             const float2* __restrict__ xsT, float* __restrict__ out,
-                                                             int32_t* __restrict__ out_i, int Ng, int Kg, int64_t ldo,
-                                                             int64_t N, int rows, int kb_per_split, int64_t split_stride,
-                                                             const float* __restrict__ residual) {
-    constexpr int RT = 4, BM = 256, GM = 128;
-    extern __shared__ __align__(16) uint8_t smem_raw[];
-    GemmPPSmem& sm = *reinterpret_cast<GemmPPSmem*>(smem_raw);
-
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int grp = wave >> 2, w4 = wave & 3;
-    const int wr = w4 >> 1, wc = w4 & 1;
-    const int g = lane >> 4, jj = lane & 15, q = jj & 7, sp = jj >> 3;
-    // tile numbering: one contiguous run of tiles per XCD, bands of 8 row blocks, rows fastest
-    const int nbx = (Ng + 3) / 4, nby = (rows + BM - 1) / BM;
-    int bx, by;
-    {
-        const int total = nbx * nby, per_xcd = (total + 7) / 8;
-        const int i = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-        if ((int)(blockIdx.x >> 3) >= per_xcd || i >= total) return;  // uniform for the workgroup
-        constexpr int kBand = 8;
-        const int band = i / (kBand * nbx), in_band = i % (kBand * nbx);
-        const int first = band * kBand, rows_in_band = min(kBand, nby - first);
-        by = first + in_band % rows_in_band;
-        bx = in_band / rows_in_band;
-    }
-    const int strip0 = bx * 4;
-    const int row0 = by * BM + grp * GM;  // first row of this group
-    const int kb0 = blockIdx.z * kb_per_split, kb1 = min(Kg, kb0 + kb_per_split);
-    const int64_t Kp = (int64_t)Kg * 128;
-
-    // ---- what this lane copies per k-group ----
-    // activations: wave w4 of a group copies its row blocks 4*w4 .. 4*w4+3 (8 rows x 128 bytes each)
-    // (all sources are a wave-uniform base pointer, which moves with the k-group, plus a 32-bit byte
-    // offset per lane; the host only launches this kernel when the tensors are below 2 GiB)
-    uint32_t aoff[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int r = (w4 * 4 + i) * 8 + (lane >> 3);  // row within the group (a multiple of 16 rows per group)
-        const int key = (r + ((r >> 3) & 1)) & 7;
-        aoff[i] = (uint32_t)(min(rows - 1, row0 + r) * (int)Kp + (((lane & 7) ^ key) * 16));
-    }
-    // activation scales: waves 0,1 of a group copy dx of rows 64*w4 + lane
-    const int xr = (w4 & 1) * 64 + lane;
-    const int64_t xrow = min(rows - 1, row0 + xr);
-    const uint8_t* xbase = nullptr;
-    uint32_t xoff = 0;
-    int64_t xstep = 0;  // bytes per k-group
-    if (!PARTIALS) {
-        if (xsT) {
-            xbase = reinterpret_cast<const uint8_t*>(xsT);
-            xoff = (uint32_t)(xrow * 8);
-            xstep = (int64_t)rows * 8;
-        } else {
-            xbase = reinterpret_cast<const uint8_t*>(xd);
-            xoff = (uint32_t)(xrow * Kg * 4);
-            xstep = 4;
-        }
-    }
-    const uint32_t lds_a = lds_off(&sm.a[0][0]);
-    const uint32_t lds_x = lds_off(&sm.dx[0][0]);
-#define LLMOPS_COPY_A(KB, BUF, I)                                                                                  \
-    copy16_to_lds(xq + (int64_t)(KB) * 128, aoff[I], lds_a + (BUF) * (BM * 128) + (grp * GM + (w4 * 4 + (I)) * 8) * 128)
-#define LLMOPS_COPY_X(KB, BUF)                                                                                     \
-    do {                                                                                                           \
-        if (!PARTIALS && w4 < 2) copy4_to_lds(xbase + (int64_t)(KB) * xstep, xoff, lds_x + (BUF) * (BM * 4) + (grp * GM + w4 * 64) * 4); \
-    } while (0)
-#define LLMOPS_COPY(KB, BUF)                                                                                       \
-    do {                                                                                                           \
-        _Pragma("unroll") for (int i = 0; i < 4; i++) LLMOPS_COPY_A(KB, BUF, i);                                   \
-        LLMOPS_COPY_X(KB, BUF);                                                                                    \
-    } while (0)
-
-    // weights (group 0; group 1 for the first k-group, while group 0 has the min term to compute): thread t
-    // of the group takes the 16-byte chunks t and t + 256 of the tile's 512 (chunk = strip (2 bits) | k8-row
-    // (4 bits) | column quad (3 bits)); its first 16 threads also the 16 chunks of fp16 scales d (strip
-    // (2 bits) | column octet (2 bits))
-    const int gtid = tid & 255;
-    uint32_t boff[2];
-    int bdst[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int ch = gtid + i * 256, st = ch >> 7, r = (ch >> 3) & 15, q4 = ch & 7;
-        boff[i] = (uint32_t)(min(Ng - 1, strip0 + st) * Kg * kBlk128 + r * 128 + q4 * 16);
-        // [strip][h = r>>3][c][g = (r&7)>>1][q4][8 * (r&1)]; c adds 512 bytes
-        bdst[i] = st * kBuStrip + ((((r >> 3) * 4) * 4 + ((r & 7) >> 1)) * 8 + q4) * 16 + (r & 1) * 8;
-    }
-    const int sst = (gtid >> 2) & 3, spart = gtid & 3;
-    const uint32_t soff = (uint32_t)(min(Ng - 1, strip0 + sst) * Kg * kBlk128 + 2048 + spart * 16);
-    v4u rb[2], rs = {0u, 0u, 0u, 0u};
-#define LLMOPS_FETCH_B(KB, WHO)                                                                            \
-    do {                                                                                                   \
-        if (grp == (WHO)) {                                                                                \
-            const uint8_t* wkb = weiq + (int64_t)(KB) * kBlk128;                                           \
-            rb[0] = *reinterpret_cast<const v4u*>(wkb + boff[0]);                                          \
-            rb[1] = *reinterpret_cast<const v4u*>(wkb + boff[1]);                                          \
-            if (gtid < 16) rs = *reinterpret_cast<const v4u*>(wkb + soff);                                 \
-        }                                                                                                  \
-    } while (0)
-#define LLMOPS_STASH_B(BUF, WHO)                                                                           \
-    do {                                                                                                   \
-        if (grp == (WHO)) {                                                                                \
-            _Pragma("unroll") for (int i = 0; i < 2; i++)                                                  \
-                _Pragma("unroll") for (int c = 0; c < 4; c++) {                                            \
-                    uint2 u;                                                                               \
-                    u.x = lo4(rb[i][c]);                                                                   \
-                    u.y = hi4(rb[i][c]);                                                                   \
-                    *reinterpret_cast<uint2*>(&sm.bu[BUF][bdst[i] + c * 512]) = u;                         \
-                }                                                                                          \
-            if (gtid < 16) {                                                                               \
-                float* dstf = sm.d[BUF] + sst * 32 + spart * 8;                                            \
-                float4 lo, hi;                                                                             \
-                lo.x = f16_bits_to_f32((uint16_t)(rs[0] & 0xFFFFu));                                       \
-                lo.y = f16_bits_to_f32((uint16_t)(rs[0] >> 16));                                           \
-                lo.z = f16_bits_to_f32((uint16_t)(rs[1] & 0xFFFFu));                                       \
-                lo.w = f16_bits_to_f32((uint16_t)(rs[1] >> 16));                                           \
-                hi.x = f16_bits_to_f32((uint16_t)(rs[2] & 0xFFFFu));                                       \
-                hi.y = f16_bits_to_f32((uint16_t)(rs[2] >> 16));                                           \
-                hi.z = f16_bits_to_f32((uint16_t)(rs[3] & 0xFFFFu));                                       \
-                hi.w = f16_bits_to_f32((uint16_t)(rs[3] >> 16));                                           \
-                *reinterpret_cast<float4*>(dstf) = lo;                                                     \
-                *reinterpret_cast<float4*>(dstf + 4) = hi;                                                 \
-            }                                                                                              \
-        }                                                                                                  \
-    } while (0)
-
-    v4f f[RT][4];
-    const int strip_l = wc * 2 + sp;          // strip (0..3) of the tile this lane's B operands come from
-    const int lrow = grp * GM + wr * 64;      // first tile row of this wave
-
-    // The accumulators start at the tile's min term (min_term_add).  Its operands are asked for ahead of the first
-    // k-group's; group 0 forms it while group 1 unpacks the first k-group's weights, group 1 in the phase it
-    // has to wait anyway (it runs one phase behind group 0).  A second and third round of 32 k-groups are
-    // fetched while the round before is being added.
-    MinTermRound<RT> mt;
-    int mroff[RT];
-#pragma unroll
-    for (int t = 0; t < RT; t++) mroff[t] = min(rows - 1, row0 + wr * 64 + t * 16 + jj) * Kg;
-    const int mstrip = min(Ng - 1, strip0 + strip_l);
-    if (kb0 < kb1) {
-        LLMOPS_COPY(kb0, 0);
-        LLMOPS_FETCH_B(kb0, 1);
-    }
-    __builtin_amdgcn_sched_barrier(0);  // the first k-group's operands are asked for first
-    if (!PARTIALS && kb0 < kb1) min_term_fetch<RT>(mt, gs, mroff, weiq, Kg, min(kb0 + 8 * g, Kg - 8), mstrip, q);
-#define LLMOPS_MIN_TERM()                                                                                  \
-    do {                                                                                                   \
-        if (!PARTIALS && kb0 < kb1) {                                                                      \
-            min_term_add<RT, true>(f, mt, min(kb0 + 8 * g, Kg - 8), kb0 + 8 * g, kb1);                     \
-            for (int k32 = kb0 + 32; k32 < kb1; k32 += 32) {                                               \
-                min_term_fetch<RT>(mt, gs, mroff, weiq, Kg, min(k32 + 8 * g, Kg - 8), mstrip, q);          \
-                min_term_add<RT, false>(f, mt, min(k32 + 8 * g, Kg - 8), k32 + 8 * g, kb1);                \
-            }                                                                                              \
-        } else {                                                                                           \
-            _Pragma("unroll") for (int t = 0; t < RT; t++)                                                 \
-                _Pragma("unroll") for (int c = 0; c < 4; c++) f[t][c] = v4f{0.f, 0.f, 0.f, 0.f};           \
-        }                                                                                                  \
-    } while (0)
-    // (s_waitcnt through the builtin, so that the compiler knows that no load of this prologue is pending in
-    // the k-group loop: left to its own bookkeeping it assumes that a further round may have been asked for and
-    // waits for "it" -- in fact for the k-group's asynchronous copies -- where the loop reuses the registers)
-    constexpr int kVmcnt0 = 0x0F70;  // vmcnt(0), the other counters left alone
-    if (grp == 1) {
-        if (kb0 < kb1) LLMOPS_STASH_B(0, 1);
-        __builtin_amdgcn_s_waitcnt(kVmcnt0);
-        __syncthreads();  // group 0 arrives here with its min term done ...
-    }
-    LLMOPS_MIN_TERM();
-    __builtin_amdgcn_s_waitcnt(kVmcnt0);
-    __syncthreads();  // ... by this one; for group 1 it is the barrier that puts it one phase behind group 0
-#undef LLMOPS_MIN_TERM
-    // A operand of row tile t, k half h: row lrow + 16t + jj, chunk 4h + g, swizzled by the row's low bits
-    const int akey = (jj + (jj >> 3)) & 7;
-    const uint32_t a_rd0 = lds_a + (lrow + jj) * 128 + (((0 + g) ^ akey) * 16);
-    const uint32_t a_rd1 = lds_a + (lrow + jj) * 128 + (((4 + g) ^ akey) * 16);
-    const int b_rd = strip_l * kBuStrip + (g * 8 + q) * 16;  // + (4h + c) * 512
-    for (int kb = kb0; kb < kb1; kb++) {
-        const int buf = (kb - kb0) & 1;
-        const bool more = kb + 1 < kb1;
-
-        // ---- matrix-core phase ----
-        // (the copies for the next k-group are issued between the MFMAs, one per four: four waves
-        // issuing all of theirs at once right after the barrier keep the address unit busy for
-        // several hundred cycles, during which none of them would reach its first MFMA)
-        const uint32_t ar0 = a_rd0 + buf * (BM * 128), ar1 = a_rd1 + buf * (BM * 128);
-        v4i a00, a01, a02, a03, a10, a11, a12, a13;
-        lds_read16_issue<0 * 2048, PARTIALS>(a00, ar0);
-        lds_read16_issue<1 * 2048, PARTIALS>(a01, ar0);
-        lds_read16_issue<2 * 2048, PARTIALS>(a02, ar0);
-        lds_read16_issue<3 * 2048, PARTIALS>(a03, ar0);
-        v4i b[2][4];
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-#pragma unroll
-            for (int c = 0; c < 4; c++) b[h][c] = *reinterpret_cast<const v4i*>(&sm.bu[buf][b_rd + (h * 4 + c) * 512]);
-        const float4 d4 = *reinterpret_cast<const float4*>(&sm.d[buf][strip_l * 32 + q * 4]);
-        v4i acc[RT][4];
-        // The int32 sums start at the bit pattern of 1.5 * 2^23: read as a float, bits + sum IS the number
-        // 1.5 * 2^23 + sum (|sum| <= 128 * 15 * 127 < 2^22), so the fold needs no convert instruction.
-        const v4i zero4 = PARTIALS ? v4i{0, 0, 0, 0} : v4i{kFoldBiasBits, kFoldBiasBits, kFoldBiasBits, kFoldBiasBits};
-#define LLMOPS_MMA4(T, H, A)                                                                              \
-    _Pragma("unroll") for (int c = 0; c < 4; c++)                                                         \
-        acc[T][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, b[H][c], (H) == 0 ? zero4 : acc[T][c], 0, 0, 0)
-        lds_ready<3, PARTIALS>(a00);
-        LLMOPS_MMA4(0, 0, a00);
-        lds_read16_issue<0 * 2048, PARTIALS>(a10, ar1);
-        if (more) LLMOPS_COPY_A(kb + 1, buf ^ 1, 0);
-        lds_ready<3, PARTIALS>(a01);
-        LLMOPS_MMA4(1, 0, a01);
-        lds_read16_issue<1 * 2048, PARTIALS>(a11, ar1);
-        if (more) LLMOPS_COPY_A(kb + 1, buf ^ 1, 1);
-        lds_ready<3, PARTIALS>(a02);
-        LLMOPS_MMA4(2, 0, a02);
-        lds_read16_issue<2 * 2048, PARTIALS>(a12, ar1);
-        if (more) LLMOPS_COPY_A(kb + 1, buf ^ 1, 2);
-        lds_ready<3, PARTIALS>(a03);
-        LLMOPS_MMA4(3, 0, a03);
-        lds_read16_issue<3 * 2048, PARTIALS>(a13, ar1);
-        if (more) LLMOPS_COPY_A(kb + 1, buf ^ 1, 3);
-        lds_ready<3, PARTIALS>(a10);
-        LLMOPS_MMA4(0, 1, a10);
-        if (more) LLMOPS_COPY_X(kb + 1, buf ^ 1);
-        lds_ready<2, PARTIALS>(a11);
-        LLMOPS_MMA4(1, 1, a11);
-        if (more) LLMOPS_FETCH_B(kb + 1, 0);
-        lds_ready<1, PARTIALS>(a12);
-        LLMOPS_MMA4(2, 1, a12);
-        lds_ready<0, PARTIALS>(a13);
-        LLMOPS_MMA4(3, 1, a13);
-#undef LLMOPS_MMA4
-        const float d[4] = {d4.x, d4.y, d4.z, d4.w};
-        const float nbd[4] = {-kFoldBias * d4.x, -kFoldBias * d4.y, -kFoldBias * d4.z, -kFoldBias * d4.w};
-        asm volatile("" : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[0][2]), "+v"(acc[0][3]), "+v"(acc[1][0]),
-                          "+v"(acc[1][1]), "+v"(acc[1][2]), "+v"(acc[1][3]), "+v"(acc[2][0]), "+v"(acc[2][1]),
-                          "+v"(acc[2][2]), "+v"(acc[2][3]), "+v"(acc[3][0]), "+v"(acc[3][1]), "+v"(acc[3][2]),
-                          "+v"(acc[3][3]));  // likewise: the MFMAs stay in the matrix-core phase
-        __syncthreads();
-
-        // ---- vector phase: fold the int32 tiles into the fp32 accumulators ----
-        if (PARTIALS) {
-            const int strip = strip0 + strip_l;
-            if (strip < Ng) {
-#pragma unroll
-                for (int t = 0; t < RT; t++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        const int row = row0 + wr * 64 + t * 16 + g * 4 + v;
-                        if (row < rows) {
-#pragma unroll
-                            for (int c = 0; c < 4; c++)
-                                out_i[((int64_t)row * ((int64_t)Ng * kGroupN) + strip * kGroupN + q * 4 + c) * Kg + kb] =
-                                    acc[t][c][v];
-                        }
-                    }
-            }
-        } else {
-#pragma unroll
-            for (int t = 0; t < RT; t++) {
-                // dx of the 4 rows this lane holds results for: rows lrow + t*16 + 4g + v
-                const float4 x4 = *reinterpret_cast<const float4*>(&sm.dx[buf][lrow + t * 16 + g * 4]);
-                const float dxv[4] = {x4.x, x4.y, x4.z, x4.w};
-                // sum * d in one fma: (bias + sum) * d - bias * d, exact before its single rounding because
-                // bias * d (2 significant bits times the 11 of an fp16) is a float; then one fma with dx
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-#pragma unroll
-                    for (int c = 0; c < 4; c++)
-                        f[t][c][v] = fmaf(fmaf(__int_as_float(acc[t][c][v]), d[c], nbd[c]), dxv[v], f[t][c][v]);
-            }
-        }
-        // the fold is register arithmetic, which the compiler may move across the barrier into the other
-        // phase; naming the accumulators as operands of an (empty) asm statement keeps it on this side
-        asm volatile("" : "+v"(f[0][0]), "+v"(f[0][1]), "+v"(f[0][2]), "+v"(f[0][3]), "+v"(f[1][0]), "+v"(f[1][1]),
-                          "+v"(f[1][2]), "+v"(f[1][3]), "+v"(f[2][0]), "+v"(f[2][1]), "+v"(f[2][2]), "+v"(f[2][3]),
-                          "+v"(f[3][0]), "+v"(f[3][1]), "+v"(f[3][2]), "+v"(f[3][3]));
-        if (kb + 1 < kb1) LLMOPS_STASH_B(buf ^ 1, 0);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies for the next k-group have landed
-        __syncthreads();
-    }
-    if (grp == 0) __syncthreads();  // pairs with group 1's last barrier
-#undef LLMOPS_COPY
-#undef LLMOPS_COPY_A
-#undef LLMOPS_COPY_X
-#undef LLMOPS_FETCH_B
-#undef LLMOPS_STASH_B
-
-    if (PARTIALS) return;
-    const int strip = strip0 + strip_l;
-    if (strip >= Ng) return;
-    float* o = out + (int64_t)blockIdx.z * split_stride;
-    const int64_t n0 = (int64_t)strip * kGroupN + q * 4;
-#pragma unroll
-    for (int t = 0; t < RT; t++)
+    for (int t = 0; t < T; t++)
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            const int row = row0 + wr * 64 + t * 16 + g * 4 + v;
+            const int row = row0 + t * 16 + g * 4 + v;
             if (row >= rows) continue;
-            float* dst = o + (int64_t)row * ldo + n0;
             // residual != nullptr only without split-K: then o is the result itself, row stride ldo
-            const float* res = residual ? residual + (int64_t)row * ldo + n0 : nullptr;
-            if (n0 + 3 < N && (ldo & 3) == 0) {
-                float4 val = make_float4(f[t][0][v], f[t][1][v], f[t][2][v], f[t][3][v]);
-                if (res) {
-                    const float4 r4 = *reinterpret_cast<const float4*>(res);
-                    val.x += r4.x, val.y += r4.y, val.z += r4.z, val.w += r4.w;
-                }
-                *reinterpret_cast<float4*>(dst) = val;
-            } else {
-#pragma unroll
-                for (int c = 0; c < 4; c++)
-                    if (n0 + c < N) dst[c] = res ? f[t][c][v] + res[c] : f[t][c][v];
-            }
+            store_pair(o + (int64_t)row * ldo + n0, residual ? residual + (int64_t)row * ldo + n0 : nullptr, f[t][0][v], f[t][1][v], n0, N, ldo);
         }
 }
 
@@ -921,154 +501,103 @@ int launch_gemm_g32(const uint8_t* w, const int8_t* xq, const float* xd, const f
 int launch_gemm_g32_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg, hipStream_t st);
 
 struct GemmPlan {
-    int RT, S, kb_per_split;  // group 32: RT = 1 (32-row tiles), kb_per_split in stages of four k-groups
+    int RT, S, kb_per_split;  // rows of a tile / 32; group 32: RT = 1 (32-row tiles), kb_per_split in stages of four k-groups
     bool lds;
 };
 
-static int g_gemm_pp_min_rows = 256;
-static int g_gemm_rt = 0;  // 0 = choose per shape; -1 = also keep 9..32 rows on the tiled kernel
+static int g_gemm_rt = 0;  // 0 = choose per shape; 1, 2, 4 (and 8, taken as 4) = that tile; -1 = also keep 9..32 rows on the tiled kernel
 static int g_gemm_fused_reduce = 1;  // split-K partial sums added by the product kernel itself (0: by a second launch)
 static int g_gemm_force_split = 0;   // > 0: the split-K factor to use whatever the estimate says (tests)
 bool gemm_rows_kernel_enabled() { return g_gemm_rt >= 0; }
 
-// Split-K factor for `tiles` output tiles on a machine with `slots` resident workgroups.
-static void gemm_split(int64_t tiles, int64_t slots, int64_t Kg, GemmPlan& p) {
-    int S = (int)((slots + tiles - 1) / tiles);
-    if (S > Kg) S = (int)Kg;
-    if (S < 1) S = 1;
-    p.kb_per_split = (int)((Kg + S - 1) / S);
-    p.S = (int)((Kg + p.kb_per_split - 1) / p.kb_per_split);
-}
-
-static GemmPlan plan_gemm(int64_t rows, int64_t Ng, int64_t Kg, int G) {
-    GemmPlan p;
-    p.lds = (G == 128);
-    if (!p.lds) {
-        p.RT = 1;
-        p.S = plan_gemm_g32(rows, Ng, Kg, g_gemm_force_split, &p.kb_per_split);
-        return p;
-    }
-    // Candidates: the 256-row kernel with two wave groups (one workgroup per CU) and the four-wave
-    // kernel with 128, 64 or 32 rows per workgroup (two, three, four workgroups per CU: bigger tiles
-    // reuse the unpacked weights over more rows but need more registers).  Measured rate per row at
-    // full occupancy (M = 2048): 1.17 : 1.0 : 0.98 : 0.77.  What decides between them at smaller M is
-    // how evenly the tiles fill the machine, so the plan takes the candidate and split-K factor with
-    // the least estimated time: rounds of resident workgroups x (rows per CU per round / efficiency)
-    // x share of K per split.  Split factors tried: the largest that still runs in one round and the
-    // smallest that fills the machine (a second round of half-length workgroups costs what one round
-    // of full-length ones does, plus the reduction of the partial sums).
-    // (the 256-row kernel's lanes address the tensors with 32-bit byte offsets)
-    const bool small = rows * Kg * 128 < ((int64_t)1 << 31) && Ng * Kg * 2176 < ((int64_t)1 << 31);
-    static const int kRT[4] = {8, 4, 2, 1};
-    static const int kRows[4] = {256, 128, 64, 32};
-    static const int kWgPerCu[4] = {1, 2, 3, 4};
-    static const double kEff[4] = {1.17, 1.0, 0.98, 0.77};
+// Row tile and split-K factor of the tiled kernel: the least estimated time (us) of 128, 64 or 32 rows x 1 .. 12 splits.  A
+// k-group of a resident round takes 1.2 / 0.95 / 0.81 us (two, three, four workgroups per compute unit), a workgroup
+// counts as its run plus 0.3 k-groups, and a round that is not full takes 1 / 0.54 / 0.85 of that plus the rest in
+// proportion; the last split of a tile to arrive adds the sums (1.7 us, 0.32 more per split and 32 rows, 0.42 us per million of them).
+// Fitted to every tile x {1 .. 8, 10, 11} splits at 17 row counts from 24 to 2048 of 4096^2, 11008 | 22016 x 4096, 4096 x 11008 and
+// 1500 x 2048: the choices are 1.4 % slower than the best measured one on average and 8 % at worst (11008 x 4096 at 64 rows: 5 splits,
+// 4 would be better), against 5 % and 65 % (1500 x 2048 at 384 rows) of the rule that counted whole rounds.
+// room: what partial sums may take (bytes).
+static void plan_gemm_tile(int64_t rows, int64_t Ng, int64_t Kg, int64_t room, GemmPlan& p) {
+    static const int kRT[3] = {4, 2, 1}, kSlots[3] = {512, 768, 1024};
+    static const double kGroupUs[3] = {1.2, 0.947, 0.811}, kPartRound[3] = {1.0, 0.541, 0.852};
+    const int force_rt = g_gemm_rt == 8 ? 4 : g_gemm_rt;
     double best = 0.0;
-    for (int i = 0; i < 4; i++) {
-        if (g_gemm_rt > 0 && kRT[i] != g_gemm_rt) continue;
-        if (kRT[i] == 8 && (!small || Kg < 8 || (g_gemm_rt != 8 && rows < g_gemm_pp_min_rows))) continue;
-        const int64_t bm = kRows[i], slots = 256 * kWgPerCu[i];
-        const int64_t tiles = ((Ng + 3) / 4) * ((rows + bm - 1) / bm);
-        const int64_t s_floor = slots / tiles, s_ceil = (slots + tiles - 1) / tiles;
-        // (a third candidate where the machine would take more: the most splits the product kernel still adds itself)
-        const int64_t s_cap = 12 * (int64_t)g_gemm_fused_reduce;
-        // Below the 256-row kernel's range a workgroup's run of k-groups is short and what a workgroup costs before
-        // and after it decides: every split factor the kernel can finish itself is tried, a workgroup counts as
-        // its run plus 3 k-groups, and a split as 2.0 * bm / Kg (measured: sweeps of every tiling x 1..12 splits at
-        // 24..256 rows on 4096^2, 11008|12288|22016 x 4096 and 4096 x 11008; the choices made this way are 1.4 %
-        // slower on average than the best measured one, against 5 % -- up to 27 % at 24..64 rows -- before).
-        const bool few_rows = rows < g_gemm_pp_min_rows && g_gemm_fused_reduce && kRT[i] != 8;
-        const int n_try = few_rows ? 12 : 3;
-        for (int it = 0; it < n_try; it++) {
-            const int64_t s_try = few_rows ? it + 1
-                                           : (it == 0 ? s_floor : (it == 1 ? s_ceil : ((s_cap > 0 && s_cap < s_floor && kRT[i] != 8) ? s_cap : s_floor)));
-            GemmPlan q = p;
-            q.RT = kRT[i];
-            int64_t S = s_try < 1 ? 1 : (s_try > Kg ? Kg : s_try);
-            if (g_gemm_force_split > 0) S = g_gemm_force_split > Kg ? Kg : g_gemm_force_split;
-            q.kb_per_split = (int)((Kg + S - 1) / S);
-            q.S = (int)((Kg + q.kb_per_split - 1) / q.kb_per_split);
-            const int64_t rounds = (tiles * q.S + slots - 1) / slots;
-            double cost = (double)rounds * (double)(bm * kWgPerCu[i]) / kEff[i] * (double)(q.kb_per_split + (few_rows ? 3 : 0)) / (double)Kg;
-            // Split-K is not free.  In the unit of this estimate (rows x share of K; about 0.014 us x Kg) the last
-            // split of a tile to arrive adds S tiles of bm rows at ~150 GB/s (0.24 * S * bm / Kg); a second launch
-            // over the partial sums costs 8-11 us whatever the shape (800 / Kg: the price at which the measured
-            // choices came out best; 4096x11008 at 40-64 rows 24-25.5 -> 21-21.8 us against 570 / Kg).
-            if (q.S > 1) {
-                const bool in_kernel = g_gemm_fused_reduce && q.S <= 12 * g_gemm_fused_reduce && kRT[i] != 8;
-                cost += in_kernel ? (few_rows ? 2.0 : 0.24) * (double)q.S * (double)bm / (double)Kg : 800.0 / (double)Kg;
-            }
-            if (best == 0.0 || cost < best) {
-                best = cost;
-                p = q;
+    for (int i = 0; i < 3; i++) {
+        if (force_rt > 0 && kRT[i] != force_rt) continue;
+        const int64_t bm = 32 * kRT[i], tiles = ((Ng + 3) / 4) * ((rows + bm - 1) / bm);
+        for (int64_t s = 1; s <= 12; s++) {
+            const int64_t want = g_gemm_force_split > 0 ? g_gemm_force_split : s;
+            const int64_t per = want >= Kg ? 1 : (Kg + want - 1) / want, S = (Kg + per - 1) / per;
+            if (S > 1 && g_gemm_force_split <= 0 && S * rows * Ng * kGroupN * 4 > room) continue;
+            const int64_t full = tiles * S / kSlots[i], rest = tiles * S % kSlots[i];
+            const double rounds = (double)full + (rest == 0 ? 0.0 : kPartRound[i] + (1.0 - kPartRound[i]) * (double)rest / kSlots[i]);
+            double t = kGroupUs[i] * ((double)per + 0.289) * rounds;
+            if (S > 1) t += 1.726 + 0.319 * (double)(S * kRT[i]) + 0.42e-6 * (double)(S * rows * Ng * kGroupN);
+            if (best == 0.0 || t < best) {
+                best = t;
+                p.RT = kRT[i], p.S = (int)S, p.kb_per_split = (int)per;
             }
         }
     }
-    if (best == 0.0) {  // a forced candidate that cannot run here: fall back to the 128-row kernel
-        p.RT = 4;
-        gemm_split(((Ng + 3) / 4) * ((rows + 127) / 128), 512, Kg, p);
+}
+
+static GemmPlan plan_gemm(int64_t rows, int64_t Ng, int64_t Kg, int G, int64_t room) {
+    GemmPlan p;
+    p.lds = (G == 128);
+    if (p.lds) {
+        plan_gemm_tile(rows, Ng, Kg, room, p);
+    } else {
+        p.RT = 1;
+        p.S = plan_gemm_g32(rows, Ng, Kg, g_gemm_force_split, &p.kb_per_split);
     }
     return p;
 }
 
-size_t gemm_workspace_bytes(int64_t rows, int64_t Ng, int64_t Kg, int G) {
-    const GemmPlan p = plan_gemm(rows, Ng, Kg, G);
+size_t gemm_workspace_bytes(int64_t rows, int64_t Ng, int64_t Kg, int G, int64_t room) {
+    const GemmPlan p = plan_gemm(rows, Ng, Kg, G, room);
     return p.S > 1 ? (size_t)p.S * rows * Ng * kGroupN * sizeof(float) : 0;
 }
 
-template <int RT>
-static int launch_gemm_lds_t(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, const float2* xsT,
-                             float* out, int64_t Ng, int64_t Kg, int64_t ldo, int64_t N, int64_t rows, const GemmPlan& p,
-                             int64_t split_stride, const float* residual, float* y_final, int64_t Ny, unsigned* counters,
-                             hipStream_t st) {
-    static bool configured = false;  // opt in to more than 64 KiB of dynamic LDS once per kernel
+// the kernel's launch needs more than 64 KiB of dynamic LDS: opted in to once per build of it
+template <int RT, bool PARTIALS>
+static int configure_gemm_tile() {
+    static bool configured = false;
     if (!configured) {
-        LLMOPS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&fc_gemm_lds_kernel<RT, false>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GemmSmem<RT>)));
+        LLMOPS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&fc_gemm_tile_kernel<RT, PARTIALS>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GemmTile<RT>)));
         configured = true;
     }
-    // (the kernel's staging loads take 32-bit offsets into the scale pairs [Kg][rows] and into a tile's rows)
+    return LLMOPS_OK;
+}
+
+template <int RT>
+static int launch_gemm_tile(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, const float2* xsT,
+                            float* out, int64_t Ng, int64_t Kg, int64_t ldo, int64_t N, int64_t rows, const GemmPlan& p,
+                            int64_t split_stride, const float* residual, float* y_final, int64_t Ny, unsigned* counters,
+                            hipStream_t st) {
+    const int bad = configure_gemm_tile<RT, false>();
+    if (bad) return bad;
+    // (the copies take 32-bit offsets into the scale pairs of a k-group and into a tile's rows and strips)
     if (rows * Kg * 8 >= ((int64_t)1 << 32) || Kg * 128 * 128 >= ((int64_t)1 << 32))
         return fail(LLMOPS_EINVAL, "fc_Q4A: rows * Kg must be below 2^29 for the tiled kernel");
     const int64_t tiles = ((Ng + 3) / 4) * ((rows + RT * 32 - 1) / (RT * 32));
     dim3 grid((unsigned)(8 * ((tiles + 7) / 8)), 1, (unsigned)p.S);  // one run of tiles per XCD
-    fc_gemm_lds_kernel<RT, false><<<grid, 256, sizeof(GemmSmem<RT>), st>>>(w, xq, xd, gs, xsT, out, nullptr, (int)Ng, (int)Kg,
-                                                                          ldo, N, (int)rows, p.kb_per_split, split_stride,
-                                                                          residual, y_final, Ny, counters);
+    fc_gemm_tile_kernel<RT, false><<<grid, 256, sizeof(GemmTile<RT>), st>>>(
+        w, xq, xd, gs, xsT, out, nullptr, (int)Ng, (int)Kg, ldo, N, (int)rows, p.kb_per_split, split_stride, residual, y_final, Ny, counters);
     return LLMOPS_OK;
 }
 
-static int launch_gemm_pp(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, const float2* xsT, float* out,
-                          int64_t Ng, int64_t Kg, int64_t ldo, int64_t N, int64_t rows, const GemmPlan& p,
-                          int64_t split_stride, const float* residual, hipStream_t st) {
-    static bool configured = false;
-    if (!configured) {
-        LLMOPS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&fc_gemm_pp_kernel<false>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GemmPPSmem)));
-        configured = true;
-    }
-    const int64_t tiles = ((Ng + 3) / 4) * ((rows + 255) / 256);
-    dim3 grid((unsigned)(8 * ((tiles + 7) / 8)), 1, (unsigned)p.S);
-    fc_gemm_pp_kernel<false><<<grid, 512, sizeof(GemmPPSmem), st>>>(w, xq, xd, gs, xsT, out, nullptr, (int)Ng, (int)Kg, ldo, N,
-                                                                   (int)rows, p.kb_per_split, split_stride, residual);
-    return LLMOPS_OK;
-}
-
-// y = product (+ residual, fp32 [rows, N], may be y itself)
+// y = product (+ residual, fp32 [rows, N], may be y itself); room: as gemm_workspace_bytes was asked with
 int launch_gemm(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, const float2* xsT, float* y,
                 float* part, unsigned* counters, int64_t rows, int64_t Ng, int64_t Kg, int G, int64_t N, const float* residual,
-                hipStream_t st) {
-    const GemmPlan p = plan_gemm(rows, Ng, Kg, G);
-    // With up to 12 splits the four-wave kernel adds the partial sums itself (the last split of a tile to arrive
-    // does), given one zeroed arrival counter per tile; otherwise a second launch adds them.  Measured (us, second
-    // launch / in kernel): 11008x4096 at 128 rows 29.3 / 25.7, at 256 rows 43.9 / 38.8; 4096x11008 at 384 rows
-    // 61.0 / 53.9, at 96 rows (11 splits) 28.6 / 24.6 - but at 128 rows (16 splits of a 128-row tile) 31.9 / 38.8:
-    // the one workgroup that adds 16 tiles takes longer than a launch that spreads them over the chip.  The
-    // 256-row kernel keeps the second launch: with one workgroup per CU nothing covers the last arrival's tail
-    // (4096x11008, 256 rows: 42.2 / 49.1; 512 rows: 66.1 / 70.4).
-    const int64_t lds_tiles = ((Ng + 3) / 4) * ((rows + p.RT * 32 - 1) / (p.RT * 32));
-    const bool fused_reduce = g_gemm_fused_reduce && p.S > 1 && p.lds && p.RT != 8 && counters != nullptr &&
-                              p.S <= 12 * g_gemm_fused_reduce && lds_tiles <= kTicketBytes / 4 && (int64_t)p.RT * 32 * Ng * kGroupN * 4 < ((int64_t)1 << 31);
+                int64_t room, hipStream_t st) {
+    const GemmPlan p = plan_gemm(rows, Ng, Kg, G, room);
+    // With up to 12 splits the tiled kernel adds the partial sums itself (the last split of a tile to arrive
+    // does), given one zeroed arrival counter per tile; otherwise a second launch adds them (8-11 us whatever the shape).
+    const int64_t tiles = ((Ng + 3) / 4) * ((rows + p.RT * 32 - 1) / (p.RT * 32));
+    const bool fused_reduce = g_gemm_fused_reduce && p.S > 1 && p.lds && counters != nullptr && p.S <= 12 * g_gemm_fused_reduce &&
+                              tiles <= kTicketBytes / 4;
     // the residual is added where the result is written: in the kernel's stores without split-K, in
     // the reduction of the partial sums with it
     const float* kres = (p.S > 1 && !fused_reduce) ? nullptr : residual;
@@ -1080,10 +609,9 @@ int launch_gemm(const uint8_t* w, const int8_t* xq, const float* xd, const float
     const int64_t ss = rows * Np;
     if (p.lds) {
         int rc;
-        if (p.RT == 8) rc = launch_gemm_pp(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, st);
-        else if (p.RT == 4) rc = launch_gemm_lds_t<4>(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, y, N, kcnt, st);
-        else if (p.RT == 2) rc = launch_gemm_lds_t<2>(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, y, N, kcnt, st);
-        else rc = launch_gemm_lds_t<1>(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, y, N, kcnt, st);
+        if (p.RT == 4) rc = launch_gemm_tile<4>(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, y, N, kcnt, st);
+        else if (p.RT == 2) rc = launch_gemm_tile<2>(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, y, N, kcnt, st);
+        else rc = launch_gemm_tile<1>(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, y, N, kcnt, st);
         if (rc) return rc;
     } else {
         const int rc = launch_gemm_g32(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p.kb_per_split, p.S, ss, kres, st);
@@ -1098,37 +626,25 @@ int launch_gemm(const uint8_t* w, const int8_t* xq, const float* xd, const float
     return LLMOPS_OK;
 }
 
-int launch_gemm_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg, int G,
-                         bool two_groups, hipStream_t st) {
-    if (G == 128 && two_groups) {
-        if (!(rows * Kg * 128 < ((int64_t)1 << 31) && Ng * Kg * 2176 < ((int64_t)1 << 31)))
-            return fail(LLMOPS_EINVAL, "the 256-row kernel addresses its operands with 32-bit offsets");
-        static bool configured = false;
-        if (!configured) {
-            LLMOPS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&fc_gemm_pp_kernel<true>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GemmPPSmem)));
-            configured = true;
-        }
-        const int64_t tiles = ((Ng + 3) / 4) * ((rows + 255) / 256);
-        dim3 grid((unsigned)(8 * ((tiles + 7) / 8)), 1, 1);
-        fc_gemm_pp_kernel<true><<<grid, 512, sizeof(GemmPPSmem), st>>>(w, xq, nullptr, nullptr, nullptr, nullptr, acc, (int)Ng,
-                                                                      (int)Kg, 0, 0, (int)rows, (int)Kg, 0, nullptr);
-    } else if (G == 128) {  // the production LDS-tiled loop, writing its int32 tiles instead of folding them
-        static bool configured = false;
-        if (!configured) {
-            LLMOPS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&fc_gemm_lds_kernel<2, true>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GemmSmem<2>)));
-            configured = true;
-        }
-        const int64_t tiles = ((Ng + 3) / 4) * ((rows + 63) / 64);
-        dim3 grid((unsigned)(8 * ((tiles + 7) / 8)), 1, 1);
-        fc_gemm_lds_kernel<2, true><<<grid, 256, sizeof(GemmSmem<2>), st>>>(w, xq, nullptr, nullptr, nullptr, nullptr, acc,
-                                                                          (int)Ng, (int)Kg, 0, 0, (int)rows, (int)Kg, 0, nullptr, nullptr, 0, nullptr);
-    } else {
-        return launch_gemm_g32_partials(w, xq, acc, rows, Ng, Kg, st);
-    }
+// the production loop, writing its int32 tiles instead of folding them
+template <int RT>
+static int launch_gemm_tile_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg, hipStream_t st) {
+    const int bad = configure_gemm_tile<RT, true>();
+    if (bad) return bad;
+    const int64_t tiles = ((Ng + 3) / 4) * ((rows + RT * 32 - 1) / (RT * 32));
+    fc_gemm_tile_kernel<RT, true><<<(unsigned)(8 * ((tiles + 7) / 8)), 256, sizeof(GemmTile<RT>), st>>>(
+        w, xq, nullptr, nullptr, nullptr, nullptr, acc, (int)Ng, (int)Kg, 0, 0, (int)rows, (int)Kg, 0, nullptr, nullptr, 0, nullptr);
     LLMOPS_LAUNCH_CHECK();
     return LLMOPS_OK;
+}
+
+int launch_gemm_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg, int G,
+                         bool rows128, hipStream_t st) {
+    if (G != 128) return launch_gemm_g32_partials(w, xq, acc, rows, Ng, Kg, st);
+    if (!rows128) return launch_gemm_tile_partials<2>(w, xq, acc, rows, Ng, Kg, st);
+    if (!(rows * Kg * 128 < ((int64_t)1 << 31) && Ng * Kg * 2176 < ((int64_t)1 << 31)))
+        return fail(LLMOPS_EINVAL, "fc_Q4A_partials with 128-row tiles: codes and weights must be below 2 GiB");
+    return launch_gemm_tile_partials<4>(w, xq, acc, rows, Ng, Kg, st);
 }
 
 }  // namespace llmops
@@ -1142,8 +658,9 @@ extern "C" void llmops_test_gemm_set_split(int splits) {
 extern "C" int llmops_test_gemm_plan(int64_t rows, int64_t Ng, int64_t Kg, int group_k, int* row_tile_factor, int* splits) {
     LLMOPS_TEST_HOOK();
     if (rows < 1 || Ng < 1 || Kg < 1 || (group_k != 32 && group_k != 128) || !row_tile_factor || !splits) return LLMOPS_EINVAL;
-    const llmops::GemmPlan p = llmops::plan_gemm(rows, Ng, Kg, group_k);
-    *row_tile_factor = p.RT;
+    const llmops::GemmPlan p = llmops::plan_gemm(rows, Ng, Kg, group_k, INT64_MAX);
+    // (128-row tiles that fill the chip unsplit, two to a compute unit, are reported as the 256 rows they cover there)
+    *row_tile_factor = p.RT == 4 && p.S == 1 && group_k == 128 && rows >= 256 && Kg >= 8 ? 8 : p.RT;
     *splits = p.S;
     return LLMOPS_OK;
 }

@@ -8,6 +8,7 @@ namespace llmops {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -17,6 +18,17 @@ union Halves8 {
     v8h h;
     uint32_t u[4];
 };
+
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+union Bf16x8 {
+    v8bf h;
+    uint32_t u[4];
+};
+// the first 8 significant bits of a float (what its upper half is as a bf16), and the upper halves of two floats
+__device__ __forceinline__ float bf_piece(float v) { return __uint_as_float(__float_as_uint(v) & 0xFFFF0000u); }
+__device__ __forceinline__ uint32_t bf_pair(float lo, float hi) {
+    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
 
 constexpr int kFoldBiasBits = 0x4B400000;  // the float 1.5 * 2^23 ...
 constexpr float kFoldBias = 12582912.0f;   // ... whose low mantissa bits count in units of 1
@@ -35,8 +47,8 @@ __device__ __forceinline__ const void* uniform_ptr(const void* p) {
     return reinterpret_cast<const void*>(((uint64_t)hi << 32) | lo);
 }
 // lane i's 16 (4) bytes at base + off (base the same for the whole wave, off a byte offset per lane)
-// land at lds_base + 16*i (4*i); counts in vmcnt like any load.  (uniform_u32 belongs to the caller whose lds_base the
-// compiler does not see to be uniform: here it cost the 256-row kernel 0.6 %)
+// land at lds_base + 16*i (4*i); counts in vmcnt like any load.  (uniform_u32 belongs to the callers whose lds_base the
+// compiler does not see to be uniform)
 __device__ __forceinline__ void copy16_to_lds(const void* base, uint32_t off, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(lds_base) : "memory", "m0");
 }
