@@ -5,9 +5,11 @@
 // decode kernel's: one workgroup per strip of 32 output columns, its 8 or 16 waves split K into
 // contiguous runs of k-groups, every wave reads each packed weight byte once, and the waves'
 // fp32 results meet in LDS.  Nothing is staged through LDS on the way in: a lane fetches exactly
-// the two dwords per (64-k half, 16-column tile) that make up its B operand of
-// v_mfma_i32_16x16x64_i8 (dword (k8-row r, column n) of a block holds k = 8r..8r+7 of that
-// column; lane (g, j) of the MFMA needs k = 16g..16g+15 of column j), unpacks them with two ANDs
+// the dwords that make up its B operands of v_mfma_i32_16x16x64_i8 (dword (k8-row r, column n) of a
+// block holds k = 8r..8r+7 of that column; lane (g, j) of the MFMA needs k = 16g..16g+15 of one column), those of columns
+// 2j and 2j + 1 together in one 8-byte load per k8-row -- column tile tau of a strip is its columns 2j + tau, whose scales
+// and mins are the two halves of one dword (a k-group takes 10 loads per lane instead of the 16 that columns j and j + 16
+// took: 16 x 11008 x 4096 14.4 -> 13.7 us for the whole call) --, unpacks them with two ANDs
 // and a shift, and takes its A operand (16 int8 codes of one activation row) straight from the
 // quantized activations in L2.  Per k-group and output element the fp32 fold is the reference's
 // (ops/op_fc.hpp:381-412): f = fma(d*dx, float(acc), f); f = fma(m, gsum, f).
@@ -21,14 +23,15 @@ namespace llmops {
 
 typedef int v4i_r __attribute__((ext_vector_type(4)));
 typedef float v4f_r __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2_r __attribute__((ext_vector_type(2)));
 
 static int g_rows_split = 1;  // 0: never cut K in two for tensors with few strips
 constexpr int kRowsBlk = 2176;
 
 template <int RT>
 struct RowsStage {
-    uint32_t w[2][2][2];  // [64-k half][16-column tile][k8-row of the pair]
-    uint32_t d[2], m[2];  // the dword that holds the fp16 scale / min of the lane's column in either tile
+    u32x2_r w[2][2];      // [64-k half][k8-row of the pair], the lane's column in either tile
+    uint32_t d, m;        // the dword that holds the fp16 scales / mins of the lane's two columns
     v4i_r a[RT][2];       // activation codes: row tile, 64-k half
     float2 xs[RT][4];     // (dx, gsum) of the 4 rows this lane holds results for
 };
@@ -55,15 +58,9 @@ __device__ __forceinline__ void rows_load(RowsStage<RT>& st, const RowsBufs& bf,
 #pragma unroll
     for (int h = 0; h < 2; h++)
 #pragma unroll
-        for (int tau = 0; tau < 2; tau++)
-#pragma unroll
-            for (int p = 0; p < 2; p++)
-                st.w[h][tau][p] = __builtin_amdgcn_raw_buffer_load_b32(rw, lw, sw + (uint32_t)((8 * h + p) * kRowBytes + 64 * tau), 2);
-#pragma unroll
-    for (int tau = 0; tau < 2; tau++) {
-        st.d[tau] = __builtin_amdgcn_raw_buffer_load_b32(rw, ls, sw + 2048u + 32u * tau, 0);
-        st.m[tau] = __builtin_amdgcn_raw_buffer_load_b32(rw, ls, sw + 2048u + 64u + 32u * tau, 0);
-    }
+        for (int p = 0; p < 2; p++) st.w[h][p] = __builtin_amdgcn_raw_buffer_load_b64(rw, lw, sw + (uint32_t)((8 * h + p) * kRowBytes), 2);
+    st.d = __builtin_amdgcn_raw_buffer_load_b32(rw, ls, sw + 2048u, 0);
+    st.m = __builtin_amdgcn_raw_buffer_load_b32(rw, ls, sw + 2048u + 64u, 0);
 #pragma unroll
     for (int t = 0; t < RT; t++) {
         const uint32_t la = bf.lane_a[t];
@@ -86,7 +83,7 @@ __device__ __forceinline__ void rows_load(RowsStage<RT>& st, const RowsBufs& bf,
 
 // DUMP: test build that stores the int32 sums of every (row, column, k-group) into `dump`
 // ([rows][Ng*32][Kg]) instead of the outputs (llmops_fc_Q4A_partials with use_mfma = 3).
-template <int RT, int NW, bool DUMP = false>
+template <int RT, int NW, int D, bool DUMP = false>
 __global__ __launch_bounds__(NW * 64, RT == 2 ? 3 : 4) void fc_rows_mfma_kernel(const uint8_t* __restrict__ weiq,
                                                                          const int8_t* __restrict__ xq,
                                                                          const float2* __restrict__ xsT,
@@ -96,7 +93,7 @@ __global__ __launch_bounds__(NW * 64, RT == 2 ? 3 : 4) void fc_rows_mfma_kernel(
                                                                          int32_t* dump = nullptr) {
     // (argument order: what the first loads need comes in the first 14 dwords, which arrive in scalar registers
     // with the wave)
-    __shared__ float red[DUMP ? 1 : NW][16 * RT][kGroupN];
+    __shared__ __align__(8) float red[DUMP ? 1 : NW][16 * RT][kGroupN];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: block offsets stay scalar
     const int g = lane >> 4, jj = lane & 15;
@@ -118,28 +115,26 @@ __global__ __launch_bounds__(NW * 64, RT == 2 ? 3 : 4) void fc_rows_mfma_kernel(
     bf.w_base = strip, bf.w_bytes = (uint32_t)Kg * (uint32_t)kRowsBlk;
     bf.xq_base = xq, bf.xq_bytes = (uint32_t)rows * (uint32_t)Kp;
     bf.xs_base = xsT, bf.xs_bytes = DUMP ? 0u : (uint32_t)Kg * (uint32_t)rows * 8u;
-    bf.lane_w = (uint32_t)(2 * g * kRowBytes + jj * 4);
-    bf.lane_s = (uint32_t)((jj >> 1) * 4);  // the dword with this column's fp16 scale; half_sh picks the half
-    const int half_sh = (jj & 1) * 16;
+    bf.lane_w = (uint32_t)(2 * g * kRowBytes + jj * 8);
+    bf.lane_s = (uint32_t)(jj * 4);
 #pragma unroll
     for (int t = 0; t < RT; t++) {
         bf.lane_a[t] = (uint32_t)min(rows - 1, 16 * t + jj) * (uint32_t)Kp + 16u * g;
         bf.lane_x[t] = (uint32_t)(16 * t + 4 * g) * 8u;
     }
 
-    // Two stages used alternately (no register copies: a copy would have to wait for the loads it copies):
-    // the k-group being multiplied waits for exactly its own loads while the next one's are in flight.
+    // (loads complete in issue order: the k-group being multiplied waits for exactly its own while the next ones' are in flight)
 #define LLMOPS_ROWS_COMPUTE(ST, KB)                                                                          \
     do {                                                                                                     \
         v4i_r b[2][2];                                                                                       \
         _Pragma("unroll") for (int h = 0; h < 2; h++) _Pragma("unroll") for (int tau = 0; tau < 2; tau++) {  \
-            const uint32_t pa = ST.w[h][tau][0], pb = ST.w[h][tau][1];                                       \
+            const uint32_t pa = ST.w[h][0][tau], pb = ST.w[h][1][tau];                                       \
             b[h][tau] = v4i_r{(int)(pa & 0x0F0F0F0Fu), (int)((pa >> 4) & 0x0F0F0F0Fu), (int)(pb & 0x0F0F0F0Fu), \
                               (int)((pb >> 4) & 0x0F0F0F0Fu)};                                               \
         }                                                                                                    \
         _Pragma("unroll") for (int tau = 0; tau < 2; tau++) {                                                \
-            const float d = f16_bits_to_f32((uint16_t)(ST.d[tau] >> half_sh));                               \
-            const float m = f16_bits_to_f32((uint16_t)(ST.m[tau] >> half_sh));                               \
+            const float d = f16_bits_to_f32((uint16_t)(ST.d >> (16 * tau)));                               \
+            const float m = f16_bits_to_f32((uint16_t)(ST.m >> (16 * tau)));                               \
             _Pragma("unroll") for (int t = 0; t < RT; t++) {                                                 \
                 v4i_r acc = v4i_r{0, 0, 0, 0};                                                               \
                 acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(ST.a[t][0], b[0][tau], acc, 0, 0, 0);            \
@@ -149,7 +144,7 @@ __global__ __launch_bounds__(NW * 64, RT == 2 ? 3 : 4) void fc_rows_mfma_kernel(
                     _Pragma("unroll") for (int v = 0; v < 4; v++) {                                          \
                         const int row_ = 16 * t + 4 * g + v;                                                 \
                         if (row_ < rows && (KB) < t1)                                                        \
-                            dump[((int64_t)row_ * Np_ + nb * kGroupN + 16 * tau + jj) * Kg + (KB)] = acc[v]; \
+                            dump[((int64_t)row_ * Np_ + nb * kGroupN + 2 * jj + tau) * Kg + (KB)] = acc[v]; \
                     }                                                                                        \
                 }                                                                                            \
                 _Pragma("unroll") for (int v = 0; v < 4; v++) {                                              \
@@ -159,30 +154,23 @@ __global__ __launch_bounds__(NW * 64, RT == 2 ? 3 : 4) void fc_rows_mfma_kernel(
             }                                                                                                \
         }                                                                                                    \
     } while (0)
-    // Four k-groups per pass, two stages in flight, nothing loaded is live across the loop's back edge (a
-    // value that is would be copied there by the register allocator, and the copy waits for its load).  A
-    // hidden size of 4096 gives a wave exactly one pass; longer runs start each pass with a fresh pair.
-    RowsStage<RT> sa, sb;
-    for (int kb = t0; kb < t1; kb += 4) {
-        rows_load<RT>(sa, bf, kb, rows, true);
-        rows_load<RT>(sb, bf, kb + 1, rows, kb + 1 < t1);
-        __builtin_amdgcn_sched_barrier(0);
-        LLMOPS_ROWS_COMPUTE(sa, kb);
-        __builtin_amdgcn_sched_barrier(0);
-        rows_load<RT>(sa, bf, kb + 2, rows, kb + 2 < t1);
-        __builtin_amdgcn_sched_barrier(0);
-        LLMOPS_ROWS_COMPUTE(sb, kb + 1);  // (a stage that was not wanted holds zeros and adds nothing)
-        __builtin_amdgcn_sched_barrier(0);
-        rows_load<RT>(sb, bf, kb + 3, rows, kb + 3 < t1);
-        __builtin_amdgcn_sched_barrier(0);
-        // (the loads above are issued whatever the run's length; only the arithmetic on zeros is skipped)
-        if (kb + 2 < t1) {
-            LLMOPS_ROWS_COMPUTE(sa, kb + 2);
+    // D k-groups per pass, all of them in flight together: with one row tile what a wave has of K where that is 2, 3 or (8
+    // waves) 4, so that it waits for memory once; 2 for longer runs and with two row tiles, which leaves registers for more
+    // waves.  Nothing loaded is live across the loop's back edge (a value that is would be copied there by the register
+    // allocator, and the copy waits for its load).
+    // Measured, us for the whole call, four k-groups per pass with two in flight / now: 16 rows 4096^2 8.9 / 8.4, 11008 x 4096
+    // 14.4 / 13.4, 22016 x 4096 19.3 / 17.8, 4096 x 11008 14.2 / 13.3, 11008^2 32.4 / 28.3 (four in flight: 33.0); 20 x 7000 x 4096
+    // 15.2 / 12.2, 32 x 4096^2 10.7 / 10.2.
+    RowsStage<RT> st[D];
+    for (int kb = t0; kb < t1; kb += D) {
+#pragma unroll
+        for (int i = 0; i < D; i++) rows_load<RT>(st[i], bf, kb + i, rows, kb + i < t1);
+#pragma unroll
+        for (int i = 0; i < D; i++) {
+            __builtin_amdgcn_sched_barrier(0);
+            LLMOPS_ROWS_COMPUTE(st[i], kb + i);  // (a stage that was not wanted holds zeros and adds nothing)
         }
         __builtin_amdgcn_sched_barrier(0);
-        if (kb + 3 < t1) {
-            LLMOPS_ROWS_COMPUTE(sb, kb + 3);
-        }
     }
 #undef LLMOPS_ROWS_COMPUTE
     if constexpr (DUMP) return;
@@ -191,9 +179,7 @@ __global__ __launch_bounds__(NW * 64, RT == 2 ? 3 : 4) void fc_rows_mfma_kernel(
 #pragma unroll
     for (int t = 0; t < RT; t++)
 #pragma unroll
-        for (int tau = 0; tau < 2; tau++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) red[wave][16 * t + 4 * g + v][16 * tau + jj] = f[t][tau][v];
+        for (int v = 0; v < 4; v++) *reinterpret_cast<float2*>(&red[wave][16 * t + 4 * g + v][2 * jj]) = make_float2(f[t][0][v], f[t][1][v]);
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < RT; i++) {
@@ -220,6 +206,19 @@ __global__ __launch_bounds__(NW * 64, RT == 2 ? 3 : 4) void fc_rows_mfma_kernel(
     }
 }
 
+// the build of the kernel for `rows` rows and k_per_wg k-groups per workgroup
+#define LLMOPS_ROWS_LAUNCH(DUMP, ...)                                                                                   \
+    do {                                                                                                                \
+        const bool wide = k_per_wg > 32;                                                                                \
+        const int64_t per_wave = (k_per_wg + (wide ? 15 : 7)) / (wide ? 16 : 8);                                        \
+        if (rows > 16) fc_rows_mfma_kernel<2, 8, 2, DUMP><<<grid, 512, 0, st>>>(__VA_ARGS__);                           \
+        else if (wide && per_wave <= 3) fc_rows_mfma_kernel<1, 16, 3, DUMP><<<grid, 1024, 0, st>>>(__VA_ARGS__);        \
+        else if (wide) fc_rows_mfma_kernel<1, 16, 2, DUMP><<<grid, 1024, 0, st>>>(__VA_ARGS__);                         \
+        else if (per_wave <= 2) fc_rows_mfma_kernel<1, 8, 2, DUMP><<<grid, 512, 0, st>>>(__VA_ARGS__);                  \
+        else if (per_wave <= 3) fc_rows_mfma_kernel<1, 8, 3, DUMP><<<grid, 512, 0, st>>>(__VA_ARGS__);                  \
+        else fc_rows_mfma_kernel<1, 8, 4, DUMP><<<grid, 512, 0, st>>>(__VA_ARGS__);                                     \
+    } while (0)
+
 // rows <= 32 (two row tiles per wave from 17 on), group 128, activations already quantized (codes [rows, Kg*128], pairs [Kg][rows])
 // `slots`: the zeroed exchange area of the FC workspace (`slot_bytes` of it), or nullptr
 int launch_fc_rows(const uint8_t* w, const int8_t* xq, const float2* xsT, float* y, int64_t rows, int64_t Ng, int64_t Kg,
@@ -234,12 +233,7 @@ int launch_fc_rows(const uint8_t* w, const int8_t* xq, const float2* xsT, float*
     // 13.3 against 13.8 us; with 32 k-groups 16 waves are slower, 15.7 against 14.1 us at 11008x4096).
     // 17..32 rows: two row tiles per wave, 8 waves (16 would not have the registers).
     const int64_t k_per_wg = split ? (Kg + 1) / 2 : Kg;
-    if (rows > 16)
-        fc_rows_mfma_kernel<2, 8><<<grid, 512, 0, st>>>(w, xq, xsT, sl, (int)Kg, (int)rows, N, y, residual);
-    else if (k_per_wg > 32)
-        fc_rows_mfma_kernel<1, 16><<<grid, 1024, 0, st>>>(w, xq, xsT, sl, (int)Kg, (int)rows, N, y, residual);
-    else
-        fc_rows_mfma_kernel<1, 8><<<grid, 512, 0, st>>>(w, xq, xsT, sl, (int)Kg, (int)rows, N, y, residual);
+    LLMOPS_ROWS_LAUNCH(false, w, xq, xsT, sl, (int)Kg, (int)rows, N, y, residual);
     LLMOPS_LAUNCH_CHECK();
     return LLMOPS_OK;
 }
@@ -253,12 +247,7 @@ int launch_fc_rows_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, in
     // only tested against nullptr in the dump build, never dereferenced
     unsigned long long* sl = split ? reinterpret_cast<unsigned long long*>(acc) : nullptr;
     const int64_t k_per_wg = split ? (Kg + 1) / 2 : Kg;
-    if (rows > 16)
-        fc_rows_mfma_kernel<2, 8, true><<<grid, 512, 0, st>>>(w, xq, nullptr, sl, (int)Kg, (int)rows, 0, nullptr, nullptr, acc);
-    else if (k_per_wg > 32)
-        fc_rows_mfma_kernel<1, 16, true><<<grid, 1024, 0, st>>>(w, xq, nullptr, sl, (int)Kg, (int)rows, 0, nullptr, nullptr, acc);
-    else
-        fc_rows_mfma_kernel<1, 8, true><<<grid, 512, 0, st>>>(w, xq, nullptr, sl, (int)Kg, (int)rows, 0, nullptr, nullptr, acc);
+    LLMOPS_ROWS_LAUNCH(true, w, xq, nullptr, sl, (int)Kg, (int)rows, 0, nullptr, nullptr, acc);
     LLMOPS_LAUNCH_CHECK();
     return LLMOPS_OK;
 }
