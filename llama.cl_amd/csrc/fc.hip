@@ -11,7 +11,7 @@ constexpr int kMaxGemvRows = 8;
 int launch_quant_x(const float* x, int64_t rows, int64_t K, int group_k, int8_t* xq, float* xd, float* gsum, float2* xsT,
                    bool exact_sum, hipStream_t stream);
 int launch_quant_x_fused(const float* x, int64_t rows, int64_t K, int group_k, const float* norm_w, float eps, bool glu_in,
-                         int8_t* xq, float* xd, float* gsum, float2* xsT, hipStream_t stream);
+                         int8_t* xq, float2* xsT, hipStream_t stream);
 int launch_strip_sumsq(const float* y, int64_t rows, int64_t N, float* out, hipStream_t st);
 size_t gemv_workspace_bytes(int64_t rows, int64_t Ng, int64_t Kg, int G);
 int launch_gemv(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, float* y, float* part,
@@ -222,7 +222,7 @@ static int fc_decode_impl(const float* x, int64_t rows, int64_t K, const int8_t*
         float* gs = reinterpret_cast<float*>(ws + lay.off_gs);
         float2* xst = reinterpret_cast<float2*>(ws + lay.off_xst);
         int rc = (norm_w != nullptr || glu == 2)
-                     ? launch_quant_x_fused(x, rows, K, group_k, norm_w, eps, glu == 2, xq, xd, gs, xst, st)
+                     ? launch_quant_x_fused(x, rows, K, group_k, norm_w, eps, glu == 2, xq, xst, st)
                      : launch_quant_x(x, rows, K, group_k, xq, xd, gs, xst, false, st);
         if (rc) return rc;
         if (out_parts > 1) {

@@ -124,9 +124,12 @@ __global__ __launch_bounds__(256) void quant_x_rows_kernel(const float* __restri
         if (item < items) {
             *reinterpret_cast<uint32_t*>(xq + item * G + sub * 4) = c;
             if (sub == 0) {
-                xd[item] = d;
-                gsum[item] = s;
-                if (xsT != nullptr) xsT[(item % Kg) * rows + item / Kg] = make_float2(d, s);
+                if (xsT != nullptr) {  // (what the product kernels read, and nothing else)
+                    xsT[(item % Kg) * rows + item / Kg] = make_float2(d, s);
+                } else {
+                    xd[item] = d;
+                    gsum[item] = s;
+                }
             }
         }
     }
@@ -141,8 +144,7 @@ __global__ __launch_bounds__(256) void quant_x_rows_kernel(const float* __restri
 // silu(gate) * up (silu_mul_kernel's expression, so the codes are those of the two launches it replaces).
 template <int U, bool GLU = false>
 __global__ __launch_bounds__(256) void quant_x_tile128_kernel(const float* __restrict__ x, int rows, int Kg, int kparts,
-                                                               int8_t* __restrict__ xq, float* __restrict__ gsum,
-                                                               float2* __restrict__ xsT) {
+                                                               int8_t* __restrict__ xq, float2* __restrict__ xsT) {
     constexpr int G = 128;
     const int sub = threadIdx.x & 31, team = threadIdx.x >> 5;
     const int rb = blockIdx.x / kparts, kp = blockIdx.x - rb * kparts;
@@ -182,10 +184,7 @@ __global__ __launch_bounds__(256) void quant_x_tile128_kernel(const float* __res
         const int kb = kb0 + u;
         if (row_ok && kb < Kg) {
             *reinterpret_cast<uint32_t*>(xq + (rbase + kb) * G + sub * 4) = c;
-            if (sub == 0) {
-                xsT[(int64_t)kb * rows + row] = make_float2(d, s);
-                gsum[rbase + kb] = s;  // [row][kg] as well: the 256-row product kernel reads a row's sums eight at a time
-            }
+            if (sub == 0) xsT[(int64_t)kb * rows + row] = make_float2(d, s);
         }
     }
 }
@@ -196,9 +195,8 @@ __global__ __launch_bounds__(256) void quant_x_tile128_kernel(const float* __res
 // codes, scales and sums as rmsnorm_out followed by that kernel).  hidden % G == 0.
 template <int VPT, int G>
 __global__ __launch_bounds__(1024) void rmsnorm_quant_kernel(const float* __restrict__ x, int64_t hidden,
-                                                              const float* __restrict__ w, float eps, int rows, int Kg,
-                                                              int8_t* __restrict__ xq, float* __restrict__ xd,
-                                                              float* __restrict__ gsum, float2* __restrict__ xsT) {
+                                                              const float* __restrict__ w, float eps, int rows,
+                                                              int8_t* __restrict__ xq, float2* __restrict__ xsT) {
     constexpr int TPG = G / 4;
     __shared__ float red[16];
     const int row = blockIdx.x;
@@ -226,12 +224,7 @@ __global__ __launch_bounds__(1024) void rmsnorm_quant_kernel(const float* __rest
                            (((uint32_t)q8_code(n.z, id) & 0xFFu) << 16) | (((uint32_t)q8_code(n.w, id) & 0xFFu) << 24);
         if (live) {
             *reinterpret_cast<uint32_t*>(xq + (int64_t)row * hidden + e) = c;
-            if ((threadIdx.x % TPG) == 0) {
-                const int64_t kb = e / G;
-                xd[(int64_t)row * Kg + kb] = d;
-                gsum[(int64_t)row * Kg + kb] = s;
-                xsT[kb * rows + row] = make_float2(d, s);
-            }
+            if ((threadIdx.x % TPG) == 0) xsT[e / G * rows + row] = make_float2(d, s);
         }
     }
 }
@@ -244,9 +237,9 @@ namespace llmops {
 // Quantization with the producer of the activations folded in (shared with fc.hip): norm_w != nullptr quantizes
 // rmsnorm(x) * norm_w, glu_in quantizes silu(gate) * up of rows [gate | up] of 2K floats; one launch instead of the
 // producer's launch, a round trip of its fp32 result through memory and the quantization launch.  Whole k-groups
-// only; xd is written with norm_w only (the group-128 product kernels read xsT and gsum).
+// only; scales and sums as the pairs that the product kernels read, xsT [Kg][rows].
 int launch_quant_x_fused(const float* x, int64_t rows, int64_t K, int group_k, const float* norm_w, float eps, bool glu_in,
-                         int8_t* xq, float* xd, float* gsum, float2* xsT, hipStream_t stream) {
+                         int8_t* xq, float2* xsT, hipStream_t stream) {
     const int64_t Kg = K / group_k;
     if (K != Kg * group_k || !aligned(x, 16) || !aligned(xq, 4) || rows >= ((int64_t)1 << 28))
         return fail(LLMOPS_EINVAL, "fused quantization: whole k-groups, 16-byte aligned rows, fewer than 2^28 rows");
@@ -255,12 +248,8 @@ int launch_quant_x_fused(const float* x, int64_t rows, int64_t K, int group_k, c
             return fail(LLMOPS_EINVAL, "fused rmsnorm + quantization: rows of at most 16384 floats, 16-byte aligned weights, no glu");
 #define LLMOPS_RQ(VPT)                                                                                                    \
     do {                                                                                                                  \
-        if (group_k == 32)                                                                                                \
-            rmsnorm_quant_kernel<VPT, 32><<<(unsigned)rows, 1024, 0, stream>>>(x, K, norm_w, eps, (int)rows, (int)Kg, xq, xd, \
-                                                                               gsum, xsT);                                \
-        else                                                                                                              \
-            rmsnorm_quant_kernel<VPT, 128><<<(unsigned)rows, 1024, 0, stream>>>(x, K, norm_w, eps, (int)rows, (int)Kg, xq, xd, \
-                                                                                gsum, xsT);                               \
+        if (group_k == 32) rmsnorm_quant_kernel<VPT, 32><<<(unsigned)rows, 1024, 0, stream>>>(x, K, norm_w, eps, (int)rows, xq, xsT); \
+        else rmsnorm_quant_kernel<VPT, 128><<<(unsigned)rows, 1024, 0, stream>>>(x, K, norm_w, eps, (int)rows, xq, xsT);   \
     } while (0)
         if (K <= 4096) LLMOPS_RQ(1);
         else if (K <= 8192) LLMOPS_RQ(2);
@@ -275,9 +264,9 @@ int launch_quant_x_fused(const float* x, int64_t rows, int64_t K, int group_k, c
         return fail(LLMOPS_EINVAL, "fused silu*up + quantization: group 128 only");
     if (rblocks * ((Kg + 3) / 4) >= 1024) {
         const int kparts = (int)((Kg + 3) / 4);
-        quant_x_tile128_kernel<4, true><<<(unsigned)(rblocks * kparts), 256, 0, stream>>>(x, (int)rows, (int)Kg, kparts, xq, gsum, xsT);
+        quant_x_tile128_kernel<4, true><<<(unsigned)(rblocks * kparts), 256, 0, stream>>>(x, (int)rows, (int)Kg, kparts, xq, xsT);
     } else {
-        quant_x_tile128_kernel<1, true><<<(unsigned)(rblocks * Kg), 256, 0, stream>>>(x, (int)rows, (int)Kg, (int)Kg, xq, gsum, xsT);
+        quant_x_tile128_kernel<1, true><<<(unsigned)(rblocks * Kg), 256, 0, stream>>>(x, (int)rows, (int)Kg, (int)Kg, xq, xsT);
     }
     LLMOPS_LAUNCH_CHECK();
     return LLMOPS_OK;
@@ -290,13 +279,13 @@ int launch_quant_x(const float* x, int64_t rows, int64_t K, int group_k, int8_t*
     const int64_t items = rows * Kg;
     if (!exact_sum && xsT != nullptr && group_k == 128 && K == Kg * group_k && aligned(x, 16) && aligned(xq, 4) &&
         rows < ((int64_t)1 << 28) && Kg < ((int64_t)1 << 20) && ((rows + 7) / 8) * Kg < ((int64_t)1 << 31)) {  // (the grid)
-        // the group-128 prefill kernels read only the codes, the transposed pairs and the sums: xd stays unwritten
+        // the group-128 prefill kernels read only the codes and the transposed pairs: xd and gsum stay unwritten
         const int64_t rblocks = (rows + 7) / 8;
         if (rblocks * ((Kg + 3) / 4) >= 1024) {  // enough workgroups with four k-groups per team
             const int kparts = (int)((Kg + 3) / 4);
-            quant_x_tile128_kernel<4><<<(unsigned)(rblocks * kparts), 256, 0, stream>>>(x, (int)rows, (int)Kg, kparts, xq, gsum, xsT);
+            quant_x_tile128_kernel<4><<<(unsigned)(rblocks * kparts), 256, 0, stream>>>(x, (int)rows, (int)Kg, kparts, xq, xsT);
         } else {
-            quant_x_tile128_kernel<1><<<(unsigned)(rblocks * Kg), 256, 0, stream>>>(x, (int)rows, (int)Kg, (int)Kg, xq, gsum, xsT);
+            quant_x_tile128_kernel<1><<<(unsigned)(rblocks * Kg), 256, 0, stream>>>(x, (int)rows, (int)Kg, (int)Kg, xq, xsT);
         }
         LLMOPS_LAUNCH_CHECK();
         return LLMOPS_OK;
