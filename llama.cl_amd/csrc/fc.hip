@@ -26,11 +26,11 @@ int launch_gemv_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64
 size_t gemm_workspace_bytes(int64_t rows, int64_t Ng, int64_t Kg, int G, int64_t room);
 int launch_gemm(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, const float2* xsT, float* y,
                 float* part, unsigned* counters, int64_t rows, int64_t Ng, int64_t Kg, int G, int64_t N, const float* residual,
-                int64_t room, hipStream_t st);
+                int64_t room, int64_t parts, hipStream_t st);
 int launch_gemm_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg, int G,
                          bool rows128, hipStream_t st);
 int launch_fc_rows(const uint8_t* w, const int8_t* xq, const float2* xsT, float* y, int64_t rows, int64_t Ng, int64_t Kg,
-                   int64_t N, const float* residual, unsigned long long* slots, size_t slot_bytes, hipStream_t st);
+                   int64_t N, const float* residual, int64_t parts, unsigned long long* slots, size_t slot_bytes, hipStream_t st);
 int launch_fc_rows_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg,
                             hipStream_t st);
 bool gemm_rows_kernel_enabled();
@@ -93,7 +93,7 @@ static int fc_check_args(const float* x, int64_t rows, int64_t K, const int8_t* 
 // the product for activations that a quantization launch has left in the workspace (more rows than the streaming
 // kernel that quantizes on the fly takes)
 static int fc_product_many_rows(const uint8_t* w, uint8_t* ws, const FcWorkspace& lay, int64_t rows, int64_t Ng, int64_t Kg,
-                                int group_k, int64_t N, const float* residual, float* y, hipStream_t st) {
+                                int group_k, int64_t N, const float* residual, float* y, int64_t parts, hipStream_t st) {
     const int8_t* xq = reinterpret_cast<const int8_t*>(ws + lay.off_xq);
     const float* xd = reinterpret_cast<const float*>(ws + lay.off_xd);
     const float* gs = reinterpret_cast<const float*>(ws + lay.off_gs);
@@ -105,10 +105,10 @@ static int fc_product_many_rows(const uint8_t* w, uint8_t* ws, const FcWorkspace
     // (us, tiled / streaming: 4096x4096 at 17 rows 20.2 / 9.9, at 32 rows 24.3 / 11.9; 4096x11008 at 24 rows
     // 22.0 / 15.7; 11008x4096 at 24 rows 19.3 / 18.8; 12288x4096 17.9 / 19.0; 22016x4096 23.0 / 27.4)
     if (rows_kernel && (rows <= 16 || (rows <= 32 && Ng < 256)))
-        return launch_fc_rows(w, xq, xst, y, rows, Ng, Kg, N, residual, reinterpret_cast<unsigned long long*>(ws + kTicketBytes),
+        return launch_fc_rows(w, xq, xst, y, rows, Ng, Kg, N, residual, parts, reinterpret_cast<unsigned long long*>(ws + kTicketBytes),
                               LLMOPS_FC_COUNTER_BYTES - kTicketBytes, st);
     return launch_gemm(w, xq, xd, gs, xst, y, reinterpret_cast<float*>(ws + lay.off_part), reinterpret_cast<unsigned*>(ws), rows, Ng,
-                       Kg, group_k, N, residual, lay.room, st);
+                       Kg, group_k, N, residual, lay.room, parts, st);
 }
 
 static int fc_impl(const float* x, int64_t rows, int64_t K, const int8_t* weiq, int64_t Ng, int64_t Kg, int group_k,
@@ -144,7 +144,7 @@ static int fc_impl(const float* x, int64_t rows, int64_t K, const int8_t* weiq, 
         float2* xst_t = reinterpret_cast<float2*>(ws + lay.off_xst);
         int rc_t = launch_quant_x(x, rows, K, group_k, xq, xd, gs, xst_t, false, st);
         if (rc_t) return rc_t;
-        if (rows > kMaxGemvRows) return launch_gemm(w, xq, xd, gs, xst_t, y, part, counters, rows, Ng, Kg, group_k, N, residual, lay.room, st);
+        if (rows > kMaxGemvRows) return launch_gemm(w, xq, xd, gs, xst_t, y, part, counters, rows, Ng, Kg, group_k, N, residual, lay.room, 1, st);
         if (residual == y) return fail(LLMOPS_EINVAL, "fc_Q4A with a short last k-group and up to 8 rows: residual must not be y");
         rc_t = launch_gemv(w, xq, xd, gs, y, part, counters, rows, Ng, Kg, group_k, N, st);
         if (rc_t == 0 && residual != nullptr) rc_t = launch_add(y, residual, rows * N, st);
@@ -158,7 +158,7 @@ static int fc_impl(const float* x, int64_t rows, int64_t K, const int8_t* weiq, 
     float2* xst = reinterpret_cast<float2*>(ws + lay.off_xst);
     int rc = launch_quant_x(x, rows, K, group_k, xq, xd, gs, xst, false, st);
     if (rc) return rc;
-    return fc_product_many_rows(w, ws, lay, rows, Ng, Kg, group_k, N, residual, y, st);
+    return fc_product_many_rows(w, ws, lay, rows, Ng, Kg, group_k, N, residual, y, 1, st);
 }
 
 extern "C" int llmops_fc_Q4A(const float* x, int64_t rows, int64_t K, const int8_t* weiq, int64_t Ng, int64_t Kg,
@@ -226,15 +226,20 @@ static int fc_decode_impl(const float* x, int64_t rows, int64_t K, const int8_t*
                      : launch_quant_x(x, rows, K, group_k, xq, xd, gs, xst, false, st);
         if (rc) return rc;
         if (out_parts > 1) {
-            // y is [out_parts][rows][N_out / out_parts]: one product per slice of strips on the same quantized rows
-            // (q, k and v of a fused q|k|v tensor come out as three dense matrices instead of one to be cut up)
+            // y is [out_parts][rows][N_out / out_parts]: q, k and v of a fused q|k|v tensor come out as three dense matrices
+            // instead of one to be cut up.  Group 128: one product whose stores know the parts (a third of the strips
+            // fills the chip less well; us with rmsnorm, 3 x 4096 x 4096, a product each / in one: 12 rows 19.1 / 14.4, 64 rows
+            // 37.8 / 19.5, 300 rows 59.4 / 41.1, 512 rows 82.2 / 52.7, 1024 rows 113.5 / 97.8 in one); group 32: a
+            // product per slice of strips on the same quantized rows.
             const int64_t ngp = Ng / out_parts, np = N_out / out_parts;
+            if (group_k == 128)
+                return fc_product_many_rows(reinterpret_cast<const uint8_t*>(weiq), ws, lay, rows, Ng, Kg, group_k, np, nullptr, y, out_parts, st);
             for (int64_t p = 0; p < out_parts && rc == 0; p++)
                 rc = fc_product_many_rows(reinterpret_cast<const uint8_t*>(weiq) + p * ngp * Kg * block_bytes(group_k), ws, lay,
-                                          rows, ngp, Kg, group_k, np, nullptr, y + p * rows * np, st);
+                                          rows, ngp, Kg, group_k, np, nullptr, y + p * rows * np, 1, st);
             return rc;
         }
-        rc = fc_product_many_rows(reinterpret_cast<const uint8_t*>(weiq), ws, lay, rows, Ng, Kg, group_k, N_out, residual, y, st);
+        rc = fc_product_many_rows(reinterpret_cast<const uint8_t*>(weiq), ws, lay, rows, Ng, Kg, group_k, N_out, residual, y, 1, st);
         if (rc == 0 && sumsq_out != nullptr) rc = launch_strip_sumsq(y, rows, N_out, sumsq_out, st);
         return rc;
     }
@@ -316,7 +321,7 @@ extern "C" int llmops_fc_Q4A_prequantized(const int8_t* xq, const float* xd, con
     hipStream_t st = as_stream(stream);
     if (rows <= kMaxGemvRows)
         return launch_gemv(w, xq, xd, gsum, y, part, reinterpret_cast<unsigned*>(ws), rows, Ng, Kg, group_k, N, st);
-    return launch_gemm(w, xq, xd, gsum, nullptr, y, part, reinterpret_cast<unsigned*>(ws), rows, Ng, Kg, group_k, N, nullptr, lay.room, st);
+    return launch_gemm(w, xq, xd, gsum, nullptr, y, part, reinterpret_cast<unsigned*>(ws), rows, Ng, Kg, group_k, N, nullptr, lay.room, 1, st);
 }
 
 extern "C" int llmops_fc_Q4A_partials(const int8_t* xq, int64_t rows, const int8_t* weiq, int64_t Ng, int64_t Kg,

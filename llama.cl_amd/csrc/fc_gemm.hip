@@ -39,7 +39,7 @@ __device__ __forceinline__ void store_pair(float* dst, const float* res, float a
 // index order (so the sum does not depend on who arrives when), adds the residual and writes the result.
 // Nobody waits for anybody.  Called by every thread of the workgroup, with LDS no longer in use once all have arrived.
 // row0 / tile_rows: first row and row count of the tile; a thread holds rows 16t + 4g + v of it, columns
-// 32*strip + 2*jj + c in f[t][c][v].
+// 32*strip + 2*jj + c in f[t][c][v]; n0: where the first of them goes in a row of y_final.
 // Where the sums of a tile lie: a row block's rows * Np floats strip by strip, a strip's rows in pairs, a pair as
 // [jj][row of the pair][c]: 16 bytes per lane, 256 of them consecutive (and the last of an odd number of rows by itself, 8 bytes
 // per lane).  Accesses of rows beyond `rows` fall outside the buffer descriptor (loads return 0, stores are dropped), as do
@@ -50,7 +50,7 @@ __device__ __forceinline__ void store_pair(float* dst, const float* res, float a
 template <int T, int SU>
 __device__ __forceinline__ void splitk_finish(const v4f (&f)[T][2], float* __restrict__ out, int64_t split_stride, int64_t Np,
                                               int row0, int tile_rows, int strip, int Ng, int jj, int g, int rows,
-                                              float* __restrict__ y_final, int64_t Ny, const float* __restrict__ residual,
+                                              float* __restrict__ y_final, int64_t Ny, int64_t n0, const float* __restrict__ residual,
                                               unsigned* counter, int tid, unsigned* ticket_sh) {
     constexpr int kAgent = 16;  // sc1: coherent at device scope, as a relaxed atomic store / load would be
     const int S = (int)gridDim.z;
@@ -85,7 +85,6 @@ __device__ __forceinline__ void splitk_finish(const v4f (&f)[T][2], float* __res
     if (*ticket_sh != (unsigned)(S - 1)) return;
     if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // next launch
     if (!strip_ok) return;
-    const int64_t n0 = (int64_t)strip * kGroupN + 2 * jj;
 #pragma unroll
     for (int t = 0; t < T; t += 2) {
         float a[4][4];
@@ -174,7 +173,7 @@ __global__ __launch_bounds__(256, (RT == 4 ? 2 : (RT == 2 ? 3 : 4))) void fc_gem
     const uint8_t* __restrict__ weiq, const int8_t* __restrict__ xq, const float* __restrict__ xd, const float* __restrict__ gs,
     const float2* __restrict__ xsT, float* __restrict__ out, int32_t* __restrict__ out_i, int Ng, int Kg, int64_t ldo, int64_t N,
     int rows, int kb_per_split, int64_t split_stride, const float* __restrict__ residual, float* __restrict__ y_final, int64_t Ny,
-    unsigned* __restrict__ counters) {
+    int part_strips, unsigned* __restrict__ counters) {
     using Tile = GemmTile<RT>;
     constexpr int BM = Tile::BM, T = Tile::T;
     extern __shared__ __align__(16) uint8_t smem_raw[];
@@ -440,15 +439,17 @@ __global__ __launch_bounds__(256, (RT == 4 ? 2 : (RT == 2 ? 3 : 4))) void fc_gem
 
     if (PARTIALS) return;
     const int strip = strip0 + wave;
+    // results in parts: part_strips strips to a dense matrix of its own (of partial sums only the finished ones are)
+    const int part = strip / part_strips;
+    const int64_t n0 = (int64_t)(strip - part * part_strips) * kGroupN + 2 * jj;
     if (counters != nullptr) {
         splitk_finish<T, (RT == 4 ? 12 : (RT == 2 ? 6 : 4))>(f, out, split_stride, ldo, row0, min(BM, rows - row0), strip, Ng, jj, g,
-                                                            rows, y_final, Ny, residual, &counters[by * nbx + bx], tid,
+                                                            rows, y_final + (int64_t)part * rows * Ny, Ny, n0, residual, &counters[by * nbx + bx], tid,
                                                             reinterpret_cast<unsigned*>(smem_raw));
         return;
     }
     if (strip >= Ng) return;
-    float* o = out + (int64_t)blockIdx.z * split_stride;
-    const int64_t n0 = (int64_t)strip * kGroupN + 2 * jj;
+    float* o = out + (int64_t)blockIdx.z * split_stride + (int64_t)part * rows * ldo;
 #pragma unroll
     for (int t = 0; t < T; t++)
 #pragma unroll
@@ -460,16 +461,17 @@ __global__ __launch_bounds__(256, (RT == 4 ? 2 : (RT == 2 ? 3 : 4))) void fc_gem
         }
 }
 
-// y[row][n] = sum over splits (index order) of part[s][row][n] (+ residual[row][n]); four columns per
+// y[p][row][n] = sum over splits (index order) of part[s][row][p * N + n] (+ residual[row][n]); four columns per
 // thread (the partial sums' row stride ldp is a multiple of 32 floats, so their 16-byte loads are aligned)
-__global__ void gemm_reduce_kernel(const float* __restrict__ part, float* __restrict__ y, int64_t rows, int64_t N,
+__global__ void gemm_reduce_kernel(const float* __restrict__ part, float* __restrict__ y, int64_t rows, int64_t N, int parts,
                                    int64_t ldp, int64_t split_stride, int S, const float* __restrict__ residual) {
     const int64_t nq = (N + 3) / 4;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * nq) return;
-    const int64_t r = i / nq, n = (i % nq) * 4;
+    if (i >= rows * nq * parts) return;
+    const int64_t r = i / nq % rows, p = i / (nq * rows), n = (i % nq) * 4;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-    float* dst = y + r * N + n;
+    part += p * N;
+    float* dst = y + (p * rows + r) * N + n;
     const float* res = residual ? residual + r * N + n : nullptr;
     const bool whole = n + 3 < N && (N & 3) == 0;
     float4 r4 = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -574,8 +576,8 @@ static int configure_gemm_tile() {
 template <int RT>
 static int launch_gemm_tile(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, const float2* xsT,
                             float* out, int64_t Ng, int64_t Kg, int64_t ldo, int64_t N, int64_t rows, const GemmPlan& p,
-                            int64_t split_stride, const float* residual, float* y_final, int64_t Ny, unsigned* counters,
-                            hipStream_t st) {
+                            int64_t split_stride, const float* residual, float* y_final, int64_t Ny, int64_t part_strips,
+                            unsigned* counters, hipStream_t st) {
     const int bad = configure_gemm_tile<RT, false>();
     if (bad) return bad;
     // (the copies take 32-bit offsets into the scale pairs of a k-group and into a tile's rows and strips)
@@ -584,14 +586,16 @@ static int launch_gemm_tile(const uint8_t* w, const int8_t* xq, const float* xd,
     const int64_t tiles = ((Ng + 3) / 4) * ((rows + RT * 32 - 1) / (RT * 32));
     dim3 grid((unsigned)(8 * ((tiles + 7) / 8)), 1, (unsigned)p.S);  // one run of tiles per XCD
     fc_gemm_tile_kernel<RT, false><<<grid, 256, sizeof(GemmTile<RT>), st>>>(
-        w, xq, xd, gs, xsT, out, nullptr, (int)Ng, (int)Kg, ldo, N, (int)rows, p.kb_per_split, split_stride, residual, y_final, Ny, counters);
+        w, xq, xd, gs, xsT, out, nullptr, (int)Ng, (int)Kg, ldo, N, (int)rows, p.kb_per_split, split_stride, residual, y_final, Ny,
+        (int)part_strips, counters);
     return LLMOPS_OK;
 }
 
-// y = product (+ residual, fp32 [rows, N], may be y itself); room: as gemm_workspace_bytes was asked with
+// y = product (+ residual, fp32 [rows, N], may be y itself); room: as gemm_workspace_bytes was asked with; parts > 1 (group 128,
+// no residual): y is [parts][rows][N], part i the columns of strips i * Ng / parts ..
 int launch_gemm(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, const float2* xsT, float* y,
                 float* part, unsigned* counters, int64_t rows, int64_t Ng, int64_t Kg, int G, int64_t N, const float* residual,
-                int64_t room, hipStream_t st) {
+                int64_t room, int64_t parts, hipStream_t st) {
     const GemmPlan p = plan_gemm(rows, Ng, Kg, G, room);
     // With up to 12 splits the tiled kernel adds the partial sums itself (the last split of a tile to arrive
     // does), given one zeroed arrival counter per tile; otherwise a second launch adds them (8-11 us whatever the shape).
@@ -606,12 +610,13 @@ int launch_gemm(const uint8_t* w, const int8_t* xq, const float* xd, const float
     float* out = p.S > 1 ? part : y;
     const int64_t ldo = p.S > 1 ? Np : N;
     const int64_t Nw = p.S > 1 ? Np : N;
+    const int64_t part_strips = p.S > 1 && !fused_reduce ? Ng : Ng / parts;
     const int64_t ss = rows * Np;
     if (p.lds) {
         int rc;
-        if (p.RT == 4) rc = launch_gemm_tile<4>(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, y, N, kcnt, st);
-        else if (p.RT == 2) rc = launch_gemm_tile<2>(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, y, N, kcnt, st);
-        else rc = launch_gemm_tile<1>(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, y, N, kcnt, st);
+        if (p.RT == 4) rc = launch_gemm_tile<4>(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, y, N, part_strips, kcnt, st);
+        else if (p.RT == 2) rc = launch_gemm_tile<2>(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, y, N, part_strips, kcnt, st);
+        else rc = launch_gemm_tile<1>(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p, ss, kres, y, N, part_strips, kcnt, st);
         if (rc) return rc;
     } else {
         const int rc = launch_gemm_g32(w, xq, xd, gs, xsT, out, Ng, Kg, ldo, Nw, rows, p.kb_per_split, p.S, ss, kres, st);
@@ -619,8 +624,8 @@ int launch_gemm(const uint8_t* w, const int8_t* xq, const float* xd, const float
     }
     LLMOPS_LAUNCH_CHECK();
     if (p.S > 1 && !fused_reduce) {
-        const int64_t total = rows * ((N + 3) / 4);
-        gemm_reduce_kernel<<<(unsigned)((total + 255) / 256), 256, 0, st>>>(part, y, rows, N, Np, ss, p.S, residual);
+        const int64_t total = parts * rows * ((N + 3) / 4);
+        gemm_reduce_kernel<<<(unsigned)((total + 255) / 256), 256, 0, st>>>(part, y, rows, N, (int)parts, Np, ss, p.S, residual);
         LLMOPS_LAUNCH_CHECK();
     }
     return LLMOPS_OK;
@@ -633,7 +638,7 @@ static int launch_gemm_tile_partials(const uint8_t* w, const int8_t* xq, int32_t
     if (bad) return bad;
     const int64_t tiles = ((Ng + 3) / 4) * ((rows + RT * 32 - 1) / (RT * 32));
     fc_gemm_tile_kernel<RT, true><<<(unsigned)(8 * ((tiles + 7) / 8)), 256, sizeof(GemmTile<RT>), st>>>(
-        w, xq, nullptr, nullptr, nullptr, nullptr, acc, (int)Ng, (int)Kg, 0, 0, (int)rows, (int)Kg, 0, nullptr, nullptr, 0, nullptr);
+        w, xq, nullptr, nullptr, nullptr, nullptr, acc, (int)Ng, (int)Kg, 0, 0, (int)rows, (int)Kg, 0, nullptr, nullptr, 0, (int)Ng, nullptr);
     LLMOPS_LAUNCH_CHECK();
     return LLMOPS_OK;
 }

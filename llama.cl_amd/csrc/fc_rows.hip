@@ -90,7 +90,7 @@ __global__ __launch_bounds__(NW * 64, RT == 2 ? 3 : 4) void fc_rows_mfma_kernel(
                                                                          unsigned long long* slots, int Kg, int rows,
                                                                          int64_t N, float* __restrict__ y,
                                                                          const float* __restrict__ residual,
-                                                                         int32_t* dump = nullptr) {
+                                                                         int part_strips, int32_t* dump = nullptr) {
     // (argument order: what the first loads need comes in the first 14 dwords, which arrive in scalar registers
     // with the wave)
     __shared__ __align__(8) float red[DUMP ? 1 : NW][16 * RT][kGroupN];
@@ -185,7 +185,8 @@ __global__ __launch_bounds__(NW * 64, RT == 2 ? 3 : 4) void fc_rows_mfma_kernel(
     for (int i = 0; i < RT; i++) {
         const int idx = threadIdx.x + NW * 64 * i;
         const int row = idx >> 5, col = idx & 31;
-        const int64_t n = (int64_t)nb * kGroupN + col;
+        const int part = nb / part_strips;  // results in parts: part_strips strips to a dense matrix of its own
+        const int64_t n = (int64_t)(nb - part * part_strips) * kGroupN + col;
         if (row < rows && n < N) {
             float v = 0.0f;
 #pragma unroll
@@ -194,14 +195,14 @@ __global__ __launch_bounds__(NW * 64, RT == 2 ? 3 : 4) void fc_rows_mfma_kernel(
                 // A slot is empty (0) or holds (1 << 32 | value bits).  Whoever finds the other half's value
                 // adds the two (a + b: the same bits whichever came first), stores the output and empties the
                 // slot for the next launch; whoever finds it empty has parked its own value and is done.
-                unsigned long long* slot = slots + ((int64_t)row * gridDim.x / 2 * kGroupN + n);
+                unsigned long long* slot = slots + ((int64_t)row * gridDim.x / 2 * kGroupN + nb * kGroupN + col);
                 const unsigned long long parked = (1ull << 32) | (unsigned long long)__float_as_uint(v);
                 const unsigned long long old = __hip_atomic_exchange(slot, parked, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 if ((old >> 32) == 0ull) continue;
                 v += __uint_as_float((unsigned)(old & 0xFFFFFFFFull));
                 __hip_atomic_store(slot, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            y[(int64_t)row * N + n] = residual ? v + residual[(int64_t)row * N + n] : v;
+            y[((int64_t)part * rows + row) * N + n] = residual ? v + residual[(int64_t)row * N + n] : v;
         }
     }
 }
@@ -220,9 +221,10 @@ __global__ __launch_bounds__(NW * 64, RT == 2 ? 3 : 4) void fc_rows_mfma_kernel(
     } while (0)
 
 // rows <= 32 (two row tiles per wave from 17 on), group 128, activations already quantized (codes [rows, Kg*128], pairs [Kg][rows])
+// parts > 1 (no residual): y is [parts][rows][N], part i the columns of strips i * Ng / parts ..
 // `slots`: the zeroed exchange area of the FC workspace (`slot_bytes` of it), or nullptr
 int launch_fc_rows(const uint8_t* w, const int8_t* xq, const float2* xsT, float* y, int64_t rows, int64_t Ng, int64_t Kg,
-                   int64_t N, const float* residual, unsigned long long* slots, size_t slot_bytes, hipStream_t st) {
+                   int64_t N, const float* residual, int64_t parts, unsigned long long* slots, size_t slot_bytes, hipStream_t st) {
     if (rows > 32) return fail(LLMOPS_EINVAL, "the streaming MFMA kernel takes at most 32 rows, got %lld", (long long)rows);
     // fewer strips than compute units and a K worth cutting: two workgroups per strip
     const bool split = slots != nullptr && g_rows_split && Ng < 256 && Kg >= 16 && (size_t)rows * Ng * kGroupN * 8 <= slot_bytes;
@@ -233,7 +235,7 @@ int launch_fc_rows(const uint8_t* w, const int8_t* xq, const float2* xsT, float*
     // 13.3 against 13.8 us; with 32 k-groups 16 waves are slower, 15.7 against 14.1 us at 11008x4096).
     // 17..32 rows: two row tiles per wave, 8 waves (16 would not have the registers).
     const int64_t k_per_wg = split ? (Kg + 1) / 2 : Kg;
-    LLMOPS_ROWS_LAUNCH(false, w, xq, xsT, sl, (int)Kg, (int)rows, N, y, residual);
+    LLMOPS_ROWS_LAUNCH(false, w, xq, xsT, sl, (int)Kg, (int)rows, N, y, residual, (int)(Ng / parts));
     LLMOPS_LAUNCH_CHECK();
     return LLMOPS_OK;
 }
@@ -247,7 +249,7 @@ int launch_fc_rows_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, in
     // only tested against nullptr in the dump build, never dereferenced
     unsigned long long* sl = split ? reinterpret_cast<unsigned long long*>(acc) : nullptr;
     const int64_t k_per_wg = split ? (Kg + 1) / 2 : Kg;
-    LLMOPS_ROWS_LAUNCH(true, w, xq, nullptr, sl, (int)Kg, (int)rows, 0, nullptr, nullptr, acc);
+    LLMOPS_ROWS_LAUNCH(true, w, xq, nullptr, sl, (int)Kg, (int)rows, 0, nullptr, nullptr, (int)Ng, acc);
     LLMOPS_LAUNCH_CHECK();
     return LLMOPS_OK;
 }
