@@ -1,16 +1,21 @@
 """Build the gfx950 shared library in-tree:  python llama.cl_amd/build.py
 
 hipcc cross-compiles for the MI355X without a GPU present.  The output,
-``llama.cl_amd/llmops/libllmops_hip.so``, is what the ``llmops`` Python module loads.
+``llama.cl_amd/llmops/libllmops_hip.so``, is what the ``llmops`` Python module loads, and beside it ``_host.so``, the
+module's own calls in native code (csrc/host, the one part that knows torch's types).
 """
 import glob
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "llmops", "libllmops_hip.so")
+HOST_SRC = os.path.join(CSRC, "host", "calls.cc")
+HOST_OUT = os.path.join(HERE, "llmops", "_host.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -58,6 +63,17 @@ def _compile(src, obj):
     return src, proc.returncode, proc.stdout.splitlines()
 
 
+def _compile_host():
+    torch_dir = os.path.dirname(importlib.util.find_spec("torch").origin)
+    inc = [os.path.join(torch_dir, "include"), os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+           "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+    cmd += [a for i in inc for a in ("-isystem", i)] + ["-Wall", "-o", HOST_OUT, HOST_SRC, "-L" + os.path.join(torch_dir, "lib")]
+    cmd += ["-ltorch_python", "-ltorch", "-ltorch_hip", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    return HOST_SRC, proc.returncode, proc.stdout.splitlines()
+
+
 def _readable(lines):
     """the host pass does not know the AMDGPU feature name and says so; that line is noise, and so are
     the resource remarks and the source lines the compiler quotes under each of them"""
@@ -87,13 +103,14 @@ def build(verbose=False, jobs=None):
         jobs = jobs or min(len(srcs), max(1, (os.cpu_count() or 2) - 1), 16)
         objs = [os.path.join(objdir, os.path.basename(s) + ".o") for s in srcs]
         with concurrent.futures.ThreadPoolExecutor(jobs) as ex:
-            results = list(ex.map(lambda so: _compile(*so), zip(srcs, objs)))
+            host = ex.submit(_compile_host)
+            results = list(ex.map(lambda so: _compile(*so), zip(srcs, objs))) + [host.result()]
         remarks, logs = [], []
         for src, rc, lines in results:
             remarks += [l for l in lines if "[-Rpass-analysis=kernel-resource-usage]" in l]
             log = _readable(lines)
             if rc != 0:
-                raise RuntimeError(f"hipcc failed on {src}:\n" + log)
+                raise RuntimeError(f"compiling {src} failed:\n" + log)
             if log.strip():
                 logs.append(log)
         check_spills(remarks)

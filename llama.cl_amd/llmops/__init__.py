@@ -188,6 +188,10 @@ def FC_dynamic_quantize_x(input, group_k, rows_variant=False):
 def fc_Q4A(input, weiq, N, residual=None):
     """fp32 [B,M,K] x packed [Ng,Kg,blk] -> fp32 [B,M,N] (ops/op_fc.hpp:286-426).
     ``residual`` (extension, fp32 [B,M,N]): returns fc_Q4A(input) + residual in the same launch."""
+    if residual is None:
+        out = (_lib._host or _lib.host()).fc_Q4A(_workspaces, input, weiq, N)
+        if out is not NotImplemented:  # (the ordinary call, in native code; what it leaves alone goes the long way)
+            return out
     _dev(input, torch.float32, 3, "input")
     _dev(weiq, torch.int8, 3, "wei_quantized")
     g = group_k_of(weiq)
@@ -367,6 +371,9 @@ def attention_rope2(q, k, v, inv_freq, kv_cache, kvc_slots, position_id, layer_i
     In place: q <- attention output, k <- rotated k, cache rows updated (ops/op_attn.hpp:721-1029).
     Extension: with qL == 1, ``position_id`` may be an int32 tensor [1] on the device; the kernels then read the
     position (and the slot) from memory, so a HIP graph that captured the call serves every following token."""
+    if (_lib._host or _lib.host()).attention_rope2(_workspaces, q, k, v, inv_freq, kv_cache, kvc_slots, position_id,
+                                                   layer_id) is not NotImplemented:
+        return
     _dev(q, torch.float32, 3, "q")
     _dev(k, torch.float32, 3, "k")
     _dev(v, torch.float32, 3, "v")

@@ -97,6 +97,25 @@ def load():
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The module's own calls in native code (csrc/host/calls.cc), bound to the library's entries."""
+    global _host
+    if _host is None:
+        lib = load()
+        try:
+            from . import _host as native
+        except ImportError as e:
+            raise ImportError(f"llmops/_host.so does not load ({e}): build it with `python llama.cl_amd/build.py`.") from e
+        native.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in (
+            "llmops_fc_Q4A_workspace_bytes", "llmops_fc_Q4A", "llmops_attention_workspace_bytes", "llmops_attention_rope",
+            "llmops_last_error")))
+        _host = native
+    return _host
+
+
 def check(rc):
     if rc != 0:
         raise RuntimeError(load().llmops_last_error().decode())
