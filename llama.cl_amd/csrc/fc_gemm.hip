@@ -463,12 +463,12 @@ __global__ __launch_bounds__(256, (RT == 4 ? 2 : (RT == 2 ? 3 : 4))) void fc_gem
 
 // y[p][row][n] = sum over splits (index order) of part[s][row][p * N + n] (+ residual[row][n]); four columns per
 // thread (the partial sums' row stride ldp is a multiple of 32 floats, so their 16-byte loads are aligned)
-__global__ void gemm_reduce_kernel(const float* __restrict__ part, float* __restrict__ y, int64_t rows, int64_t N, int parts,
+__global__ void gemm_reduce_kernel(const float* __restrict__ part, float* __restrict__ y, int64_t rows, int64_t N,
                                    int64_t ldp, int64_t split_stride, int S, const float* __restrict__ residual) {
     const int64_t nq = (N + 3) / 4;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * nq * parts) return;
-    const int64_t r = i / nq % rows, p = i / (nq * rows), n = (i % nq) * 4;
+    if (i >= rows * nq) return;
+    const int64_t r = i / nq, n = (i % nq) * 4, p = blockIdx.y;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
     part += p * N;
     float* dst = y + (p * rows + r) * N + n;
@@ -624,8 +624,8 @@ int launch_gemm(const uint8_t* w, const int8_t* xq, const float* xd, const float
     }
     LLMOPS_LAUNCH_CHECK();
     if (p.S > 1 && !fused_reduce) {
-        const int64_t total = parts * rows * ((N + 3) / 4);
-        gemm_reduce_kernel<<<(unsigned)((total + 255) / 256), 256, 0, st>>>(part, y, rows, N, (int)parts, Np, ss, p.S, residual);
+        const int64_t total = rows * ((N + 3) / 4);
+        gemm_reduce_kernel<<<dim3((unsigned)((total + 255) / 256), (unsigned)parts), 256, 0, st>>>(part, y, rows, N, Np, ss, p.S, residual);
         LLMOPS_LAUNCH_CHECK();
     }
     return LLMOPS_OK;
