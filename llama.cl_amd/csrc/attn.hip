@@ -59,13 +59,30 @@ __device__ __forceinline__ void store_cache<__half>(__half* dst, float v) {
     *dst = __float2half_rn(v);
 }
 
-// q,k,v [B,qL,H,S].  One workgroup per (b, l, h); thread i handles element i (and i+half).
-template <typename T>
+// q,k,v [B,qL,H,S].  One workgroup of a wave per (b, l, h); thread i handles element i (and i+half).  TABLES: before those, `tables`
+// workgroups each write 64 entries of row_token: the (last) token of this call that a cache row belongs to, or -1.  (us for the
+// whole call, 32 heads, with a launch that filled the table with -1 and a scattered store per token / so: 64 tokens 17.9 / 17.2,
+// 300 behind 300 50.0 / 48.3, 1024 tokens 84.6 / 82.1, 2048 tokens 175 / 172.)
+template <typename T, bool TABLES>
 __global__ void attn_prep_kernel(float* __restrict__ q, float* __restrict__ k, const float* __restrict__ v, int64_t qL,
                                  int64_t H, int64_t S, const float* __restrict__ inv_freq, int64_t half,
                                  T* __restrict__ kc, T* __restrict__ vc, int64_t maxlen, const int32_t* __restrict__ slots,
-                                 int position_id, int32_t* __restrict__ row_token) {
-    const int64_t h = blockIdx.x % H, l = (blockIdx.x / H) % qL, b = blockIdx.x / (H * qL);
+                                 int position_id, int32_t* __restrict__ row_token, int64_t kvLen, unsigned tables) {
+    if (TABLES && blockIdx.x < tables) {
+        __shared__ int32_t token[64];
+        const int64_t row0 = (int64_t)blockIdx.x * 64;
+        token[threadIdx.x] = -1;
+        __syncthreads();
+        for (int64_t l = threadIdx.x; l < qL; l += 64) {
+            const int64_t at = (int64_t)slots[l] - row0;
+            if (at >= 0 && at < 64) atomicMax(&token[at], (int32_t)l);
+        }
+        __syncthreads();
+        if (row0 + threadIdx.x < kvLen) row_token[row0 + threadIdx.x] = token[threadIdx.x];
+        return;
+    }
+    const int64_t item = TABLES ? blockIdx.x - tables : blockIdx.x;
+    const int64_t h = item % H, l = (item / H) % qL, b = item / (H * qL);
     const int64_t base = ((b * qL + l) * H + h) * S;
     const int slot = slots[l];
     // slots live in device memory and cannot be validated on the host: a slot outside the cache is
@@ -73,10 +90,6 @@ __global__ void attn_prep_kernel(float* __restrict__ q, float* __restrict__ k, c
     const bool slot_ok = slot >= 0 && slot < maxlen;
     T* kdst = kc + ((b * H + h) * maxlen + (slot_ok ? slot : 0)) * S;
     T* vdst = vc + ((b * H + h) * maxlen + (slot_ok ? slot : 0)) * S;
-    if (row_token != nullptr && blockIdx.x < qL && threadIdx.x == 0) {
-        const int s0 = slots[blockIdx.x];
-        if (s0 >= 0 && s0 < maxlen) row_token[s0] = (int32_t)blockIdx.x;
-    }
     for (int64_t i = threadIdx.x; i < S; i += blockDim.x) {
         if (i < half) {
             float q0 = q[base + i], q1 = q[base + i + half];
@@ -99,11 +112,6 @@ __global__ void attn_prep_kernel(float* __restrict__ q, float* __restrict__ k, c
     }
 }
 
-__global__ void fill_i32_kernel(int32_t* p, int64_t n, int32_t v) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
 __device__ __forceinline__ float4 load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 __device__ __forceinline__ float4 load4(const __half* p) {
     const uint2 u = *reinterpret_cast<const uint2*>(p);
@@ -116,6 +124,32 @@ __device__ __forceinline__ float2 load2(const float* p) { return *reinterpret_ca
 __device__ __forceinline__ float2 load2(const __half* p) {
     const uint32_t u = *reinterpret_cast<const uint32_t*>(p);
     return __half22float2(*reinterpret_cast<const __half2*>(&u));
+}
+
+// a value as the cache holds it
+template <typename T>
+__device__ __forceinline__ float cache_round(float v);
+template <>
+__device__ __forceinline__ float cache_round<float>(float v) {
+    return v;
+}
+template <>
+__device__ __forceinline__ float cache_round<__half>(float v) {
+    return __half2float(__float2half_rn(v));
+}
+template <typename T>
+__device__ __forceinline__ void store4(T* dst, float4 v);
+template <>
+__device__ __forceinline__ void store4<float>(float* dst, float4 v) {
+    *reinterpret_cast<float4*>(dst) = v;
+}
+template <>
+__device__ __forceinline__ void store4<__half>(__half* dst, float4 v) {
+    const __half2 a = __floats2half2_rn(v.x, v.y), b = __floats2half2_rn(v.z, v.w);
+    uint2 u;
+    u.x = *reinterpret_cast<const uint32_t*>(&a);
+    u.y = *reinterpret_cast<const uint32_t*>(&b);
+    *reinterpret_cast<uint2*>(dst) = u;
 }
 
 // ---- split-KV attention of few query tokens over a short cache ----
@@ -254,18 +288,17 @@ constexpr float kFewMax = 0x1p56f, kFewMin = 0x1p-90f;
 __device__ __forceinline__ float max_abs(float m, float4 v) {
     return fmaxf(fmaxf(fmaxf(fmaxf(m, fabsf(v.x)), fabsf(v.y)), fabsf(v.z)), fabsf(v.w));  // (in this order: two v_max3_f32)
 }
-// the wave's 32 x qL scores before scaling, into the layout of the MFMA's result; krow, q0: the lane's row and the first
-// query from dim 8 * hf on; buf: 32 * 32 floats of the wave's own
-template <typename T>
-__device__ __forceinline__ void few_scores_fp32(const T* krow, const float* q0, int qL, int64_t q_stride, float* buf, int c32,
-                                                          int hf, v16f& pr) {
+// the wave's 32 x qL scores before scaling, into the layout of the MFMA's result; k_at(d), q_at(l, d): four dims from
+// d + 8 * hf on of the lane's row and of query l; buf: 32 * 32 floats of the wave's own
+template <typename K, typename Q>
+__device__ __forceinline__ void few_scores_fp32(K k_at, Q q_at, int qL, float* buf, int c32, int hf, v16f& pr) {
     for (int l = 0; l < qL; l++) {
         float s = 0.0f;
 #pragma unroll 1
         for (int i = 0; i < 8; i++) {
 #pragma unroll
             for (int e = 0; e < 8; e += 4) {
-                const float4 a = load4(krow + 16 * i + e), w = load4(q0 + l * q_stride + 16 * i + e);
+                const float4 a = k_at(16 * i + e), w = q_at(l, 16 * i + e);
                 s = fmaf(a.x, w.x, s), s = fmaf(a.y, w.y, s), s = fmaf(a.z, w.z, s), s = fmaf(a.w, w.w, s);
             }
         }
@@ -280,9 +313,10 @@ __device__ __forceinline__ void few_scores_fp32(const T* krow, const float* q0, 
         pr[4 * jj] = x.x, pr[4 * jj + 1] = x.y, pr[4 * jj + 2] = x.z, pr[4 * jj + 3] = x.w;
     }
 }
-// the wave's 64 output elements of the lane's query; dst: the lane's place in the first of the 16 result registers
-template <typename T>
-__device__ __forceinline__ void few_outputs_fp32(const T* vbase, int p0, int kvLen, int c32, int hf, const v16f& pr, float* dst) {
+// the wave's 64 output elements of the lane's query; v_at(row, col): four columns of a row of the wave's 32; dst: the lane's
+// place in the first of the 16 result registers
+template <typename V>
+__device__ __forceinline__ void few_outputs_fp32(V v_at, int hf, const v16f& pr, float* dst) {
     float w[2][16];  // [half that holds the row][register]
 #pragma unroll
     for (int r = 0; r < 16; r++) {
@@ -295,7 +329,7 @@ __device__ __forceinline__ void few_outputs_fp32(const T* vbase, int p0, int kvL
         float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int row = 0; row < 32; row++) {
-            const float4 v = load4(vbase + (int64_t)min(p0 + row, kvLen - 1) * 128 + col);
+            const float4 v = v_at(row, col);
             const float p = w[(row >> 2) & 1][4 * (row >> 3) + (row & 3)];
             a.x = fmaf(p, v.x, a.x), a.y = fmaf(p, v.y, a.y), a.z = fmaf(p, v.z, a.z), a.w = fmaf(p, v.w, a.w);
         }
@@ -303,38 +337,135 @@ __device__ __forceinline__ void few_outputs_fp32(const T* vbase, int p0, int kvL
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(256, 2) void attn_few_kernel(const float* __restrict__ q, const T* __restrict__ kc,
-                                                           const T* __restrict__ vc, int qL, int64_t H, int64_t maxlen, int kvLen,
-                                                           const int32_t* __restrict__ slots, float* __restrict__ part, int nchunks) {
-    constexpr int S = 128, P = sizeof(T) == 4 ? 3 : 2;
-    __shared__ __align__(16) int tok[4][32];
-    __shared__ float wm[4][64], wl[4][64];
-    __shared__ __align__(16) float os[4][16][64][4];  // [wave][4j + v][lane][c]
+// ROPE: rotation and cache update happen here too (a launch and its gap less).
+// Every workgroup rotates the queries on their way to LDS, a thread per token and pair of dims.  The rows that this call
+// writes are nobody's cache rows: they are masked, and their stale contents kept out of the products, wherever they lie in the
+// cache; one more workgroup per head (the last chunk: FRESH) takes the call's own k and v in their place, rotates k, and
+// writes k and the cache -- memory that no other workgroup uses.  Rotary pairs are 64 dims apart (other widths and the
+// unrotated build: attn_prep_kernel before).
+struct FewSmem {
+    int tok[4][32];
+    float wm[4][64], wl[4][64];
+    float os[4][16][64][4];  // [wave][4j + v][lane][c]
+    // Until the outputs, 22 rows of 132 floats lie behind the first 4 KB of an os[w] (which are the fp32 path's): the rotated
+    // queries in os[3] and os[2], the FRESH workgroup's rotated k in os[1] and os[0].  (132: 16-byte reads of 32 rows at once
+    // fall on different banks)
+    __device__ __forceinline__ float* row(int l, int first) { return (l < 22 ? &os[first][4][0][0] + l * 132 : &os[first - 1][4][0][0] + (l - 22) * 132); }
+};
+template <typename T, bool ROPE, bool FRESH>
+__device__ __forceinline__ void attn_few_body(FewSmem& sm, const float* __restrict__ q, T* __restrict__ kc, T* __restrict__ vc, int qL, int64_t H, int64_t maxlen,
+                                              int kvLen, const int32_t* __restrict__ slots, float* __restrict__ part, int nchunks,
+                                              float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ inv_freq,
+                                              int position_id) {
+    constexpr int S = 128, P = sizeof(T) == 4 ? 3 : 2, IT = 8;  // (qL < 32: at most 8 tokens per wave)
+    auto& tok = sm.tok;
+    auto &wm = sm.wm, &wl = sm.wl;
+    auto& os = sm.os;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int hf = lane >> 5, c32 = lane & 31;
     const int chunk = blockIdx.x % nchunks;
     const int64_t bh = blockIdx.x / nchunks, b = bh / H, h = bh % H;
-    const int p0 = chunk * 128 + wave * 32;  // this wave's first cache row
-    const T* kbase = kc + bh * maxlen * S;
-    const T* vbase = vc + bh * maxlen * S;
+    const int p0 = chunk * 128 + wave * 32;  // this wave's first cache row (FRESH: wave 0's row is token c32)
+    T* kbase = kc + bh * maxlen * S;
+    T* vbase = vc + bh * maxlen * S;
+    const int64_t tokens = b * qL * H * S + h * S, stride = H * S;  // where the head's q, k, v rows start, and their distance
     const T* krow = kbase + (int64_t)min(p0 + c32, kvLen - 1) * S + 8 * hf;
-    float4 kr[16], vr[16], qr[16];
-    const float* qrow = q + ((b * qL + min(c32, qL - 1)) * H + h) * S + 8 * hf;
+    // row r of the wave's 32, four columns
+    const auto v_at = [&](int row, int col) {
+        if (!FRESH) return load4(vbase + (int64_t)min(p0 + row, kvLen - 1) * S + col);
+        const float4 x = load4(v + tokens + min(row, qL - 1) * stride + col);
+        return make_float4(cache_round<T>(x.x), cache_round<T>(x.y), cache_round<T>(x.z), cache_round<T>(x.w));
+    };
+    // (loads return in order: what masks and rotation need first)
+    const int my_slot = ROPE ? slots[min(lane, qL - 1)] : 0;  // (fewer than 32 tokens: a lane per slot)
+    float freq = 0.0f, qa[IT], qb[IT];
+    float4 qr[16];  // (unrotated build: the lane's query straight from memory)
+    if (ROPE) {
+        freq = inv_freq[lane];
 #pragma unroll
-    for (int i = 0; i < 8; i++) qr[2 * i] = load4(qrow + 16 * i), qr[2 * i + 1] = load4(qrow + 16 * i + 4);
+        for (int it = 0; it < IT; it++) {
+            const float* at = q + tokens + min(wave + 4 * it, qL - 1) * stride + lane;
+            qa[it] = at[0], qb[it] = at[64];
+        }
+    } else {
+        const float* at = q + tokens + min(c32, qL - 1) * stride + 8 * hf;
 #pragma unroll
-    for (int i = 0; i < 8; i++) kr[2 * i] = load4(krow + 16 * i), kr[2 * i + 1] = load4(krow + 16 * i + 4);
+        for (int i = 0; i < 8; i++) qr[2 * i] = load4(at + 16 * i), qr[2 * i + 1] = load4(at + 16 * i + 4);
+    }
+    float4 kr[16], vr[16];
+    if (!FRESH) {
 #pragma unroll
-    for (int r = 0; r < 16; r++) vr[r] = load4(vbase + (int64_t)min(p0 + 8 * (r >> 2) + 4 * hf + (r & 3), kvLen - 1) * S + 4 * c32);
+        for (int i = 0; i < 8; i++) kr[2 * i] = load4(krow + 16 * i), kr[2 * i + 1] = load4(krow + 16 * i + 4);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r++) vr[r] = v_at(8 * (r >> 2) + 4 * hf + (r & 3), 4 * c32);
     __builtin_amdgcn_sched_barrier(0);
-    {
-        // which token of this call wrote the lane's cache row (-1: none); rows past the end belong to nobody
+    if (!FRESH) {
+        // which token of this call wrote the lane's cache row (-1: none); rows past the end belong to nobody, and with ROPE
+        // neither do those of this call
         const int row = p0 + c32;
         int t = -1;
-        for (int l = 0; l < qL; l++) t = slots[l] == row ? l : t;
-        tok[wave][c32] = row < kvLen ? t : INT_MAX;
+        for (int l = 0; l < qL; l++) t = (ROPE ? __builtin_amdgcn_readlane(my_slot, l) : slots[l]) == row ? l : t;
+        tok[wave][c32] = row < kvLen && (!ROPE || t == -1) ? t : INT_MAX;
     }
+    if (ROPE) {
+#pragma unroll 1
+        for (int l = wave; l < qL; l += 4) {  // (a loop of its own: one copy of the long code behind cosf and sinf)
+            const float xita = freq * (float)(l + position_id);
+            float* to = sm.row(l, 3);
+            sincosf(xita, &to[lane + 64], &to[lane]);
+        }
+    }
+#pragma unroll
+    for (int it = 0; it < IT; it++) {
+        const int l = wave + 4 * it;  // (uniform)
+        if (!ROPE || l >= qL) break;
+        float* to = sm.row(l, 3);
+        const float c = to[lane], s = to[lane + 64];
+        to[lane] = c * qa[it] - s * qb[it];
+        to[lane + 64] = s * qa[it] + c * qb[it];
+        if (FRESH) {
+            const int slot = __builtin_amdgcn_readlane(my_slot, l);
+            // (of several tokens with one slot the last one's row stays)
+            const bool last = !__any(lane > l && lane < qL && my_slot == slot), stored = last && slot >= 0 && slot < maxlen;
+            float* at = k + tokens + l * stride + lane;
+            const float* vat = v + tokens + l * stride + lane;
+            const float k0 = at[0], k1 = at[64], r0 = c * k0 - s * k1, r1 = s * k0 + c * k1;
+            at[0] = r0, at[64] = r1;
+            if (stored) {
+                T *kdst = kbase + (int64_t)slot * S + lane, *vdst = vbase + (int64_t)slot * S + lane;
+                store_cache(kdst, r0), store_cache(kdst + 64, r1);
+                store_cache(vdst, vat[0]), store_cache(vdst + 64, vat[64]);
+            }
+            float* kto = sm.row(l, 1);
+            kto[lane] = cache_round<T>(r0), kto[lane + 64] = cache_round<T>(r1);
+            if (lane == 0) tok[0][l] = last && slot >= 0 && slot < kvLen ? l : INT_MAX;
+        }
+    }
+    if (FRESH) {
+        if (wave > 0 || lane >= qL) {
+            if (lane < 32) tok[wave][lane] = INT_MAX;
+        }
+    }
+    if (ROPE) __syncthreads();
+    // no product with what a row holds that nobody sees: a weight of 0 does not take away an infinity
+    const auto unseen = [&](int row) { return ROPE && tok[wave][row] == INT_MAX; };
+    if (FRESH) {
+        const float* mine = sm.row(min(c32, qL - 1), 1) + 8 * hf;
+#pragma unroll
+        for (int i = 0; i < 8; i++) kr[2 * i] = load4(mine + 16 * i), kr[2 * i + 1] = load4(mine + 16 * i + 4);
+    }
+    if (ROPE && (FRESH || __any(unseen(c32)))) {
+        const bool none = unseen(c32);
+#pragma unroll
+        for (int i = 0; i < 16; i++) kr[i] = make_float4(none ? 0.f : kr[i].x, none ? 0.f : kr[i].y, none ? 0.f : kr[i].z, none ? 0.f : kr[i].w);
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const bool off = unseen(8 * (r >> 2) + 4 * hf + (r & 3));
+            vr[r] = make_float4(off ? 0.f : vr[r].x, off ? 0.f : vr[r].y, off ? 0.f : vr[r].z, off ? 0.f : vr[r].w);
+        }
+    }
+    const float* qrow = sm.row(min(c32, qL - 1), 3) + 8 * hf;
     // (two accumulators for the leading products and one for the small ones: fewer roundings at full size)
     v16f s0[2], s1;
 #pragma unroll
@@ -344,8 +475,9 @@ __global__ __launch_bounds__(256, 2) void attn_few_kernel(const float* __restric
         Bf3 a, w;
         split_bf<P>(a, 0, kr[2 * i].x, kr[2 * i].y), split_bf<P>(a, 1, kr[2 * i].z, kr[2 * i].w);
         split_bf<P>(a, 2, kr[2 * i + 1].x, kr[2 * i + 1].y), split_bf<P>(a, 3, kr[2 * i + 1].z, kr[2 * i + 1].w);
-        split_bf<3>(w, 0, qr[2 * i].x, qr[2 * i].y), split_bf<3>(w, 1, qr[2 * i].z, qr[2 * i].w);
-        split_bf<3>(w, 2, qr[2 * i + 1].x, qr[2 * i + 1].y), split_bf<3>(w, 3, qr[2 * i + 1].z, qr[2 * i + 1].w);
+        const float4 q0 = ROPE ? load4(qrow + 16 * i) : qr[2 * i], q1 = ROPE ? load4(qrow + 16 * i + 4) : qr[2 * i + 1];
+        split_bf<3>(w, 0, q0.x, q0.y), split_bf<3>(w, 1, q0.z, q0.w);
+        split_bf<3>(w, 2, q1.x, q1.y), split_bf<3>(w, 3, q1.z, q1.w);
         s0[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[0].h, w.p[0].h, s0[i & 1], 0, 0, 0);
         if (P == 3) s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[2].h, w.p[0].h, s1, 0, 0, 0);
         s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[0].h, w.p[2].h, s1, 0, 0, 0);
@@ -361,7 +493,12 @@ __global__ __launch_bounds__(256, 2) void attn_few_kernel(const float* __restric
 #pragma unroll
     for (int r = 0; r < 16; r++) z = fmaf(pr[r], 0.0f, z);
     if (__builtin_expect(__any(z != 0.0f), 0))
-        few_scores_fp32<T>(krow, q + (b * qL * H + h) * S + 8 * hf, qL, H * S, &os[wave][0][0][0], c32, hf, pr);
+        few_scores_fp32(
+            [&](int d) {
+                if (unseen(c32)) return make_float4(0.f, 0.f, 0.f, 0.f);
+                return FRESH ? load4(sm.row(min(c32, qL - 1), 1) + 8 * hf + d) : load4(krow + d);
+            },
+            [&](int l, int d) { return load4((ROPE ? sm.row(l, 3) : q + tokens + l * stride) + 8 * hf + d); }, qL, &os[wave][0][0][0], c32, hf, pr);
     float mx = -FLT_MAX;
 #pragma unroll
     for (int jj = 0; jj < 4; jj++) {
@@ -394,7 +531,8 @@ __global__ __launch_bounds__(256, 2) void attn_few_kernel(const float* __restric
     for (int r = 0; r < 16; r++) big[r & 1] = max_abs(big[r & 1], vr[r]);
     big[0] = fmaxf(big[0], big[1]);
     if (__builtin_expect(__any(big[0] > kFewMax || (big[0] < kFewMin && big[0] > 0.0f)), 0)) {
-        few_outputs_fp32<T>(vbase, p0, kvLen, c32, hf, pr, &os[wave][0][lane][0]);
+        few_outputs_fp32([&](int row, int col) { return unseen(row) ? make_float4(0.f, 0.f, 0.f, 0.f) : v_at(row, col); }, hf, pr,
+                         &os[wave][0][lane][0]);
     } else {
         v16f o[4];
 #pragma unroll
@@ -452,6 +590,17 @@ __global__ __launch_bounds__(256, 2) void attn_few_kernel(const float* __restric
         for (int w = 0; w < 4; w++) l += wl[w][lane] + wl[w][lane + 32];
         *reinterpret_cast<float2*>(rec) = make_float2(mx, l);
     }
+}
+template <typename T, bool ROPE>
+__global__ __launch_bounds__(256, 2) void attn_few_kernel(const float* __restrict__ q, T* __restrict__ kc, T* __restrict__ vc, int qL, int64_t H, int64_t maxlen,
+                                                           int kvLen, const int32_t* __restrict__ slots, float* __restrict__ part,
+                                                           int nchunks, float* __restrict__ k, const float* __restrict__ v,
+                                                           const float* __restrict__ inv_freq, int position_id) {
+    __shared__ __align__(16) FewSmem sm;
+    if (ROPE && blockIdx.x % nchunks == nchunks - 1)
+        attn_few_body<T, ROPE, true>(sm, q, kc, vc, qL, H, maxlen, kvLen, slots, part, nchunks, k, v, inv_freq, position_id);
+    else
+        attn_few_body<T, ROPE, false>(sm, q, kc, vc, qL, H, maxlen, kvLen, slots, part, nchunks, k, v, inv_freq, position_id);
 }
 
 // Merge of the chunk records of one query: out = sum_c exp(m_c - M) o_c / sum_c exp(m_c - M) s_c.
@@ -557,31 +706,6 @@ __global__ __launch_bounds__(128) void attn_merge_kernel(float* __restrict__ q, 
 // The position may come from device memory (pos_dev != nullptr): a HIP graph of a decode step captures the
 // launch once, for the largest kv length (the grid and the record layout are sized by `nchunks`), and every
 // replay reads the current position; workgroups whose chunk lies beyond the current kv length leave at once.
-template <typename T>
-__device__ __forceinline__ float cache_round(float v);
-template <>
-__device__ __forceinline__ float cache_round<float>(float v) {
-    return v;
-}
-template <>
-__device__ __forceinline__ float cache_round<__half>(float v) {
-    return __half2float(__float2half_rn(v));
-}
-template <typename T>
-__device__ __forceinline__ void store4(T* dst, float4 v);
-template <>
-__device__ __forceinline__ void store4<float>(float* dst, float4 v) {
-    *reinterpret_cast<float4*>(dst) = v;
-}
-template <>
-__device__ __forceinline__ void store4<__half>(__half* dst, float4 v) {
-    const __half2 a = __floats2half2_rn(v.x, v.y), b = __floats2half2_rn(v.z, v.w);
-    uint2 u;
-    u.x = *reinterpret_cast<const uint32_t*>(&a);
-    u.y = *reinterpret_cast<const uint32_t*>(&b);
-    *reinterpret_cast<uint2*>(dst) = u;
-}
-
 // rotate the lane's 4 elements (index e4 = first element) of a 128-wide head vector at `base`;
 // cs = cos table [half], sn = sin table [half] of the current position (LDS)
 __device__ __forceinline__ float4 rope4(const float* base, int e4, const float* cs, const float* sn, int half) {
@@ -1503,12 +1627,28 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
     const bool tiled = plan.kernel == 3;
     if (!tiled && (int64_t)bhq * nchunks > max_records)
         return fail(LLMOPS_EWORKSPACE, "attention workspace too small for %lld chunk records", (long long)bhq * nchunks);
-    if (tiled) {
-        fill_i32_kernel<<<(unsigned)((maxlen + 255) / 256), 256, 0, st>>>(row_token, maxlen, -1);
+    // All tokens of a head together: rotation and cache update ride in the same launch where the rotary pairs suit it, the
+    // workspace has a record more per query, and the workgroup more per head makes no compute unit take one more: then the
+    // launch saved is worth more than what every workgroup does for it, 1.2 us (us, separate / together, 32 heads: 8 tokens
+    // behind 500 18.4 / 16.3, 31 behind 97 20.5 / 18.4, 16 behind 1500 26.4 / 24.5, halves 23.1 / 21.6; 4 behind 1000 20.2 / 21.1, 31
+    // behind 3500 48.3 / 48.7; 128 heads, 16 behind 500 34.3 / 35.7).
+    const int64_t wgs = B * H * nchunks, wgs_rope = wgs + B * H;
+    if (plan.kernel == 2 && half == 64 && (int64_t)bhq * (nchunks + 1) <= max_records && wgs_rope <= 512 && (wgs > 256) == (wgs_rope > 256)) {
+        attn_few_kernel<T, true><<<(unsigned)wgs_rope, 256, 0, st>>>(q, kc, vc, (int)qL, H, maxlen, (int)kvLen, slots, part,
+                                                                                   nchunks + 1, k, v, inv_freq, position_id);
         LLMOPS_LAUNCH_CHECK();
+        attn_merge_kernel<<<(unsigned)bhq, 128, 0, st>>>(q, part, qL, H, nchunks + 1);
+        LLMOPS_LAUNCH_CHECK();
+        return LLMOPS_OK;
     }
-    attn_prep_kernel<T><<<(unsigned)(B * qL * H), 64, 0, st>>>(q, k, v, qL, H, S, inv_freq, half, kc, vc, maxlen, slots,
-                                                              position_id, tiled ? row_token : nullptr);
+    if (tiled) {
+        const unsigned tables = (unsigned)((kvLen + 63) / 64);
+        attn_prep_kernel<T, true><<<(unsigned)(B * qL * H) + tables, 64, 0, st>>>(q, k, v, qL, H, S, inv_freq, half, kc, vc, maxlen, slots,
+                                                                                 position_id, row_token, kvLen, tables);
+    } else {
+        attn_prep_kernel<T, false><<<(unsigned)(B * qL * H), 64, 0, st>>>(q, k, v, qL, H, S, inv_freq, half, kc, vc, maxlen, slots,
+                                                                         position_id, nullptr, 0, 0);
+    }
     LLMOPS_LAUNCH_CHECK();
     if (tiled) {
         // enough query tokens to share K/V tiles: the MFMA kernel reads the cache once per 128 queries
@@ -1532,7 +1672,8 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
         return LLMOPS_OK;
     }
     if (plan.kernel == 2)
-        attn_few_kernel<T><<<(unsigned)(B * H * nchunks), 256, 0, st>>>(q, kc, vc, (int)qL, H, maxlen, (int)kvLen, slots, part, nchunks);
+        attn_few_kernel<T, false><<<(unsigned)(B * H * nchunks), 256, 0, st>>>(q, kc, vc, (int)qL, H, maxlen, (int)kvLen, slots, part,
+                                                                               nchunks, nullptr, nullptr, nullptr, 0);
     else if (plan.pw == 16)
         attn_split_kernel<T, 16><<<(unsigned)(bhq * nchunks), 256, 0, st>>>(q, kc, vc, qL, H, maxlen, kvLen, slots, part, nchunks);
     else if (plan.pw == 8)
