@@ -210,8 +210,17 @@ static int fc_decode_impl(const float* x, int64_t rows, int64_t K, const int8_t*
     if (workspace_bytes < need)
         return fail(LLMOPS_EWORKSPACE, "fc_Q4A needs %zu workspace bytes, got %zu", need, workspace_bytes);
     uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
-    if (rows > kMaxGemvRows) {
-        // More rows than the streaming kernel takes: the producer is folded into the quantization launch instead
+    // From two rows on a producer costs the streaming kernel more than the launch that the other way takes: every strip's
+    // workgroup forms it again for every row.  Without one the rows count as in fc_Q4A, with one they are one fewer.  (us,
+    // streaming / quantization launch and product, 2 and 8 rows: rmsnorm, 12288 x 4096 17.9 / 13.4 and 36.6 / 13.3, 22016 x 4096
+    // 25.0 / 17.1 and 53.8 / 17.8, 55296 x 4096 54.4 / 30.3 and 122.6 / 32.1; silu * up, 4096 x 11008, 3 and 8 rows 13.0 / 12.8 and
+    // 27.7 / 12.2; residual, 4096 x 4096, 4 and 8 rows 9.3 / 8.6 and 11.0 / 8.7.)
+    const int rows_from = (Ng > 256 ? g_rows_from_large : g_rows_from_small) - (norm_w != nullptr || glu == 2 ? 1 : 0);
+    const bool quantize_first = group_k == 128 && Ng >= 64 && gemm_rows_kernel_enabled() && glu != 1 && rows >= rows_from &&
+                                ((norm_w == nullptr && glu != 2) || aligned(x, 16)) &&
+                                (norm_w == nullptr || (K <= 16384 && aligned(norm_w, 16)));
+    if (rows > kMaxGemvRows || quantize_first) {
+        // More rows than the streaming kernel takes or is good at: the producer is folded into the quantization launch instead
         // (its fp32 result never goes through memory), the residual into the product's stores, and the sums of
         // squares take a launch of their own.  The statistic of the rmsnorm is computed from the row (sumsq_in is
         // not needed: the launch has the whole row in registers).

@@ -196,8 +196,9 @@ class LlamaDecoder:
         H, F = self.configs["hidden_size"], self.configs["intermediate_size"]
         n1, n2 = ops["input_layernorm"], ops["post_attention_layernorm"]
         rows = hidden_states.shape[0] * hidden_states.shape[1]
-        many = rows > 8  # a prompt or a batch: the sums of squares are not handed on (the norms read their rows)
-        if many:  # q, k and v as three dense [B,qL,H*S] tensors straight from the product
+        # a prompt or a batch: the sums of squares are not handed on (the norms read their rows)
+        many = rows > 8 or (rows > 1 and all(llmops.group_k_of(ops[n].weight) == 128 for n in ("o_proj", "down_proj")))
+        if rows > 8:  # q, k and v as three dense [B,qL,H*S] tensors straight from the product
             q, k, v = llmops.fc_Q4A_decode(hidden_states, ops["qkv_proj"].weight, 3 * H, norm=(n1.weight, n1.eps), out_parts=3)
         else:
             qkv = llmops.fc_Q4A_decode(hidden_states, ops["qkv_proj"].weight, 3 * H, norm=(n1.weight, n1.eps), sumsq_in=sumsq)
