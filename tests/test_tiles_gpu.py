@@ -1,0 +1,135 @@
+"""Edges of the tiled product, of the weight-streaming one and of the launches that were folded together, against the oracle.
+Outputs are fp32 sums of exact int32 group sums: 1e-5 of the largest, as elsewhere."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import max_rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    import llmops
+    return llmops
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _inputs(rows, N, K, seed):
+    rng = np.random.default_rng(seed)
+    return (rng.standard_normal((1, rows, K)).astype(np.float32), (rng.standard_normal((N, K)) * 0.02).astype(np.float32),
+            rng.standard_normal((1, rows, N)).astype(np.float32))
+
+
+@pytest.mark.parametrize("tile", [1, 2, 4])
+@pytest.mark.parametrize("rows,N,Kg,split", [
+    (17, 33, 1, 1), (31, 64, 2, 1), (33, 130, 3, 3), (65, 257, 5, 2), (127, 96, 6, 3), (129, 160, 7, 7), (40, 1000, 13, 12), (131, 32, 25, 12)])
+def test_tiled_product_edges(ops, orc, tile, rows, N, Kg, split):
+    """Row counts around a tile and a row tile, odd ones (whose last row has a place of its own among the partial sums),
+    columns that end inside a strip and strips inside a tile, runs of one k-group up, runs shorter and longer than the LDS slots and than the
+    four k-groups whose min term is formed together; with the residual, and parts against the slices of the whole."""
+    from llmops import _lib
+    lib = _lib.load()
+    x, w, res = _inputs(rows, N, 128 * Kg, rows + Kg)
+    pw = orc.quant_w(w, 128)
+    want = orc.fc(x, pw, N)
+    lib.llmops_test_gemm_set_tuning(tile)
+    lib.llmops_test_gemm_set_split(split)
+    try:
+        got = ops.fc_Q4A(dev(x), dev(pw), N).cpu().numpy()
+        got_res = ops.fc_Q4A(dev(x), dev(pw), N, residual=dev(res)).cpu().numpy()
+        strips = pw.shape[0] - pw.shape[0] % 3
+        if strips:
+            p3 = dev(pw[:strips])
+            whole = ops.fc_Q4A_decode(dev(x), p3, strips * 32)
+            parts = ops.fc_Q4A_decode(dev(x), p3, strips * 32, out_parts=3)
+            assert torch.equal(torch.cat(list(parts), dim=-1), whole)
+    finally:
+        lib.llmops_test_gemm_set_tuning(0)
+        lib.llmops_test_gemm_set_split(0)
+    assert max_rel_err(got, want) <= 1e-5
+    assert max_rel_err(got_res, want + res) <= 1e-5
+
+
+@pytest.mark.parametrize("rows", [40, 300])
+def test_tiled_product_sums_that_overflow(ops, orc, rows):
+    """A row whose group sum is beyond fp32 although its values are not: infinite outputs where the min says so, in that
+    row and nowhere else."""
+    x, w, _ = _inputs(rows, 96, 640, 3)
+    x[0, 7, 128:256] = 3e36
+    pw = orc.quant_w(w, 128)
+    want = orc.fc(x, pw, 96)
+    got = ops.fc_Q4A(dev(x), dev(pw), 96).cpu().numpy()
+    assert np.isinf(want[0, 7]).all() and np.array_equal(got[0, 7], want[0, 7])
+    other = np.arange(rows) != 7
+    assert max_rel_err(got[0, other], want[0, other]) <= 1e-5
+
+
+@pytest.mark.parametrize("rows", [3, 16, 17, 32])
+@pytest.mark.parametrize("N,Kg", [(2048, 1), (2050, 15), (2048, 16), (2080, 35), (2048, 49), (8224, 33), (8224, 66)])
+def test_few_row_product_runs(ops, orc, rows, N, Kg):
+    """The weight-streaming product where a wave has one k-group, 2, 3, 4 or more of them, halves of K and all of it."""
+    x, w, _ = _inputs(rows, N, 128 * Kg, rows + Kg)
+    pw = orc.quant_w(w, 128)
+    assert max_rel_err(ops.fc_Q4A(dev(x), dev(pw), N).cpu().numpy(), orc.fc(x, pw, N)) <= 1e-5
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("N,K,off", [(2048, 512, 0), (2048, 512, 2), (8224, 256, 0), (96, 512, 0)])
+def test_two_to_eight_rows_with_a_producer(ops, orc, rows, N, K, off):
+    """rmsnorm, silu(gate) * up and residual around the product of few rows against the separate operators, on either
+    side of the rule that sends them to the quantization launch: rows, strips (64, more than 256, too few), an input that
+    does not start on 16 bytes."""
+    rng = np.random.default_rng(rows + N + off)
+    pw = ops.offline_FC_quant_Q4A(dev((rng.standard_normal((N, K)) * 0.02).astype(np.float32)), 128)
+
+    def shifted(shape):  # (a dense tensor that starts 4 * off bytes behind an allocation)
+        flat = dev(rng.standard_normal(int(np.prod(shape)) + off).astype(np.float32))
+        return flat[off:].view(shape)
+
+    x, gu, nw = shifted((1, rows, K)), shifted((1, rows, 2 * K)), dev(rng.standard_normal(K).astype(np.float32))
+    res = dev(rng.standard_normal((1, rows, N)).astype(np.float32))
+
+    def close(got, want):
+        assert max_rel_err(got.cpu().numpy(), want.cpu().numpy()) <= 1e-5
+
+    close(ops.fc_Q4A_decode(x, pw, N, residual=res), ops.fc_Q4A(x, pw, N) + res)
+    if off == 0:
+        close(ops.fc_Q4A_decode(x, pw, N, norm=(nw, 1e-5)), ops.fc_Q4A(ops.rmsnorm_out(x, nw, 1e-5), pw, N))
+    close(ops.fc_Q4A_decode(gu, pw, N, glu_in=True), ops.fc_Q4A(ops.silu_mul(gu), pw, N))
+    y, ss = ops.fc_Q4A_decode(x, pw, N, residual=res, want_sumsq=True)
+    pad = torch.nn.functional.pad(y.reshape(rows, N).double(), (0, -N % 32))
+    assert ((ss.double() - (pad ** 2).reshape(rows, -1, 32).sum(-1)).abs() <= 1e-5 * ss.double().abs().clamp(min=1e-3)).all()
+
+
+@pytest.mark.parametrize("cache_dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("qL,past,H", [(16, 300, 32), (31, 96, 32), (9, 1000, 32), (22, 200, 16), (23, 200, 16)])
+def test_attention_does_not_read_the_rows_it_replaces(ops, qL, past, H, cache_dtype):
+    """What the cache held where the call's own rows go, and behind them, must not matter, be it infinities or NaN; rotary
+    pairs 64 dims apart (one launch for rotation and scores) and 32 (two)."""
+    S, rows = 128, past + qL + 40
+    gen = torch.Generator(device="cuda").manual_seed(qL)
+    q, k, v = (torch.randn(1, qL, H * S, generator=gen, device="cuda") for _ in range(3))
+    clean = torch.randn(2, 1, H, rows, S, generator=gen, device="cuda").to(cache_dtype)
+    slots = torch.arange(past, past + qL, dtype=torch.int32, device="cuda")
+    slots[2], slots[qL - 1] = 5, rows + 7  # one inside the old rows, one outside the cache
+    for half in (64, 32):
+        inv = 1.0 / (10000.0 ** (torch.arange(half, device="cuda").float() / half))
+        outs = []
+        for stale in (0.0, float("nan"), float("inf")):
+            cache = clean.clone()
+            cache[:, :, :, past:past + qL - 1] = stale
+            cache[:, :, :, past + 2] = 1.0  # (row of no token: an old row like the others)
+            cache[:, :, :, past + qL - 1:] = stale  # (behind all tokens but one that has no row)
+            cache[:, :, :, past + qL - 1] = 1.0
+            cache[:, :, :, 5] = stale
+            a = [q.clone(), k.clone()]
+            ops.attention_rope2(a[0], a[1], v, inv, cache, slots, past, 0)
+            outs.append(a + [cache[:, :, :, :past + qL]])  # (what lies behind stays as it was)
+        for o in outs[1:]:
+            assert all(torch.equal(s, t) for s, t in zip(o, outs[0]))
+        assert torch.isfinite(outs[0][0]).all()
