@@ -402,10 +402,10 @@ __global__ __launch_bounds__(256, (RT == 4 ? 2 : (RT == 2 ? 3 : 4))) void fc_gem
         fold(P - 1);
         if (!PARTIALS && (since == 3 || kb + 1 == kb1)) {
             // Min term sum_kb m[n,kb]*gsum[row,kb]: a rank-Kg product, done four k-groups at a time straight into the fp32
-            // accumulators; lane (jj, g) has gsum of row jj and m of its columns for the group with index g of the four.
-            // gsum = three and m = two bf16 pieces, exactly and at any scale (as in fc_gemm_g32_kernel); the six products of a
-            // k-group fit into the eight slots that a lane has in v_mfma_f32_16x16x32_bf16.  An infinity has no pieces: it is
-            // in the first product alone, zeros stand for it in the others.
+            // accumulators by v_mfma_f32_16x16x4_f32; lane (jj, g) has gsum of row jj and m of its columns for the group with
+            // index g of the four.  (On the bf16 matrix cores, both factors in exact pieces, it is no faster -- 2048 x 11008 x 4096
+            // 158.7 to 159.9 us against 160.1 to 162.9, 2048 x 4096 x 11008 151.5 against 151 -- and its sums lose more: rms error
+            // against 64 bits 1.85e-7 of the outputs at K = 4096 where this has 1.62e-7.)
             int mine = ring - since + g;
             mine += mine < 0 ? kMinRing : 0;
             const bool live = g <= since;
@@ -415,22 +415,14 @@ __global__ __launch_bounds__(256, (RT == 4 ? 2 : (RT == 2 ? 3 : 4))) void fc_gem
 #pragma unroll
             for (int t = 0; t < T; t++) gv[t] = gsr[t * 16];
             __builtin_amdgcn_sched_barrier(0);
-            Bf16x8 mb[2];
+            float mv[2];
 #pragma unroll
-            for (int c = 0; c < 2; c++) {
-                const float mv = live ? f16_bits_to_f32((uint16_t)(c == 0 ? mh & 0xFFFFu : mh >> 16)) : 0.0f;
-                const float mf = __builtin_isinf(mv) ? 0.0f : mv, m2 = mf - bf_piece(mf);
-                mb[c].u[0] = bf_pair(mv, mf), mb[c].u[1] = __float_as_uint(mf);
-                mb[c].u[2] = bf_pair(m2, m2), mb[c].u[3] = __float_as_uint(m2);
-            }
+            for (int c = 0; c < 2; c++) mv[c] = live ? f16_bits_to_f32((uint16_t)(c == 0 ? mh & 0xFFFFu : mh >> 16)) : 0.0f;
 #pragma unroll
             for (int t = 0; t < T; t++) {
                 gv[t] = live ? gv[t] : 0.0f;
-                const float gf = __builtin_isinf(gv[t]) ? 0.0f : gv[t], g2 = gf - bf_piece(gf), g3 = g2 - bf_piece(g2);
-                Bf16x8 ga;
-                ga.u[0] = bf_pair(gv[t], g2), ga.u[2] = bf_pair(gf, g2), ga.u[1] = ga.u[3] = __float_as_uint(g3);
 #pragma unroll
-                for (int c = 0; c < 2; c++) f[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga.h, mb[c].h, f[t][c], 0, 0, 0);
+                for (int c = 0; c < 2; c++) f[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(gv[t], mv[c], f[t][c], 0, 0, 0);
             }
         }
         since = since == 3 ? 0 : since + 1;

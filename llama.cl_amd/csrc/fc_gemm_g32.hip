@@ -42,6 +42,17 @@ constexpr int kG32Rows = 32;       // rows and strips of a tile
 constexpr int kG32Strips = 8;
 constexpr int kG32Gps = 4;         // k-groups per stage
 
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+union Bf16x8 {
+    v8bf h;
+    uint32_t u[4];
+};
+// the first 8 significant bits of a float (what its upper half is as a bf16), and the upper halves of two floats
+__device__ __forceinline__ float bf_piece(float v) { return __uint_as_float(__float_as_uint(v) & 0xFFFF0000u); }
+__device__ __forceinline__ uint32_t bf_pair(float lo, float hi) {
+    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+
 // PARTIALS: test build that stores the int32 sums of every (row, column, k-group) into out_i ([rows][Ng*32][Kg])
 // WIDE: lane offsets of 64 bits, for a K whose eight strips are 4 GiB and more (K above 26.8 million)
 template <bool PARTIALS, bool WIDE>

@@ -12,23 +12,6 @@ typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-union Halves8 {
-    v8h h;
-    uint32_t u[4];
-};
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-union Bf16x8 {
-    v8bf h;
-    uint32_t u[4];
-};
-// the first 8 significant bits of a float (what its upper half is as a bf16), and the upper halves of two floats
-__device__ __forceinline__ float bf_piece(float v) { return __uint_as_float(__float_as_uint(v) & 0xFFFF0000u); }
-__device__ __forceinline__ uint32_t bf_pair(float lo, float hi) {
-    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
 
 constexpr int kFoldBiasBits = 0x4B400000;  // the float 1.5 * 2^23 ...
 constexpr float kFoldBias = 12582912.0f;   // ... whose low mantissa bits count in units of 1
@@ -62,10 +45,5 @@ __device__ __forceinline__ void copy16_to_lds(const void* base, uint64_t off, ui
 __device__ __forceinline__ void copy4_to_lds(const void* base, uint64_t off, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(reinterpret_cast<uint64_t>(base) + off), "s"(lds_base) : "memory", "m0");
 }
-
-// 16 bytes from a 4-byte boundary
-struct __attribute__((packed, aligned(4))) Float4U {
-    float v[4];
-};
 
 }  // namespace llmops
