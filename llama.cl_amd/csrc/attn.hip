@@ -4,7 +4,8 @@
 // One query token: attn_decode_kernel (everything in one launch) and attn_merge_kernel.  More:
 //   1. attn_prep_kernel   rotate q and k in place (rope_embed, ops/op_attn.hpp:44-94), write the
 //                         rotated k and the v rows into the cache at slots[p] (:764-773), and
-//                         from 32 tokens on record which cache rows were written by which token of this call.
+//                         from 32 tokens on record which cache rows were written by which token of this call
+//                         (attn_few_kernel does the first two itself where that saves time).
 //   2. below 32 tokens    attn_split_kernel or attn_few_kernel: a workgroup takes a chunk of cache rows and leaves
 //                         per query the chunk's score maximum, its sum of exponentials and its weighted V sum.
 //      from 32 on         attn_prefill_kernel: 128 queries to a workgroup, the cache rows in one piece or in several.
