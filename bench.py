@@ -41,7 +41,7 @@ MEASURED_TRAFFIC_PROFILE = "profiles/fc_gemv_fused_kernel__hbm_traffic_pmc.md"
 PROFILE_SOURCES = {
     "profiles/fc_gemv_fused_kernel__hbm_traffic_pmc.md": (("fc_gemv.hip", "gemv_device.h"), "13290cb794320013"),
     "profiles/fc_gemv_fused_kernel__vector_alu_pmc.md": (("fc_gemv.hip", "gemv_device.h"), "13290cb794320013"),
-    "profiles/fc_gemm_kernels__prefill_g128_pmc.md": (("fc_gemm.hip", "gemm_device.h", "fc_rows.hip", "q8_act.hip"), "7b780da08a380fc9"),
+    "profiles/fc_gemm_kernels__prefill_g128_pmc.md": (("fc_gemm.hip", "gemm_device.h", "fc_rows.hip", "q8_act.hip"), "8a34ec47bbe352e1"),
     "profiles/attn_prefill_kernel__prompt_2048_pmc.md": (("attn.hip",), "b8d23a92c7c2c397"),
     "profiles/fc_gemm_g32_attn_few_quant_w_kernels__pmc.md": (("fc_gemm_g32.hip", "gemm_device.h", "attn.hip", "q4_pack.hip"), "ddfe6c3880745663"),
 }

@@ -100,10 +100,11 @@ static int fc_product_many_rows(const uint8_t* w, uint8_t* ws, const FcWorkspace
     const float2* xst = reinterpret_cast<const float2*>(ws + lay.off_xst);
     const bool rows_kernel = group_k == 128 && Ng >= 64 && gemm_rows_kernel_enabled();
     // up to 16 rows are still bound by the weight stream: one strip per workgroup, MFMA inner product
-    // (measured against the tiled kernel: 15 vs 18 us at 16 rows, 11008x4096).  17..32 rows (two row tiles
-    // per wave) only win for tensors of fewer than 256 strips, where the tiled kernel has too few tiles
-    // (us, tiled / streaming: 4096x4096 at 17 rows 20.2 / 9.9, at 32 rows 24.3 / 11.9; 4096x11008 at 24 rows
-    // 22.0 / 15.7; 11008x4096 at 24 rows 19.3 / 18.8; 12288x4096 17.9 / 19.0; 22016x4096 23.0 / 27.4)
+    // (us, tiled / streaming: 16 rows 11008x4096 14.6 / 13.5, 22016x4096 21.3 / 17.9).  17..32 rows (two row tiles
+    // per wave) win for tensors of fewer than 256 strips, where the tiled kernel has too few tiles (4096x4096 at 17 rows
+    // 15.4 / 9.5, at 32 rows 13.7 / 10.4; 4096x11008 at 24 rows 16.4 / 15.0), and mostly not beyond (11008x4096 at 17 rows
+    // 17.2 / 16.0, at 24 rows 15.4 / 16.8, at 32 rows 16.2 / 17.7; 22016x4096 at 24 rows 23.3 / 22.1; 55296x4096 at 32 rows
+    // 38.6 / 46.2; 11008x11008 at 24 rows 27.0 / 35.6)
     if (rows_kernel && (rows <= 16 || (rows <= 32 && Ng < 256)))
         return launch_fc_rows(w, xq, xst, y, rows, Ng, Kg, N, residual, parts, reinterpret_cast<unsigned long long*>(ws + kTicketBytes),
                               LLMOPS_FC_COUNTER_BYTES - kTicketBytes, st);
@@ -133,11 +134,11 @@ static int fc_impl(const float* x, int64_t rows, int64_t K, const int8_t* weiq, 
     // weight byte grows with the row count (every row is quantized and dotted separately), while the time of
     // the weight-streaming MFMA kernel below hardly depends on it, separate quantization launch included
     // (us, streaming / MFMA):
-    //   4096x4096 (128 strips):    2 rows  6.0 /  8.0, 3 rows  7.5 /  8.2, 4 rows  8.3 /  8.2, 8 rows 10.2 /  8.4
-    //   4096x11008 (128 strips):   2 rows  9.3 / 11.6, 3 rows 11.5 / 11.8, 4 rows 13.0 / 12.0, 8 rows 20.3 / 12.5
-    //   8192x4096 (256 strips):    2 rows  6.7 /  8.9, 3 rows  8.1 /  8.6, 4 rows  8.8 /  8.6, 8 rows 14.5 /  8.9
-    //   12288x4096 (384 strips):   2 rows  9.3 / 12.0, 3 rows 13.4 / 11.6, 4 rows 15.6 / 11.7, 8 rows 22.4 / 12.2
-    //   22016x4096 (688 strips):   2 rows 12.8 / 16.1, 3 rows 20.1 / 16.0, 4 rows 22.2 / 15.3, 8 rows 31.0 / 16.1
+    //   4096x4096 (128 strips):    2 rows  6.4 /  7.7, 3 rows  8.0 /  7.9, 4 rows  8.9 /  7.8, 8 rows 10.5 /  7.9
+    //   4096x11008 (128 strips):   2 rows  9.2 / 12.0, 3 rows 11.0 / 12.2, 4 rows 12.2 / 12.2, 8 rows 20.3 / 12.6
+    //   8192x4096 (256 strips):    2 rows  7.2 /  9.5, 3 rows  8.6 /  8.9, 4 rows  9.5 /  9.0, 8 rows 14.9 /  9.1
+    //   12288x4096 (384 strips):   2 rows  9.6 / 12.4, 3 rows 13.8 / 12.7, 4 rows 15.7 / 12.8, 8 rows 22.9 / 13.1
+    //   22016x4096 (688 strips):   2 rows 13.1 / 16.1, 3 rows 19.9 / 16.2, 4 rows 22.9 / 16.4, 8 rows 31.8 / 16.7
     if (k_tail) {
         // K is not a whole number of k-groups (no shape the reference is used with): the general quantization kernel
         // pads the last group's codes with zeros, as FC_dynamic_quantize_x does, and the product runs on the codes

@@ -148,8 +148,8 @@ __device__ __forceinline__ void splitk_finish(const v4f (&f)[T][2], float* __res
 // A 256 x 128 tile with two wave groups (one workgroup per compute unit, 20 % less to copy) takes 165 to 170 us at
 // 2048 x 11008 x 4096 where 128 rows take 156: nothing covers its barriers, its first fetch and its stores.
 // Measured, us for the whole call in a graph, kernels before (weights and codes through registers below 512 rows, two wave
-// groups in alternating phases from there on) and now: 128 x 4096 x 11008 27.5 / 24.4, 300 x 4090 x 11008 46 / 39, 512 x 4096^2
-// 33.8 / 27.7, 512 x 22016 x 4096 102.5 / 88, 512 x 4096 x 11008 57 / 53, 2048 x 11008 x 4096 164 / 157, 2048 x 4096 x 11008 153 / 150.
+// groups in alternating phases from there on) and now: 128 x 4096 x 11008 27.5 / 23.4, 300 x 4090 x 11008 46 / 39, 512 x 4096^2
+// 33.8 / 27.7, 512 x 22016 x 4096 102.5 / 90, 512 x 4096 x 11008 57 / 53, 2048 x 11008 x 4096 164 / 157, 2048 x 4096 x 11008 153 / 151.
 constexpr int kBlk128 = 2176;
 constexpr int kStages = 3;    // LDS slots of a k-group: one is multiplied, one has landed, one is on its way
 constexpr int kMinRing = 6;   // LDS slots of sums and mins: the last four k-groups and the two ahead
