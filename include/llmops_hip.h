@@ -136,13 +136,17 @@ int llmops_fc_Q4A_residual(const float* x, int64_t rows, int64_t K, const int8_t
                            int group_k, int64_t N, const float* residual, float* y, void* workspace,
                            size_t workspace_bytes, llmops_stream_t stream);
 
-/* fc_Q4A with the neighbouring ops of chatllama/main.py:344-375 folded in.  Up to 8 rows (a decode step) it is
- * one launch.  With more rows (a batch of decode steps, a prompt) the producer of the input -- rmsnorm, or
- * silu(gate)*up -- runs inside the quantization launch, so that its fp32 result never passes through memory,
- * the residual is added in the product's stores and the sums of squares take a launch of their own; the codes,
- * scales and results are those of the separate ops (llmops_rmsnorm_out / llmops_silu_mul, then llmops_fc_Q4A).
- * More than 8 rows need whole 16-byte aligned rows, take glu 0 or 2 (2 with group 128 only), hidden sizes up to
- * 16384 with norm_w, and compute the rmsnorm's statistic from the row (sumsq_in is accepted and not read).
+/* fc_Q4A with the neighbouring ops of chatllama/main.py:344-375 folded in.  One row (a decode step) is one launch.
+ * So are 2..8 rows with group 32, with fewer than 64 strips, with glu 1, with rmsnorm'ed rows of more than 16384
+ * floats or of which x or norm_w does not start on 16 bytes (glu 2: x); other 2..8 rows are, where that is the faster
+ * way for their sizes and options.  The rest (a batch of decode steps, a prompt) take a launch each for quantization
+ * and product: the producer of the input -- rmsnorm, or silu(gate)*up -- runs inside the quantization launch, so that its
+ * fp32 result never passes through memory, the residual is added in the product's stores and the sums of squares
+ * take a launch of their own; the codes, scales and results are those of the separate ops (llmops_rmsnorm_out /
+ * llmops_silu_mul, then llmops_fc_Q4A), and the rmsnorm's statistic is computed from the row (sumsq_in is accepted
+ * and not read).  Either way results are the same up to the rounding of fp32 sums.
+ * More than 8 rows need whole 16-byte aligned rows, take glu 0 or 2 (2 with group 128 only) and hidden sizes up to
+ * 16384 with norm_w.
  * Each option may be left out (NULL / 0):
  *   norm_w, eps : x is rmsnorm'ed first (clone + rmsnorm, ops/op_misc.hpp:142-181); needs K % 4 == 0
  *   residual    : y += residual (iadd, ops/op_misc.hpp:55-79), fp32 [rows,N_out]

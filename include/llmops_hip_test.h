@@ -61,6 +61,12 @@ void llmops_test_fc_rows_set_split(int on);
  * 256 strips and for larger ones (defaults 4 and 3; values below 2 restore them) */
 void llmops_test_fc_set_row_routing(int rows_from_small, int rows_from_large);
 
+/* llmops_fc_Q4A_decode (host arithmetic only, no launch): whether a call of these sizes and options (norm, sumsq_in,
+ * sumsq_out: given or not; everything on 16 bytes) goes to a quantization launch and a product (1) or to the streaming
+ * kernel in one launch (0).  Reads the knob above. */
+int llmops_test_fc_decode_route(int64_t rows, int64_t K, int64_t Ng, int64_t Kg, int group_k, int norm, int sumsq_in, int glu,
+                                int sumsq_out, int* quantize_first);
+
 /* decode attention (one query token): force the cache rows per wavefront (fp32 cache 4, 8, 16; fp16 cache 8, 16,
  * 32; a chunk is 4 times that); 0 = choose */
 void llmops_test_attn_set_decode_plan(int rows_per_wave);

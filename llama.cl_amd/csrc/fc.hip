@@ -175,6 +175,39 @@ extern "C" int llmops_fc_Q4A_residual(const float* x, int64_t rows, int64_t K, c
     return fc_impl(x, rows, K, weiq, Ng, Kg, group_k, N, residual, y, workspace, workspace_bytes, stream);
 }
 
+// Up to 8 rows: whether the producer, the product and the sums of squares are launches of their own (quantization, the
+// weight-streaming MFMA product, launch_strip_sumsq) instead of one launch of the streaming kernel.  That one forms a
+// producer in every strip's workgroup again for every row, and quantizes and multiplies row by row: a row costs it 0.5 us
+// (64 strips x 4 k-groups) to 3 us (688 x 32) and more with a producer, hardly anything the other way, where the second
+// launch costs 1.5 to 3 us and the sums 1.9.  In a graph, weights not from a cache, us, streaming / separate launches, at
+// rows either side of where the line lies (strips x k-groups):
+//   residual:             64x4 4 rows 4.3 / 5.3, 5 5.3 / 5.3; 64x16 4 5.9 / 6.6, 5 7.2 / 6.7; 128x32 3 7.4 / 7.1; 128x86 3 10.1 / 10.3,
+//                         4 11.4 / 10.3; 256x32 3 7.9 / 8.2, 4 9.1 / 8.3; 384x32 2 8.8 / 10.9, 3 13.3 / 11.0; 688x32 3 19.2 / 14.3
+//   .. and sums:          64x4 8 rows 6.7 / 7.1; 64x16 6 8.0 / 8.6, 8 9.2 / 8.7; 128x32 5 9.0 / 9.2, 6 9.5 / 9.2; 128x86 4 12.0 / 12.4,
+//                         5 15.9 / 12.4; 256x32 4 9.4 / 10.2, 5 11.7 / 10.2; 384x32 2 9.2 / 12.9, 3 14.1 / 13.1
+//   rmsnorm:              64x4 2 rows 5.8 / 5.0, 3 8.1 / 5.3; 128x32 3 12.6 / 7.5; 128x86 2 11.3 / 12.3, 3 15.4 / 12.2;
+//                         384x32 2 16.5 / 11.5; 688x32 2 23.8 / 14.6
+//   .. and sums:          64x16 2 rows 7.2 / 8.6, 3 10.1 / 8.9; 128x32 2 9.2 / 9.4, 3 12.9 / 9.5; 384x32 2 17.4 / 13.3
+//   .. sums handed in:    64x4 4 rows 5.0 / 5.3, 5 6.5 / 5.3; 64x16 4 6.8 / 6.9, 5 9.3 / 6.8; 128x32 2 6.7 / 7.5, 3 9.2 / 7.5; 256x32 2
+//                         7.2 / 8.6, 3 9.7 / 8.6; 384x32 2 10.4 / 11.3, 3 17.1 / 11.5; 688x32 2 14.9 / 14.5
+//   silu * up, residual:  64x4 4 rows 4.9 / 5.2, 5 6.1 / 5.2; 64x16 4 6.8 / 6.6; 128x32 2 6.8 / 7.0, 3 8.7 / 7.1; 128x86 2 9.6 / 10.2, 3
+//                         12.1 / 10.3; 384x32 2 11.2 / 11.0; 688x32 2 15.5 / 14.1
+//   .. and sums:          64x4 7 rows 7.4 / 7.2, 8 7.9 / 7.2; 64x16 5 8.9 / 8.6; 128x32 3 9.1 / 9.2, 4 10.4 / 9.2; 128x86 3 12.7 / 12.3;
+//                         256x32 3 9.6 / 10.2, 4 11.1 / 10.2; 384x32 2 11.2 / 12.9, 3 16.8 / 13.1
+static bool decode_quantizes_first(int64_t rows, int64_t K, int64_t Ng, int64_t Kg, int group_k, bool norm, bool sums_in, int glu, bool sums_out) {
+    if (group_k != 128 || Ng < 64 || !gemm_rows_kernel_enabled() || glu == 1 || (norm && K > 16384)) return false;
+    const bool large = Ng > 256;
+    const int64_t blocks = Ng * Kg;
+    int from = large ? g_rows_from_large : g_rows_from_small;  // (as in fc_Q4A)
+    if (norm && !sums_in) return rows >= from - 1;
+    const bool producer = norm || glu == 2;
+    if (large) return rows >= from - (producer && !sums_out && (glu == 2 || blocks >= 16384) ? 1 : 0);
+    if (blocks < 2048) from += 1;
+    else if (producer) from -= 1;
+    if (sums_out) from += blocks < 512 ? (producer ? 3 : 4) : (producer || blocks >= 8192 ? 1 : 2);
+    return rows >= from;
+}
+
 static int fc_decode_impl(const float* x, int64_t rows, int64_t K, const int8_t* weiq, int64_t Ng, int64_t Kg, int group_k,
                           int64_t N_out, const float* norm_w, float eps, const float* residual, int glu,
                           const float* sumsq_in, int64_t sumsq_parts, float* sumsq_out, float* y, int64_t out_parts,
@@ -211,15 +244,9 @@ static int fc_decode_impl(const float* x, int64_t rows, int64_t K, const int8_t*
     if (workspace_bytes < need)
         return fail(LLMOPS_EWORKSPACE, "fc_Q4A needs %zu workspace bytes, got %zu", need, workspace_bytes);
     uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
-    // From two rows on a producer costs the streaming kernel more than the launch that the other way takes: every strip's
-    // workgroup forms it again for every row.  Without one the rows count as in fc_Q4A, with one they are one fewer.  (us,
-    // streaming / quantization launch and product, 2 and 8 rows: rmsnorm, 12288 x 4096 17.9 / 13.4 and 36.6 / 13.3, 22016 x 4096
-    // 25.0 / 17.1 and 53.8 / 17.8, 55296 x 4096 54.4 / 30.3 and 122.6 / 32.1; silu * up, 4096 x 11008, 3 and 8 rows 13.0 / 12.8 and
-    // 27.7 / 12.2; residual, 4096 x 4096, 4 and 8 rows 9.3 / 8.6 and 11.0 / 8.7.)
-    const int rows_from = (Ng > 256 ? g_rows_from_large : g_rows_from_small) - (norm_w != nullptr || glu == 2 ? 1 : 0);
-    const bool quantize_first = group_k == 128 && Ng >= 64 && gemm_rows_kernel_enabled() && glu != 1 && rows >= rows_from &&
-                                ((norm_w == nullptr && glu != 2) || aligned(x, 16)) &&
-                                (norm_w == nullptr || (K <= 16384 && aligned(norm_w, 16)));
+    const bool sums_in = sumsq_in != nullptr && sumsq_parts <= 256;  // (what the streaming kernel reads)
+    const bool quantize_first = decode_quantizes_first(rows, K, Ng, Kg, group_k, norm_w != nullptr, sums_in, glu, sumsq_out != nullptr) &&
+                                ((norm_w == nullptr && glu != 2) || aligned(x, 16)) && (norm_w == nullptr || aligned(norm_w, 16));
     if (rows > kMaxGemvRows || quantize_first) {
         // More rows than the streaming kernel takes or is good at: the producer is folded into the quantization launch instead
         // (its fp32 result never goes through memory), the residual into the product's stores, and the sums of
@@ -265,6 +292,14 @@ extern "C" int llmops_fc_Q4A_decode(const float* x, int64_t rows, int64_t K, con
                                     void* workspace, size_t workspace_bytes, llmops_stream_t stream) {
     return fc_decode_impl(x, rows, K, weiq, Ng, Kg, group_k, N_out, norm_w, eps, residual, glu, sumsq_in, sumsq_parts, sumsq_out, y,
                           1, workspace, workspace_bytes, stream);
+}
+
+extern "C" int llmops_test_fc_decode_route(int64_t rows, int64_t K, int64_t Ng, int64_t Kg, int group_k, int norm, int sumsq_in, int glu,
+                                           int sumsq_out, int* quantize_first) {
+    LLMOPS_TEST_HOOK();
+    LLMOPS_REQUIRE(valid_group(group_k) && rows > 0 && K > 0 && Ng > 0 && Kg > 0 && quantize_first != nullptr);
+    *quantize_first = rows > kMaxGemvRows || decode_quantizes_first(rows, K, Ng, Kg, group_k, norm != 0, sumsq_in != 0, glu, sumsq_out != 0);
+    return LLMOPS_OK;
 }
 
 extern "C" int llmops_fc_Q4A_decode_parts(const float* x, int64_t rows, int64_t K, const int8_t* weiq, int64_t Ng, int64_t Kg,

@@ -237,7 +237,8 @@ def interleave_gate_up(gate_packed, up_packed):
 
 def fc_Q4A_decode(input, weiq, N_out, norm=None, residual=None, glu=False, sumsq_in=None, want_sumsq=False,
                   glu_in=False, attn_records=None, out_parts=1):
-    """Extension: fc_Q4A with its neighbours of the decode step folded in (one launch for B*M <= 8).
+    """Extension: fc_Q4A with its neighbours of the decode step folded in (one launch for one row, and for up to 8 where that
+    is the faster way).
 
     norm=(weight, eps): input is rmsnorm'ed first;  residual: added to the result;
     glu=True: ``weiq`` holds interleaved gate/up strips (``interleave_gate_up``) and the result is
@@ -249,9 +250,10 @@ def fc_Q4A_decode(input, weiq, N_out, norm=None, residual=None, glu=False, sumsq
     columns i*N_out/p ..), e.g. q, k and v of a fused q|k|v projection, instead of one tensor to be cut up and copied.
     want_sumsq=True returns ``(out, sumsq)`` where ``sumsq``
     [B*M, strips] holds the sum of squares of every 32 outputs; passed as ``sumsq_in`` to the FC that
-    rmsnorms ``out`` it saves that FC the pass over the row.  With more than 8 rows the rmsnorm or the
-    silu(gate)*up runs inside the quantization launch (same codes as the separate ops give), the residual inside the
-    product; shapes that launch does not take, and glu=True, are composed from the separate ops."""
+    rmsnorms ``out`` it saves that FC the pass over the row where that FC is one launch.  With more than 8 rows (group 128: with
+    2 to 8 too where that is faster) the rmsnorm or the silu(gate)*up runs inside the quantization launch (same codes as the
+    separate ops give; ``sumsq_in`` is not needed), the residual inside the product, the sums of squares behind it; with more than 8
+    rows shapes that launch does not take, and glu=True, are composed from the separate ops."""
     if attn_records is not None:
         # input = the attention output still in chunk records (attention_rope2_records); merged on the way in
         r = attn_records

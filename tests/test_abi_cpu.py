@@ -134,6 +134,31 @@ def test_gemm_planner_choices(lib):
     assert lib.llmops_test_gemm_plan(i64(0), i64(1), i64(1), 128, None, None) != 0
 
 
+@pytest.mark.parametrize("form,sizes", [
+    # (strips, k-groups): the last row count that measured faster in one launch, the first that did in separate ones
+    ("residual", {(64, 4): (4, 6), (64, 16): (4, 5), (128, 32): (3, 4), (128, 86): (3, 4), (256, 32): (3, 4), (384, 32): (2, 3), (688, 32): (2, 3)}),
+    ("residual sums", {(64, 4): (8, 9), (64, 16): (6, 8), (128, 32): (5, 6), (128, 86): (4, 5), (256, 32): (4, 5), (384, 32): (2, 3), (688, 32): (2, 3)}),
+    ("norm", {(64, 4): (1, 3), (64, 16): (1, 3), (128, 32): (1, 3), (128, 86): (2, 3), (256, 32): (1, 3), (384, 32): (1, 2), (688, 32): (1, 2)}),
+    ("norm sums", {(64, 4): (2, 3), (64, 16): (2, 3), (128, 32): (2, 3), (128, 86): (2, 3), (256, 32): (2, 3), (384, 32): (1, 2), (688, 32): (1, 2)}),
+    ("norm sums_in", {(64, 4): (4, 5), (64, 16): (3, 5), (128, 32): (2, 3), (256, 32): (2, 3), (384, 32): (2, 3), (688, 32): (1, 2)}),
+    ("glu", {(64, 4): (4, 5), (64, 16): (3, 5), (128, 32): (2, 3), (128, 86): (2, 3), (256, 32): (2, 3), (384, 32): (1, 2), (688, 32): (1, 2)}),
+    ("glu sums", {(64, 4): (6, 8), (64, 16): (4, 6), (128, 32): (2, 4), (128, 86): (2, 4), (256, 32): (3, 4), (384, 32): (2, 3), (688, 32): (2, 3)})])
+def test_rows_from_which_a_decode_projection_is_quantized_first(lib, form, sizes):
+    opts, first = form.split(), ctypes.c_int(-1)
+    i64 = ctypes.c_int64
+
+    def separate(rows, strips, groups, group_k=128, glu=2 if "glu" in opts else 0):
+        assert lib.llmops_test_fc_decode_route(i64(rows), i64(groups * group_k), i64(strips), i64(groups), group_k, int("norm" in opts),
+                                               int("sums_in" in opts), glu, int("sums" in opts), ctypes.byref(first)) == 0
+        return first.value
+
+    for (strips, groups), (one, many) in sizes.items():
+        assert [separate(r, strips, groups) for r in (1, one, many, 9)] == [0, 0, 1, 1], (form, strips, groups)
+        # what the quantization and the product behind it do not take: one launch up to 8 rows
+        assert not separate(8, 63, groups) and not separate(8, strips, groups, group_k=32)
+        assert "norm" in opts or not separate(8, strips, groups, glu=1)
+
+
 def test_python_ops_refuse_host_tensors():
     """The product path has no CPU fallback: host tensors raise instead of being computed elsewhere."""
     import torch
