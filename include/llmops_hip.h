@@ -166,6 +166,11 @@ int llmops_fc_Q4A_decode(const float* x, int64_t rows, int64_t K, const int8_t* 
                          const float* sumsq_in, int64_t sumsq_parts, float* sumsq_out, float* y, void* workspace,
                          size_t workspace_bytes, llmops_stream_t stream);
 
+/* 1 if a call with norm_w and these sizes would be one launch, in which every strip's workgroup forms the rmsnorm's
+ * statistic: then the FC that produces x had better leave it in sumsq_out, for sumsq_in here.  0 if the quantization
+ * launch forms it anyway and sumsq_out would be a launch for nothing.  (Host arithmetic; nothing is launched.) */
+int llmops_fc_Q4A_decode_wants_sumsq(int64_t rows, int64_t K, int64_t Ng, int64_t Kg, int group_k, int glu);
+
 /* llmops_fc_Q4A_decode for more than 8 rows whose result is wanted as out_parts dense matrices, y laid out
  * [out_parts][rows][N_out / out_parts] (Ng % out_parts == 0, N_out == Ng*32): the strips of part p are strips
  * p*Ng/out_parts .. of weiq.  A q|k|v projection over weights stacked along N (chatllama/main.py:347-349 runs three

@@ -294,6 +294,10 @@ extern "C" int llmops_fc_Q4A_decode(const float* x, int64_t rows, int64_t K, con
                           1, workspace, workspace_bytes, stream);
 }
 
+extern "C" int llmops_fc_Q4A_decode_wants_sumsq(int64_t rows, int64_t K, int64_t Ng, int64_t Kg, int group_k, int glu) {
+    return rows <= kMaxGemvRows && !decode_quantizes_first(rows, K, Ng, Kg, group_k, true, false, glu, false);
+}
+
 extern "C" int llmops_test_fc_decode_route(int64_t rows, int64_t K, int64_t Ng, int64_t Kg, int group_k, int norm, int sumsq_in, int glu,
                                            int sumsq_out, int* quantize_first) {
     LLMOPS_TEST_HOOK();

@@ -196,8 +196,9 @@ class LlamaDecoder:
         H, F = self.configs["hidden_size"], self.configs["intermediate_size"]
         n1, n2 = ops["input_layernorm"], ops["post_attention_layernorm"]
         rows = hidden_states.shape[0] * hidden_states.shape[1]
-        # a prompt or a batch: the sums of squares are not handed on (the norms read their rows)
-        many = rows > 8 or (rows > 1 and all(llmops.group_k_of(ops[n].weight) == 128 for n in ("o_proj", "down_proj")))
+        following = self.layers[i + 1]["qkv_proj"] if i + 1 < len(self.layers) else self.lm_head
+        to_gate_up, to_following = (self._wants_sumsq(ops["gate_up_proj"], rows, not self.stacked_gate_up),
+                                    self._wants_sumsq(following, rows, False))
         if rows > 8:  # q, k and v as three dense [B,qL,H*S] tensors straight from the product
             q, k, v = llmops.fc_Q4A_decode(hidden_states, ops["qkv_proj"].weight, 3 * H, norm=(n1.weight, n1.eps), out_parts=3)
         else:
@@ -213,22 +214,25 @@ class LlamaDecoder:
                                                    attn_records=recs)
         else:
             llmops.attention_rope2(q, k, v, self.inv_freq, kv_cache, kv_cache_slots, position_id, i)
-            if many:
-                attn_output, ss = llmops.fc_Q4A_decode(q, ops["o_proj"].weight, H, residual=hidden_states), None
-            else:
-                attn_output, ss = llmops.fc_Q4A_decode(q, ops["o_proj"].weight, H, residual=hidden_states, want_sumsq=True)
+            attn_output, ss = self._decode_fc(to_gate_up, q, ops["o_proj"].weight, H, residual=hidden_states)
         if self.stacked_gate_up:
-            gate_up = llmops.fc_Q4A_decode(attn_output, ops["gate_up_proj"].weight, 2 * F, norm=(n2.weight, n2.eps),
-                                           sumsq_in=ss)
-            if many:
-                return llmops.fc_Q4A_decode(gate_up, ops["down_proj"].weight, H, residual=attn_output, glu_in=True), None
-            return llmops.fc_Q4A_decode(gate_up, ops["down_proj"].weight, H, residual=attn_output, want_sumsq=True,
-                                        glu_in=True)
-        act = llmops.fc_Q4A_decode(attn_output, ops["gate_up_proj"].weight, F, norm=(n2.weight, n2.eps), glu=True,
-                                   sumsq_in=ss)
-        if many:
-            return llmops.fc_Q4A_decode(act, ops["down_proj"].weight, H, residual=attn_output), None
-        return llmops.fc_Q4A_decode(act, ops["down_proj"].weight, H, residual=attn_output, want_sumsq=True)
+            act = llmops.fc_Q4A_decode(attn_output, ops["gate_up_proj"].weight, 2 * F, norm=(n2.weight, n2.eps), sumsq_in=ss)
+        else:
+            act = llmops.fc_Q4A_decode(attn_output, ops["gate_up_proj"].weight, F, norm=(n2.weight, n2.eps), glu=True,
+                                       sumsq_in=ss)
+        return self._decode_fc(to_following, act, ops["down_proj"].weight, H, residual=attn_output, glu_in=self.stacked_gate_up)
+
+    @staticmethod
+    def _wants_sumsq(op, rows, glu):
+        """whether the FC that makes ``op``'s input should hand on its sums of squares for op's rmsnorm"""
+        if rows == 1 or rows > 8:  # (one launch; the norm reads its rows in the quantization launch)
+            return rows == 1
+        g, (Ng, Kg, _) = llmops.group_k_of(op.weight), op.weight.shape
+        return bool(llmops._lib.load().llmops_fc_Q4A_decode_wants_sumsq(rows, Kg * g, Ng, Kg, g, int(glu)))
+
+    @staticmethod
+    def _decode_fc(sums, *args, **kw):
+        return llmops.fc_Q4A_decode(*args, want_sumsq=True, **kw) if sums else (llmops.fc_Q4A_decode(*args, **kw), None)
 
     def capture_decode(self, kv_cache, slot, position_id, stream=None):
         """Capture one decode step (batch 1, one token) as a HIP graph that serves every position: the token id,

@@ -73,6 +73,37 @@ def test_forward_prefill_then_decode(orc, plan):
         assert np.abs(kv.cache.cpu().numpy() - cache_h).max() <= 5e-2
 
 
+@pytest.mark.parametrize("cfg,rows,handed_on", [
+    (dict(CFG), 3, [True, True]),                                                        # too few strips for the product of few rows
+    (dict(CFG, intermediate_size=2048, vocab_size=2080), 3, [False, True, False, False]),  # .. but gate|up and the logits have enough
+    (dict(CFG, intermediate_size=2048, vocab_size=2080), 2, [True, True]),
+    (dict(CFG, intermediate_size=2048, vocab_size=2080), 9, [False, False])])
+def test_short_prompts_hand_on_the_sums_that_are_read(monkeypatch, cfg, rows, handed_on):
+    """2..8 tokens: o and down leave sums of squares exactly where the FC behind them is one launch, which reads them
+    (handed_on: per layer o, down; two values: the same in both layers); the result is that of the separate operators."""
+    import llmops
+    from llmops.decode import LlamaDecoder
+    from llmops.opset import KVCache
+    model = LlamaDecoder(cfg, group_k=128, seed=3)
+    wanted, fc = [], llmops.fc_Q4A_decode
+
+    def recording(input, weiq, N_out, **kw):
+        if "norm" in kw:
+            wanted.append(kw.get("sumsq_in") is not None)
+        return fc(input, weiq, N_out, **kw)
+
+    monkeypatch.setattr(llmops, "fc_Q4A_decode", recording)
+    ids = torch.arange(rows, device="cuda").reshape(1, rows)
+    slots = torch.arange(rows, dtype=torch.int32, device="cuda")
+    out = model.forward(ids, KVCache(cfg, 1, 64).cache, slots, 0)
+    assert wanted == [False] + (handed_on * 2)[:4]  # (the first norm has no FC in front)
+    apart = LlamaDecoder(cfg, group_k=128, seed=3)
+    monkeypatch.setattr(apart, "_wants_sumsq", lambda *a: False, raising=True)
+    want = apart.forward(ids, KVCache(cfg, 1, 64).cache, slots, 0)
+    # (a statistic summed in another order flips 8-bit codes now and then)
+    assert float((out - want).norm() / want.norm()) <= 0.03
+
+
 def test_layer_ops_teacher_forced(orc):
     """Every op of one layer, each checked against the oracle evaluated on the GPU's own input to that op."""
     import llmops
