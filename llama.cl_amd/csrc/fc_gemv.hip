@@ -128,34 +128,49 @@ __device__ __forceinline__ void finish_strip(float f[MT][4], float (*red)[MT][kG
     // travels inside the atomic, so there is nothing to order, and the cost is one round trip to memory
     // instead of three (store and acknowledgement, ticket, loads).
     if (slots != nullptr) {
+        const bool live = mine && n < N;
+        unsigned long long* slot = slots + ((int64_t)tr * Np + n);
         float done = 0.0f;  // the finished output if this thread is the one that finished it, else 0
-        if (mine && n < N) {
-            unsigned long long* slot = slots + ((int64_t)tr * Np + n);
+        bool found = false;
+        if (live) {
             const unsigned long long parked = (1ull << 32) | (unsigned long long)__float_as_uint(v);
             const unsigned long long old = __hip_atomic_exchange(slot, parked, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if ((old >> 32) != 0ull) {
+            found = (old >> 32) != 0ull;
+            if (found) {
                 const float both = v + __uint_as_float((unsigned)(old & 0xFFFFFFFFull));
                 done = has_residual ? both + residual_value : both;
                 y[(int64_t)tr * N + n] = done;
-                __hip_atomic_store(slot, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
-        if (sumsq_out == nullptr) return;
-        // The strip's sum of squares: each of the two workgroups knows the squares of the outputs it finished;
-        // the two partial sums meet through one more exchange per (row, strip), in slots behind the outputs'
-        // (p0 + p1: the same bits whichever came first).
-        float sq = done * done;
-#pragma unroll
-        for (int o = 16; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
-        if (mine && (lane_id_now() & 31) == 0) {
-            const int64_t strips = (int64_t)gridDim.x / S;
-            unsigned long long* slot = slots + (int64_t)rows * Np + ((int64_t)tr * strips + nb);
-            const unsigned long long parked = (1ull << 32) | (unsigned long long)__float_as_uint(sq);
-            const unsigned long long old = __hip_atomic_exchange(slot, parked, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if ((old >> 32) != 0ull) {
-                sumsq_out[(int64_t)tr * strips + nb] = sq + __uint_as_float((unsigned)(old & 0xFFFFFFFFull));
-                __hip_atomic_store(slot, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (sumsq_out == nullptr) {
+            if (found) __hip_atomic_store(slot, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
+        }
+        // The strip's sum of squares is formed by one workgroup, in one order.  Mostly one of the two finishes all of a row's 32
+        // outputs and has what it needs.  Where each finishes some (seen in 8 to 17 % of the launches of 128 strips x 86
+        // k-groups), sums of what either has, added up, would depend on which outputs those are: there the finished outputs stay
+        // in their slots, and who comes second to one more exchange per (row, strip), in slots behind the outputs', takes the
+        // other's from them and empties all slots.
+        const int half = lane & 32;
+        const uint32_t mine_of_row = (uint32_t)(__ballot(found) >> half), of_row = (uint32_t)(__ballot(live) >> half);
+        const bool mixed = mine_of_row != 0u && mine_of_row != of_row;  // (both workgroups see it)
+        if (found)
+            __hip_atomic_store(slot, mixed ? (2ull << 32) | (unsigned long long)__float_as_uint(done) : 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int64_t strips = (int64_t)gridDim.x / S;
+        if (mixed) {
+            unsigned long long* second_slot = slots + (int64_t)rows * Np + ((int64_t)tr * strips + nb);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's outputs have been acknowledged
+            int second = 0;
+            if ((lane & 31) == 0) second = __hip_atomic_exchange(second_slot, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0ull;
+            second = __shfl(second, half, 64);
+            if (second) {
+                if (live && !found) done = __uint_as_float((unsigned)__hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                strip_sumsq(done, mine, tr, nb, (int)strips, sumsq_out);
+                if (live) __hip_atomic_store(slot, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if ((lane & 31) == 0) __hip_atomic_store(second_slot, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
+        } else if (mine_of_row != 0u) {
+            strip_sumsq(done, mine, tr, nb, (int)strips, sumsq_out);
         }
         return;
     }

@@ -104,6 +104,42 @@ def test_short_prompts_hand_on_the_sums_that_are_read(monkeypatch, cfg, rows, ha
     assert float((out - want).norm() / want.norm()) <= 0.03
 
 
+@pytest.mark.parametrize("rows,N", [(1, 4096), (1, 4090), (2, 4090)])
+def test_sums_of_squares_are_the_same_bits_in_every_launch(rows, N):
+    """The two halves of K of a down projection each finish some of a strip's outputs now and then (one launch in ten of
+    this size); the sums of squares, which the next rmsnorm reads, must not show it.  While another stream is busy too,
+    and with the hand-off area empty afterwards."""
+    import llmops
+    K, n = 11008, 50
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    w = llmops.offline_FC_quant_Q4A(torch.randn(N, K, generator=gen, device="cuda") * 0.02, 128)
+    x, res = (torch.randn(1, rows, k, generator=gen, device="cuda") for k in (2 * K, N))
+    busy, stream, other = torch.randn(32 << 20, device="cuda"), torch.cuda.Stream(), torch.cuda.Stream()
+
+    def call():
+        return llmops.fc_Q4A_decode(x, w, N, residual=res, want_sumsq=True, glu_in=True)
+
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        y0, s0 = call()
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            outs = [call() for _ in range(n)]
+        for i in range(60):
+            if i % 2:
+                with torch.cuda.stream(other):
+                    busy.mul_(1.0)
+            graph.replay()
+            stream.synchronize()
+            for y, s in outs:
+                assert torch.equal(y, y0) and torch.equal(s, s0)
+        head = llmops._workspace(x.device, 1)[:3 << 20]  # (counters and exchange slots)
+        assert not head.any()
+    pad = torch.nn.functional.pad(y0.reshape(rows, N).double(), (0, -N % 32))
+    assert torch.allclose(s0.double(), (pad ** 2).reshape(rows, -1, 32).sum(-1), rtol=2e-6, atol=0)
+
+
 def test_layer_ops_teacher_forced(orc):
     """Every op of one layer, each checked against the oracle evaluated on the GPU's own input to that op."""
     import llmops
