@@ -33,8 +33,8 @@ int llmops_test_calib_copy(const void* src, void* dst, int64_t bytes, int workgr
 void llmops_test_fc_set_tuning(int target_workgroups, int waves_per_workgroup);
 
 /* prefill GEMM planner knob: force the row-tile factor of the LDS-tiled MFMA kernel (1, 2 or 4:
- * 32, 64 or 128 rows per workgroup; 8: as 4); 0 = choose per shape; -1 = choose
- * per shape and send 9..16 rows to the tiled kernel too instead of the weight-streaming MFMA kernel */
+ * 32, 64 or 128 rows per workgroup); 0 (and what is none of these) = choose per shape; -1 = choose
+ * per shape and send 9..32 rows to the tiled kernel too instead of the weight-streaming MFMA kernel */
 void llmops_test_gemm_set_tuning(int row_tile_factor);
 
 /* prefill GEMM with split-K: the product kernel adds the partial sums itself (the last split of a tile to
@@ -48,8 +48,8 @@ void llmops_test_gemm_set_reduce(int in_kernel);
 void llmops_test_gemm_set_split(int splits);
 
 /* prefill GEMM: what the planner chooses for a product of `rows` rows with a packed tensor of Ng strips x Kg
- * k-groups (host arithmetic only, no launch): the row-tile factor (1, 2, 4: 32, 64, 128 rows per workgroup; 8: 128
- * rows, unsplit, two workgroups to a compute unit) and the split-K factor.  Reads the knobs above. */
+ * k-groups (host arithmetic only, no launch): the row-tile factor (1, 2, 4: 32, 64, 128 rows per workgroup; group 32
+ * has 32-row tiles only) and the split-K factor.  Reads the knobs above. */
 int llmops_test_gemm_plan(int64_t rows, int64_t Ng, int64_t Kg, int group_k, int* row_tile_factor, int* splits);
 
 /* weight-streaming MFMA kernel (3..16 rows, 17..32 for tensors of fewer than 256 strips): two workgroups per strip with half of K each for tensors of

@@ -501,7 +501,7 @@ struct GemmPlan {
     bool lds;
 };
 
-static int g_gemm_rt = 0;  // 0 = choose per shape; 1, 2, 4 (and 8, taken as 4) = that tile; -1 = also keep 9..32 rows on the tiled kernel
+static int g_gemm_rt = 0;  // 0 = choose per shape; 1, 2, 4 = that tile; -1 = also keep 9..32 rows on the tiled kernel
 static int g_gemm_fused_reduce = 1;  // split-K partial sums added by the product kernel itself (0: by a second launch)
 static int g_gemm_force_split = 0;   // > 0: the split-K factor to use whatever the estimate says (tests)
 bool gemm_rows_kernel_enabled() { return g_gemm_rt >= 0; }
@@ -517,10 +517,9 @@ bool gemm_rows_kernel_enabled() { return g_gemm_rt >= 0; }
 static void plan_gemm_tile(int64_t rows, int64_t Ng, int64_t Kg, int64_t room, GemmPlan& p) {
     static const int kRT[3] = {4, 2, 1}, kSlots[3] = {512, 768, 1024};
     static const double kGroupUs[3] = {1.2, 0.947, 0.811}, kPartRound[3] = {1.0, 0.541, 0.852};
-    const int force_rt = g_gemm_rt == 8 ? 4 : g_gemm_rt;
     double best = 0.0;
     for (int i = 0; i < 3; i++) {
-        if (force_rt > 0 && kRT[i] != force_rt) continue;
+        if (g_gemm_rt > 0 && kRT[i] != g_gemm_rt) continue;
         const int64_t bm = 32 * kRT[i], tiles = ((Ng + 3) / 4) * ((rows + bm - 1) / bm);
         for (int64_t s = 1; s <= 12; s++) {
             const int64_t want = g_gemm_force_split > 0 ? g_gemm_force_split : s;
@@ -648,8 +647,9 @@ int launch_gemm_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64
 
 }  // namespace llmops
 
-extern "C" void llmops_test_gemm_set_tuning(int rows_per_wave_tile) {
-    if (llmops::test_hooks_enabled(__func__)) llmops::g_gemm_rt = rows_per_wave_tile;
+extern "C" void llmops_test_gemm_set_tuning(int row_tile_factor) {
+    const bool known = row_tile_factor == -1 || row_tile_factor == 1 || row_tile_factor == 2 || row_tile_factor == 4;
+    if (llmops::test_hooks_enabled(__func__)) llmops::g_gemm_rt = known ? row_tile_factor : 0;
 }
 extern "C" void llmops_test_gemm_set_split(int splits) {
     if (llmops::test_hooks_enabled(__func__)) llmops::g_gemm_force_split = splits < 0 ? 0 : splits;
@@ -658,8 +658,7 @@ extern "C" int llmops_test_gemm_plan(int64_t rows, int64_t Ng, int64_t Kg, int g
     LLMOPS_TEST_HOOK();
     if (rows < 1 || Ng < 1 || Kg < 1 || (group_k != 32 && group_k != 128) || !row_tile_factor || !splits) return LLMOPS_EINVAL;
     const llmops::GemmPlan p = llmops::plan_gemm(rows, Ng, Kg, group_k, INT64_MAX);
-    // (128-row tiles that fill the chip unsplit, two to a compute unit, are reported as the 256 rows they cover there)
-    *row_tile_factor = p.RT == 4 && p.S == 1 && group_k == 128 && rows >= 256 && Kg >= 8 ? 8 : p.RT;
+    *row_tile_factor = p.RT;
     *splits = p.S;
     return LLMOPS_OK;
 }

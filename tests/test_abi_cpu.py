@@ -105,8 +105,8 @@ def test_test_hooks_are_refused_unless_the_process_asks_for_them():
 
 def test_gemm_planner_choices(lib):
     """The prefill GEMM's planner is host arithmetic: what it chooses for the shapes its rules were measured
-    on (row-tile factor 1, 2, 4 = 32, 64, 128 rows per workgroup, 8 = the 256-row kernel; split-K factor),
-    and that every plan covers K exactly once."""
+    on (row-tile factor 1, 2, 4 = 32, 64, 128 rows per workgroup; split-K factor), and that every plan covers K
+    exactly once."""
     i64, ci = ctypes.c_int64, ctypes.c_int
 
     def plan(rows, N, K, G=128):
@@ -115,10 +115,10 @@ def test_gemm_planner_choices(lib):
                                          ctypes.byref(S)) == 0
         return rt.value, S.value
 
-    # many rows: the 256-row kernel, no split where the tiles fill the machine
-    assert plan(2048, 11008, 4096) == (8, 1)
-    assert plan(2048, 4096, 11008) == (8, 1)
-    assert plan(2048, 4096, 512)[0] != 8          # fewer than 8 k-groups: its min-term prologue reads 8 at a time
+    # many rows: 128-row tiles, no split where they fill the machine (16 x 32 tiles are two to a compute unit)
+    assert plan(2048, 11008, 4096) == (4, 1)
+    assert plan(2048, 4096, 11008) == (4, 1)
+    assert plan(2048, 4096, 512) == (4, 1)
     # few rows: 32-row tiles and as many splits as still leave runs of 4 k-groups (not 11 runs of 3)
     assert plan(32, 11008, 4096) == (1, 8)
     assert plan(64, 11008, 4096) == (1, 5)
@@ -128,10 +128,19 @@ def test_gemm_planner_choices(lib):
         for N, K in ((4096, 4096), (11008, 4096), (4096, 11008), (352, 640), (22016, 4096), (64, 128)):
             rt, S = plan(rows, N, K)
             Kg = (K + 127) // 128
-            assert rt in (1, 2, 4, 8) and 1 <= S <= Kg
+            assert rt in (1, 2, 4) and 1 <= S <= Kg
             per = (Kg + S - 1) // S
             assert (Kg + per - 1) // per == S     # S splits of `per` k-groups, the last possibly short, none empty
     assert lib.llmops_test_gemm_plan(i64(0), i64(1), i64(1), 128, None, None) != 0
+    # a forced tile is the tile reported, and what is no tile is not forced
+    try:
+        for forced, want in ((1, 1), (2, 2), (4, 4), (8, 4), (3, 4), (0, 4)):
+            lib.llmops_test_gemm_set_tuning(forced)
+            assert plan(2048, 11008, 4096)[0] == want
+    finally:
+        lib.llmops_test_gemm_set_tuning(0)
+    # group 32: 32-row tiles, stages of four k-groups
+    assert plan(512, 11008, 4096, 32)[0] == 1 and plan(64, 4096, 4096, 32)[0] == 1
 
 
 @pytest.mark.parametrize("form,sizes", [

@@ -118,7 +118,7 @@ def test_quant_x_rows_variant_vs_oracle(ops, orc, G, rows, K):
 
 
 # ---- int32 partial sums -------------------------------------------------------------------------
-INNER_LOOPS = [(32, 0), (32, 1), (128, 0), (128, 1), (128, 2)]  # (group, use_mfma); 2 = 256-row kernel, group 128 only
+INNER_LOOPS = [(32, 0), (32, 1), (128, 0), (128, 1), (128, 2)]  # (group, use_mfma); 2 = 128-row instead of 64-row tiles, group 128 only
 
 
 @pytest.mark.parametrize("G,mfma", INNER_LOOPS)
@@ -593,13 +593,12 @@ def test_fc_prefill_mid_rows_vs_oracle(ops, orc, rows, N, K):
     assert np.array_equal(ye, (xe.astype(np.float64) @ we.astype(np.float64).T).astype(np.float32).reshape(1, rows, N))
 
 
-@pytest.mark.parametrize("tiling", [1, 2, 4, 8])
+@pytest.mark.parametrize("tiling", [1, 2, 4])
 @pytest.mark.parametrize("rows,N,K", [(70, 2070, 1024), (300, 2070, 1024), (515, 352, 4096), (1024, 4096, 512)])
 def test_fc_prefill_every_tiling_vs_oracle(ops, orc, tiling, rows, N, K):
-    """The group-128 MFMA kernels with each row tiling forced in turn (32, 64, 128 rows per workgroup, and
-    the 256-row kernel whose two wave groups alternate phases), on shapes with ragged row and column
-    edges, with and without split-K: output against the oracle, the residual epilogue, and the
-    closed-form construction exactly."""
+    """The group-128 tiled kernel with each row tiling forced in turn (32, 64, 128 rows per workgroup), on shapes
+    with ragged row and column edges, with and without split-K: output against the oracle, the residual epilogue,
+    and the closed-form construction exactly."""
     from llmops import _lib
     lib = _lib.load()
     rng = np.random.default_rng(rows + N + tiling)
@@ -624,12 +623,10 @@ def test_fc_prefill_every_tiling_vs_oracle(ops, orc, tiling, rows, N, K):
 @pytest.mark.parametrize("split", [0, 3])
 @pytest.mark.parametrize("K", [1024, 5120, 11008])
 def test_fc_prefill_min_term_at_any_activation_scale(ops, orc, K, split):
-    """The 256-row kernel forms the min term sum_kg m * gsum once per tile from fp16 halves of the group
-    sums, 32 k-groups per MFMA, and falls back to fp32 MFMAs for a round in which some row's sums are too
-    small or too large for that.  Rows of ordinary, tiny, huge and zero activations side by side; 8
-    k-groups (a quarter of one MFMA's 32), 40 (a short second batch of 32) and 86 (a short third), with
-    and without split-K (splits that start off a multiple of 8): every ROW to 1e-5 of its own largest
-    output, which is what the fallback exists for."""
+    """The tiled kernel forms the min term sum_kg m * gsum four k-groups at a time on the fp32 matrix cores.  Rows of
+    ordinary, tiny, huge (sums beyond fp16) and zero activations side by side in 128-row tiles; 8, 40 and 86 k-groups in
+    one run and in three (runs that end inside the four): every ROW to 1e-5 of its own largest output, so that no
+    row's sums can have been rounded at another row's scale or at fewer than fp32's bits."""
     from llmops import _lib
     lib = _lib.load()
     rows, N = 300, 1056
@@ -642,7 +639,7 @@ def test_fc_prefill_min_term_at_any_activation_scale(ops, orc, K, split):
     w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
     pw = orc.quant_w(w, 128)
     want = orc.fc(x, pw, N)
-    lib.llmops_test_gemm_set_tuning(8)
+    lib.llmops_test_gemm_set_tuning(4)
     lib.llmops_test_gemm_set_split(split)
     try:
         got = host(ops.fc_Q4A(dev(x), dev(pw), N))
@@ -881,10 +878,10 @@ def test_fc_short_last_group(ops, orc, G, rows, N, K):
 
 
 @pytest.mark.parametrize("rows,N,K", [(300, 160, 1100), (300, 160, 5000), (513, 352, 4100)])
-def test_fc_256_row_kernel_short_last_group(ops, orc, rows, N, K):
-    """The 256-row kernel (forced) on a K that is not a whole number of k-groups: its min-term prologue reads a
-    row's group sums eight at a time from rows of 9, 40 and 33 floats (4-byte aligned only), the last k-group
-    is zero padded by the quantization."""
+def test_fc_128_row_tiles_short_last_group(ops, orc, rows, N, K):
+    """128-row tiles (forced) on a K that is not a whole number of k-groups, the last of which the quantization pads with
+    zeros: 9, 40 and 33 k-groups, the min term of the last one formed by itself or as the fourth of four, and rows that
+    end inside a tile."""
     from llmops import _lib
     lib = _lib.load()
     rng = np.random.default_rng(rows + N + K)
@@ -893,7 +890,7 @@ def test_fc_256_row_kernel_short_last_group(ops, orc, rows, N, K):
     x = rng.standard_normal((1, rows, K)).astype(np.float32)
     res = rng.standard_normal((1, rows, N)).astype(np.float32)
     want = orc.fc(x, pw, N)
-    lib.llmops_test_gemm_set_tuning(8)
+    lib.llmops_test_gemm_set_tuning(4)
     try:
         got = host(ops.fc_Q4A(dev(x), dev(pw), N))
         got_res = host(ops.fc_Q4A(dev(x), dev(pw), N, residual=dev(res)))

@@ -7,7 +7,7 @@
   fp32 output, ops/op_fc.hpp:408) and is compared to rounding.
 * The weight-streaming int8 MFMA kernel of 3..32 rows: its int32 sums (fc_Q4A_partials, use_mfma=3).
 * Config 3 (group 128, M in {16,128,512,2048}, 4096->11008 and 11008->4096): the GPU output against the oracle
-  on a sample of rows (FC rows are independent), and the 256-row kernel's int32 sums at 2048 rows.
+  on a sample of rows (FC rows are independent), and the int32 sums of its 128-row tiles at 2048 rows.
 
 Compared domain of the quantizer: finite activations whose group maximum is a normal fp32 number well inside the
 range (|x| in about [1e-30, 1e30]).  NaN, infinities and groups so small that 1/d overflows go through x86's
@@ -180,8 +180,9 @@ def test_config3_prefill_gemm_full_size_vs_oracle(orc, M, N, K):
 
 
 @pytest.mark.parametrize("strips,K", [(4, 4096), (8, 11008)])
-def test_config3_256_row_kernel_int32_sums_at_2048_rows(orc, strips, K):
-    """fc_gemm_pp_kernel (use_mfma=2) at 2048 rows on a subset of strips: int32 sums of sampled rows bit-equal"""
+def test_config3_tiled_kernel_int32_sums_at_2048_rows(orc, strips, K):
+    """fc_gemm_tile_kernel with 128-row tiles (use_mfma=2) at 2048 rows on a subset of strips: int32 sums of sampled rows
+    bit-equal"""
     import llmops
     rng = np.random.default_rng(strips + K)
     M = 2048

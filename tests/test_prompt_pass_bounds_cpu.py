@@ -36,7 +36,7 @@ def product(m, name, rows, Ng, Kg, N, ws_bytes, y_bytes, y_off=0, w_bytes=None, 
     off_xst = up(off_gs + rows * Kg * 4)
     off_part = up(off_xst + rows * Kg * 8 + 256)
     w_bytes = Ng * Kg * BLK if w_bytes is None else w_bytes
-    bm = 256 if rt == 8 else rt * 32
+    bm = rt * 32
     nbx, nby = -(-Ng // 4), -(-rows // bm)
     kper = -(-Kg // S)
     bx, by = np.arange(nbx)[:, None], np.arange(nby)[None, :]
