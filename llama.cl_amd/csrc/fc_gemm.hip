@@ -627,6 +627,8 @@ int launch_gemm(const uint8_t* w, const int8_t* xq, const float* xd, const float
 // the production loop, writing its int32 tiles instead of folding them
 template <int RT>
 static int launch_gemm_tile_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg, hipStream_t st) {
+    if (Kg * 128 * (RT * 32) >= ((int64_t)1 << 32))  // (32-bit offsets into a tile's rows)
+        return fail(LLMOPS_EINVAL, "fc_Q4A_partials: K must be below 2^32 / %d for tiles of that many rows", RT * 32);
     const int bad = configure_gemm_tile<RT, true>();
     if (bad) return bad;
     const int64_t tiles = ((Ng + 3) / 4) * ((rows + RT * 32 - 1) / (RT * 32));
@@ -639,10 +641,7 @@ static int launch_gemm_tile_partials(const uint8_t* w, const int8_t* xq, int32_t
 int launch_gemm_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg, int G,
                          bool rows128, hipStream_t st) {
     if (G != 128) return launch_gemm_g32_partials(w, xq, acc, rows, Ng, Kg, st);
-    if (!rows128) return launch_gemm_tile_partials<2>(w, xq, acc, rows, Ng, Kg, st);
-    if (!(rows * Kg * 128 < ((int64_t)1 << 31) && Ng * Kg * 2176 < ((int64_t)1 << 31)))
-        return fail(LLMOPS_EINVAL, "fc_Q4A_partials with 128-row tiles: codes and weights must be below 2 GiB");
-    return launch_gemm_tile_partials<4>(w, xq, acc, rows, Ng, Kg, st);
+    return rows128 ? launch_gemm_tile_partials<4>(w, xq, acc, rows, Ng, Kg, st) : launch_gemm_tile_partials<2>(w, xq, acc, rows, Ng, Kg, st);
 }
 
 }  // namespace llmops

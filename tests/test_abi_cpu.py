@@ -73,6 +73,10 @@ def test_argument_validation_without_device(lib):
     rc = lib.llmops_attention_rope_decode(vp(256), vp(256), vp(256), i64(2200), i64(32), i64(128), vp(256), i64(64), vp(256), 0,
                                           i64(2), i64(16), vp(256), vp(256), 0, vp(256), ctypes.c_size_t(1 << 40), vp(0))
     assert rc == 1 and b"65535 heads" in lib.llmops_last_error()
+    # int32 sums by tiles of 64 and 128 rows: a tile's rows are addressed with 32 bits
+    for use_mfma, groups in ((1, 1 << 19), (2, 1 << 18)):
+        rc = lib.llmops_fc_Q4A_partials(vp(256), i64(64), vp(256), i64(1), i64(groups), 128, vp(256), use_mfma, vp(0))
+        assert rc == 1 and b"K must be below" in lib.llmops_last_error()
     rc = lib.llmops_fc_workspace_reset(vp(0), ctypes.c_size_t(1 << 20), vp(0))
     assert rc == 1 and b"workspace != nullptr" in lib.llmops_last_error()
     # the entry point that allocates nothing validates its arguments before it enqueues anything (no device here:

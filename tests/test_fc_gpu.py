@@ -144,6 +144,18 @@ def test_partials_extreme_codes(ops, orc, G, mfma):
     assert np.array_equal(got, orc.fc_partials(xq, wq))
 
 
+def test_partials_of_more_than_2_gib_of_codes(ops, orc):
+    """Codes and sums beyond 2^31 bytes, whose offsets do not fit 31 bits: either tile, and the oracle on rows around there."""
+    rows = (1 << 24) + 5
+    rng = np.random.default_rng(4)
+    wq = orc.quant_w((rng.standard_normal((32, 128)) * 0.02).astype(np.float32), 128)
+    xq = torch.randint(-127, 128, (rows, 128), generator=torch.Generator(device="cuda").manual_seed(1), device="cuda", dtype=torch.int8)
+    got = [ops.fc_Q4A_partials(xq, dev(wq), use_mfma=m) for m in (1, 2)]
+    assert torch.equal(*got)
+    some = torch.tensor([0, 1, 127, 128, (1 << 23) - 1, 1 << 23, (1 << 24) - 1, 1 << 24, rows - 1])
+    assert np.array_equal(host(got[1][some.cuda()]), orc.fc_partials(host(xq[some.cuda()]), wq))
+
+
 # ---- fp32 output --------------------------------------------------------------------------------
 @pytest.mark.parametrize("G", [32, 128])
 def test_fc_golden(ops, G):
