@@ -115,10 +115,13 @@ int llmops_fc_workspace_reset(void* workspace, size_t workspace_bytes, llmops_st
 
 /* fc_Q4A for callers that cannot allocate device memory or carry a workspace around: code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the
- * reference.  Same arguments, kernels and results as llmops_fc_Q4A, but the workspace is a fixed array of
+ * reference.  Same arguments and kernels as llmops_fc_Q4A, but the workspace is a fixed array of
  * LLMOPS_FC_NOALLOC_SCRATCH_BYTES inside the library's device image (every device the library runs on
  * holds its own copy until the process ends).  The call allocates and frees nothing.  Sizes whose
- * workspace (llmops_fc_Q4A_workspace_bytes) exceeds the array are refused with LLMOPS_EWORKSPACE.
+ * workspace (llmops_fc_Q4A_workspace_bytes) fits the array give the same bits as llmops_fc_Q4A.  Of larger ones, more
+ * than 8 rows with group 128 are taken where the array holds the codes and scales: K is then split over fewer
+ * workgroups than llmops_fc_Q4A would, or over none, so that fp32 sums may be rounded in another order.  The rest
+ * is refused with LLMOPS_EWORKSPACE.
  * Every call on a device shares that device's array: calls that can overlap on one device (two streams,
  * two host threads) race and must use llmops_fc_Q4A with a workspace each instead.  The first call on a
  * device looks the array's address up (hipGetSymbolAddress); make that call outside stream capture. */

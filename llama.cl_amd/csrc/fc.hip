@@ -42,7 +42,8 @@ struct FcWorkspace {
     int64_t room;  // what partial sums may take
 };
 
-// limit: bytes that the workspace has, where that is fixed (the tiled product then splits K no further than they allow)
+// limit: bytes that the workspace has, where that is fixed (the tiled product then splits K no further than they allow; what
+// fits without the limit is split as without it)
 static FcWorkspace fc_layout(int64_t rows, int64_t Ng, int64_t Kg, int G, size_t limit = 0) {
     FcWorkspace w;
     size_t o = LLMOPS_FC_COUNTER_BYTES;
@@ -56,7 +57,7 @@ static FcWorkspace fc_layout(int64_t rows, int64_t Ng, int64_t Kg, int G, size_t
     // (+256: the weight-streaming MFMA kernel fetches the pairs of whole 16-row tiles, up to 31 pairs past the last row)
     o = align_up(o + (size_t)rows * Kg * 2 * sizeof(float) + 256, 256);
     w.off_part = o;
-    w.room = limit == 0 ? INT64_MAX : (int64_t)limit - (int64_t)o - 256;
+    w.room = limit == 0 ? INT64_MAX : (int64_t)limit - (int64_t)o;  // (multiples of 256 both)
     o = align_up(o + (rows <= kMaxGemvRows ? gemv_workspace_bytes(rows, Ng, Kg, G) : gemm_workspace_bytes(rows, Ng, Kg, G, w.room)), 256);
     w.total = o;
     return w;

@@ -216,7 +216,8 @@ def fc_Q4A(input, weiq, N, residual=None):
 def fc_Q4A_noalloc(input, weiq, N, out):
     """Extension: fc_Q4A into a caller-provided ``out`` (fp32 [B,M,N]) without allocating anything -- the
     workspace is a fixed array inside the library (``llmops_fc_Q4A_noalloc``).  For callers that cannot
-    allocate (graph capture, serving loops); sizes beyond the array raise.  Calls that overlap on one device race."""
+    allocate (graph capture, serving loops); sizes that do not fit the array raise, or split K less and may then differ
+    in rounding.  Calls that overlap on one device race."""
     _dev(input, torch.float32, 3, "input")
     _dev(weiq, torch.int8, 3, "wei_quantized")
     _dev(out, torch.float32, 3, "out")
