@@ -7,6 +7,7 @@ module's own calls in native code (csrc/host, the one part that knows torch's ty
 import glob
 import importlib.util
 import os
+import re
 import subprocess
 import sys
 import sysconfig
@@ -64,10 +65,18 @@ def _compile(src, obj):
 
 
 def _compile_host():
-    torch_dir = os.path.dirname(importlib.util.find_spec("torch").origin)
+    if os.path.exists(HOST_OUT):
+        os.remove(HOST_OUT)
+    spec = importlib.util.find_spec("torch")
+    if spec is None:
+        return HOST_SRC, 0, ["torch is not installed: llmops/_host.so is left out (the C library does not need it)"]
+    torch_dir = os.path.dirname(spec.origin)
+    with open(os.path.join(torch_dir, "version.py")) as fh:
+        version = re.search(r"^__version__ = ['\"]([^'\"]+)", fh.read(), re.M).group(1)
     inc = [os.path.join(torch_dir, "include"), os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
            "/opt/rocm/include", sysconfig.get_paths()["include"]]
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           '-DLLMOPS_BUILT_FOR="torch %s, Python %d.%d"' % ((version,) + sys.version_info[:2])]
     cmd += [a for i in inc for a in ("-isystem", i)] + ["-Wall", "-o", HOST_OUT, HOST_SRC, "-L" + os.path.join(torch_dir, "lib")]
     cmd += ["-ltorch_python", "-ltorch", "-ltorch_hip", "-ltorch_cpu", "-lc10_hip", "-lc10"]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
@@ -104,7 +113,7 @@ def build(verbose=False, jobs=None):
         objs = [os.path.join(objdir, os.path.basename(s) + ".o") for s in srcs]
         with concurrent.futures.ThreadPoolExecutor(jobs) as ex:
             host = ex.submit(_compile_host)
-            results = list(ex.map(lambda so: _compile(*so), zip(srcs, objs))) + [host.result()]
+            results = list(ex.map(lambda so: _compile(*so), zip(srcs, objs)))
         remarks, logs = [], []
         for src, rc, lines in results:
             remarks += [l for l in lines if "[-Rpass-analysis=kernel-resource-usage]" in l]
@@ -118,6 +127,10 @@ def build(verbose=False, jobs=None):
         proc = subprocess.run(link, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
         if proc.returncode != 0:
             raise RuntimeError("link failed:\n" + proc.stdout)
+        src, rc, lines = host.result()
+        if rc != 0:
+            raise RuntimeError(f"compiling {src} failed ({OUT} is built; without _host.so the module calls it through ctypes):\n" + "\n".join(lines))
+        logs += lines
         if verbose and logs:
             print("\n".join(logs))
     finally:

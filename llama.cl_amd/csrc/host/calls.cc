@@ -147,4 +147,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, null
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__host(void) {
+    PyObject* m = PyModule_Create(&module);
+    if (m != nullptr && PyModule_AddStringConstant(m, "built_for", LLMOPS_BUILT_FOR) != 0) {  // (compared before anything is called)
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

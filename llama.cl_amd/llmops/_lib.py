@@ -1,6 +1,8 @@
 """ctypes binding of libllmops_hip.so (the C ABI declared in include/llmops_hip.h)."""
 import ctypes
 import os
+import sys
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libllmops_hip.so")
@@ -102,15 +104,33 @@ def load():
 _host = None
 
 
+class _PythonCalls:
+    """in the place of _host.so where that does not load: leaves every call to the Python functions"""
+
+    @staticmethod
+    def fc_Q4A(*args):
+        return NotImplemented
+
+    attention_rope2 = fc_Q4A
+
+
 def host():
-    """The module's own calls in native code (csrc/host/calls.cc), bound to the library's entries."""
+    """The module's own calls in native code (csrc/host/calls.cc), bound to the library's entries.  They only shorten
+    calls: without them (not built, or built for another torch or Python) the Python functions do the same work."""
     global _host
     if _host is None:
         lib = load()
         try:
+            import torch
             from . import _host as native
+            here = "torch %s, Python %d.%d" % ((torch.__version__,) + sys.version_info[:2])
+            if native.built_for != here:
+                raise ImportError(f"built for {native.built_for}, this is {here}")
         except ImportError as e:
-            raise ImportError(f"llmops/_host.so does not load ({e}): build it with `python llama.cl_amd/build.py`.") from e
+            warnings.warn(f"llmops/_host.so does not load ({e}): calls go through ctypes, which takes some us more each; "
+                          "`python llama.cl_amd/build.py` builds it", RuntimeWarning, stacklevel=3)
+            _host = _PythonCalls
+            return _host
         native.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in (
             "llmops_fc_Q4A_workspace_bytes", "llmops_fc_Q4A", "llmops_attention_workspace_bytes", "llmops_attention_rope",
             "llmops_last_error")))

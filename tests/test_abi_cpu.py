@@ -185,6 +185,38 @@ def test_python_ops_refuse_host_tensors():
         llmops.fc_Q4A(torch.zeros(1, 1, 128), torch.zeros(1, 1, 2176, dtype=torch.int8), 32)
 
 
+@pytest.mark.parametrize("native,why", [("None", "_host"), ("types.SimpleNamespace(built_for='torch 0.1, Python 3.10')", "torch 0.1")])
+def test_calls_without_the_native_module(native, why):
+    """Where _host.so is missing, or built for another torch, the Python functions take the calls, with their own errors, and
+    say so once."""
+    import subprocess
+    import sys
+    code = f"""
+import sys, types, warnings
+sys.path.insert(0, {os.path.dirname(os.path.dirname(LIB))!r})
+sys.modules["llmops._host"] = {native}
+import torch, llmops
+llmops.__dict__.pop("_host", None)
+if sys.modules["llmops._host"] is not None:
+    llmops._host = sys.modules["llmops._host"]
+with warnings.catch_warnings(record=True) as said:
+    warnings.simplefilter("always")
+    for call in (lambda: llmops.fc_Q4A(torch.zeros(1, 1, 128), torch.zeros(1, 1, 2176, dtype=torch.int8), 32),
+                 lambda: llmops.attention_rope2(*[torch.zeros(1, 1, 128)] * 3, torch.zeros(64), torch.zeros(2, 1, 1, 4, 128), torch.zeros(1, dtype=torch.int32), 0, 0)):
+        for _ in range(2):
+            try:
+                call()
+            except RuntimeError as e:
+                print(e)
+print([str(w.message) for w in said])
+"""
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, out.stderr
+    lines = out.stdout.splitlines()
+    assert len(lines) == 5 and all("on the HIP device" in l for l in lines[:4])
+    assert lines[4].count("_host.so does not load") == 1 and why in lines[4]
+
+
 def test_kvcache_slot_manager():
     """KVCache.prepare mirrors chatllama/main.py:60-125: ring buffer, protected system slots, early stop."""
     import torch
