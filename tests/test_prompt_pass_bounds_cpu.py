@@ -1,13 +1,15 @@
-"""Host model of the addresses of a prompt pass (LlamaDecoder.forward, fused plan, more than 8 rows, group 128): for every
+"""Host model of the addresses of a prompt pass (LlamaDecoder.forward, fused plan, 33 tokens and more, group 128): for every
 launch the first and last byte of each pointer, from the launch's arguments and the kernels' index expressions, against the
-size of the allocation behind it.  Plans and workspace sizes come from the library itself (no GPU needed)."""
+part of the allocation that is meant.  Plans and workspace sizes come from the library itself (no GPU needed)."""
 import ctypes
 
 import numpy as np
 import pytest
 
 COUNTERS = 3 << 20          # LLMOPS_FC_COUNTER_BYTES
+TICKETS = 65536             # kTicketBytes: arrival counters, one per tile
 BLK = 2176                  # a packed block of group 128
+LANES = np.arange(64)
 
 
 def up(v, a=256):
@@ -18,64 +20,137 @@ class Model:
     def __init__(self, lib):
         self.lib, self.seen, self.bad = lib, [], []
 
-    def touch(self, launch, what, size, lo, hi):
-        """bytes [lo, hi) of an allocation of `size` bytes"""
+    def touch(self, launch, what, region, lo, hi):
+        """bytes [lo, hi) that must lie in `region`: a size, or (first byte, end)"""
+        first, end = region if isinstance(region, tuple) else (0, region)
         self.seen.append((launch, what))
-        if not (0 <= lo < hi <= size):
-            self.bad.append((launch, what, lo, hi, size))
+        if not (first <= lo < hi <= end):
+            self.bad.append((launch, what, lo, hi, first, end))
+
+    def need(self, rows, Ng, Kg, G=128):
+        return self.lib.llmops_fc_Q4A_workspace_bytes(rows, Kg * G, Ng, Kg, G)
+
+    def plan(self, rows, Ng, Kg, G=128):
+        rt, S = ctypes.c_int(), ctypes.c_int()
+        assert self.lib.llmops_test_gemm_plan(rows, Ng, Kg, G, ctypes.byref(rt), ctypes.byref(S)) == 0
+        return rt.value, S.value
 
 
-def product(m, name, rows, Ng, Kg, N, ws_bytes, y_bytes, y_off=0, w_bytes=None, w_off=0, residual=False):
-    """launch_gemm on a workspace laid out as fc_layout lays it out"""
-    rt, S = ctypes.c_int(), ctypes.c_int()
-    assert m.lib.llmops_test_gemm_plan(rows, Ng, Kg, 128, ctypes.byref(rt), ctypes.byref(S)) == 0
-    rt, S = rt.value, S.value
-    off_xq = COUNTERS
-    off_xd = up(off_xq + rows * Kg * 128)
-    off_gs = up(off_xd + rows * Kg * 4)
+def layout(rows, Kg, G, ws):
+    """fc_layout: codes, scales, sums, pairs (and what the few-row product reads past them), partial sums"""
+    at = {"codes": (COUNTERS, COUNTERS + rows * Kg * G)}
+    off_gs = up(up(COUNTERS + rows * Kg * G) + rows * Kg * 4)
     off_xst = up(off_gs + rows * Kg * 4)
-    off_part = up(off_xst + rows * Kg * 8 + 256)
-    w_bytes = Ng * Kg * BLK if w_bytes is None else w_bytes
-    bm = rt * 32
-    nbx, nby = -(-Ng // 4), -(-rows // bm)
-    kper = -(-Kg // S)
-    bx, by = np.arange(nbx)[:, None], np.arange(nby)[None, :]
-    strips = np.minimum(Ng - 1, bx * 4 + np.array([0, 3])[:, None, None])
-    row = np.minimum(rows - 1, by * bm + np.array([0, bm - 1])[:, None, None])
-    launch = "%s: product of %d x %d strips, %d-row tiles, %d splits" % (name, rows, Ng, bm, S)
-    assert kper * (S - 1) < Kg                                                  # every split has k-groups
-    m.touch(launch, "codes", ws_bytes, off_xq + int(row.min()) * Kg * 128, off_xq + int(row.max()) * Kg * 128 + (Kg - 1) * 128 + 128)
-    m.touch(launch, "pairs", ws_bytes, off_xst, off_xst + ((Kg - 1) * rows + int(row.max())) * 8 + 8)
-    m.touch(launch, "weights", w_bytes, w_off + int(strips.min()) * Kg * BLK, w_off + (int(strips.max()) * Kg + Kg - 1) * BLK + BLK)
-    if rt == 8:  # the min term reads eight k-groups of a row's sums and of a strip's mins at a time
-        assert Kg >= 8 and rows * Kg * 128 < 1 << 31 and Ng * Kg * BLK < 1 << 31   # 32-bit offsets
-        starts = np.minimum(np.concatenate([np.arange(z * kper, min(Kg, (z + 1) * kper), 32) for z in range(S)])[:, None] + 8 * np.arange(4), Kg - 8)
-        m.touch(launch, "sums", ws_bytes, off_gs + int(starts.min()) * 4, off_gs + (int(row.max()) * Kg + int(starts.max())) * 4 + 32)
-    in_kernel = S > 1 and rt != 8 and S <= 12 and nbx * nby <= 65536 // 4
+    at["pairs"] = (off_xst, off_xst + rows * Kg * 8)
+    at["partial sums"] = (up(off_xst + rows * Kg * 8 + 256), ws)
+    return at
+
+
+def tiles_of_the_grid(nbx, nby):
+    """(bx, by) of every workgroup that has a tile: runs of tiles per XCD, bands of 8 row blocks"""
+    total, out = nbx * nby, []
+    per = -(-total // 8)
+    for block in range(8 * per):
+        i = (block & 7) * per + (block >> 3)
+        if i < total:
+            band, in_band = divmod(i, 8 * nbx)
+            rows_in_band = min(8, nby - band * 8)
+            out.append((in_band // rows_in_band, band * 8 + in_band % rows_in_band))
+    return out
+
+
+def product(m, name, rows, Ng, Kg, N, ws_bytes, y_bytes, parts=1, residual=False):
+    """launch_gemm, group 128: fc_gemm_tile_kernel (and gemm_reduce_kernel) on a workspace laid out as fc_layout does;
+    results [parts][rows][N]"""
+    rt, S = m.plan(rows, Ng, Kg)
+    assert rt in (1, 2, 4)
+    at = layout(rows, Kg, 128, ws_bytes)
+    BM, per, Kp = 32 * rt, -(-Kg // S), Kg * 128
+    nbx, nby = -(-Ng // 4), -(-rows // BM)
+    launch = "%s: product of %d rows x %d strips, %d-row tiles, %d splits" % (name, rows, Ng, BM, S)
+    assert (S - 1) * per < Kg <= S * per                                        # every split has k-groups, together all of them
+    grid = tiles_of_the_grid(nbx, nby)
+    assert len(grid) == nbx * nby and len(set(grid)) == len(grid) and max(grid) <= (nbx - 1, nby - 1)
+    codes, pairs, weights = [], [], []
+    for by in range(nby):
+        row0 = by * BM
+        # codes: wave w's copy i has rows (w * RT + i) * 8 + lane / 8, a 16-byte chunk of 128 per lane
+        r = ((np.arange(4)[:, None, None] * rt + np.arange(rt)[:, None]) * 8 + (LANES >> 3)).ravel()
+        chunk = np.tile(LANES & 7, 4 * rt) ^ ((r >> 1) & 7)
+        assert len(set(zip(r, chunk))) == BM * 8 and r.max() == BM - 1
+        off = (np.minimum(rows - 1, row0 + r) - row0) * Kp + chunk * 16
+        assert 0 <= off.min() and off.max() < 1 << 32                           # 32-bit lane offsets
+        codes += [row0 * Kp + off.min(), row0 * Kp + off.max() + (Kg - 1) * 128 + 16]
+        # scales and sums: 64 rows to a copy, 4 bytes per lane, from the pairs [Kg][rows]
+        row = np.minimum(rows - 1, row0 + np.arange(max(1, BM // 64))[:, None] * 64 + np.minimum(LANES, BM - 1))
+        assert row.max() * 8 < 1 << 32
+        pairs += [row.min() * 8, (Kg - 1) * rows * 8 + row.max() * 8 + 4 + 4]
+    for bx in range(nbx):
+        base, strip = bx * 4 * Kg * BLK, (np.minimum(Ng - 1, bx * 4 + np.arange(4)) - bx * 4) * Kg * BLK
+        nib = strip[:, None, None] + (np.arange(2) * 1024)[:, None] + (2 * ((LANES >> 3) & 3) + (LANES >> 5)) * 128 + (LANES & 7) * 16
+        assert len(set(nib[0].ravel())) == 128 and nib[0].max() + 16 == 2048    # a strip's nibbles, each once
+        tail = strip[LANES >> 4] + (LANES & 15) * 4 + 2048                      # scales, and 64 bytes on the mins
+        assert nib.max() < 1 << 32 and tail.max() + 64 < 1 << 32
+        weights += [base + nib.min(), base + (Kg - 1) * BLK + max(nib.max() + 16, tail.max() + 64 + 4)]
+    for what, seen, region in (("codes", codes, at["codes"]), ("pairs", pairs, at["pairs"]), ("weights", weights, (0, Ng * Kg * BLK))):
+        m.touch(launch, what, region, region[0] + int(min(seen)), region[0] + int(max(seen)))
+    # LDS: the last copies of a slot end where the slot's codes, nibbles, scales and row scales end
+    stage = BM * 128 + 4 * 2048 + 256 + BM * 4
+    smem = 3 * stage + 6 * BM * 4 + 6 * 256
+    m.touch(launch, "LDS", smem, 0, 2 * stage + BM * 128 + 4 * 2 * 1024 + 256 + (max(1, BM // 64) - 1) * 256 + 4 * min(64, BM))
+    m.touch(launch, "LDS", smem, 3 * stage, 3 * stage + 6 * BM * 4 + 5 * 256 + 64 * 4)
+    assert smem <= 160 << 10 and {1: 4, 2: 3, 4: 2}[rt] * smem <= 160 << 10     # (as many workgroups to a compute unit as planned)
+    Np, part_strips = Ng * 32, Ng // parts
+    assert Ng % parts == 0 and (parts == 1 or N == part_strips * 32)
+    last_strip = [((s // part_strips) * rows + rows - 1) * N + min(N, (s - s // part_strips * part_strips) * 32 + 32) for s in range(Ng)]
     if S > 1:
-        m.touch(launch, "partial sums", ws_bytes, off_part, off_part + ((S - 1) * rows * Ng * 32 + (rows - 1) * Ng * 32 + Ng * 32) * 4)
-        if in_kernel:
-            m.touch(launch, "counters", 65536, 0, (int(by.max()) * nbx + int(bx.max())) * 4 + 4)
+        first = at["partial sums"][0]
+        if S <= 12 and nbx * nby <= TICKETS // 4:
+            # a row block's sums strip by strip, pairs of rows in 16 bytes per lane, the last of an odd number by itself in 8
+            ends = []
+            for by in range(nby):
+                tile_rows = min(BM, rows - by * BM)
+                rr = np.arange(0, tile_rows, 2)
+                end = np.where(rr + 1 < tile_rows, rr * 128 + 15 * 16 + 16, rr * 128 + 15 * 8 + 8).max()
+                assert end == tile_rows * 128                                   # (a strip's place, filled)
+                ends.append(((by * BM) * Np + (Ng - 1) * 32 * tile_rows) * 4 + int(end))
+            m.touch(launch, "partial sums", at["partial sums"], first, first + (S - 1) * rows * Np * 4 + max(ends))
+            m.touch(launch, "counters", TICKETS, 0, max(by * nbx + bx for bx, by in grid) * 4 + 4)
         else:
+            m.touch(launch, "partial sums", at["partial sums"], first, first + ((S - 1) * rows * Np + (rows - 1) * Np + Np) * 4)
             launch += ", then the sum"
-    m.touch(launch, "result", y_bytes, y_off, y_off + ((rows - 1) * N + N) * 4)
+            m.touch(launch, "partial sums", at["partial sums"], first,
+                    first + ((parts - 1) * N + (S - 1) * rows * Np + (rows - 1) * Np + (N + 3) // 4 * 4) * 4)
+    m.touch(launch, "result", y_bytes, 0, max(last_strip) * 4)
     if residual:
-        m.touch(launch, "residual", y_bytes, y_off, y_off + ((rows - 1) * N + N) * 4)
-    return off_part
+        m.touch(launch, "residual", y_bytes, 0, max(last_strip) * 4)
 
 
-def quantization(m, name, rows, Kg, ws_bytes, x_bytes, glu=False):
-    """rmsnorm_quant_kernel, quant_x_tile128_kernel: codes, scales or pairs, sums"""
-    off_xq = COUNTERS
-    off_xd = up(off_xq + rows * Kg * 128)
-    off_gs = up(off_xd + rows * Kg * 4)
-    off_xst = up(off_gs + rows * Kg * 4)
-    K = Kg * 128
+def product_g32_part(m, name, rows, Ng, Kg, ws_bytes):
+    """launch_gemm, group 32: partial sums [split][rows][Ng * 32], added by a second launch"""
+    _, S = m.plan(rows, Ng, Kg, 32)
+    at = layout(rows, Kg, 32, ws_bytes)["partial sums"]
+    if S > 1:
+        m.touch(name, "partial sums", at, at[0], at[0] + S * rows * Ng * 32 * 4)
+
+
+def quantization(m, name, rows, Kg, ws_bytes, x_bytes, glu=False, norm=False):
+    """rmsnorm_quant_kernel (norm), quant_x_tile128_kernel: codes and the pairs [Kg][rows], nothing else"""
+    at, K = layout(rows, Kg, 128, ws_bytes), Kg * 128
+    if norm:
+        vpt = 1 if K <= 4096 else 2 if K <= 8192 else 4
+        e = np.arange(vpt * 1024) * 4
+        last = int(e[e < K].max()) + 4
+        assert last == K
+        m.touch(name, "norm weights", K * 4, 0, last * 4)
+    else:
+        # 8 rows x 1 or 4 k-groups to a workgroup; rows and k-groups past the end re-read the last and store nothing
+        U = 4 if -(-rows // 8) * -(-Kg // 4) >= 1024 else 1
+        kb = np.minimum(np.arange(-(-Kg // U) * U), Kg - 1)
+        assert kb.max() == Kg - 1
     m.touch(name, "input", x_bytes, 0, ((rows - 1) * (2 if glu else 1) * K + (2 * K if glu else K)) * 4)
-    m.touch(name, "codes", ws_bytes, off_xq, off_xq + (rows - 1) * K + K)
-    m.touch(name, "scales", ws_bytes, off_xd, off_xd + ((rows - 1) * Kg + Kg - 1) * 4 + 4)
-    m.touch(name, "sums", ws_bytes, off_gs, off_gs + ((rows - 1) * Kg + Kg - 1) * 4 + 4)
-    m.touch(name, "pairs", ws_bytes, off_xst, off_xst + ((Kg - 1) * rows + rows - 1) * 8 + 8)
+    m.touch(name, "codes", at["codes"], at["codes"][0], at["codes"][0] + (rows - 1) * K + K)
+    m.touch(name, "pairs", at["pairs"], at["pairs"][0], at["pairs"][0] + ((Kg - 1) * rows + rows - 1) * 8 + 8)
 
 
 def attention(m, rows, H, past, maxlen, half):
@@ -83,62 +158,87 @@ def attention(m, rows, H, past, maxlen, half):
     q_bytes, plane = rows * H * S * 4, H * maxlen * S * e
     ws_bytes = m.lib.llmops_attention_workspace_bytes(1, rows, H, S, maxlen)
     head = 65536
+    part = head + up(maxlen * 4)
     k, r, n = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     assert m.lib.llmops_test_attn_plan(1, rows, H, maxlen, past, int(half), ctypes.byref(k), ctypes.byref(r), ctypes.byref(n)) == 0
+    assert k.value == 3 and (n.value - 1) * r.value < min(past + rows, maxlen) <= n.value * r.value
     kv = min(past + rows, maxlen)
-    name = "attention, kernel %d, %d pieces of %d rows" % (k.value, n.value, r.value)
     slot = np.arange(past, past + rows)
+    # rotation, cache update and, by workgroups of their own in front, the table of which token wrote a cache row
+    tables = -(-kv // 64)
+    table = np.arange(tables * 64)
+    m.touch("rotation", "token of a cache row", (head, part), head, head + int(table[table < kv].max()) * 4 + 4)
+    m.touch("rotation", "slots", rows * 4, 0, (rows - 1) * 4 + 4)
     for what, lo in (("k rows of the cache", 0), ("v rows of the cache", plane)):
-        m.touch("rotation", what, 2 * plane, lo + int(slot.min()) * S * e, lo + ((H - 1) * maxlen + int(slot.max())) * S * e + S * e)
-        m.touch(name, what, 2 * plane, lo, lo + ((H - 1) * maxlen + kv - 1) * S * e + S * e)
+        m.touch("rotation", what, (lo, lo + plane), lo + int(slot.min()) * S * e, lo + ((H - 1) * maxlen + int(slot.max())) * S * e + S * e)
     for what in ("q", "k", "v"):
         m.touch("rotation", what, q_bytes, 0, (((rows - 1) * H + H - 1) * S + S - 1) * 4 + 4)
-    part = head + up(maxlen * 4)
-    if k.value == 3:
-        m.touch("fill", "token of a cache row", ws_bytes, head, head + maxlen * 4)
-        m.touch("rotation", "token of a cache row", part, head + int(slot.min()) * 4, head + int(slot.max()) * 4 + 4)
-        m.touch(name, "token of a cache row", part, head, head + (kv - 1) * 4 + 4)
-    if n.value > 1 or k.value < 3:
-        m.touch(name, "records", ws_bytes, part, part + ((H * rows - 1) * n.value + n.value - 1) * 520 + 520)
+    name = "attention, %d pieces of %d rows" % (n.value, r.value)
+    for what, lo in (("k rows of the cache", 0), ("v rows of the cache", plane)):
+        m.touch(name, what, (lo, lo + plane), lo, lo + ((H - 1) * maxlen + kv - 1) * S * e + S * e)
+    m.touch(name, "token of a cache row", (head, head + kv * 4), head, head + (kv - 1) * 4 + 4)  # (what the table's workgroups wrote)
+    if n.value > 1:
+        m.touch(name, "records", (part, ws_bytes), part, part + ((H * rows - 1) * n.value + n.value - 1) * 520 + 520)
     m.touch(name, "output", q_bytes, 0, ((rows - 1) * H + H - 1) * S * 4 + S * 4)
 
 
-@pytest.mark.parametrize("rows", [33, 200, 300, 384, 512, 513, 1000, 2048])
+@pytest.mark.parametrize("rows", [33, 65, 200, 300, 383, 384, 512, 513, 1000, 2048])
 @pytest.mark.parametrize("past,half", [(0, False), (700, True)])
 def test_every_address_of_a_prompt_pass(rows, past, half):
     from llmops import _lib
     lib = _lib.load()
     m, H, F, V, heads, table = Model(lib), 4096, 11008, 55296, 32, 1024
     maxlen = max(256, up(past + rows))
-    need = lambda Ng, Kg: lib.llmops_fc_Q4A_workspace_bytes(rows, Kg * 128, Ng, Kg, 128)
     m.touch("embedding", "output", rows * H * 4, 0, (rows - 1) * H * 4 + ((H // 4 - 1) * 4 + 4) * 4)
     m.touch("embedding", "rows", table * H, 0, (table - 1) * H + (H // 4 - 1) * 4 + 4)
-    # q, k, v: three products of 128 strips on one quantization; the workspace is the larger of what whole and part need
-    ws = max(need(384, 32), need(128, 32))
-    quantization(m, "rmsnorm and quantization", rows, 32, ws, rows * H * 4)
-    layouts = {product(m, "q, k, v part %d" % p, rows, 128, 32, H, ws, 3 * rows * H * 4, p * rows * H * 4, 384 * 32 * BLK, p * 128 * 32 * BLK)
-               for p in range(3)}
-    assert len(layouts) == 1
+    # q, k, v: one product of 384 strips whose stores know the three parts (the call asks for a part's workspace too)
+    ws = max(m.need(rows, 384, 32), m.need(rows, 128, 32))
+    quantization(m, "rmsnorm and quantization", rows, 32, ws, rows * H * 4, norm=True)
+    product(m, "q, k and v", rows, 384, 32, H, m.need(rows, 384, 32), 3 * rows * H * 4, parts=3)
     attention(m, rows, heads, past, maxlen, half)
-    quantization(m, "quantization of o's input", rows, 32, need(128, 32), rows * H * 4)
-    product(m, "o", rows, 128, 32, H, need(128, 32), rows * H * 4, residual=True)
-    quantization(m, "rmsnorm and quantization", rows, 32, need(688, 32), rows * H * 4)
-    product(m, "gate and up", rows, 688, 32, 2 * F, need(688, 32), rows * 2 * F * 4)
-    quantization(m, "silu * up and quantization", rows, 86, need(128, 86), rows * 2 * F * 4, glu=True)
-    product(m, "down", rows, 128, 86, H, need(128, 86), rows * H * 4, residual=True)
-    quantization(m, "rmsnorm and quantization", rows, 32, need(1728, 32), rows * H * 4)
-    product(m, "logits", rows, 1728, 32, V, need(1728, 32), rows * V * 4)
+    quantization(m, "quantization of o's input", rows, 32, m.need(rows, 128, 32), rows * H * 4)
+    product(m, "o", rows, 128, 32, H, m.need(rows, 128, 32), rows * H * 4, residual=True)
+    quantization(m, "rmsnorm and quantization", rows, 32, m.need(rows, 688, 32), rows * H * 4, norm=True)
+    product(m, "gate and up", rows, 688, 32, 2 * F, m.need(rows, 688, 32), rows * 2 * F * 4)
+    quantization(m, "silu * up and quantization", rows, 86, m.need(rows, 128, 86), rows * 2 * F * 4, glu=True)
+    product(m, "down", rows, 128, 86, H, m.need(rows, 128, 86), rows * H * 4, residual=True)
+    quantization(m, "rmsnorm and quantization", rows, 32, m.need(rows, 1728, 32), rows * H * 4, norm=True)
+    product(m, "logits", rows, 1728, 32, V, m.need(rows, 1728, 32), rows * V * 4)
     assert not m.bad, m.bad
     assert len(m.seen) > 60
 
 
-def test_the_model_finds_a_workspace_that_is_too_small():
-    """What the q|k|v product once did: a part's partial sums in a workspace sized for the whole."""
+@pytest.mark.parametrize("rows,Ng,Kg,N,parts", [(45, 3, 1, 96, 1), (131, 7, 5, 210, 1), (300, 128, 86, 4090, 1), (97, 33, 8, 352, 3), (4096, 128, 32, 4096, 1)])
+def test_ragged_products_stay_inside(rows, Ng, Kg, N, parts):
+    """Rows, strips and columns that end inside a tile, a strip and a pair of rows; every split that the kernel finishes itself
+    and one more than that, and a plan forced on every tile."""
     from llmops import _lib
     lib = _lib.load()
     m = Model(lib)
-    whole, part = (lib.llmops_fc_Q4A_workspace_bytes(512, 4096, n, 32, 128) for n in (384, 128))
-    product(m, "q", 512, 128, 32, 4096, whole, 512 * 4096 * 4)
-    assert [b[1] for b in m.bad] == ["partial sums"] and m.bad[0][3] <= part
-    # (not even the module's smallest workspace, 16 MiB, held them)
-    assert m.bad[0][3] > 16 << 20
+    try:
+        for tile in (0, 1, 2, 4):
+            for split in (0, 1, 2, 5, 12, 13):
+                lib.llmops_test_gemm_set_tuning(tile)
+                lib.llmops_test_gemm_set_split(split)
+                product(m, "tile %d" % tile, rows, Ng, Kg, N, m.need(rows, Ng, Kg), parts * rows * N * 4, parts=parts, residual=parts == 1)
+    finally:
+        lib.llmops_test_gemm_set_tuning(0)
+        lib.llmops_test_gemm_set_split(0)
+    assert not m.bad, m.bad
+
+
+def test_the_model_finds_a_workspace_that_is_too_small():
+    """A part of q|k|v with groups of 32, which are products of their own, in a workspace sized for the whole; and partial sums
+    of the tiled product with 256 bytes too few."""
+    from llmops import _lib
+    m = Model(_lib.load())
+    whole, part = m.need(512, 384, 128, 32), m.need(512, 128, 128, 32)
+    assert whole < part
+    product_g32_part(m, "q", 512, 128, 128, part)
+    assert not m.bad
+    product_g32_part(m, "q", 512, 128, 128, whole)
+    assert [b[1] for b in m.bad] == ["partial sums"] and m.bad[0][3] == part
+    m.bad.clear()
+    assert m.plan(300, 128, 86)[1] > 1
+    product(m, "down", 300, 128, 86, 4096, m.need(300, 128, 86) - 256, 300 * 4096 * 4)
+    assert [b[1] for b in m.bad] == ["partial sums"]
