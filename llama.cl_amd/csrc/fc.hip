@@ -103,9 +103,10 @@ static int fc_product_many_rows(const uint8_t* w, uint8_t* ws, const FcWorkspace
     // up to 16 rows are still bound by the weight stream: one strip per workgroup, MFMA inner product
     // (us, tiled / streaming: 16 rows 11008x4096 14.6 / 13.5, 22016x4096 21.3 / 17.9).  17..32 rows (two row tiles
     // per wave) win for tensors of fewer than 256 strips, where the tiled kernel has too few tiles (4096x4096 at 17 rows
-    // 15.4 / 9.5, at 32 rows 13.7 / 10.4; 4096x11008 at 24 rows 16.4 / 15.0), and mostly not beyond (11008x4096 at 17 rows
-    // 17.2 / 16.0, at 24 rows 15.4 / 16.8, at 32 rows 16.2 / 17.7; 22016x4096 at 24 rows 23.3 / 22.1; 55296x4096 at 32 rows
-    // 38.6 / 46.2; 11008x11008 at 24 rows 27.0 / 35.6)
+    // 15.4 / 9.5, at 32 rows 13.7 / 10.4; 4096x11008 at 24 rows 16.4 / 15.0).  From there on neither is ahead throughout: the
+    // tiled kernel, taken for all, is behind by about 1.2 us at some sizes (11008x4096 at 17 rows 17.2 / 16.0, 22016x4096 at 24 rows
+    // 23.3 / 22.1) and ahead by 1.4 to 8.6 at others (11008x4096 at 24 rows 15.4 / 16.8, at 32 rows 16.2 / 17.7; 55296x4096 at
+    // 32 rows 38.6 / 46.2; 11008x11008 at 24 rows 27.0 / 35.6)
     if (rows_kernel && (rows <= 16 || (rows <= 32 && Ng < 256)))
         return launch_fc_rows(w, xq, xst, y, rows, Ng, Kg, N, residual, parts, reinterpret_cast<unsigned long long*>(ws + kTicketBytes),
                               LLMOPS_FC_COUNTER_BYTES - kTicketBytes, st);
@@ -235,8 +236,9 @@ static int fc_decode_impl(const float* x, int64_t rows, int64_t K, const int8_t*
         LLMOPS_REQUIRE(glu != 1 && residual == nullptr && sumsq_out == nullptr && (Ng % out_parts) == 0 &&
                        N_out == Ng * kGroupN);
     const FcWorkspace lay = fc_layout(rows, Ng, Kg, group_k);
-    // (parts are products of their own with fewer strips each, and fewer strips are split over K more often: a part can
-    // need more room for partial sums than the whole; the offsets in front of them are the same)
+    // (with groups of 32 parts are products of their own with fewer strips each, and fewer strips are split over K more often:
+    // a part can need more room for partial sums than the whole; the offsets in front of them are the same.  One size is
+    // asked for with either group, as the header says, although with groups of 128 the whole's is used)
     size_t need = lay.total;
     if (out_parts > 1) {
         const size_t part_need = fc_layout(rows, Ng / out_parts, Kg, group_k).total;

@@ -139,10 +139,11 @@ __device__ __forceinline__ void splitk_finish(const v4f (&f)[T][2], float* __res
 //     (2 x 2 waves of 64 x 64 unpack twice as much: 32-row tiles 2 to 7 % slower, 128 rows even), codes are read by all four.
 //     (The weights as the A operand, a row and eight adjacent columns in a lane: 2 % faster with 128 rows, but eight scales to
 //     convert instead of two, 2 to 6 % slower with 32 and 64.)
-//   * codes, nibbles, scales, sums and mins are copied to LDS asynchronously (global_load_lds) two k-groups ahead: no
-//     registers, no LDS store instructions.  (Through registers one k-group ahead: 5 to 13 % slower, 512 x 22016 x 4096 103 us
-//     against 90.)  Codes, scales and nibbles have three slots; sums and mins six, since the min term is formed for four
-//     k-groups together.
+//   * codes, nibbles, scales, sums and mins are copied to LDS asynchronously (global_load_lds), asked for two k-groups before
+//     they are multiplied and waited for one k-group later, where everyone passes the same barrier: what is on its way has the
+//     time of one k-group.  No registers, no LDS store instructions.  (Through registers: 5 to 13 % slower, 512 x 22016 x
+//     4096 103 us against 90.)  Codes, scales and nibbles have three slots; sums and mins six, since the min term is formed
+//     for four k-groups together.
 //   * the first operands of a k-group are read from LDS while the last row tiles of the one before are multiplied, and the
 //     fold of one pair of row tiles runs beside the products of the next: the order is pinned.
 // A 256 x 128 tile with two wave groups (one workgroup per compute unit, 20 % less to copy) takes 165 to 170 us at
@@ -151,7 +152,7 @@ __device__ __forceinline__ void splitk_finish(const v4f (&f)[T][2], float* __res
 // groups in alternating phases from there on) and now: 128 x 4096 x 11008 27.5 / 23.4, 300 x 4090 x 11008 46 / 39, 512 x 4096^2
 // 33.8 / 27.7, 512 x 22016 x 4096 102.5 / 90, 512 x 4096 x 11008 57 / 53, 2048 x 11008 x 4096 164 / 157, 2048 x 4096 x 11008 153 / 151.
 constexpr int kBlk128 = 2176;
-constexpr int kStages = 3;    // LDS slots of a k-group: one is multiplied, one has landed, one is on its way
+constexpr int kStages = 3;    // LDS slots of a k-group: one is multiplied, one has landed (its first operands are read), one is on its way
 constexpr int kMinRing = 6;   // LDS slots of sums and mins: the last four k-groups and the two ahead
 template <int RT>
 struct GemmTile {

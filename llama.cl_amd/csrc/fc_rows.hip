@@ -230,9 +230,8 @@ int launch_fc_rows(const uint8_t* w, const int8_t* xq, const float2* xsT, float*
     const bool split = slots != nullptr && g_rows_split && Ng < 256 && Kg >= 16 && (size_t)rows * Ng * kGroupN * 8 <= slot_bytes;
     const unsigned grid = (unsigned)(split ? 2 * Ng : Ng);
     unsigned long long* sl = split ? slots : nullptr;
-    // A wave has four k-groups in flight per pass: 8 waves cover 32 k-groups per workgroup in one pass (a hidden
-    // size of 4096); longer runs take 16 waves rather than a second pass (4096x11008 in two halves, 16 rows:
-    // 13.3 against 13.8 us; with 32 k-groups 16 waves are slower, 15.7 against 14.1 us at 11008x4096).
+    // 8 waves cover 32 k-groups per workgroup in one pass of up to four k-groups each (a hidden size of 4096); longer runs take
+    // 16 waves rather than longer ones (with 32 k-groups 16 waves of two are slower: 18.9 against 13.2 us at 16 x 11008 x 4096).
     // 17..32 rows: two row tiles per wave, 8 waves (16 would not have the registers).
     const int64_t k_per_wg = split ? (Kg + 1) / 2 : Kg;
     LLMOPS_ROWS_LAUNCH(false, w, xq, xsT, sl, (int)Kg, (int)rows, N, y, residual, (int)(Ng / parts));

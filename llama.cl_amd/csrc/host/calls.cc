@@ -2,10 +2,11 @@
 // call of the C entry.  A small call is shorter than the Python around it (one row of a 4096 x 4096 product: 5.4 us on the
 // device, 10.9 us per call through ctypes and 5.2 us so; one token of attention over 2048 rows of halves 21.2 and 14.1).
 //
-// These are shortcuts for the ordinary case and decide nothing: whatever is not ordinary -- a tensor subclass, tracing or
-// vmap, a mode that intercepts calls, a stream under capture, a workspace that is missing or too small, any argument that
-// a check would refuse -- returns NotImplemented with nothing done, and the Python function takes the call, workspace
-// policy and error messages included.  Nothing is kept between calls but the addresses of the C entries.
+// These are shortcuts for the ordinary case and decide nothing: whatever is not ordinary -- a tensor subclass, vmap, a mode
+// that intercepts calls, a stream under capture, a workspace that is missing or too small, any argument that a check
+// would refuse -- returns NotImplemented with nothing done, and the Python function takes the call, workspace policy and
+// error messages included.  (torch.jit.trace does not stop them: neither way can it record more than the output's
+// allocation.)  Nothing is kept between calls but the addresses of the C entries.
 #include <Python.h>
 
 #include <ATen/ATen.h>
