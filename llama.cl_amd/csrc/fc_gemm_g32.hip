@@ -2,14 +2,18 @@
 // /root/reference/ops/op_fc.hpp:381-412).
 //
 // What bounds it: with a group of 32 every v_mfma_i32_32x32x32_i8 (32 cycles) is a whole k-group of its tile, and its 16
-// results per lane are folded into the fp32 accumulators with 32 vector instructions: the vector ALU (about 60 ns per
-// step and SIMD in a loop of nothing else, against 14 ns of matrix core) is the limit, so everything else is kept off it
-// and out of its way (counters at 512 x 11008 x 4096: the vector ALU issues 66 % of the time, 64 of a wave's 108 vector
-// instructions per k-group are the fold; the matrix cores are busy 15 %; waves wait 24 %):
+// results per lane are folded into the fp32 accumulators with 32 vector instructions.  Products and vector instructions of a
+// SIMD's waves hardly overlap (registers only: 8 such MFMAs take 256 cycles, 64 fold instructions 296 in one wave and 296 in
+// two waves together, both 360 in one wave, 680 in two, 1000 in three): a step of 32 x 64 is 96 cycles of products, the min
+// term's included, and about 98 vector instructions of 2 cycles.  So everything else is kept off the vector ALU and out of
+// its way, and three workgroups share a compute unit (a stage of four k-groups: one alone 0.95 us, two 1.24, three 1.46):
+//   * 168 registers: the operands of one k-group are in registers, those of the next on their way from LDS, and not those of a
+//     whole stage (216, two workgroups: 512 x 11008 x 4096, whose 688 tiles are then more than a round, 105.5 us against 87.2,
+//     128 x 11008 x 4096 40.9 / 35.0, 2048 x 4096^2 133 / 127).
 //   * tile 32 rows x 256 columns, four waves side by side (each 32 x 64 = two strips): a strip's weights are unpacked by
 //     one wave only, and the rows' codes and scales are read from LDS by all four.  (Sixty-four rows x 128 columns, two
-//     waves either way: 0 to 3 % slower at almost every size, 512 x 11008 x 4096 by 2 %; 128 x 128 with 64 x 64 per wave by
-//     7 %: its 256 registers leave two waves per SIMD.)
+//     waves either way, measured with two workgroups to a compute unit: 0 to 3 % slower at almost every size; 128 x 128 with
+//     64 x 64 per wave: 7 %.)
 //   * a stage is four k-groups.  Codes, packed blocks, scales and sums are all copied to LDS asynchronously
 //     (global_load_lds) one stage ahead: no registers, no LDS store instructions, 16 bytes per lane where the layout has
 //     them.  (Weights taken straight from memory into operand registers, one dword per lane and load, cost more than
@@ -27,9 +31,6 @@
 //     gsum every eight groups / now: K = 512 1.16 / 2.91 / 1.16, 1024 1.36 / 3.04 / 1.30, 4096 2.22 / 3.54 / 1.58, 11008
 //     2.18 / 3.52 / 1.79.  (Four groups at a time, a bf16 and a half-length bf16 product: 1.20 / 1.25 / 1.51 / 1.72, and
 //     0 to 2 % faster.)
-// Measured (us for the whole call in a graph, before -- one wave per 64 rows x 64 columns, operands straight from memory,
-// three instructions per fold -- and now): 512 x 11008 x 4096 330 / 109, 512 x 4096 x 11008 230 / 97, 2048 x 4096^2
-// 291 / 133, 64 x 4096^2 40 / 20.5, 9 x 4096 x 11008 33 / 20.4, 300 x 1024 x 2048 35 / 18.5.
 #include <type_traits>
 
 #include "gemm_device.h"
@@ -56,7 +57,7 @@ __device__ __forceinline__ uint32_t bf_pair(float lo, float hi) {
 // PARTIALS: test build that stores the int32 sums of every (row, column, k-group) into out_i ([rows][Ng*32][Kg])
 // WIDE: lane offsets of 64 bits, for a K whose eight strips are 4 GiB and more (K above 26.8 million)
 template <bool PARTIALS, bool WIDE>
-__global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __restrict__ weiq, const int8_t* __restrict__ xq,
+__global__ __launch_bounds__(256, 3) void fc_gemm_g32_kernel(const uint8_t* __restrict__ weiq, const int8_t* __restrict__ xq,
                                                               const float* __restrict__ xd, const float* __restrict__ gs,
                                                               const float2* __restrict__ xsT, float* __restrict__ out,
                                                               int32_t* __restrict__ out_i, int Ng, int Kg, int64_t ldo, int64_t N,
@@ -152,75 +153,72 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
     __syncthreads();
 
     const int akey = (j + ((j >> 3) & 1)) & 7;
-    int a_rd[4];
-#pragma unroll
-    for (int ks = 0; ks < 4; ks++) a_rd[ks] = j * 128 + (((2 * ks + h) ^ akey) * 16);
 
     for (int st = st0; st < st1; st++) {
         const int buf = (st - st0) & 1;
         const bool more = st + 1 < st1;
-        v4i af[4];
-        float4 xf[2][4];
-        // lane half h holds the tile rows 8b + 4h + v (result register 4b + v)
-        auto load_x = [&](int kk) {
-            if (PARTIALS) return;
+        const int nk = min(GPS, kg1 - st * GPS);
+        v4i af[2];
+        uint32_t raw[2][2];
+        uint16_t dbits[2];
+        float4 xf[4];
+        auto load_ops = [&](int kk) {
+            af[kk & 1] = *reinterpret_cast<const v4i*>(&sa[buf][j * 128 + (((2 * kk + h) ^ akey) * 16)]);
 #pragma unroll
-            for (int b = 0; b < 4; b++) xf[kk & 1][b] = *reinterpret_cast<const float4*>(&sx[buf][kk * BM + 8 * b + 4 * h]);
+            for (int s = 0; s < 2; s++) {
+                const uint8_t* bs = &sbn[buf][(2 * wave + s) * 2048 + h * 128 + j * 4 + kk * 512];
+                raw[s][0] = *reinterpret_cast<const uint32_t*>(bs), raw[s][1] = *reinterpret_cast<const uint32_t*>(bs + 256);
+                dbits[s] = sdm[buf][kk * (STRIPS * 64) + (2 * wave + s) * 64 + j];
+            }
         };
+        // lane half h holds the tile rows 8b + 4h + v (result register 4b + v)
+        auto load_x = [&](int kk, int b) {
+            if (!PARTIALS) xf[b] = *reinterpret_cast<const float4*>(&sx[buf][kk * BM + 8 * b + 4 * h]);
+        };
+        load_ops(0);
 #pragma unroll
-        for (int ks = 0; ks < 4; ks++) af[ks] = *reinterpret_cast<const v4i*>(&sa[buf][a_rd[ks]]);
-        load_x(0);
-        v4i bu[2][4];
-        float d[2][4];
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const uint8_t* bs = &sbn[buf][(2 * wave + s) * 2048 + h * 128 + j * 4];
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                const uint32_t w0 = *reinterpret_cast<const uint32_t*>(bs + ks * 512), w1 = *reinterpret_cast<const uint32_t*>(bs + ks * 512 + 256);
-                bu[s][ks] = v4i{(int)lo4(w0), (int)hi4(w0), (int)lo4(w1), (int)hi4(w1)};
-                // (k-groups past the end: d = 0 and nothing is added)
-                const uint16_t bits = sdm[buf][ks * (STRIPS * 64) + (2 * wave + s) * 64 + j];
-                d[s][ks] = f16_bits_to_f32(st * GPS + ks < kg1 ? bits : (uint16_t)0);
-                // converted once, not inside every fma of the fold (v_fma_mix runs at half the rate of v_fma)
-                asm volatile("" : "+v"(d[s][ks]));
-            }
-        }
-        // Min term operands: lane half h has the stage's k-groups h and 2 + h.  The row's sum g = g1 + g2 + g3 and the
-        // column's min m = m1 + m2 in bf16 pieces (g3 and m2 have at most 8 bits left, so their low halves are zero; the low
-        // half of m meets that of g3).
-        Bf16x8 ga[2], ma[2][2];  // [pair of k-groups], [strip][pair]
-        if (!PARTIALS) {
-#pragma unroll
-            for (int p = 0; p < 2; p++) {
-                const float sum = sg[buf][(2 * p + h) * BM + j];
-                const float g1 = st * GPS + 2 * p + h < kg1 ? sum : 0.0f;  // (k-groups past the end add nothing)
-                const float g2 = g1 - bf_piece(g1), g3 = g2 - bf_piece(g2);
-                ga[p].u[0] = ga[p].u[2] = bf_pair(g1, g2), ga[p].u[1] = ga[p].u[3] = __float_as_uint(g3);
-#pragma unroll
-                for (int s = 0; s < 2; s++) {
-                    const float m = f16_bits_to_f32(sdm[buf][(2 * p + h) * (STRIPS * 64) + (2 * wave + s) * 64 + 32 + j]), m2 = m - bf_piece(m);
-                    ma[s][p].u[0] = bf_pair(m, m), ma[s][p].u[1] = __float_as_uint(m);
-                    ma[s][p].u[2] = bf_pair(m2, m2), ma[s][p].u[3] = __float_as_uint(m2);
-                }
-            }
-        }
+        for (int b = 0; b < 4; b++) load_x(0, b);
         __builtin_amdgcn_sched_barrier(0);
         if (more) copy_stage(st + 1, buf ^ 1);
         __builtin_amdgcn_sched_barrier(0);
 
-        v16i acc[2];  // steps (k-group i >> 1, strip i & 1) alternate between the two
-        auto mma = [&](int i) { acc[i & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i >> 1], bu[i & 1][i >> 1], bias, 0, 0, 0); };
-        mma(0);
-        __builtin_amdgcn_sched_barrier(0);
+        v4i bu[2];
+        float d[2][2];  // scales [k-group, odd or even][strip]
+        auto unpack = [&](int kk) {
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int s = i & 1, kk = i >> 1;
-            if (s == 0 && kk + 1 < GPS) load_x(kk + 1);
-            if (i + 1 < 8) {
-                mma(i + 1);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int s = 0; s < 2; s++) {
+                bu[s] = v4i{(int)lo4(raw[s][0]), (int)hi4(raw[s][0]), (int)lo4(raw[s][1]), (int)hi4(raw[s][1])};
+                d[kk & 1][s] = f16_bits_to_f32(dbits[s]);
+                // converted once, not inside every fma of the fold (v_fma_mix runs at half the rate of v_fma)
+                asm volatile("" : "+v"(d[kk & 1][s]));
             }
+        };
+        // Min term operands: lane half h has the k-groups 2p + h of the stage.  The row's sum g = g1 + g2 + g3 and the
+        // column's min m = m1 + m2 in bf16 pieces (g3 and m2 have at most 8 bits left, so their low halves are zero; the low
+        // half of m meets that of g3).
+        Bf16x8 ga, ma[2];
+        float gsum;
+        uint16_t mbits[2];
+        auto load_min = [&](int p) {
+            gsum = sg[buf][(2 * p + h) * BM + j];
+#pragma unroll
+            for (int s = 0; s < 2; s++) mbits[s] = sdm[buf][(2 * p + h) * (STRIPS * 64) + (2 * wave + s) * 64 + 32 + j];
+        };
+        auto min_ops = [&](int p) {
+            const float g1 = 2 * p + h < nk ? gsum : 0.0f;  // (k-groups past the end add nothing)
+            const float g2 = g1 - bf_piece(g1), g3 = g2 - bf_piece(g2);
+            ga.u[0] = ga.u[2] = bf_pair(g1, g2), ga.u[1] = ga.u[3] = __float_as_uint(g3);
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                const float m = f16_bits_to_f32(mbits[s]), m2 = m - bf_piece(m);
+                ma[s].u[0] = bf_pair(m, m), ma[s].u[1] = __float_as_uint(m);
+                ma[s].u[2] = bf_pair(m2, m2), ma[s].u[3] = __float_as_uint(m2);
+            }
+        };
+        v16i acc[2];  // steps (k-group i >> 1, strip i & 1) alternate between the two
+        auto mma = [&](int i) { acc[i & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[(i >> 1) & 1], bu[i & 1], bias, 0, 0, 0); };
+        auto fold = [&](int i) {
+            const int s = i & 1, kk = i >> 1;
             if (PARTIALS) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
@@ -228,20 +226,44 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
                     if (strip0 + s < Ng && row < rows && kg < Kg)
                         out_i[((int64_t)row * ((int64_t)Ng * kGroupN) + (strip0 + s) * kGroupN + j) * Kg + kg] = acc[s][r];
                 }
-            } else {
-                const float dd = d[s][kk], nbd = -kFoldBias * dd;
+                return;
+            }
+            const float dd = d[kk & 1][s], nbd = -kFoldBias * dd;
 #pragma unroll
-                for (int b = 0; b < 4; b++) {
-                    const float4 x = xf[kk & 1][b];
-                    f[s][4 * b + 0] = fmaf(fmaf(__int_as_float(acc[s][4 * b + 0]), dd, nbd), x.x, f[s][4 * b + 0]);
-                    f[s][4 * b + 1] = fmaf(fmaf(__int_as_float(acc[s][4 * b + 1]), dd, nbd), x.y, f[s][4 * b + 1]);
-                    f[s][4 * b + 2] = fmaf(fmaf(__int_as_float(acc[s][4 * b + 2]), dd, nbd), x.z, f[s][4 * b + 2]);
-                    f[s][4 * b + 3] = fmaf(fmaf(__int_as_float(acc[s][4 * b + 3]), dd, nbd), x.w, f[s][4 * b + 3]);
+            for (int b = 0; b < 4; b++) {
+                const float xv[4] = {xf[b].x, xf[b].y, xf[b].z, xf[b].w};
+                float t[4];
+#pragma unroll
+                for (int v = 0; v < 4; v++) t[v] = fmaf(__int_as_float(acc[s][4 * b + v]), dd, nbd);
+#pragma unroll
+                for (int v = 0; v < 4; v++) f[s][4 * b + v] = fmaf(t[v], xv[v], f[s][4 * b + v]);
+                if (s == 1 && kk + 1 < GPS) {
+                    asm volatile("" : "+v"(f[s]));
+                    load_x(kk + 1, b);
                 }
-                // (the strip's next fold is two steps away: nothing waits for the product)
-                if ((kk & 1) == 0) f[s] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ga[kk >> 1].h, ma[s][kk >> 1].h, f[s], 0, 0, 0);
+            }
+            // (the strip's next fold is two steps away: nothing waits for the product)
+            if ((kk & 1) == 0) f[s] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ga.h, ma[s].h, f[s], 0, 0, 0);
+        };
+        unpack(0);
+        mma(0);
+#pragma unroll
+        for (int kk = 0; kk < GPS; kk++) {
+            if (kk >= nk) break;  // (uniform: the last stage may have fewer k-groups)
+            __builtin_amdgcn_sched_barrier(0);
+            mma(2 * kk + 1);
+            if (kk + 1 < GPS) load_ops(kk + 1);
+            if (!PARTIALS && (kk & 1) == 0) load_min(kk >> 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (!PARTIALS && (kk & 1) == 0) min_ops(kk >> 1);
+            fold(2 * kk);
+            __builtin_amdgcn_sched_barrier(0);
+            if (kk + 1 < GPS) {
+                unpack(kk + 1);
+                mma(2 * kk + 2);
             }
             __builtin_amdgcn_sched_barrier(0);
+            fold(2 * kk + 1);
         }
         __builtin_amdgcn_s_waitcnt(kVmcnt0);  // this wave's copies for the next stage have landed
         __syncthreads();
@@ -263,10 +285,11 @@ __global__ __launch_bounds__(256, 2) void fc_gemm_g32_kernel(const uint8_t* __re
     }
 }
 
-// Split-K factor.  Estimated time in us: a workgroup's run of stages plus half a stage, 1.43 us each, times how many
-// workgroups a compute unit has to run (two fit, and two together take 1.3 times what one does alone); the second launch
-// that adds the partial sums 2 us, 2 more per four splits (its loads in flight) and their traffic.  Measured against every
-// factor of 1, 2, 3, 4, 6, 8, 12, 16, 24 at 9 .. 2048 rows of five shapes: 0.9 % slower than the best on average, 9 % at worst.
+// Split-K factor.  Estimated time in us: a workgroup's run of stages, 0.95 us each, times how many workgroups a compute unit
+// has to run (three fit; two together take 1.3, three 1.53 times what one does alone); the second launch that adds the partial
+// sums 0.44 us per four splits (its loads in flight) and their traffic.  Against every factor of 1 .. 6, 8, 10, 12, 16, 20, 24 at 19
+// row counts from 9 to 2048 of seven shapes: 1.3 % slower than the best on average, 10 % at worst (32 x 22016 x 4096, 8 splits
+// where 4 are best; the rule of two workgroups to a compute unit: 2.3 %, 23 %).
 // Partial sums never take a workspace that fits the built-in scratch of llmops_fc_Q4A_noalloc beyond it.
 int plan_gemm_g32(int64_t rows, int64_t Ng, int64_t Kg, int force_split, int* st_per_split) {
     const int64_t nst = (Kg + kG32Gps - 1) / kG32Gps;
@@ -279,9 +302,9 @@ int plan_gemm_g32(int64_t rows, int64_t Ng, int64_t Kg, int force_split, int* st
         if (force_split > 0 && s != (force_split < nst ? (force_split < 24 ? force_split : 24) : nst)) continue;
         const int64_t per = (nst + s - 1) / s, S = (nst + per - 1) / per;
         if (S > 1 && room >= 0 && S * rows * Ng * kGroupN * 4 > room && force_split <= 0) continue;
-        const int64_t full = tiles * S / 512, rest = tiles * S % 512;
-        double t = 1.43 * ((double)per + 0.5) * ((double)full * 1.3 + (rest == 0 ? 0.0 : rest <= 256 ? 1.0 : 1.3));
-        if (S > 1) t += 2.0 + 2.0 * (double)((S + 3) / 4) + 0.5e-6 * (double)S * (double)rows * (double)(Ng * kGroupN);
+        const int64_t full = tiles * S / 768, rest = tiles * S % 768;
+        double t = 0.95 * (double)per * ((double)full * 1.53 + (rest == 0 ? 0.0 : rest <= 256 ? 1.0 : rest <= 512 ? 1.3 : 1.53));
+        if (S > 1) t += 0.44 * (double)((S + 3) / 4) + 1.16e-6 * (double)S * (double)rows * (double)(Ng * kGroupN);
         if (best == 0.0 || t < best) best = t, best_s = S, best_per = per;
     }
     *st_per_split = (int)best_per;

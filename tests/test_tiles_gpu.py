@@ -69,6 +69,27 @@ def test_tiled_product_sums_that_overflow(ops, orc, rows):
     assert max_rel_err(got[0, other], want[0, other]) <= 1e-5
 
 
+@pytest.mark.parametrize("rows,N", [(9, 70), (33, 300)])
+@pytest.mark.parametrize("Kg", [1, 2, 3, 4, 5, 6, 7, 10])
+def test_group32_product_last_stage(ops, orc, rows, N, Kg):
+    """The group-32 product's stages of four k-groups where the last has one, two, three or all of them, in the only stage and
+    behind others: int32 sums exactly; outputs, a row of huge and one of zero activations among them, to 1e-5 of each row's
+    own largest (sums of Kg products: Kg * 2^-24)."""
+    x, w, res = _inputs(rows, N, 32 * Kg, rows + Kg)
+    x[0, 2] *= 30000.0
+    x[0, 3] = 0.0
+    pw = orc.quant_w(w, 32)
+    rng = np.random.default_rng(Kg)
+    xq = rng.integers(-127, 128, (rows, 32 * Kg)).astype(np.int8)
+    assert np.array_equal(ops.fc_Q4A_partials(dev(xq), dev(pw), use_mfma=1).cpu().numpy(), orc.fc_partials(xq, pw))
+    want = orc.fc(x, pw, N)
+    got = ops.fc_Q4A(dev(x), dev(pw), N).cpu().numpy()
+    scale = np.abs(want[0]).max(axis=1, keepdims=True)
+    assert (np.abs(got[0] - want[0]) <= 1e-5 * scale).all() and (got[0, 3] == 0.0).all()
+    got = ops.fc_Q4A(dev(x), dev(pw), N, residual=dev(res)).cpu().numpy()
+    assert (np.abs(got[0] - (want + res)[0]) <= 1e-5 * np.maximum(scale, np.abs(res[0]).max())).all()
+
+
 @pytest.mark.parametrize("rows", [3, 16, 17, 32])
 @pytest.mark.parametrize("N,Kg", [(2048, 1), (2050, 15), (2048, 16), (2080, 35), (2048, 49), (8224, 33), (8224, 66)])
 def test_few_row_product_runs(ops, orc, rows, N, Kg):
