@@ -85,6 +85,14 @@ __device__ __forceinline__ float silu_times(float gate, float up) {
     return up * (gate * __builtin_amdgcn_rcpf(1.0f + expf(-gate)));
 }
 
+// Codes of a group-128 product in the order of the A operands of v_mfma_i32_16x16x64_i8 (fc_rows.hip): sixteen rows (n, fewer at
+// the end) after sixteen rows, k-group after k-group, 16 k-values (chunk 0 .. 7 of the k-group) of all n rows after the next 16.
+// Byte offset of the chunk of a row; as many bytes in all as row by row.
+__device__ __forceinline__ int64_t tile_code_offset(int64_t row, int64_t rows, int64_t Kg, int64_t kb, int chunk) {
+    const int64_t first = row & ~(int64_t)15, n = rows - first < 16 ? rows - first : 16;
+    return first * Kg * 128 + ((kb * 8 + chunk) * n + (row - first)) * 16;
+}
+
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));

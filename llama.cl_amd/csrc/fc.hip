@@ -9,9 +9,9 @@ namespace llmops {
 constexpr int kMaxGemvRows = 8;
 
 int launch_quant_x(const float* x, int64_t rows, int64_t K, int group_k, int8_t* xq, float* xd, float* gsum, float2* xsT,
-                   bool exact_sum, hipStream_t stream);
+                   bool exact_sum, bool* tile, hipStream_t stream);
 int launch_quant_x_fused(const float* x, int64_t rows, int64_t K, int group_k, const float* norm_w, float eps, bool glu_in,
-                         int8_t* xq, float2* xsT, hipStream_t stream);
+                         int8_t* xq, float2* xsT, bool tiled, hipStream_t stream);
 int launch_strip_sumsq(const float* y, int64_t rows, int64_t N, float* out, hipStream_t st);
 size_t gemv_workspace_bytes(int64_t rows, int64_t Ng, int64_t Kg, int G);
 int launch_gemv(const uint8_t* w, const int8_t* xq, const float* xd, const float* gs, float* y, float* part,
@@ -29,11 +29,17 @@ int launch_gemm(const uint8_t* w, const int8_t* xq, const float* xd, const float
                 int64_t room, int64_t parts, hipStream_t st);
 int launch_gemm_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg, int G,
                          bool rows128, hipStream_t st);
-int launch_fc_rows(const uint8_t* w, const int8_t* xq, const float2* xsT, float* y, int64_t rows, int64_t Ng, int64_t Kg,
+int launch_fc_rows(const uint8_t* w, const int8_t* xq, bool tiled, const float2* xsT, float* y, int64_t rows, int64_t Ng, int64_t Kg,
                    int64_t N, const float* residual, int64_t parts, unsigned long long* slots, size_t slot_bytes, hipStream_t st);
 int launch_fc_rows_partials(const uint8_t* w, const int8_t* xq, int32_t* acc, int64_t rows, int64_t Ng, int64_t Kg,
                             hipStream_t st);
+bool stream_fits(int64_t rows, int64_t Kg);
+bool stream_forced();
+bool streams(int64_t rows, int64_t Ng, int64_t Kg, int group_k);  // below
+double stream_estimate(int64_t rows, int64_t Ng, int64_t Kg, size_t slot_bytes);
 bool gemm_rows_kernel_enabled();
+bool gemm_tile_forced();
+double gemm_tile_estimate(int64_t rows, int64_t Ng, int64_t Kg);
 
 static inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
@@ -91,24 +97,32 @@ static int fc_check_args(const float* x, int64_t rows, int64_t K, const int8_t* 
     return LLMOPS_OK;
 }
 
+// Whether the product of quantized activations (group 128) is the weight-streaming kernel's or the tiled one's.  Up to 16
+// rows are bound by the weight stream (tiled / streaming, us: 9 x 1024 x 512 7.6 / 5.0, 16 x 512 x 4096 9.6 / 6.5).  Above, the
+// streaming kernel fetches every row's codes for each strip again, the tiled one shares them between four strips but needs splits
+// of K and barriers: whichever is estimated to take less, with 7 us on the tiled side, which its estimate leaves out.  Of 190 sizes (17 ..
+// 512 rows of 13 shapes from 1024 x 512 to 11008 x 11008) two are up to 5 % slower than by the other kernel (384 x 4096 x 11008 43.7 /
+// 45.8) and six stay up to 20 % behind it (96 x 22016 x 4096 35.3 / 29.5): 64 x 4096^2 14.1 / 9.0, 128 x 4096 x 11008 25.1 / 22.6, 256 x
+// 4096^2 20.9 / 16.3, 512 x 2048^2 15.5 / 12.8; 256 x 22016 x 4096 48.1 / 57.3, 128 x 11008 x 11008 43.6 / 49.1.  Beyond 512 rows
+// it was not measured.
+bool llmops::streams(int64_t rows, int64_t Ng, int64_t Kg, int group_k) {
+    if (group_k != 128 || rows > 512 || !gemm_rows_kernel_enabled() || !stream_fits(rows, Kg)) return false;
+    if (rows <= 16 && Ng >= 64) return true;
+    if (rows <= kMaxGemvRows || gemm_tile_forced()) return false;
+    if (stream_forced()) return true;
+    return stream_estimate(rows, Ng, Kg, LLMOPS_FC_COUNTER_BYTES - kTicketBytes) <= gemm_tile_estimate(rows, Ng, Kg) + 7.0;
+}
+
 // the product for activations that a quantization launch has left in the workspace (more rows than the streaming
-// kernel that quantizes on the fly takes)
-static int fc_product_many_rows(const uint8_t* w, uint8_t* ws, const FcWorkspace& lay, int64_t rows, int64_t Ng, int64_t Kg,
+// kernel that quantizes on the fly takes); streamed: what streams() says; tiled: the codes are in the order of tile_code_offset
+static int fc_product_many_rows(const uint8_t* w, uint8_t* ws, const FcWorkspace& lay, bool streamed, bool tiled, int64_t rows, int64_t Ng, int64_t Kg,
                                 int group_k, int64_t N, const float* residual, float* y, int64_t parts, hipStream_t st) {
     const int8_t* xq = reinterpret_cast<const int8_t*>(ws + lay.off_xq);
     const float* xd = reinterpret_cast<const float*>(ws + lay.off_xd);
     const float* gs = reinterpret_cast<const float*>(ws + lay.off_gs);
     const float2* xst = reinterpret_cast<const float2*>(ws + lay.off_xst);
-    const bool rows_kernel = group_k == 128 && Ng >= 64 && gemm_rows_kernel_enabled();
-    // up to 16 rows are still bound by the weight stream: one strip per workgroup, MFMA inner product
-    // (us, tiled / streaming: 16 rows 11008x4096 14.6 / 13.5, 22016x4096 21.3 / 17.9).  17..32 rows (two row tiles
-    // per wave) win for tensors of fewer than 256 strips, where the tiled kernel has too few tiles (4096x4096 at 17 rows
-    // 15.4 / 9.5, at 32 rows 13.7 / 10.4; 4096x11008 at 24 rows 16.4 / 15.0).  From there on neither is ahead throughout: the
-    // tiled kernel, taken for all, is behind by about 1.2 us at some sizes (11008x4096 at 17 rows 17.2 / 16.0, 22016x4096 at 24 rows
-    // 23.3 / 22.1) and ahead by 1.4 to 8.6 at others (11008x4096 at 24 rows 15.4 / 16.8, at 32 rows 16.2 / 17.7; 55296x4096 at
-    // 32 rows 38.6 / 46.2; 11008x11008 at 24 rows 27.0 / 35.6)
-    if (rows_kernel && (rows <= 16 || (rows <= 32 && Ng < 256)))
-        return launch_fc_rows(w, xq, xst, y, rows, Ng, Kg, N, residual, parts, reinterpret_cast<unsigned long long*>(ws + kTicketBytes),
+    if (streamed)
+        return launch_fc_rows(w, xq, tiled, xst, y, rows, Ng, Kg, N, residual, parts, reinterpret_cast<unsigned long long*>(ws + kTicketBytes),
                               LLMOPS_FC_COUNTER_BYTES - kTicketBytes, st);
     return launch_gemm(w, xq, xd, gs, xst, y, reinterpret_cast<float*>(ws + lay.off_part), reinterpret_cast<unsigned*>(ws), rows, Ng,
                        Kg, group_k, N, residual, lay.room, parts, st);
@@ -145,7 +159,7 @@ static int fc_impl(const float* x, int64_t rows, int64_t K, const int8_t* weiq, 
         // K is not a whole number of k-groups (no shape the reference is used with): the general quantization kernel
         // pads the last group's codes with zeros, as FC_dynamic_quantize_x does, and the product runs on the codes
         float2* xst_t = reinterpret_cast<float2*>(ws + lay.off_xst);
-        int rc_t = launch_quant_x(x, rows, K, group_k, xq, xd, gs, xst_t, false, st);
+        int rc_t = launch_quant_x(x, rows, K, group_k, xq, xd, gs, xst_t, false, nullptr, st);
         if (rc_t) return rc_t;
         if (rows > kMaxGemvRows) return launch_gemm(w, xq, xd, gs, xst_t, y, part, counters, rows, Ng, Kg, group_k, N, residual, lay.room, 1, st);
         if (residual == y) return fail(LLMOPS_EINVAL, "fc_Q4A with a short last k-group and up to 8 rows: residual must not be y");
@@ -153,15 +167,16 @@ static int fc_impl(const float* x, int64_t rows, int64_t K, const int8_t* weiq, 
         if (rc_t == 0 && residual != nullptr) rc_t = launch_add(y, residual, rows * N, st);
         return rc_t;
     }
-    const bool rows_kernel = group_k == 128 && Ng >= 64 && gemm_rows_kernel_enabled();
+    const bool streamed = streams(rows, Ng, Kg, group_k), rows_kernel = Ng >= 64 && streamed;
     const bool gemv = rows <= kMaxGemvRows && !(rows_kernel && rows >= (Ng > 256 ? g_rows_from_large : g_rows_from_small));
     if (gemv)
         return launch_gemv_fused(w, x, y, part, counters, rows, Ng, Kg, group_k, N, residual, nullptr, 0.0f, 0, nullptr, 0,
                                  nullptr, st);
     float2* xst = reinterpret_cast<float2*>(ws + lay.off_xst);
-    int rc = launch_quant_x(x, rows, K, group_k, xq, xd, gs, xst, false, st);
+    bool tiled = streamed;
+    int rc = launch_quant_x(x, rows, K, group_k, xq, xd, gs, xst, false, &tiled, st);
     if (rc) return rc;
-    return fc_product_many_rows(w, ws, lay, rows, Ng, Kg, group_k, N, residual, y, 1, st);
+    return fc_product_many_rows(w, ws, lay, streamed, tiled, rows, Ng, Kg, group_k, N, residual, y, 1, st);
 }
 
 extern "C" int llmops_fc_Q4A(const float* x, int64_t rows, int64_t K, const int8_t* weiq, int64_t Ng, int64_t Kg,
@@ -197,7 +212,7 @@ extern "C" int llmops_fc_Q4A_residual(const float* x, int64_t rows, int64_t K, c
 //   .. and sums:          64x4 7 rows 7.4 / 7.2, 8 7.9 / 7.2; 64x16 5 8.9 / 8.6; 128x32 3 9.1 / 9.2, 4 10.4 / 9.2; 128x86 3 12.7 / 12.3;
 //                         256x32 3 9.6 / 10.2, 4 11.1 / 10.2; 384x32 2 11.2 / 12.9, 3 16.8 / 13.1
 static bool decode_quantizes_first(int64_t rows, int64_t K, int64_t Ng, int64_t Kg, int group_k, bool norm, bool sums_in, int glu, bool sums_out) {
-    if (group_k != 128 || Ng < 64 || !gemm_rows_kernel_enabled() || glu == 1 || (norm && K > 16384)) return false;
+    if (Ng < 64 || rows > kMaxGemvRows || !streams(rows, Ng, Kg, group_k) || glu == 1 || (norm && K > 16384)) return false;
     const bool large = Ng > 256;
     const int64_t blocks = Ng * Kg;
     int from = large ? g_rows_from_large : g_rows_from_small;  // (as in fc_Q4A)
@@ -261,9 +276,11 @@ static int fc_decode_impl(const float* x, int64_t rows, int64_t K, const int8_t*
         float* xd = reinterpret_cast<float*>(ws + lay.off_xd);
         float* gs = reinterpret_cast<float*>(ws + lay.off_gs);
         float2* xst = reinterpret_cast<float2*>(ws + lay.off_xst);
+        const bool streamed = streams(rows, Ng, Kg, group_k);
+        bool tiled = streamed;
         int rc = (norm_w != nullptr || glu == 2)
-                     ? launch_quant_x_fused(x, rows, K, group_k, norm_w, eps, glu == 2, xq, xst, st)
-                     : launch_quant_x(x, rows, K, group_k, xq, xd, gs, xst, false, st);
+                     ? launch_quant_x_fused(x, rows, K, group_k, norm_w, eps, glu == 2, xq, xst, tiled, st)
+                     : launch_quant_x(x, rows, K, group_k, xq, xd, gs, xst, false, &tiled, st);
         if (rc) return rc;
         if (out_parts > 1) {
             // y is [out_parts][rows][N_out / out_parts]: q, k and v of a fused q|k|v tensor come out as three dense matrices
@@ -273,13 +290,13 @@ static int fc_decode_impl(const float* x, int64_t rows, int64_t K, const int8_t*
             // product per slice of strips on the same quantized rows.
             const int64_t ngp = Ng / out_parts, np = N_out / out_parts;
             if (group_k == 128)
-                return fc_product_many_rows(reinterpret_cast<const uint8_t*>(weiq), ws, lay, rows, Ng, Kg, group_k, np, nullptr, y, out_parts, st);
+                return fc_product_many_rows(reinterpret_cast<const uint8_t*>(weiq), ws, lay, streamed, tiled, rows, Ng, Kg, group_k, np, nullptr, y, out_parts, st);
             for (int64_t p = 0; p < out_parts && rc == 0; p++)
-                rc = fc_product_many_rows(reinterpret_cast<const uint8_t*>(weiq) + p * ngp * Kg * block_bytes(group_k), ws, lay,
+                rc = fc_product_many_rows(reinterpret_cast<const uint8_t*>(weiq) + p * ngp * Kg * block_bytes(group_k), ws, lay, false, false,
                                           rows, ngp, Kg, group_k, np, nullptr, y + p * rows * np, 1, st);
             return rc;
         }
-        rc = fc_product_many_rows(reinterpret_cast<const uint8_t*>(weiq), ws, lay, rows, Ng, Kg, group_k, N_out, residual, y, 1, st);
+        rc = fc_product_many_rows(reinterpret_cast<const uint8_t*>(weiq), ws, lay, streamed, tiled, rows, Ng, Kg, group_k, N_out, residual, y, 1, st);
         if (rc == 0 && sumsq_out != nullptr) rc = launch_strip_sumsq(y, rows, N_out, sumsq_out, st);
         return rc;
     }

@@ -506,6 +506,7 @@ static int g_gemm_rt = 0;  // 0 = choose per shape; 1, 2, 4 = that tile; -1 = al
 static int g_gemm_fused_reduce = 1;  // split-K partial sums added by the product kernel itself (0: by a second launch)
 static int g_gemm_force_split = 0;   // > 0: the split-K factor to use whatever the estimate says (tests)
 bool gemm_rows_kernel_enabled() { return g_gemm_rt >= 0; }
+bool gemm_tile_forced() { return g_gemm_rt != 0 || g_gemm_force_split > 0; }
 
 // Row tile and split-K factor of the tiled kernel: the least estimated time (us) of 128, 64 or 32 rows x 1 .. 12 splits.  A
 // k-group of a resident round takes 1.2 / 0.95 / 0.81 us (two, three, four workgroups per compute unit), a workgroup
@@ -515,7 +516,7 @@ bool gemm_rows_kernel_enabled() { return g_gemm_rt >= 0; }
 // 1500 x 2048: the choices are 1.4 % slower than the best measured one on average and 8 % at worst (11008 x 4096 at 64 rows: 5 splits,
 // 4 would be better), against 5 % and 65 % (1500 x 2048 at 384 rows) of the rule that counted whole rounds.
 // room: what partial sums may take (bytes).
-static void plan_gemm_tile(int64_t rows, int64_t Ng, int64_t Kg, int64_t room, GemmPlan& p) {
+static double plan_gemm_tile(int64_t rows, int64_t Ng, int64_t Kg, int64_t room, GemmPlan& p) {
     static const int kRT[3] = {4, 2, 1}, kSlots[3] = {512, 768, 1024};
     static const double kGroupUs[3] = {1.2, 0.947, 0.811}, kPartRound[3] = {1.0, 0.541, 0.852};
     double best = 0.0;
@@ -536,6 +537,13 @@ static void plan_gemm_tile(int64_t rows, int64_t Ng, int64_t Kg, int64_t room, G
             }
         }
     }
+    return best;
+}
+
+// estimated time of the tiled kernel (group 128), us
+double gemm_tile_estimate(int64_t rows, int64_t Ng, int64_t Kg) {
+    GemmPlan p;
+    return plan_gemm_tile(rows, Ng, Kg, INT64_MAX, p);
 }
 
 static GemmPlan plan_gemm(int64_t rows, int64_t Ng, int64_t Kg, int G, int64_t room) {

@@ -142,9 +142,10 @@ __global__ __launch_bounds__(256) void quant_x_rows_kernel(const float* __restri
 // store into a line of its own, 16 KB from the next.  Codes and scales as in quant_x_rows_kernel.
 // GLU: x is [rows, 2*Kg*G], a row holding the gate and the up projection side by side, and what is quantized is
 // silu(gate) * up (silu_mul_kernel's expression, so the codes are those of the two launches it replaces).
+// tiled: codes in the order of tile_code_offset instead of row by row (the 8 rows' 16 bytes are then neighbours).
 template <int U, bool GLU = false>
 __global__ __launch_bounds__(256) void quant_x_tile128_kernel(const float* __restrict__ x, int rows, int Kg, int kparts,
-                                                               int8_t* __restrict__ xq, float2* __restrict__ xsT) {
+                                                               int8_t* __restrict__ xq, float2* __restrict__ xsT, bool tiled) {
     constexpr int G = 128;
     const int sub = threadIdx.x & 31, team = threadIdx.x >> 5;
     const int rb = blockIdx.x / kparts, kp = blockIdx.x - rb * kparts;
@@ -183,7 +184,8 @@ __global__ __launch_bounds__(256) void quant_x_tile128_kernel(const float* __res
                            (((uint32_t)q8_code(v[u].z, id) & 0xFFu) << 16) | (((uint32_t)q8_code(v[u].w, id) & 0xFFu) << 24);
         const int kb = kb0 + u;
         if (row_ok && kb < Kg) {
-            *reinterpret_cast<uint32_t*>(xq + (rbase + kb) * G + sub * 4) = c;
+            const int64_t at = tiled ? tile_code_offset(row, rows, Kg, kb, sub >> 2) + (sub & 3) * 4 : (rbase + kb) * G + sub * 4;
+            *reinterpret_cast<uint32_t*>(xq + at) = c;
             if (sub == 0) xsT[(int64_t)kb * rows + row] = make_float2(d, s);
         }
     }
@@ -196,7 +198,7 @@ __global__ __launch_bounds__(256) void quant_x_tile128_kernel(const float* __res
 template <int VPT, int G>
 __global__ __launch_bounds__(1024) void rmsnorm_quant_kernel(const float* __restrict__ x, int64_t hidden,
                                                               const float* __restrict__ w, float eps, int rows,
-                                                              int8_t* __restrict__ xq, float2* __restrict__ xsT) {
+                                                              int8_t* __restrict__ xq, float2* __restrict__ xsT, bool tiled) {
     constexpr int TPG = G / 4;
     __shared__ float red[16];
     const int row = blockIdx.x;
@@ -223,7 +225,8 @@ __global__ __launch_bounds__(1024) void rmsnorm_quant_kernel(const float* __rest
         const uint32_t c = ((uint32_t)q8_code(n.x, id) & 0xFFu) | (((uint32_t)q8_code(n.y, id) & 0xFFu) << 8) |
                            (((uint32_t)q8_code(n.z, id) & 0xFFu) << 16) | (((uint32_t)q8_code(n.w, id) & 0xFFu) << 24);
         if (live) {
-            *reinterpret_cast<uint32_t*>(xq + (int64_t)row * hidden + e) = c;
+            const int64_t at = tiled ? tile_code_offset(row, rows, hidden / 128, e / 128, (int)(e % 128) >> 4) + (e & 15) : (int64_t)row * hidden + e;
+            *reinterpret_cast<uint32_t*>(xq + at) = c;
             if ((threadIdx.x % TPG) == 0) xsT[e / G * rows + row] = make_float2(d, s);
         }
     }
@@ -237,9 +240,11 @@ namespace llmops {
 // Quantization with the producer of the activations folded in (shared with fc.hip): norm_w != nullptr quantizes
 // rmsnorm(x) * norm_w, glu_in quantizes silu(gate) * up of rows [gate | up] of 2K floats; one launch instead of the
 // producer's launch, a round trip of its fp32 result through memory and the quantization launch.  Whole k-groups
-// only; scales and sums as the pairs that the product kernels read, xsT [Kg][rows].
+// only; scales and sums as the pairs that the product kernels read, xsT [Kg][rows]; tiled (group 128): codes in the order
+// of tile_code_offset.
 int launch_quant_x_fused(const float* x, int64_t rows, int64_t K, int group_k, const float* norm_w, float eps, bool glu_in,
-                         int8_t* xq, float2* xsT, hipStream_t stream) {
+                         int8_t* xq, float2* xsT, bool tiled, hipStream_t stream) {
+    if (tiled && group_k != 128) return fail(LLMOPS_EINVAL, "fused quantization: codes in tiles with group 128 only");
     const int64_t Kg = K / group_k;
     if (K != Kg * group_k || !aligned(x, 16) || !aligned(xq, 4) || rows >= ((int64_t)1 << 28))
         return fail(LLMOPS_EINVAL, "fused quantization: whole k-groups, 16-byte aligned rows, fewer than 2^28 rows");
@@ -248,8 +253,8 @@ int launch_quant_x_fused(const float* x, int64_t rows, int64_t K, int group_k, c
             return fail(LLMOPS_EINVAL, "fused rmsnorm + quantization: rows of at most 16384 floats, 16-byte aligned weights, no glu");
 #define LLMOPS_RQ(VPT)                                                                                                    \
     do {                                                                                                                  \
-        if (group_k == 32) rmsnorm_quant_kernel<VPT, 32><<<(unsigned)rows, 1024, 0, stream>>>(x, K, norm_w, eps, (int)rows, xq, xsT); \
-        else rmsnorm_quant_kernel<VPT, 128><<<(unsigned)rows, 1024, 0, stream>>>(x, K, norm_w, eps, (int)rows, xq, xsT);   \
+        if (group_k == 32) rmsnorm_quant_kernel<VPT, 32><<<(unsigned)rows, 1024, 0, stream>>>(x, K, norm_w, eps, (int)rows, xq, xsT, false); \
+        else rmsnorm_quant_kernel<VPT, 128><<<(unsigned)rows, 1024, 0, stream>>>(x, K, norm_w, eps, (int)rows, xq, xsT, tiled); \
     } while (0)
         if (K <= 4096) LLMOPS_RQ(1);
         else if (K <= 8192) LLMOPS_RQ(2);
@@ -264,28 +269,31 @@ int launch_quant_x_fused(const float* x, int64_t rows, int64_t K, int group_k, c
         return fail(LLMOPS_EINVAL, "fused silu*up + quantization: group 128 only");
     if (rblocks * ((Kg + 3) / 4) >= 1024) {
         const int kparts = (int)((Kg + 3) / 4);
-        quant_x_tile128_kernel<4, true><<<(unsigned)(rblocks * kparts), 256, 0, stream>>>(x, (int)rows, (int)Kg, kparts, xq, xsT);
+        quant_x_tile128_kernel<4, true><<<(unsigned)(rblocks * kparts), 256, 0, stream>>>(x, (int)rows, (int)Kg, kparts, xq, xsT, tiled);
     } else {
-        quant_x_tile128_kernel<1, true><<<(unsigned)(rblocks * Kg), 256, 0, stream>>>(x, (int)rows, (int)Kg, (int)Kg, xq, xsT);
+        quant_x_tile128_kernel<1, true><<<(unsigned)(rblocks * Kg), 256, 0, stream>>>(x, (int)rows, (int)Kg, (int)Kg, xq, xsT, tiled);
     }
     LLMOPS_LAUNCH_CHECK();
     return LLMOPS_OK;
 }
 
-// shared with fc.hip
+// shared with fc.hip; tile: in, whether the codes may be left in the order of tile_code_offset; out, whether they were
 int launch_quant_x(const float* x, int64_t rows, int64_t K, int group_k, int8_t* xq, float* xd, float* gsum, float2* xsT,
-                   bool exact_sum, hipStream_t stream) {
+                   bool exact_sum, bool* tile, hipStream_t stream) {
+    const bool tiled = tile != nullptr && *tile;
+    if (tile != nullptr) *tile = false;
     const int64_t Kg = (K + group_k - 1) / group_k;
     const int64_t items = rows * Kg;
     if (!exact_sum && xsT != nullptr && group_k == 128 && K == Kg * group_k && aligned(x, 16) && aligned(xq, 4) &&
         rows < ((int64_t)1 << 28) && Kg < ((int64_t)1 << 20) && ((rows + 7) / 8) * Kg < ((int64_t)1 << 31)) {  // (the grid)
         // the group-128 prefill kernels read only the codes and the transposed pairs: xd and gsum stay unwritten
         const int64_t rblocks = (rows + 7) / 8;
+        if (tile != nullptr) *tile = tiled;
         if (rblocks * ((Kg + 3) / 4) >= 1024) {  // enough workgroups with four k-groups per team
             const int kparts = (int)((Kg + 3) / 4);
-            quant_x_tile128_kernel<4><<<(unsigned)(rblocks * kparts), 256, 0, stream>>>(x, (int)rows, (int)Kg, kparts, xq, xsT);
+            quant_x_tile128_kernel<4><<<(unsigned)(rblocks * kparts), 256, 0, stream>>>(x, (int)rows, (int)Kg, kparts, xq, xsT, tiled);
         } else {
-            quant_x_tile128_kernel<1><<<(unsigned)(rblocks * Kg), 256, 0, stream>>>(x, (int)rows, (int)Kg, (int)Kg, xq, xsT);
+            quant_x_tile128_kernel<1><<<(unsigned)(rblocks * Kg), 256, 0, stream>>>(x, (int)rows, (int)Kg, (int)Kg, xq, xsT, tiled);
         }
         LLMOPS_LAUNCH_CHECK();
         return LLMOPS_OK;
@@ -325,7 +333,7 @@ extern "C" int llmops_FC_dynamic_quantize_x(const float* x, int64_t rows, int64_
     LLMOPS_REQUIRE(aligned(xq, 2));
     const int64_t Kg = (K + group_k - 1) / group_k;
     LLMOPS_REQUIRE(rows * Kg < ((int64_t)1 << 33));
-    return launch_quant_x(x, rows, K, group_k, xq, xd, gsum, nullptr, true, as_stream(stream));
+    return launch_quant_x(x, rows, K, group_k, xq, xd, gsum, nullptr, true, nullptr, as_stream(stream));
 }
 
 extern "C" int llmops_FC_dynamic_quantize_x_rows(const float* x, int64_t rows, int64_t K, int group_k, int8_t* xq,
@@ -335,5 +343,5 @@ extern "C" int llmops_FC_dynamic_quantize_x_rows(const float* x, int64_t rows, i
     LLMOPS_REQUIRE(rows > 0 && K > 0 && (K % group_k) == 0);
     LLMOPS_REQUIRE(aligned(x, 16) && aligned(xq, 4));
     LLMOPS_REQUIRE(rows * (K / group_k) < ((int64_t)1 << 33));
-    return launch_quant_x(x, rows, K, group_k, xq, xd, gsum, nullptr, false, as_stream(stream));
+    return launch_quant_x(x, rows, K, group_k, xq, xd, gsum, nullptr, false, nullptr, as_stream(stream));
 }

@@ -72,6 +72,8 @@ SIGNATURES = {
     "llmops_test_fc_set_row_routing": (None, [c_int, c_int]),
     "llmops_test_fc_decode_route": (c_int, [c_i64, c_i64, c_i64, c_i64, c_int, c_int, c_int, c_int, c_int, c_ptr]),
     "llmops_test_fc_rows_set_split": (None, [c_int]),
+    "llmops_test_fc_stream_set": (None, [c_int, c_int, c_int, c_int]),
+    "llmops_test_fc_stream_plan": (c_int, [c_i64, c_i64, c_i64, c_ptr, c_ptr, c_ptr, c_ptr]),
     "llmops_test_attn_set_decode_plan": (None, [c_int]),
     "llmops_test_attn_plan": (c_int, [c_i64, c_i64, c_i64, c_i64, c_int, c_int, c_ptr, c_ptr, c_ptr]),
     "llmops_test_fc_decode_attn_dump": (c_int, [c_ptr, c_ptr, c_i64, c_i64, c_ptr, c_i64, c_i64, c_i64, c_ptr, c_ptr, c_ptr, c_ptr,

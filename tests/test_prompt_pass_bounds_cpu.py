@@ -242,3 +242,88 @@ def test_the_model_finds_a_workspace_that_is_too_small():
     assert m.plan(300, 128, 86)[1] > 1
     product(m, "down", 300, 128, 86, 4096, m.need(300, 128, 86) - 256, 300 * 4096 * 4)
     assert [b[1] for b in m.bad] == ["partial sums"]
+
+
+def streamed(m, name, rows, Ng, Kg, N, ws_bytes, y_bytes, build, parts=1):
+    """launch_fc_rows: fc_stream_kernel on codes in the order of tile_code_offset; results [parts][rows][N]"""
+    rt, sw, nw, halves = build
+    at, Kp = layout(rows, Kg, 128, ws_bytes), Kg * 128
+    blocks, units = -(-rows // (16 * rt)), -(-Ng // sw)
+    launch = "%s: streamed product of %d rows x %d strips, %d row tiles, %d strips, %d waves%s" % (name, rows, Ng, rt, sw, nw, ", halves" if halves else "")
+    per = 2 if halves else 1
+    block = np.arange(-(-units // 8) * 8 * blocks * per)
+    inn = block % (8 * blocks * per)
+    nb0, rb, split = (block // (8 * blocks * per) * 8 + (inn & 7)) * sw, (inn >> 3) % blocks, (inn >> 3) // blocks
+    live = nb0 < Ng
+    seen = set(zip(nb0[live], rb[live], split[live]))
+    assert len(seen) == live.sum() == units * blocks * per                       # every (strips, row block, half) once
+    runs = []
+    for sp in range(per):
+        lo, hi = sp * Kg // per, (sp + 1) * Kg // per
+        runs += [(lo + w * (hi - lo) // nw, lo + (w + 1) * (hi - lo) // nw) for w in range(nw)]
+    assert [r[0] for r in runs] == [0] + [r[1] for r in runs][:-1] and runs[-1][1] == Kg   # the waves' runs cover K once
+    # codes: what the quantization writes fills rows * Kp bytes, each chunk of 16 once, and the loads find a row's chunks
+    row, g, jj = np.arange(rows), LANES >> 4, LANES & 15
+    first, n = row & ~15, np.minimum(16, rows - (row & ~15))
+    kbs = sorted({0, Kg // 2, Kg - 1})
+    wrote = {}
+    for kb in kbs:
+        for chunk in range(8):
+            for r, o in zip(row, first * Kp + ((kb * 8 + chunk) * n + (row - first)) * 16):
+                assert o not in wrote
+                wrote[o] = (r, kb, chunk)
+    assert max(wrote) + 16 == at["codes"][1] - at["codes"][0] == rows * Kp
+    for b in range(blocks):
+        for t in range(rt):
+            top = min(b * 16 * rt + 16 * t, (rows - 1) & ~15)
+            cnt = min(16, rows - top)
+            lane = top * Kp + (g * cnt + np.minimum(jj, cnt - 1)) * 16
+            for kb in kbs:
+                for h in range(2):
+                    off = lane + (kb * 2 + h) * cnt * 64
+                    assert off.max() < 1 << 32
+                    assert [wrote[o] for o in off] == [(top + min(j, cnt - 1), kb, 4 * h + gg) for j, gg in zip(jj, g)]
+    m.touch(launch, "codes", at["codes"], at["codes"][0], at["codes"][0] + max(wrote) + 16)
+    lane_x = np.minimum(rows - 1, np.arange(blocks)[:, None] * 16 * rt + np.minimum(LANES, 16 * rt - 1)) * 8
+    m.touch(launch, "pairs", at["pairs"], at["pairs"][0], at["pairs"][0] + (Kg - 1) * rows * 8 + int(lane_x.max()) + 8)
+    lane_w = 2 * g * 128 + jj * 8 + 9 * 128
+    assert lane_w.max() + 8 == 2048
+    m.touch(launch, "weights", Ng * Kg * BLK, 0, (Ng - 1) * Kg * BLK + (Kg - 1) * BLK + 2048 + 64 + 15 * 4 + 4)
+    assert nw * (32 // sw * (32 * sw + 8) * 4 + 512) <= 64 << 10                # LDS, static
+    if halves:
+        m.touch(launch, "exchange slots", COUNTERS - TICKETS, 0, ((rows - 1) * Ng + Ng - 1) * 32 * 8 + 32 * 8)
+    part_strips = Ng // parts
+    m.touch(launch, "result", y_bytes, 0, max(((s // part_strips) * rows + rows - 1) * N + min(N, (s % part_strips) * 32 + 32) for s in range(Ng)) * 4)
+
+
+@pytest.mark.parametrize("Ng,Kg,N,parts", [(128, 32, 4096, 1), (384, 32, 4096, 3), (688, 32, 22016, 1), (128, 86, 4096, 1), (16, 4, 500, 1), (3, 1, 70, 1)])
+def test_streamed_products_stay_inside(Ng, Kg, N, parts):
+    """The route and the build that are chosen at 1 to 512 rows, and every build forced at ragged ones; above 512 rows never."""
+    from llmops import _lib
+    lib = _lib.load()
+    m, out = Model(lib), [ctypes.c_int() for _ in range(4)]
+
+    def chosen(rows):
+        assert lib.llmops_test_fc_stream_plan(rows, Ng, Kg, *[ctypes.byref(o) for o in out]) == 0
+        return tuple(o.value for o in out) if out[0].value else None
+
+    took = []
+    for rows in (1, 9, 16, 17, 32, 33, 48, 64, 65, 100, 128, 200, 512, 513, 2048):
+        build = chosen(rows)
+        if build:
+            took.append(rows)
+            streamed(m, "chosen", rows, Ng, Kg, N, m.need(rows, Ng, Kg), parts * rows * N * 4, build, parts)
+    assert 513 not in took and 2048 not in took and 48 in took and (9 in took) and ((1 in took) == (Ng >= 64))
+    try:
+        for rt in (1, 2, 3, 4):
+            for sw in (1, 2):
+                for nw in (4, 8):
+                    for halves in (0, 1):
+                        lib.llmops_test_fc_stream_set(rt, sw, nw, halves)
+                        for rows in (9, 45, 131):
+                            build = chosen(rows)
+                            assert build[:3] == (rt, sw, nw)
+                            streamed(m, "forced", rows, Ng, Kg, N, m.need(rows, Ng, Kg), parts * rows * N * 4, build, parts)
+    finally:
+        lib.llmops_test_fc_stream_set(0, 0, 0, 0)
+    assert not m.bad, m.bad

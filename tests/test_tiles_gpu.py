@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+import oracle
 from conftest import max_rel_err
 
 pytestmark = pytest.mark.gpu
@@ -88,6 +89,54 @@ def test_group32_product_last_stage(ops, orc, rows, N, Kg):
     assert (np.abs(got[0] - want[0]) <= 1e-5 * scale).all() and (got[0, 3] == 0.0).all()
     got = ops.fc_Q4A(dev(x), dev(pw), N, residual=dev(res)).cpu().numpy()
     assert (np.abs(got[0] - (want + res)[0]) <= 1e-5 * np.maximum(scale, np.abs(res[0]).max())).all()
+
+
+@pytest.mark.parametrize("halves", [0, 1])
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("strips", [1, 2])
+@pytest.mark.parametrize("row_tiles", [1, 2, 3, 4])
+def test_streaming_product_every_build(ops, orc, row_tiles, strips, waves, halves):
+    """Every build of the weight-streaming product, forced: rows that end inside a row tile, one past it and past a row block, columns
+    inside a strip, strips inside a pair (and fewer than the eight of a round of the XCDs), waves with no k-group, one and several; K in
+    halves; residual, in place too; results in parts; the same bits again (the exchange slots are left empty)."""
+    from llmops import _lib
+    lib = _lib.load()
+    lib.llmops_test_fc_stream_set(row_tiles, strips, waves, halves)
+    try:
+        for rows, N, Kg in ((9, 33, 1), (17, 290, 5), (16 * row_tiles + 1, 96, 9), (33, 130, 17), (129, 1000, 3)):
+            x, w, res = _inputs(rows, N, 128 * Kg, rows + Kg)
+            pw = orc.quant_w(w, 128)
+            want = orc.fc(x, pw, N)
+            tx, tw, tr = dev(x), dev(pw), dev(res)
+            got = ops.fc_Q4A(tx, tw, N)
+            assert max_rel_err(got.cpu().numpy(), want) <= 1e-5
+            assert torch.equal(ops.fc_Q4A(tx, tw, N), got)
+            assert max_rel_err(ops.fc_Q4A(tx, tw, N, residual=tr).cpu().numpy(), want + res) <= 1e-5
+            if pw.shape[0] >= 3:
+                p3 = dev(pw[:pw.shape[0] - pw.shape[0] % 3])
+                whole = ops.fc_Q4A_decode(tx, p3, p3.shape[0] * 32)
+                assert torch.equal(torch.cat(list(ops.fc_Q4A_decode(tx, p3, p3.shape[0] * 32, out_parts=3)), dim=-1), whole)
+            # codes row by row: an input that does not start on 16 bytes takes the general quantization
+            flat = torch.empty(tx.numel() + 2, device="cuda")
+            flat[2:] = tx.flatten()
+            assert max_rel_err(ops.fc_Q4A(flat[2:].view(tx.shape), tw, N).cpu().numpy(), want) <= 1e-5
+    finally:
+        lib.llmops_test_fc_stream_set(0, 0, 0, 0)
+
+
+@pytest.mark.parametrize("rows", [9, 16, 31, 33, 100, 500])
+@pytest.mark.parametrize("N,K", [(512, 512), (4096, 4096), (2090, 1024)])
+def test_streaming_product_exact_and_with_a_producer(ops, orc, rows, N, K):
+    """Whatever build is chosen: whole-numbered inputs whose result is exact, and rmsnorm and silu(gate) * up in the quantization launch, whose
+    codes are those of the separate operators: the same bits."""
+    xe, we = oracle.closed_form_fc_inputs(rows, N, K, seed=rows)
+    got = ops.fc_Q4A(dev(xe.reshape(1, rows, K)), ops.offline_FC_quant_Q4A(dev(we), 128), N).cpu().numpy()
+    assert np.array_equal(got, (xe.astype(np.float64) @ we.astype(np.float64).T).astype(np.float32).reshape(1, rows, N))
+    rng = np.random.default_rng(rows)
+    pw = ops.offline_FC_quant_Q4A(dev((rng.standard_normal((N, K)) * 0.02).astype(np.float32)), 128)
+    x, gu, nw = (dev(rng.standard_normal(s).astype(np.float32)) for s in ((1, rows, K), (1, rows, 2 * K), (K,)))
+    assert torch.equal(ops.fc_Q4A_decode(x, pw, N, norm=(nw, 1e-5)), ops.fc_Q4A(ops.rmsnorm_out(x, nw, 1e-5), pw, N))
+    assert torch.equal(ops.fc_Q4A_decode(gu, pw, N, glu_in=True), ops.fc_Q4A(ops.silu_mul(gu), pw, N))
 
 
 @pytest.mark.parametrize("rows", [3, 16, 17, 32])
