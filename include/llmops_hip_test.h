@@ -52,12 +52,12 @@ void llmops_test_gemm_set_split(int splits);
  * has 32-row tiles only) and the split-K factor.  Reads the knobs above. */
 int llmops_test_gemm_plan(int64_t rows, int64_t Ng, int64_t Kg, int group_k, int* row_tile_factor, int* splits);
 
-/* weight-streaming MFMA kernel (3..512 rows where it is estimated to be the faster one, group 128): whether two workgroups
+/* weight-streaming MFMA kernel (3..1024 rows where it is estimated to be the faster one, group 128): whether two workgroups
  * may have half of K of a strip each (default on; 0 switches it off, for comparisons and tests) */
 void llmops_test_fc_rows_set_split(int on);
 
 /* weight-streaming MFMA kernel: force the build -- row tiles of 16 (1..4) and strips (1, 2) of a workgroup, its waves (4, 8), K in halves
- * where the exchange area has the room -- and send 9..512 rows to it; row_tiles 0 (and what is no build) = choose per shape */
+ * where the exchange area has the room -- and send 17..1024 rows to it; row_tiles 0 (and what is no build) = choose per shape */
 void llmops_test_fc_stream_set(int row_tiles, int strips, int waves, int halves);
 
 /* weight-streaming MFMA kernel (host arithmetic only, no launch): the build that a product of `rows` quantized rows with a
@@ -66,7 +66,7 @@ int llmops_test_fc_stream_plan(int64_t rows, int64_t Ng, int64_t Kg, int* row_ti
 
 /* llmops_fc_Q4A with 2..8 rows, group 128: from how many rows the weight-streaming MFMA kernel (separate
  * quantization launch) replaces the streaming kernel that quantizes on the fly, for tensors of up to
- * 256 strips and for larger ones (defaults 4 and 3; values below 2 restore them) */
+ * 256 strips and for larger ones (values below 2: as the sizes say) */
 void llmops_test_fc_set_row_routing(int rows_from_small, int rows_from_large);
 
 /* llmops_fc_Q4A_decode (host arithmetic only, no launch): whether a call of these sizes and options (norm, sumsq_in,

@@ -80,8 +80,28 @@ extern "C" size_t llmops_fc_Q4A_workspace_bytes(int64_t rows, int64_t K, int64_t
 }
 
 // from how many rows the weight-streaming MFMA kernel takes over from the streaming kernel that quantizes
-// on the fly: tensors of up to 256 strips / of more
-static int g_rows_from_small = 4, g_rows_from_large = 3;
+// on the fly, where tests say it: tensors of up to 256 strips / of more; 0: rows_from() below, and in
+// decode_quantizes_first 4 / 3
+static int g_rows_from_small = 0, g_rows_from_large = 0;
+
+// .. in fc_Q4A.  The first kernel's work per weight byte grows with the row count (every row is quantized and dotted separately), the
+// second's time hardly depends on it, separate quantization launch included, which is what it needs up to 8 rows.
+// us, weights from memory, first / second, at rows either side of the line:
+//   4096x4096 (128 strips): 2 rows 5.8 / 6.8, 3 7.4 / 6.9, 8 9.7 / 7.0; 512x4096: 2 5.2 / 5.9, 3 6.8 / 6.0, 8 9.1 / 6.0
+//   4096x11008:             2 rows 8.7 / 10.8, 3 10.7 / 10.9 (from a cache 12.2 / 10.9), 4 12.4 / 10.4, 8 19.6 / 10.6
+//   6000x4096 (188), 8192x4096 (256): 3 rows 7.5 / 7.7 and 8.2 / 8.2, 4 8.5 / 7.8 and 9.1 / 8.2
+//   11008x4096, 12288x4096: 2 rows 9.1 / 11.4 and 9.3 / 11.5, 3 13.1 / 10.5 and 13.7 / 11.4
+//   1500x2048, 2048x2048:   3 rows 5.1 / 5.5, 4 5.7 / 5.5; 1024x512 .. 4096x512, 1024x1024: 4 4.2 / 5.0, 5 5.2 / 5.0
+//   8192x1024:              5 rows 5.5 / 5.7, 6 5.8 / 5.8, 8 6.5 / 5.8
+//   Under 16 strips the first kernel stays up to 8 rows, though it is the slower one from 3 on (352x2048: 4 rows 5.4 / 5.3, 8 8.4 / 5.3):
+//   the bits of its dump build are those of fc_Q4A there.
+static int rows_from(int64_t Ng, int64_t Kg) {
+    const int forced = Ng > 256 ? g_rows_from_large : g_rows_from_small;
+    if (forced > 0) return forced;
+    if (Ng < 16) return kMaxGemvRows + 1;
+    if (Kg < 12) return 5;
+    return Kg >= 32 && (Ng <= 128 || Ng > 256) ? 3 : 4;
+}
 
 // argument checks of fc_Q4A that do not involve the workspace
 static int fc_check_args(const float* x, int64_t rows, int64_t K, const int8_t* weiq, int64_t Ng, int64_t Kg, int group_k,
@@ -103,14 +123,18 @@ static int fc_check_args(const float* x, int64_t rows, int64_t K, const int8_t* 
 // of K and barriers: whichever is estimated to take less, with 7 us on the tiled side, which its estimate leaves out.  Of 190 sizes (17 ..
 // 512 rows of 13 shapes from 1024 x 512 to 11008 x 11008) two are up to 5 % slower than by the other kernel (384 x 4096 x 11008 43.7 /
 // 45.8) and six stay up to 20 % behind it (96 x 22016 x 4096 35.3 / 29.5): 64 x 4096^2 14.1 / 9.0, 128 x 4096 x 11008 25.1 / 22.6, 256 x
-// 4096^2 20.9 / 16.3, 512 x 2048^2 15.5 / 12.8; 256 x 22016 x 4096 48.1 / 57.3, 128 x 11008 x 11008 43.6 / 49.1.  Beyond 512 rows
-// it was not measured.
+// 4096^2 20.9 / 16.3, 512 x 2048^2 15.5 / 12.8; 256 x 22016 x 4096 48.1 / 57.3, 128 x 11008 x 11008 43.6 / 49.1.  Up to 11 k-groups
+// the tiled path's quantization costs less and most of this kernel's time is its results: 4.75 (40 x 4096 x 512 8.8 / 5.7,
+// 384 x 4096 x 512 10.0 / 9.5; 448 rows 10.05 / 10.7, 300 x 6000 x 512 10.4 / 10.7).  From 513 rows on the estimates are less even:
+// 2 (600 x 512 x 4096 17.0 / 13.3, 900 x 2048^2 19.6 / 17.8, 1000 x 1500 x 3072 26.4 / 21.0; 1000 x 600 x 11008 34.7 / 35.4,
+// 800 x 600 x 11008 31.0 / 33.8, 600 x 4096^2 does not come near); beyond 1024 rows what there is to gain is a few percent.
 bool llmops::streams(int64_t rows, int64_t Ng, int64_t Kg, int group_k) {
-    if (group_k != 128 || rows > 512 || !gemm_rows_kernel_enabled() || !stream_fits(rows, Kg)) return false;
-    if (rows <= 16 && Ng >= 64) return true;
-    if (rows <= kMaxGemvRows || gemm_tile_forced()) return false;
+    if (group_k != 128 || rows > 1024 || !gemm_rows_kernel_enabled() || !stream_fits(rows, Kg)) return false;
+    if (rows <= 16) return true;
+    if (gemm_tile_forced()) return false;
     if (stream_forced()) return true;
-    return stream_estimate(rows, Ng, Kg, LLMOPS_FC_COUNTER_BYTES - kTicketBytes) <= gemm_tile_estimate(rows, Ng, Kg) + 7.0;
+    const double ahead = rows > 512 ? 2.0 : Kg < 12 ? 4.75 : 7.0;
+    return stream_estimate(rows, Ng, Kg, LLMOPS_FC_COUNTER_BYTES - kTicketBytes) <= gemm_tile_estimate(rows, Ng, Kg) + ahead;
 }
 
 // the product for activations that a quantization launch has left in the workspace (more rows than the streaming
@@ -146,15 +170,6 @@ static int fc_impl(const float* x, int64_t rows, int64_t K, const int8_t* weiq, 
     float* part = reinterpret_cast<float*>(ws + lay.off_part);
     hipStream_t st = as_stream(stream);
     const uint8_t* w = reinterpret_cast<const uint8_t*>(weiq);
-    // few rows: one launch, the streaming kernel quantizes the activations it needs on the fly.  Its work per
-    // weight byte grows with the row count (every row is quantized and dotted separately), while the time of
-    // the weight-streaming MFMA kernel below hardly depends on it, separate quantization launch included
-    // (us, streaming / MFMA):
-    //   4096x4096 (128 strips):    2 rows  6.4 /  7.7, 3 rows  8.0 /  7.9, 4 rows  8.9 /  7.8, 8 rows 10.5 /  7.9
-    //   4096x11008 (128 strips):   2 rows  9.2 / 12.0, 3 rows 11.0 / 12.2, 4 rows 12.2 / 12.2, 8 rows 20.3 / 12.6
-    //   8192x4096 (256 strips):    2 rows  7.2 /  9.5, 3 rows  8.6 /  8.9, 4 rows  9.5 /  9.0, 8 rows 14.9 /  9.1
-    //   12288x4096 (384 strips):   2 rows  9.6 / 12.4, 3 rows 13.8 / 12.7, 4 rows 15.7 / 12.8, 8 rows 22.9 / 13.1
-    //   22016x4096 (688 strips):   2 rows 13.1 / 16.1, 3 rows 19.9 / 16.2, 4 rows 22.9 / 16.4, 8 rows 31.8 / 16.7
     if (k_tail) {
         // K is not a whole number of k-groups (no shape the reference is used with): the general quantization kernel
         // pads the last group's codes with zeros, as FC_dynamic_quantize_x does, and the product runs on the codes
@@ -167,9 +182,8 @@ static int fc_impl(const float* x, int64_t rows, int64_t K, const int8_t* weiq, 
         if (rc_t == 0 && residual != nullptr) rc_t = launch_add(y, residual, rows * N, st);
         return rc_t;
     }
-    const bool streamed = streams(rows, Ng, Kg, group_k), rows_kernel = Ng >= 64 && streamed;
-    const bool gemv = rows <= kMaxGemvRows && !(rows_kernel && rows >= (Ng > 256 ? g_rows_from_large : g_rows_from_small));
-    if (gemv)
+    const bool streamed = streams(rows, Ng, Kg, group_k);
+    if (rows <= kMaxGemvRows && !(streamed && rows >= rows_from(Ng, Kg)))  // (one launch)
         return launch_gemv_fused(w, x, y, part, counters, rows, Ng, Kg, group_k, N, residual, nullptr, 0.0f, 0, nullptr, 0,
                                  nullptr, st);
     float2* xst = reinterpret_cast<float2*>(ws + lay.off_xst);
@@ -215,7 +229,7 @@ static bool decode_quantizes_first(int64_t rows, int64_t K, int64_t Ng, int64_t 
     if (Ng < 64 || rows > kMaxGemvRows || !streams(rows, Ng, Kg, group_k) || glu == 1 || (norm && K > 16384)) return false;
     const bool large = Ng > 256;
     const int64_t blocks = Ng * Kg;
-    int from = large ? g_rows_from_large : g_rows_from_small;  // (as in fc_Q4A)
+    int from = large ? (g_rows_from_large > 0 ? g_rows_from_large : 3) : g_rows_from_small > 0 ? g_rows_from_small : 4;
     if (norm && !sums_in) return rows >= from - 1;
     const bool producer = norm || glu == 2;
     if (large) return rows >= from - (producer && !sums_out && (glu == 2 || blocks >= 16384) ? 1 : 0);
@@ -412,8 +426,8 @@ extern "C" int llmops_fc_Q4A_partials(const int8_t* xq, int64_t rows, const int8
 
 extern "C" void llmops_test_fc_set_row_routing(int rows_from_small, int rows_from_large) {
     if (!test_hooks_enabled(__func__)) return;
-    g_rows_from_small = rows_from_small >= 2 ? rows_from_small : 4;
-    g_rows_from_large = rows_from_large >= 2 ? rows_from_large : 3;
+    g_rows_from_small = rows_from_small >= 2 ? rows_from_small : 0;
+    g_rows_from_large = rows_from_large >= 2 ? rows_from_large : 0;
 }
 
 // ---- fc_Q4A for callers that cannot allocate ---------------------------------------------------

@@ -298,7 +298,7 @@ def streamed(m, name, rows, Ng, Kg, N, ws_bytes, y_bytes, build, parts=1):
 
 @pytest.mark.parametrize("Ng,Kg,N,parts", [(128, 32, 4096, 1), (384, 32, 4096, 3), (688, 32, 22016, 1), (128, 86, 4096, 1), (16, 4, 500, 1), (3, 1, 70, 1)])
 def test_streamed_products_stay_inside(Ng, Kg, N, parts):
-    """The route and the build that are chosen at 1 to 512 rows, and every build forced at ragged ones; above 512 rows never."""
+    """The route and the build that are chosen at 1 to 1024 rows, and every build forced at ragged ones; above 1024 rows never."""
     from llmops import _lib
     lib = _lib.load()
     m, out = Model(lib), [ctypes.c_int() for _ in range(4)]
@@ -308,12 +308,12 @@ def test_streamed_products_stay_inside(Ng, Kg, N, parts):
         return tuple(o.value for o in out) if out[0].value else None
 
     took = []
-    for rows in (1, 9, 16, 17, 32, 33, 48, 64, 65, 100, 128, 200, 512, 513, 2048):
+    for rows in (1, 9, 16, 17, 32, 33, 48, 64, 65, 100, 128, 200, 512, 1000, 1025, 2048):
         build = chosen(rows)
         if build:
             took.append(rows)
             streamed(m, "chosen", rows, Ng, Kg, N, m.need(rows, Ng, Kg), parts * rows * N * 4, build, parts)
-    assert 513 not in took and 2048 not in took and 48 in took and (9 in took) and ((1 in took) == (Ng >= 64))
+    assert 1025 not in took and 2048 not in took and 48 in took and 9 in took
     try:
         for rt in (1, 2, 3, 4):
             for sw in (1, 2):

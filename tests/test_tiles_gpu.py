@@ -139,6 +139,18 @@ def test_streaming_product_exact_and_with_a_producer(ops, orc, rows, N, K):
     assert torch.equal(ops.fc_Q4A_decode(gu, pw, N, glu_in=True), ops.fc_Q4A(ops.silu_mul(gu), pw, N))
 
 
+@pytest.mark.parametrize("N,Kg", [(70, 11), (96, 12), (4096, 32), (4128, 32), (8224, 31), (8224, 32)])
+def test_rows_either_side_of_the_streaming_kernel(ops, orc, N, Kg):
+    """fc_Q4A on either side of the lines between the kernel that quantizes on the fly (2 to 4 rows) and the weight-streaming one, and
+    between that and the tiles (around 512 and 1024 rows)."""
+    for rows in (2, 3, 4, 5, 8) + ((512, 513, 1024, 1025) if N < 100 else ()):
+        x, w, res = _inputs(rows, N, 128 * Kg, rows + Kg)
+        pw = orc.quant_w(w, 128)
+        want = orc.fc(x, pw, N)
+        assert max_rel_err(ops.fc_Q4A(dev(x), dev(pw), N).cpu().numpy(), want) <= 1e-5
+        assert max_rel_err(ops.fc_Q4A(dev(x), dev(pw), N, residual=dev(res)).cpu().numpy(), want + res) <= 1e-5
+
+
 @pytest.mark.parametrize("rows", [3, 16, 17, 32])
 @pytest.mark.parametrize("N,Kg", [(2048, 1), (2050, 15), (2048, 16), (2080, 35), (2048, 49), (8224, 33), (8224, 66)])
 def test_few_row_product_runs(ops, orc, rows, N, Kg):
