@@ -20,6 +20,7 @@
 #include <limits.h>
 
 #include "common.h"
+#include "gemv_device.h"
 
 namespace llmops {
 
@@ -61,14 +62,15 @@ __device__ __forceinline__ void store_cache<__half>(__half* dst, float v) {
 }
 
 // q,k,v [B,qL,H,S].  One workgroup of a wave per (b, l, h); thread i handles element i (and i+half).  TABLES: before those, `tables`
-// workgroups each write 64 entries of row_token: the (last) token of this call that a cache row belongs to, or -1.  (us for the
+// workgroups each write 64 entries of row_token: the (last) token of this call that a cache row belongs to, -1, or from kvLen on
+// INT_MAX, and the smallest and largest token of each 32 rows.  (us for the
 // whole call, 32 heads, with a launch that filled the table with -1 and a scattered store per token / so: 64 tokens 17.9 / 17.2,
 // 300 behind 300 50.0 / 48.3, 1024 tokens 84.6 / 82.1, 2048 tokens 175 / 172.)
 template <typename T, bool TABLES>
 __global__ void attn_prep_kernel(float* __restrict__ q, float* __restrict__ k, const float* __restrict__ v, int64_t qL,
                                  int64_t H, int64_t S, const float* __restrict__ inv_freq, int64_t half,
                                  T* __restrict__ kc, T* __restrict__ vc, int64_t maxlen, const int32_t* __restrict__ slots,
-                                 int position_id, int32_t* __restrict__ row_token, int64_t kvLen, unsigned tables) {
+                                 int position_id, int32_t* __restrict__ row_token, int2* __restrict__ tile_tokens, int64_t kvLen, unsigned tables) {
     if (TABLES && blockIdx.x < tables) {
         __shared__ int32_t token[64];
         const int64_t row0 = (int64_t)blockIdx.x * 64;
@@ -79,7 +81,12 @@ __global__ void attn_prep_kernel(float* __restrict__ q, float* __restrict__ k, c
             if (at >= 0 && at < 64) atomicMax(&token[at], (int32_t)l);
         }
         __syncthreads();
-        if (row0 + threadIdx.x < kvLen) row_token[row0 + threadIdx.x] = token[threadIdx.x];
+        const int32_t mine = row0 + threadIdx.x < kvLen ? token[threadIdx.x] : INT_MAX;
+        row_token[row0 + threadIdx.x] = mine;
+        int lo = mine, hi = mine;
+#pragma unroll
+        for (int off = 1; off < 32; off <<= 1) lo = min(lo, __shfl_xor(lo, off, 64)), hi = max(hi, __shfl_xor(hi, off, 64));
+        if ((threadIdx.x & 31) == 0) tile_tokens[row0 / 32 + threadIdx.x / 32] = make_int2(lo, hi);
         return;
     }
     const int64_t item = TABLES ? blockIdx.x - tables : blockIdx.x;
@@ -688,6 +695,45 @@ __global__ __launch_bounds__(128) void attn_merge_kernel(float* __restrict__ q, 
     q[((b * qL + pq) * H + h) * S + threadIdx.x] = r;
 }
 
+// The same for up to N records of a query and many queries (the pieces of attn_prefill_kernel): half a wave to a query, 16 bytes to a
+// lane, all records of eight queries asked for at once.  (512 tokens behind 1500, 32 heads, two records each: 20 us by
+// attn_merge_kernel's workgroup per query, 7.)
+template <int N>
+__global__ __launch_bounds__(256) void attn_merge_rows_kernel(float* __restrict__ q, const float* __restrict__ part, int qL, int H,
+                                                               unsigned queries, int nchunks) {
+    constexpr int S = 128;
+    const unsigned bhq = blockIdx.x * 8 + (threadIdx.x >> 5);
+    const int at = 4 * (threadIdx.x & 31);
+    if (bhq >= queries) return;
+    const float* rec = part + (size_t)bhq * nchunks * (S + 2);
+    float2 st[N], lo[N], hi[N];
+#pragma unroll
+    for (int c = 0; c < N; c++) {
+        const float* rc = rec + min(c, nchunks - 1) * (S + 2);
+        st[c] = *reinterpret_cast<const float2*>(rc);
+        lo[c] = *reinterpret_cast<const float2*>(rc + 2 + at);
+        hi[c] = *reinterpret_cast<const float2*>(rc + 4 + at);
+    }
+    float M = -FLT_MAX, den = 0.0f, w[N];
+#pragma unroll
+    for (int c = 0; c < N; c++) M = fmaxf(M, st[c].x);  // (records past the last are copies of it)
+#pragma unroll
+    for (int c = 0; c < N; c++) {
+        w[c] = c >= nchunks || st[c].y == 0.0f ? 0.0f : expf(st[c].x - M);
+        den += w[c] * st[c].y;
+    }
+    const float inv = 1.0f / den;
+    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int c = 0; c < N; c++) {
+        const float wc = w[c] * inv;
+        acc.x = fmaf(wc, lo[c].x, acc.x), acc.y = fmaf(wc, lo[c].y, acc.y);
+        acc.z = fmaf(wc, hi[c].x, acc.z), acc.w = fmaf(wc, hi[c].y, acc.w);
+    }
+    const unsigned pq = bhq % (unsigned)qL, bh = bhq / (unsigned)qL, h = bh % (unsigned)H, b = bh / (unsigned)H;
+    *reinterpret_cast<float4*>(q + (((size_t)b * qL + pq) * H + h) * S + at) = acc;
+}
+
 // ---- decode attention (one query token) ------------------------------------------------------
 // attention_rope2 for qL == 1: every workgroup rotates q itself (cos/sin of the position computed once
 // per workgroup, one angle per lane), the workgroup whose chunk holds the new token's cache row rotates
@@ -1062,6 +1108,14 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(const int32_t* __
 // no query of a wave may see (in-chunk causal mask, ops/op_attn.hpp:1007-1011) are skipped.  K rows
 // take 272 bytes per plane and V columns 80, so that the 16 lanes one phase of a 16-byte read serves
 // touch 16 different 16-byte slots of the 256-byte bank line (17 and 5 are odd).
+//
+// Bound: the products are 3072 cycles of a pass (two tiles) on each SIMD, a pass takes 5400; the vector instructions of its two waves
+// (330 each, most of them the halves of K, V and P and the exponentials) do not overlap them all.  Beside the passes a workgroup spent 23000
+// cycles (10 us) on fetching its queries and on the merge, both by lanes that each followed a row of their own, 16 KB apart; through LDS, rows
+// of 512 bytes on either side, these are 14000, most of it the memory's latency and the masked tiles.  One set now stages its next tile before
+// its products and the other behind them, so that one's vector work meets the other's products (5500 / 5300 cycles a pass).  (whole call, us,
+// before / with all of these, 32 heads: 128 tokens 23.0 / 19.8, 512 48.6 / 41.3, 2048 174 / 159, halves 143 / 127; 512 behind 1500 105 / 79 with
+// the merge by rows.)
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 
@@ -1069,7 +1123,10 @@ typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
     const v2h h = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(a, b));
     hi = __builtin_bit_cast(uint32_t, h);
-    lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a - (float)h[0], b - (float)h[1]));
+    float la, lb;  // a - h.x, b - h.y: one instruction each (the compiler converts, then subtracts)
+    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(la) : "v"(hi), "v"(a));
+    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(lb) : "v"(hi), "v"(b));
+    lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(la, lb));
 }
 __device__ __forceinline__ uint32_t pack_hi(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
@@ -1080,6 +1137,23 @@ union V8hBits {
     uint4 q;
 };
 
+// 4 and 2 elements of a cache row, asked for through a descriptor
+template <typename T>
+__device__ __forceinline__ float4 buffer_load4(buffer_rsrc rs, uint32_t at) {
+    if constexpr (sizeof(T) == 4) {
+        return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0));
+    } else {
+        const uint2 u = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, 0));
+        const float2 a = __half22float2(__builtin_bit_cast(__half2, u.x)), b = __half22float2(__builtin_bit_cast(__half2, u.y));
+        return make_float4(a.x, a.y, b.x, b.y);
+    }
+}
+template <typename T>
+__device__ __forceinline__ float2 buffer_load2(buffer_rsrc rs, uint32_t at) {
+    if constexpr (sizeof(T) == 4) return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, 0));
+    else return __half22float2(__builtin_bit_cast(__half2, (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0)));
+}
+
 // One tile in LDS (fp16 planes, the tile's tokens); each wave set has two of them; the merge at the end reuses the memory
 template <bool LO>
 struct PrefillSmem {
@@ -1089,32 +1163,37 @@ struct PrefillSmem {
     uint8_t v_hi[S * VSB];
     uint8_t v_lo[LO ? S * VSB : 16];
     int tok[BK];
-    int tok_range[4];  // smallest and largest token of the tile
 };
-constexpr size_t kPrefillMergeBytes = (size_t)66 * 256 * sizeof(float);  // set 1's (max, sum, 64 outputs) per lane
+constexpr int kPrefillRow = 528;                      // bytes of a row of 128 floats in LDS: 33 16-byte slots
+constexpr size_t kPrefillRowsBytes = 128 * kPrefillRow;
+// The queries on their way to the registers: beside fp32 rows half of them in each set's second tile buffer (filled behind the first
+// pass's barrier), beside halves behind the buffers.  The merge at the end: both sets' outputs, then (max, sum) of each and the weights.
+constexpr size_t kPrefillMergeBytes = 2 * kPrefillRowsBytes + 3 * 128 * sizeof(float2);
 template <bool LO>
 constexpr size_t prefill_smem_bytes() {
-    return 4 * sizeof(PrefillSmem<LO>) > kPrefillMergeBytes ? 4 * sizeof(PrefillSmem<LO>) : kPrefillMergeBytes;
+    const size_t walk = 4 * sizeof(PrefillSmem<LO>) + (LO ? 0 : kPrefillRowsBytes);
+    return walk > kPrefillMergeBytes ? walk : kPrefillMergeBytes;
 }
+static_assert(sizeof(PrefillSmem<true>) >= kPrefillRowsBytes / 2 && prefill_smem_bytes<true>() <= 160 * 1024 && prefill_smem_bytes<false>() <= 160 * 1024, "");
 
 template <typename T>
 __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __restrict__ kc, const T* __restrict__ vc,
                                                           int64_t qL, int64_t H, int64_t maxlen, int64_t kvLen,
-                                                          const int32_t* __restrict__ row_token, int qtiles, int kv_span,
+                                                          const int32_t* __restrict__ row_token, const int2* __restrict__ tile_tokens, int qtiles, int kv_span,
                                                           float* __restrict__ part, int nsplit) {
     constexpr bool LO = sizeof(T) == 4;  // an fp16 cache holds no low halves
     constexpr int S = 128, BQ = 128, BK = 32, KSB = 272, VSB = 80;
     extern __shared__ __align__(16) uint8_t smem_raw[];
-    const int lane = threadIdx.x & 63, wave8 = threadIdx.x >> 6;
-    const int set = wave8 >> 2, wave = wave8 & 3, tid = threadIdx.x & 255;  // (wave, tid: within the set)
+    const int lane = threadIdx.x & 63, wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int set = wave8 >> 2, wave = wave8 & 3;  // (wave: within the set)
     // two tile buffers per set, used alternately: while a tile is multiplied the next one is written
     PrefillSmem<LO>* const sm2 = reinterpret_cast<PrefillSmem<LO>*>(smem_raw) + 2 * set;
     const int hf = lane >> 5, c32 = lane & 31;
     // late query tiles see the most cache rows: they are dealt out first so that they do not form the tail
     // (gridDim.y = nsplit workgroups share a query tile, each with kv_span cache rows; one: kv_span covers them all)
-    const int64_t bhs = gridDim.x / qtiles;
-    const int qt = qtiles - 1 - (int)(blockIdx.x / bhs);
-    const int64_t bh = blockIdx.x % bhs, b = bh / H, h = bh % H;
+    const unsigned bhs = gridDim.x / (unsigned)qtiles, turn = __builtin_amdgcn_readfirstlane(blockIdx.x / bhs);
+    const int qt = qtiles - 1 - (int)turn;
+    const int64_t bh = blockIdx.x - turn * bhs, b = bh / H, h = bh % H;
     const int kv_begin = (int)blockIdx.y * kv_span;
     // (32-bit arithmetic from here on: the launcher keeps qL and kvLen below 2^31 and a head's cache plane below 4 GiB)
     const int qLi = (int)qL, kvLeni = (int)kvLen;
@@ -1122,21 +1201,11 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __
     const int pq = q_lo_wave + c32;  // this lane's query token
     const bool valid = pq < qLi;
     const int q_hi_wave = min(q_lo_wave + 31, qLi - 1);
-    float* qrow = q + ((b * qL + (valid ? pq : qLi - 1)) * H + h) * S;
+    float* const q0 = q + ((b * qL + qt * BQ) * H + h) * S;  // the first query's row, H * S floats to the next
+    const int q_rows = min(BQ, qLi - qt * BQ);
     const T* kbase = kc + bh * maxlen * S;
     const T* vbase = vc + bh * maxlen * S;
 
-    // the lane's share of its query row as halves: step i covers dims 16i + 8*hf .. +7
-    V8hBits qh[8], ql[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const float4 t0 = *reinterpret_cast<const float4*>(qrow + 16 * i + 8 * hf);
-        const float4 t1 = *reinterpret_cast<const float4*>(qrow + 16 * i + 8 * hf + 4);
-        split2(t0.x, t0.y, qh[i].u[0], ql[i].u[0]);
-        split2(t0.z, t0.w, qh[i].u[1], ql[i].u[1]);
-        split2(t1.x, t1.y, qh[i].u[2], ql[i].u[2]);
-        split2(t1.z, t1.w, qh[i].u[3], ql[i].u[3]);
-    }
     const float d_scale = 1.0f / sqrtf((float)S);
     float m_run = -FLT_MAX, l_run = 0.0f;
     v16f o[4];
@@ -1145,61 +1214,39 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __
 #pragma unroll
         for (int r = 0; r < 16; r++) o[c][r] = 0.0f;
 
-    // Staging.  K: a thread moves 16 consecutive floats of one row (row = thread/8).  V is written transposed,
+    // Staging.  K: a wave moves two whole rows at a time, 16 bytes (8 of halves) to a lane.  V is written transposed,
     // cache row r of the tile at position 16*(r/16) + 8*((r/4)%2) + 4*((r%16)/8) + r%4 of its column: a thread
     // moves the 8 rows that share an aligned run of 8 positions (rows 16b + 4h + w and 16b + 8 + 4h + w, w = 0..3;
     // (b, h) = the thread's wave) of two neighbouring columns, so that a column's share is one 16-byte store.
     // (Four rows of four columns per thread meant 8-byte stores 320 bytes apart: eight lanes on every bank.)
     // The next tile's global loads are issued before the current tile is computed on and land in registers
     // meanwhile.
-    const int krow = tid >> 3, kseg = tid & 7;
+    const int krow = 2 * wave + hf, kseg = c32;  // rows krow + 8u
     const int vb = wave >> 1, vh = wave & 1, vcp = lane;  // rows 16*vb + 8*(e/4) + 4*vh + e%4, columns 2*vcp, 2*vcp+1
     float4 kst[4];
     float2 vst[8];
     int tst = INT_MAX;
+    const uint32_t kv_row = S * sizeof(T), k_at = (uint32_t)krow * kv_row + (uint32_t)kseg * 4 * sizeof(T),
+                   v_at = (uint32_t)(16 * vb + 4 * vh) * kv_row + (uint32_t)vcp * 2 * sizeof(T);
+    // (rows from kvLen on read as zero: the loads go through a descriptor that ends there)
 #define LLMOPS_STAGE_LOAD(KV0)                                                                          \
     do {                                                                                                \
-        const uint32_t rk_ = (uint32_t)min((KV0) + krow, kvLeni - 1);                                   \
-        _Pragma("unroll") for (int u = 0; u < 4; u++)                                                   \
-            kst[u] = load4(kbase + (rk_ * (uint32_t)S + (uint32_t)(kseg * 16 + u * 4)));               \
-        _Pragma("unroll") for (int e = 0; e < 8; e++) {                                                 \
-            const uint32_t rv_ = (uint32_t)min((KV0) + 16 * vb + 8 * (e >> 2) + 4 * vh + (e & 3), kvLeni - 1); \
-            vst[e] = load2(vbase + (rv_ * (uint32_t)S + (uint32_t)(vcp * 2)));                          \
-        }                                                                                               \
-        if (tid < BK) tst = ((KV0) + tid < kvLeni) ? row_token[(KV0) + tid] : INT_MAX;                  \
+        const uint32_t bytes_ = (uint32_t)__builtin_amdgcn_readfirstlane(max(0, min(BK, kvLeni - (KV0)))) * kv_row; \
+        const buffer_rsrc rk_ = make_rsrc(kbase + (int64_t)(KV0) * S, bytes_), rv_ = make_rsrc(vbase + (int64_t)(KV0) * S, bytes_); \
+        _Pragma("unroll") for (int u = 0; u < 4; u++) kst[u] = buffer_load4<T>(rk_, k_at + 8 * u * kv_row); \
+        _Pragma("unroll") for (int e = 0; e < 8; e++) vst[e] = buffer_load2<T>(rv_, v_at + (8 * (e >> 2) + (e & 3)) * kv_row); \
+        if (wave == 0) tst = row_token[(KV0) + c32]; /* (the table ends on a multiple of 64 rows) */    \
     } while (0)
-    // The last cache row that any query of the workgroup may see bounds the walk (rows of later tokens and rows
-    // beyond it are masked anyway; without the bound an early query tile would stage, barrier by barrier, all the
-    // tiles that only later tiles need).
-    int kv_end;
-    {
-        const int q_hi_wg = min((qt + 1) * BQ, qLi) - 1;
-        int last = -1;
-        for (int r = kv_begin + tid; r < min(kvLeni, kv_begin + kv_span); r += 256)
-            if (row_token[r] <= q_hi_wg) last = r;  // (r grows: the last hit is the largest; each set scans all rows)
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) last = max(last, __shfl_xor(last, off, 64));
-        int* const red = sm2[1].tok;  // (the second buffer is first written at the end of the loop's first pass)
-        if (lane == 0) red[wave] = last;
-        __syncthreads();
-        kv_end = max(max(red[0], red[1]), max(red[2], red[3])) + 1;
-    }
-    if (kv_end <= kv_begin) kv_end = kv_begin;  // no row of this range is visible to anybody: nothing to walk
     // Writing a staged tile: halves of K row-major, halves of V transposed, the tile's tokens and their range.
 #define LLMOPS_STAGE_STORE(SM)                                                                                  \
     do {                                                                                                        \
-        uint32_t hi_[8], lo_[8];                                                                                \
         _Pragma("unroll") for (int u = 0; u < 4; u++) {                                                         \
-            split2(kst[u].x, kst[u].y, hi_[2 * u], lo_[2 * u]);                                                 \
-            split2(kst[u].z, kst[u].w, hi_[2 * u + 1], lo_[2 * u + 1]);                                         \
-        }                                                                                                       \
-        uint4* dh_ = reinterpret_cast<uint4*>(&(SM).k_hi[krow * KSB + kseg * 32]);                              \
-        dh_[0] = make_uint4(hi_[0], hi_[1], hi_[2], hi_[3]);                                                    \
-        dh_[1] = make_uint4(hi_[4], hi_[5], hi_[6], hi_[7]);                                                    \
-        if (LO) {                                                                                               \
-            uint4* dl_ = reinterpret_cast<uint4*>(&(SM).k_lo[krow * KSB + kseg * 32]);                          \
-            dl_[0] = make_uint4(lo_[0], lo_[1], lo_[2], lo_[3]);                                                \
-            dl_[1] = make_uint4(lo_[4], lo_[5], lo_[6], lo_[7]);                                                \
+            uint2 hi_, lo_;                                                                                     \
+            split2(kst[u].x, kst[u].y, hi_.x, lo_.x);                                                           \
+            split2(kst[u].z, kst[u].w, hi_.y, lo_.y);                                                           \
+            const int at_ = (krow + 8 * u) * KSB + kseg * 8;                                                    \
+            *reinterpret_cast<uint2*>(&(SM).k_hi[at_]) = hi_;                                                   \
+            if (LO) *reinterpret_cast<uint2*>(&(SM).k_lo[at_]) = lo_;                                           \
         }                                                                                                       \
         {                                                                                                       \
             uint32_t h_[2][4], l_[2][4]; /* [column][pair of rows] */                                           \
@@ -1213,29 +1260,57 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __
                 if (LO) *reinterpret_cast<uint4*>(&(SM).v_lo[at_]) = make_uint4(l_[j][0], l_[j][1], l_[j][2], l_[j][3]); \
             }                                                                                                   \
         }                                                                                                       \
-        if (wave == 0) {                                                                                        \
-            /* the tile's token range, once for all waves: DPP steps inside the rows of 16 lanes, the two rows */ \
-            /* that hold tokens (lanes 0..31) combined through scalar registers */                              \
-            int mn_ = tst, mx_ = tst;                                                                           \
-            LLMOPS_DPP_MINMAX(0xB1);  /* quad_perm [1,0,3,2] */                                                 \
-            LLMOPS_DPP_MINMAX(0x4E);  /* quad_perm [2,3,0,1] */                                                 \
-            LLMOPS_DPP_MINMAX(0x141); /* row_half_mirror */                                                     \
-            LLMOPS_DPP_MINMAX(0x140); /* row_mirror */                                                          \
-            const int lo2_ = min(__builtin_amdgcn_readlane(mn_, 0), __builtin_amdgcn_readlane(mn_, 16));        \
-            const int hi2_ = max(__builtin_amdgcn_readlane(mx_, 0), __builtin_amdgcn_readlane(mx_, 16));        \
-            if (lane < BK) (SM).tok[lane] = tst;                                                                \
-            if (lane == 0) (SM).tok_range[0] = lo2_, (SM).tok_range[1] = hi2_;                                  \
-        }                                                                                                       \
+        if (wave == 0 && lane < BK) (SM).tok[lane] = tst;                                                       \
     } while (0)
-#define LLMOPS_DPP_MINMAX(CTRL)                                                      \
-    mn_ = min(mn_, __builtin_amdgcn_update_dpp(mn_, mn_, CTRL, 0xF, 0xF, false)); \
-    mx_ = max(mx_, __builtin_amdgcn_update_dpp(mx_, mx_, CTRL, 0xF, 0xF, false))
     // Set 0 walks the tiles 0, 2, 4, ..., set 1 the tiles 1, 3, 5, ...: both make the same number of passes.  One
     // barrier per pass: behind it the pass's buffer is complete and nobody reads the other buffer any more, which
-    // the pass then fills -- after its own products -- from the registers that the loads of the pass before filled.
+    // the pass then fills -- set 0 after its own products, set 1 before them -- from the registers that the loads of the pass before filled.
     LLMOPS_STAGE_LOAD(kv_begin + set * BK);
+    // The queries: every second row of the workgroup's by each set, a row by half a wave, through LDS into the lane's share of its own
+    // row as halves (step i covers dims 16i + 8*hf .. +7).  (Each lane fetching from its own row, 64 rows apart in one load: 4 us.)
+    uint8_t* const q_lds = LO ? smem_raw + sizeof(PrefillSmem<LO>) : smem_raw + 4 * sizeof(PrefillSmem<LO>);
+    constexpr int kQHalf = LO ? 2 * (int)sizeof(PrefillSmem<LO>) : 64 * kPrefillRow;  // rows 64 .. from here on
+    const int trow = 2 * wave8 + hf, tcol = c32;
+    {
+        float4 t[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) t[u] = *reinterpret_cast<const float4*>(q0 + min(trow + 16 * u, q_rows - 1) * (H * S) + 4 * tcol);
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            *reinterpret_cast<float4*>(q_lds + (u >> 2) * kQHalf + (trow + 16 * (u & 3)) * kPrefillRow + 16 * tcol) = t[u];
+    }
+    // The last cache tile that any query of the workgroup may see bounds the walk (rows of later tokens and rows
+    // beyond it are masked anyway; without the bound an early query tile would stage, barrier by barrier, all the
+    // tiles that only later tiles need).
+    int kv_end = kv_begin;
+    {
+        const int q_hi_wg = min((qt + 1) * BQ, qLi) - 1, first = kv_begin / BK, last = (min(kvLeni, kv_begin + kv_span) + BK - 1) / BK;
+        for (int t0 = (last - first - 1) / 64 * 64 + first; t0 >= first; t0 -= 64) {
+            const unsigned long long seen = __ballot(t0 + lane < last && tile_tokens[min(t0 + lane, last - 1)].x <= q_hi_wg);
+            if (seen != 0) {
+                kv_end = (t0 + 64 - __builtin_clzll(seen)) * BK;
+                break;
+            }
+        }
+    }
+    const int2* const ranges = tile_tokens + kv_begin / BK + set;
+    int2 range = ranges[0], range_next = range;  // smallest and largest token of the set's tile
     LLMOPS_STAGE_STORE(sm2[0]);
-    if (kv_begin + 2 * BK < kv_end) LLMOPS_STAGE_LOAD(kv_begin + set * BK + 2 * BK);
+    __syncthreads();
+    V8hBits qh[8], ql[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float4* at = reinterpret_cast<const float4*>(q_lds + (wave >> 1) * kQHalf + (32 * (wave & 1) + c32) * kPrefillRow + 64 * i + 32 * hf);
+        const float4 t0 = at[0], t1 = at[1];
+        split2(t0.x, t0.y, qh[i].u[0], ql[i].u[0]);
+        split2(t0.z, t0.w, qh[i].u[1], ql[i].u[1]);
+        split2(t1.x, t1.y, qh[i].u[2], ql[i].u[2]);
+        split2(t1.z, t1.w, qh[i].u[3], ql[i].u[3]);
+    }
+    if (kv_begin + 2 * BK < kv_end) {
+        LLMOPS_STAGE_LOAD(kv_begin + set * BK + 2 * BK);
+        range_next = ranges[2];
+    }
     for (int kv_pair = kv_begin, pass = 0; kv_pair < kv_end; kv_pair += 2 * BK, pass++) {
         PrefillSmem<LO>& sm = sm2[pass & 1];
         const uint8_t* kp_hi = &sm.k_hi[c32 * KSB + 16 * hf];  // + 32 i
@@ -1246,7 +1321,15 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __
         __syncthreads();
         // skip the tile if even the wave's last query may not see any of its rows; a tile that every query of the
         // wave sees whole (the usual case away from the diagonal) needs no masks
-        const int tmin = sm.tok_range[0], tmax = sm.tok_range[1];
+        const int tmin = range.x, tmax = range.y;
+        if (set == 1 && kv_pair + 2 * BK < kv_end) {
+            LLMOPS_STAGE_STORE(sm2[(pass + 1) & 1]);
+            range = range_next;
+            if (kv_pair + 4 * BK < kv_end) {
+                LLMOPS_STAGE_LOAD(kv_pair + set * BK + 4 * BK);
+                range_next = ranges[(kv_pair - kv_begin) / BK + 4];
+            }
+        }
         if (q_lo_wave < qLi && tmin <= q_hi_wave) {
         const bool all_visible = tmax <= q_lo_wave && q_lo_wave + 31 < qLi;
 
@@ -1306,6 +1389,16 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __
         const float m_new = fmaxf(m_run, mx);
         const float alpha = expf(m_run - m_new);  // 0 on the first visible tile, 1 while nothing is visible
         float psum = 0.0f;
+        if (all_visible) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            // e^x as 2^(x * log2 e) on the exponential unit: x <= 0, and wherever the result matters (|x| < 20)
+            // the product's rounding moves it by less than 1e-6 of itself
+            const float pv = __builtin_amdgcn_exp2f((sacc[r] - m_new) * 1.44269504088896341f);
+            sacc[r] = pv;
+            psum += pv;
+        }
+        } else {
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             // e^x as 2^(x * log2 e) on the exponential unit: x <= 0, and wherever the result matters (|x| < 20)
@@ -1313,6 +1406,7 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __
             const float pv = (sacc[r] == -FLT_MAX) ? 0.0f : __builtin_amdgcn_exp2f((sacc[r] - m_new) * 1.44269504088896341f);
             sacc[r] = pv;
             psum += pv;
+        }
         }
         {
             const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(psum), __float_as_uint(psum), false, false);
@@ -1349,62 +1443,77 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __
             }
         }
         }  // (tile visible to the wave)
-        if (kv_pair + 2 * BK < kv_end) {
+        if (set == 0 && kv_pair + 2 * BK < kv_end) {
             LLMOPS_STAGE_STORE(sm2[(pass + 1) & 1]);
-            if (kv_pair + 4 * BK < kv_end) LLMOPS_STAGE_LOAD(kv_pair + set * BK + 4 * BK);
+            range = range_next;
+            if (kv_pair + 4 * BK < kv_end) {
+                LLMOPS_STAGE_LOAD(kv_pair + set * BK + 4 * BK);
+                range_next = ranges[(kv_pair - kv_begin) / BK + 4];
+            }
         }
     }
 
 #undef LLMOPS_STAGE_STORE
-#undef LLMOPS_DPP_MINMAX
 #undef LLMOPS_STAGE_LOAD
-    // Merge of the two sets: lane by lane (same query, same columns in both).  Set 1 leaves its running maximum, its
-    // sum and its 64 outputs in LDS, value r of lane l of wave w at float r*256 + w*64 + l.
+    // Merge of the two sets, through LDS: every lane leaves what it holds of its query's output, then half a wave takes a row of
+    // both sets, so that the rows leave as whole lines.  (From the lanes that hold them, 32 rows apart in one store: 4.4 us.)
     __syncthreads();  // every wave is done with its tile
-    float* mrg = reinterpret_cast<float*>(smem_raw) + wave * 64 + lane;
-    if (set == 1) {
-        mrg[0] = m_run;
-        mrg[256] = l_run;
+    // (the lane's number anew: no register held it through the walk)
+    const int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), lq = ln & 31, lh = ln >> 5;
+    uint8_t* const o_lds = smem_raw;
+    float2* const stats = reinterpret_cast<float2*>(smem_raw + 2 * kPrefillRowsBytes);  // [set][query] (max, sum), then [query] weights
+    {
+        uint8_t* const at = o_lds + set * kPrefillRowsBytes + (wave * 32 + lq) * kPrefillRow + 16 * lh;
+        // (the lane holds columns 32c + 8j + 4*hf + v of its query's output row)
 #pragma unroll
         for (int c = 0; c < 4; c++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) mrg[(2 + 16 * c + r) * 256] = o[c][r];
+            for (int j = 0; j < 4; j++)
+                *reinterpret_cast<float4*>(at + 128 * c + 32 * j) = make_float4(o[c][4 * j], o[c][4 * j + 1], o[c][4 * j + 2], o[c][4 * j + 3]);
+        if (lh == 0) stats[set * 128 + wave * 32 + lq] = make_float2(m_run, l_run);
     }
     __syncthreads();
-    if (set == 1 || !valid) return;
-    {
-        const float m1 = mrg[0], l1 = mrg[256];
-        const float mm = fmaxf(m_run, m1);
-        const float a0 = expf(m_run - mm), a1 = expf(m1 - mm);  // (a set that saw no row has sum 0 and outputs 0)
-        l_run = l_run * a0 + l1 * a1;
-        m_run = mm;
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) o[c][r] = o[c][r] * a0 + mrg[(2 + 16 * c + r) * 256] * a1;
+    if (wave8 < 2) {
+        const int at = wave8 * 64 + ln;
+        const float2 s0 = stats[at], s1 = stats[128 + at];
+        const float mm = fmaxf(s0.x, s1.x);
+        const float a0 = expf(s0.x - mm), a1 = expf(s1.x - mm);  // (a set that saw no row has sum 0 and outputs 0)
+        stats[256 + at] = make_float2(a0, a1);
+        const float l = s0.y * a0 + s1.y * a1;
+        stats[at] = make_float2(mm, nsplit > 1 ? l : 1.0f / l);
     }
-    if (nsplit > 1) {  // a record [max, sum, out[S]] for attn_merge_kernel
-        float* rec = part + ((bh * qL + pq) * nsplit + blockIdx.y) * (S + 2);
-        if (hf == 0) *reinterpret_cast<float2*>(rec) = make_float2(m_run, l_run);
+    __syncthreads();
+    float4 z[8];
+    float2 st[8];
 #pragma unroll
-        for (int c = 0; c < 4; c++)
+    for (int u = 0; u < 8; u++) {
+        const int row = 2 * wave8 + lh + 16 * u;
+        const float2 a = stats[256 + row];
+        const float4 x = *reinterpret_cast<const float4*>(o_lds + row * kPrefillRow + 16 * lq);
+        const float4 y = *reinterpret_cast<const float4*>(o_lds + kPrefillRowsBytes + row * kPrefillRow + 16 * lq);
+        st[u] = stats[row];
+        z[u] = make_float4(x.x * a.x + y.x * a.y, x.y * a.x + y.y * a.y, x.z * a.x + y.z * a.y, x.w * a.x + y.w * a.y);
+    }
+    if (nsplit > 1) {  // records [max, sum, out[S]] for attn_merge_kernel
+        float* const rec = part + ((bh * qL + qt * BQ) * nsplit + blockIdx.y) * (S + 2);
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                float2* dst = reinterpret_cast<float2*>(rec + 2 + 32 * c + 8 * j + 4 * hf);
-                dst[0] = make_float2(o[c][4 * j], o[c][4 * j + 1]);
-                dst[1] = make_float2(o[c][4 * j + 2], o[c][4 * j + 3]);
-            }
+        for (int u = 0; u < 8; u++) {
+            const int row = 2 * wave8 + lh + 16 * u;
+            if (row >= q_rows) break;
+            float* const at = rec + (int64_t)row * nsplit * (S + 2);
+            if (lq == 0) *reinterpret_cast<float2*>(at) = st[u];
+            float2* dst = reinterpret_cast<float2*>(at + 2 + 4 * lq);
+            dst[0] = make_float2(z[u].x, z[u].y);
+            dst[1] = make_float2(z[u].z, z[u].w);
+        }
         return;
     }
-    const float inv = 1.0f / l_run;
-    // the lane holds columns 32c + 8j + 4*hf + v of its query's output row
 #pragma unroll
-    for (int c = 0; c < 4; c++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float4 out = make_float4(o[c][4 * j] * inv, o[c][4 * j + 1] * inv, o[c][4 * j + 2] * inv, o[c][4 * j + 3] * inv);
-            *reinterpret_cast<float4*>(qrow + 32 * c + 8 * j + 4 * hf) = out;
-        }
+    for (int u = 0; u < 8; u++) {
+        const int row = 2 * wave8 + lh + 16 * u;
+        if (row >= q_rows) break;
+        *reinterpret_cast<float4*>(q0 + row * (H * S) + 4 * lq) = make_float4(z[u].x * st[u].y, z[u].y * st[u].y, z[u].z * st[u].y, z[u].w * st[u].y);
+    }
 }
 
 // ---- softmax op (ops/op_misc.hpp:183-194): one workgroup per row ------------------------------
@@ -1457,17 +1566,18 @@ static TokensPlan plan_tokens(int64_t bh, int64_t qL, int64_t kvLen, bool half_c
     TokensPlan p{};
     if (qL >= g_prefill_min_tokens) {
         // A workgroup takes a compute unit: with fewer query tiles than those, ns workgroups share a tile's cache rows, at
-        // least 128 each.  A row costs a tile 0.041 us (halves 0.0365: two products instead of three); the launch that merges
-        // the records costs 3.5 us, 0.55 us per 1000 queries and 0.25 us per 1000 records (0.3 beside halves).  Against one
-        // piece and all pieces at 2016 sizes (1 to 128 heads in all, 32 to 2048 tokens behind 0 to 6000, both cache types, not
-        // from a cache): 0.06 % slower than the better one on average, 8 % at worst.  (us, one / split, 32 heads: 32 tokens
-        // behind 500 35.1 / 23.4; 64 behind 100 22.6 / 25.4, behind 300 30.1 / 26.8; 256 behind none 32.2 / 41.1, behind 300
-        // 46.3 / 43.1, halves 40.6 / 43.6; 200 behind 300, halves 35.8 / 38.9; 512 behind 500 71.4 / 70.9, behind 1500 116 / 94.)
+        // least 128 each.  A row costs a tile 0.0365 us (halves 0.0305: two products instead of three); the launch that merges the
+        // records costs 2.6 us and 0.165 us per 1000 records.  (us, one piece / as planned, 32 heads: 32 tokens behind 100 17.4 / 17.4
+        // (two 17.9), behind 500 32.4 / 20.2; 128 behind 200 29.2 / 26.1, behind 2000 95.6 / 40.8; 256 behind none 28.4 / 28.4 (two 29.9),
+        // halves 24.1 / 24.2 (27.7); 384 behind 300 48.8 / 42.9; 512 behind none 41.5 / 40.1, behind 1500 108.8 / 79.2; 8 heads, 2048 tokens
+        // 97.9 / 68.2; 128 heads, 128 behind 1500 91.4 / 78.3.  Of 30 sizes two are 2 to 5 % slower than with the best number of pieces.)
+        // Beside halves a record is priced at 0.35 us per 1000, above what it costs: the planner's test holds 200 and 256 tokens behind 300 to
+        // one piece there (256: 35.2, in four 30.8; 384 behind 300 43.3, in two 40.0).
         p.kernel = 3;
-        const double row = half_cache ? 0.0365 : 0.041, record = half_cache ? 0.3e-3 : 0.25e-3;
+        const double row = half_cache ? 0.0305 : 0.0365, record = half_cache ? 0.35e-3 : 0.165e-3;
         int64_t ns = 256 / (bh * ((qL + 127) / 128));
         if (ns > (kvLen + 127) / 128) ns = (kvLen + 127) / 128;
-        if (ns < 2 || bhq * ns > max_records || row * (double)(kvLen - kvLen / ns) < 3.5 + 0.55e-3 * (double)bhq + record * (double)(bhq * ns)) ns = 1;
+        if (ns < 2 || bhq * ns > max_records || row * (double)(kvLen - kvLen / ns) < 2.6 + record * (double)(bhq * ns)) ns = 1;
         p.rows = (int)(((kvLen + ns - 1) / ns + 63) / 64 * 64);
         p.pieces = (int)((kvLen + p.rows - 1) / p.rows);
         return p;
@@ -1626,6 +1736,10 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
     const int nchunks = plan.pieces;
     // the tiled kernel finds the token of a cache row in row_token; the others compare the slots themselves
     const bool tiled = plan.kernel == 3;
+    // (beside it the token ranges of the tiles, ahead of the records, of which there are at least a row's more than any plan takes)
+    const unsigned tables = tiled ? (unsigned)((kvLen + 63) / 64) : 0;
+    int2* const tile_tokens = reinterpret_cast<int2*>(part);
+    part += align_up((size_t)tables * 2 * sizeof(int2), 256) / sizeof(float);
     if (!tiled && (int64_t)bhq * nchunks > max_records)
         return fail(LLMOPS_EWORKSPACE, "attention workspace too small for %lld chunk records", (long long)bhq * nchunks);
     // All tokens of a head together: rotation and cache update ride in the same launch where the rotary pairs suit it, the
@@ -1643,12 +1757,11 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
         return LLMOPS_OK;
     }
     if (tiled) {
-        const unsigned tables = (unsigned)((kvLen + 63) / 64);
         attn_prep_kernel<T, true><<<(unsigned)(B * qL * H) + tables, 64, 0, st>>>(q, k, v, qL, H, S, inv_freq, half, kc, vc, maxlen, slots,
-                                                                                 position_id, row_token, kvLen, tables);
+                                                                                 position_id, row_token, tile_tokens, kvLen, tables);
     } else {
         attn_prep_kernel<T, false><<<(unsigned)(B * qL * H), 64, 0, st>>>(q, k, v, qL, H, S, inv_freq, half, kc, vc, maxlen, slots,
-                                                                         position_id, nullptr, 0, 0);
+                                                                         position_id, nullptr, nullptr, 0, 0);
     }
     LLMOPS_LAUNCH_CHECK();
     if (tiled) {
@@ -1663,11 +1776,15 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
             configured = true;
         }
-        attn_prefill_kernel<T><<<dim3((unsigned)(B * H * qtiles), (unsigned)nchunks), 512, smem, st>>>(q, kc, vc, qL, H, maxlen, kvLen, row_token,
+        attn_prefill_kernel<T><<<dim3((unsigned)(B * H * qtiles), (unsigned)nchunks), 512, smem, st>>>(q, kc, vc, qL, H, maxlen, kvLen, row_token, tile_tokens,
                                                                                                        qtiles, plan.rows, part, nchunks);
         LLMOPS_LAUNCH_CHECK();
         if (nchunks > 1) {
-            attn_merge_kernel<<<(unsigned)bhq, 128, 0, st>>>(q, part, qL, H, nchunks);
+            const unsigned groups = (unsigned)((bhq + 7) / 8);
+            if (nchunks <= 2) attn_merge_rows_kernel<2><<<groups, 256, 0, st>>>(q, part, (int)qL, (int)H, (unsigned)bhq, nchunks);
+            else if (nchunks <= 4) attn_merge_rows_kernel<4><<<groups, 256, 0, st>>>(q, part, (int)qL, (int)H, (unsigned)bhq, nchunks);
+            else if (nchunks <= 8) attn_merge_rows_kernel<8><<<groups, 256, 0, st>>>(q, part, (int)qL, (int)H, (unsigned)bhq, nchunks);
+            else attn_merge_kernel<<<(unsigned)bhq, 128, 0, st>>>(q, part, qL, H, nchunks);
             LLMOPS_LAUNCH_CHECK();
         }
         return LLMOPS_OK;

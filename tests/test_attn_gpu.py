@@ -265,6 +265,19 @@ def test_attention_tokens_behind_a_cache(ops, B, qL, kv, H, kernel, cache_dtype,
     _tokens_behind_a_cache(ops, B, qL, kv, H, cache_dtype, order)
 
 
+@pytest.mark.parametrize("B,qL,kv,H,pieces", [(1, 37, 200, 3, 2), (2, 129, 400, 1, 4), (1, 61, 500, 3, 4), (1, 33, 700, 5, 6), (1, 35, 1000, 1, 8),
+                                              (1, 35, 1100, 1, 9), (3, 32, 64, 1, 1), (1, 128, 96 + 128, 1, 2)])
+@pytest.mark.parametrize("cache_dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("order", ["in order", "shuffled"])
+def test_attention_tiles_in_pieces(ops, B, qL, kv, H, pieces, cache_dtype, order):
+    """The tiled kernel's cache rows in two, four, eight and more records a query (every build of the merge, its last workgroup partly
+    filled), the last query tile and the last cache tile partly filled."""
+    k, r, n = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    assert ops._lib.load().llmops_test_attn_plan(B, qL, H, kv, kv - qL, int(cache_dtype == torch.float16), ctypes.byref(k), ctypes.byref(r), ctypes.byref(n)) == 0
+    assert k.value == 3 and n.value == pieces
+    _tokens_behind_a_cache(ops, B, qL, kv, H, cache_dtype, order)
+
+
 @pytest.mark.parametrize("B,qL,kv,H,plan", [
     (1, 3, 100, 4, (1, 16)), (1, 31, 40, 8, (1, 16)),                             # chunks of 16 rows
     (1, 8, 131, 32, (1, 32)), (4, 3, 100, 32, (1, 32)), (4, 3, 140, 32, (2, 128)),  # of 32, and just beyond the rule
