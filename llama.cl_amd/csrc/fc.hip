@@ -84,23 +84,24 @@ extern "C" size_t llmops_fc_Q4A_workspace_bytes(int64_t rows, int64_t K, int64_t
 // decode_quantizes_first 4 / 3
 static int g_rows_from_small = 0, g_rows_from_large = 0;
 
-// .. in fc_Q4A.  The first kernel's work per weight byte grows with the row count (every row is quantized and dotted separately), the
-// second's time hardly depends on it, separate quantization launch included, which is what it needs up to 8 rows.
-// us, weights from memory, first / second, at rows either side of the line:
-//   4096x4096 (128 strips): 2 rows 5.8 / 6.8, 3 7.4 / 6.9, 8 9.7 / 7.0; 512x4096: 2 5.2 / 5.9, 3 6.8 / 6.0, 8 9.1 / 6.0
-//   4096x11008:             2 rows 8.7 / 10.8, 3 10.7 / 10.9 (from a cache 12.2 / 10.9), 4 12.4 / 10.4, 8 19.6 / 10.6
+// .. in fc_Q4A.  The first kernel's work per weight byte grows with the row count (every row is quantized and dotted separately); the
+// second's time hardly depends on it up to 16 rows, but it has a launch more, and a program that issues call by call needs 8.4 us for two
+// launches, 5.2 for one: below that only a captured graph would have what the second saves.  us in a graph, weights from memory, first / second:
+//   4096x4096 (128 strips): 2 rows 5.8 / 6.8, 3 7.4 / 6.9 (call by call 6.9 / 8.6), 4 8.0 / 7.0, 8 9.7 / 7.0
 //   6000x4096 (188), 8192x4096 (256): 3 rows 7.5 / 7.7 and 8.2 / 8.2, 4 8.5 / 7.8 and 9.1 / 8.2
 //   11008x4096, 12288x4096: 2 rows 9.1 / 11.4 and 9.3 / 11.5, 3 13.1 / 10.5 and 13.7 / 11.4
-//   1500x2048, 2048x2048:   3 rows 5.1 / 5.5, 4 5.7 / 5.5; 1024x512 .. 4096x512, 1024x1024: 4 4.2 / 5.0, 5 5.2 / 5.0
-//   8192x1024:              5 rows 5.5 / 5.7, 6 5.8 / 5.8, 8 6.5 / 5.8
-//   Under 16 strips the first kernel stays up to 8 rows, though it is the slower one from 3 on (352x2048: 4 rows 5.4 / 5.3, 8 8.4 / 5.3):
-//   the bits of its dump build are those of fc_Q4A there.
+//   4096x11008:             2 rows 8.7 / 10.8, 3 10.7 / 10.9 (from a cache 12.2 / 10.9), 4 12.4 / 10.4, 8 19.6 / 10.6; 2500x11008: 3 14.9 / 9.7
+//   1500x2048, 2048x2048:   4 rows 5.7 / 5.5, 8 8.3 / 5.5
+//   1024x512 .. 4096x1024:  4 rows 4.2 / 5.0, 8 6.3 / 5.3 (call by call 6.3 / 8.6)
+//   512x4096 (16):          3 rows 6.8 / 6.0, 6 8.3 / 6.0 (call by call 8.3 / 8.4), 8 9.1 / 6.0; 600x11008: 3 8.6 / 7.7, 4 9.2 / 7.7, 8 12.4 / 7.8
+//   Under 16 strips the first kernel stays up to 8 rows: the bits of its dump build are those of fc_Q4A there.
 static int rows_from(int64_t Ng, int64_t Kg) {
     const int forced = Ng > 256 ? g_rows_from_large : g_rows_from_small;
     if (forced > 0) return forced;
-    if (Ng < 16) return kMaxGemvRows + 1;
-    if (Kg < 12) return 5;
-    return Kg >= 32 && (Ng <= 128 || Ng > 256) ? 3 : 4;
+    if (Ng < 16 || Kg < 12) return kMaxGemvRows + 1;
+    if (Ng < 64) return Kg < 24 ? kMaxGemvRows + 1 : Kg < 64 ? 6 : 4;
+    if (Ng > 256 || Kg >= 64) return 3;
+    return Kg < 24 ? 5 : 4;
 }
 
 // argument checks of fc_Q4A that do not involve the workspace

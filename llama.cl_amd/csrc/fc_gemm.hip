@@ -516,21 +516,27 @@ bool gemm_tile_forced() { return g_gemm_rt != 0 || g_gemm_force_split > 0; }
 // 1500 x 2048: the choices are 1.4 % slower than the best measured one on average and 8 % at worst (11008 x 4096 at 64 rows: 5 splits,
 // 4 would be better), against 5 % and 65 % (1500 x 2048 at 384 rows) of the rule that counted whole rounds.
 // room: what partial sums may take (bytes).
-static double plan_gemm_tile(int64_t rows, int64_t Ng, int64_t Kg, int64_t room, GemmPlan& p) {
+template <typename I>
+static double plan_gemm_tile_in(I rows, I Ng, I Kg, int64_t room, GemmPlan& p) {
     static const int kRT[3] = {4, 2, 1}, kSlots[3] = {512, 768, 1024};
     static const double kGroupUs[3] = {1.2, 0.947, 0.811}, kPartRound[3] = {1.0, 0.541, 0.852};
     double best = 0.0;
+    const double part_us = 0.42e-6 * (double)rows * (double)(Ng * kGroupN);
     for (int i = 0; i < 3; i++) {
         if (g_gemm_rt > 0 && kRT[i] != g_gemm_rt) continue;
-        const int64_t bm = 32 * kRT[i], tiles = ((Ng + 3) / 4) * ((rows + bm - 1) / bm);
-        for (int64_t s = 1; s <= 12; s++) {
-            const int64_t want = g_gemm_force_split > 0 ? g_gemm_force_split : s;
-            const int64_t per = want >= Kg ? 1 : (Kg + want - 1) / want, S = (Kg + per - 1) / per;
-            if (S > 1 && g_gemm_force_split <= 0 && S * rows * Ng * kGroupN * 4 > room) continue;
-            const int64_t full = tiles * S / kSlots[i], rest = tiles * S % kSlots[i];
+        const I bm = 32 * kRT[i], tiles = ((Ng + 3) / 4) * ((rows + bm - 1) / bm), slots = kSlots[i];
+        I last = 0;
+        for (I s = 1; s <= 12; s++) {
+            const I want = g_gemm_force_split > 0 ? (I)g_gemm_force_split : s;
+            const I per = want >= Kg ? 1 : (Kg + want - 1) / want;
+            if (per == last) continue;
+            last = per;
+            const I S = (Kg + per - 1) / per;
+            if (S > 1 && g_gemm_force_split <= 0 && (int64_t)S * (int64_t)rows * (int64_t)Ng * kGroupN * 4 > room) continue;
+            const I full = tiles * S / slots, rest = tiles * S - full * slots;
             const double rounds = (double)full + (rest == 0 ? 0.0 : kPartRound[i] + (1.0 - kPartRound[i]) * (double)rest / kSlots[i]);
             double t = kGroupUs[i] * ((double)per + 0.289) * rounds;
-            if (S > 1) t += 1.726 + 0.319 * (double)(S * kRT[i]) + 0.42e-6 * (double)(S * rows * Ng * kGroupN);
+            if (S > 1) t += 1.726 + 0.319 * (double)(S * kRT[i]) + (double)S * part_us;
             if (best == 0.0 || t < best) {
                 best = t;
                 p.RT = kRT[i], p.S = (int)S, p.kb_per_split = (int)per;
@@ -538,6 +544,24 @@ static double plan_gemm_tile(int64_t rows, int64_t Ng, int64_t Kg, int64_t room,
         }
     }
     return best;
+}
+
+static double plan_gemm_tile(int64_t rows, int64_t Ng, int64_t Kg, int64_t room, GemmPlan& p) {
+    // (a call plans up to three times, and programs repeat their sizes: the last plan of the thread; 0.2 us each)
+    static thread_local struct {
+        int64_t rows = 0, Ng = 0, Kg = 0, room = 0;
+        int rt = 0, split = 0;
+        GemmPlan plan{};
+        double us = 0.0;
+    } last;
+    if (last.rows != rows || last.Ng != Ng || last.Kg != Kg || last.room != room || last.rt != g_gemm_rt || last.split != g_gemm_force_split) {
+        last.us = rows * Ng < ((int64_t)1 << 31) && Kg < ((int64_t)1 << 24)
+                      ? plan_gemm_tile_in<unsigned>((unsigned)rows, (unsigned)Ng, (unsigned)Kg, room, last.plan)
+                      : plan_gemm_tile_in<int64_t>(rows, Ng, Kg, room, last.plan);
+        last.rows = rows, last.Ng = Ng, last.Kg = Kg, last.room = room, last.rt = g_gemm_rt, last.split = g_gemm_force_split;
+    }
+    p.RT = last.plan.RT, p.S = last.plan.S, p.kb_per_split = last.plan.kb_per_split;
+    return last.us;
 }
 
 // estimated time of the tiled kernel (group 128), us

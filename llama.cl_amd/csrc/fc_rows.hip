@@ -264,27 +264,36 @@ static StreamPlan plan_stream(int64_t rows, int64_t Ng, int64_t Kg, size_t slot_
         return best;
     }
     const bool may_split = g_rows_split && Kg >= 2 && (size_t)rows * Ng * kGroupN * 8 <= slot_bytes;
-    const int strips = (int)Ng, groups = (int)Kg, n_rows = (int)rows;
-    for (int RT = 1; RT <= 4 && 16 * (RT - 1) < n_rows; RT++) {
-        const int blocks = (n_rows + 16 * RT - 1) / (16 * RT);
-        for (int SW = 1; SW <= 2; SW++)
-            for (int NW = 4; NW <= 8; NW += 4)
+    // (a call plans more than once, and programs repeat their sizes: the last plan of the thread; 0.3 us each)
+    static thread_local struct {
+        int64_t rows = 0, Ng = 0, Kg = 0;
+        bool may_split = false;
+        StreamPlan plan{};
+    } last;
+    if (last.rows == rows && last.Ng == Ng && last.Kg == Kg && last.may_split == may_split) return last.plan;
+    const unsigned strips = (unsigned)Ng, groups = (unsigned)Kg, n_rows = (unsigned)rows;  // (Ng <= kTicketBytes / 4, rows <= 2^25 here)
+    const double stored = 0.103e-6 * (double)(Ng * Kg * kRowsBlk), exchange = 0.615 + 4.9e-6 * (double)(rows * Ng * kGroupN);
+    for (int RT = 1; RT <= 4 && 16u * (RT - 1) < n_rows; RT++) {
+        const unsigned blocks = (n_rows + 16 * RT - 1) / (16 * RT);
+        for (int SW = 1; SW <= 2; SW++) {
+            // (as many for every XCD: the strips go round them)
+            const unsigned units = ((strips + SW - 1) / SW + 7) / 8 * 8 * blocks;
+            const double step = 0.103 + 0.038 * RT * SW, wave = 0.25 * (0.114 * SW + 0.0733 * RT), write = 0.347 * RT * SW;
+            for (int NW = 4; NW <= 8; NW += 4) {
+                const unsigned place = kPlace[RT - 1][SW - 1][NW / 8];
                 for (int split = 0; split <= (may_split ? 1 : 0); split++) {
-                    // (as many for every XCD: the strips go round them)
-                    const int64_t wgs = (int64_t)(((strips + SW - 1) / SW + 7) / 8 * 8) * blocks * (split + 1);
-                    const int run = (((groups + split) >> split) + NW - 1) / NW, place = kPlace[RT - 1][SW - 1][NW / 8];
-                    const auto round = [&](int64_t n) {
-                        return 0.565 + run * (0.103 + 0.038 * RT * SW + (double)(n * NW) / 4.0 * (0.114 * SW + 0.0733 * RT)) +
-                               0.347 * (double)(RT * SW * n);
-                    };
-                    const int64_t full = wgs / (256 * place), rest = wgs - full * 256 * place;
-                    double us = (double)full * round(place) + (rest ? round((rest + 255) / 256) : 0.0);
-                    if (split) us += 0.615 + 4.9e-6 * (double)(rows * Ng * kGroupN);
+                    const unsigned wgs = units << split, run = (((groups + split) >> split) + NW - 1) / NW;
+                    const auto round = [&](unsigned n) { return 0.565 + run * (step + (double)(n * NW) * wave) + write * (double)n; };
+                    const unsigned full = wgs / (256 * place), rest = wgs - full * 256 * place;
+                    double us = (full ? (double)full * round(place) : 0.0) + (rest ? round((rest + 255) / 256) : 0.0) + stored;
+                    if (split) us += exchange;
                     if (place == 1 && full > 0) us += 1.41 * (double)(rest ? full : full - 1);
-                    us += 0.103e-6 * (double)(Ng * Kg * kRowsBlk);
                     if (best.RT == 0 || us < best.us) best = StreamPlan{RT, SW, NW, split != 0, us};
                 }
+            }
+        }
     }
+    last.rows = rows, last.Ng = Ng, last.Kg = Kg, last.may_split = may_split, last.plan = best;
     return best;
 }
 
