@@ -5,7 +5,8 @@
 //   1. attn_prep_kernel   rotate q and k in place (rope_embed, ops/op_attn.hpp:44-94), write the
 //                         rotated k and the v rows into the cache at slots[p] (:764-773), and
 //                         from 32 tokens on record which cache rows were written by which token of this call
-//                         (attn_few_kernel does the first two itself where that saves time).
+//                         (attn_few_kernel does the first two itself where that saves time).  From 32 tokens on, all dimensions
+//                         rotating, attn_prep_rows_kernel: the same without q, which attn_prefill_kernel rotates.
 //   2. below 32 tokens    attn_split_kernel or attn_few_kernel: a workgroup takes a chunk of cache rows and leaves
 //                         per query the chunk's score maximum, its sum of exponentials and its weighted V sum.
 //      from 32 on         attn_prefill_kernel: 128 queries to a workgroup, the cache rows in one piece or in several.
@@ -28,13 +29,21 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 
 // ---- rope ------------------------------------------------------------------------------------
 // theta = inv_freq[i] * (float)pos, cosf/sinf in fp32 (CosSin_cache::update, ops/op_attn.hpp:25-32)
-__device__ __forceinline__ void rope_pair(float& x0, float& x1, float inv_freq, int pos) {
-    const float xita = inv_freq * (float)pos;
-    const float c = cosf(xita), s = sinf(xita);
+__device__ __forceinline__ void rotate_pair(float& x0, float& x1, float c, float s) {
     const float y0 = c * x0 - s * x1;
     const float y1 = s * x0 + c * x1;
     x0 = y0;
     x1 = y1;
+}
+__device__ __forceinline__ void rotate4(float4& a, float4& b, float4 c, float4 s) {
+    rotate_pair(a.x, b.x, c.x, s.x);
+    rotate_pair(a.y, b.y, c.y, s.y);
+    rotate_pair(a.z, b.z, c.z, s.z);
+    rotate_pair(a.w, b.w, c.w, s.w);
+}
+__device__ __forceinline__ void rope_pair(float& x0, float& x1, float inv_freq, int pos) {
+    const float xita = inv_freq * (float)pos;
+    rotate_pair(x0, x1, cosf(xita), sinf(xita));
 }
 
 // x [B,H,L,S] in place; one thread per rotated pair
@@ -61,6 +70,26 @@ __device__ __forceinline__ void store_cache<__half>(__half* dst, float v) {
     *dst = __float2half_rn(v);
 }
 
+// A workgroup's 64 entries of row_token (64 rows from 64 blockIdx.x on) and the two token ranges that go with them
+__device__ __forceinline__ void fill_row_tokens(int32_t* token, int64_t qL, const int32_t* __restrict__ slots, int32_t* __restrict__ row_token,
+                                                int2* __restrict__ tile_tokens, int64_t kvLen) {
+    const int64_t row0 = (int64_t)blockIdx.x * 64;
+    if (threadIdx.x < 64) token[threadIdx.x] = -1;
+    __syncthreads();
+    for (int64_t l = threadIdx.x; l < qL; l += blockDim.x) {
+        const int64_t at = (int64_t)slots[l] - row0;
+        if (at >= 0 && at < 64) atomicMax(&token[at], (int32_t)l);
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int32_t mine = row0 + threadIdx.x < kvLen ? token[threadIdx.x] : INT_MAX;
+    row_token[row0 + threadIdx.x] = mine;
+    int lo = mine, hi = mine;
+#pragma unroll
+    for (int off = 1; off < 32; off <<= 1) lo = min(lo, __shfl_xor(lo, off, 64)), hi = max(hi, __shfl_xor(hi, off, 64));
+    if ((threadIdx.x & 31) == 0) tile_tokens[row0 / 32 + threadIdx.x / 32] = make_int2(lo, hi);
+}
+
 // q,k,v [B,qL,H,S].  One workgroup of a wave per (b, l, h); thread i handles element i (and i+half).  TABLES: before those, `tables`
 // workgroups each write 64 entries of row_token: the (last) token of this call that a cache row belongs to, -1, or from kvLen on
 // INT_MAX, and the smallest and largest token of each 32 rows.  (us for the
@@ -73,20 +102,7 @@ __global__ void attn_prep_kernel(float* __restrict__ q, float* __restrict__ k, c
                                  int position_id, int32_t* __restrict__ row_token, int2* __restrict__ tile_tokens, int64_t kvLen, unsigned tables) {
     if (TABLES && blockIdx.x < tables) {
         __shared__ int32_t token[64];
-        const int64_t row0 = (int64_t)blockIdx.x * 64;
-        token[threadIdx.x] = -1;
-        __syncthreads();
-        for (int64_t l = threadIdx.x; l < qL; l += 64) {
-            const int64_t at = (int64_t)slots[l] - row0;
-            if (at >= 0 && at < 64) atomicMax(&token[at], (int32_t)l);
-        }
-        __syncthreads();
-        const int32_t mine = row0 + threadIdx.x < kvLen ? token[threadIdx.x] : INT_MAX;
-        row_token[row0 + threadIdx.x] = mine;
-        int lo = mine, hi = mine;
-#pragma unroll
-        for (int off = 1; off < 32; off <<= 1) lo = min(lo, __shfl_xor(lo, off, 64)), hi = max(hi, __shfl_xor(hi, off, 64));
-        if ((threadIdx.x & 31) == 0) tile_tokens[row0 / 32 + threadIdx.x / 32] = make_int2(lo, hi);
+        fill_row_tokens(token, qL, slots, row_token, tile_tokens, kvLen);
         return;
     }
     const int64_t item = TABLES ? blockIdx.x - tables : blockIdx.x;
@@ -158,6 +174,57 @@ __device__ __forceinline__ void store4<__half>(__half* dst, float4 v) {
     u.x = *reinterpret_cast<const uint32_t*>(&a);
     u.y = *reinterpret_cast<const uint32_t*>(&b);
     *reinterpret_cast<uint2*>(dst) = u;
+}
+
+// The same ahead of attn_prefill_kernel where all 128 dimensions rotate (half 64): q stays as it is and is rotated by that kernel's
+// workgroups on its way to their LDS; they take the cosines and sines from `turns` ([qL][cos 64, sin 64]).  Bound by memory, and q is 2/7 of
+// what the kernel above moves.  A wave computes its token's 64 angles once, a lane each, for eight heads, 16 bytes to a lane.
+// (The case of a whole call as a program makes it, q and k put back before it, us, both launches by the kernel above / so, the same bits: 32
+// heads, 2048 tokens 185 / 174, 384 tokens halves 35.1 / 31.4, 128 behind 2000 37.9 / 35.5, 32 tokens 13.9 / 13.8; batches of 2 x 1000 137 / 124,
+// 4 x 40 behind 100 halves 21.7 / 19.6, 8 x 200 behind 50 99 / 88.)
+template <typename T>
+__global__ __launch_bounds__(256) void attn_prep_rows_kernel(float* __restrict__ k, const float* __restrict__ v, int qL, int H, const float* __restrict__ inv_freq,
+                                                             T* __restrict__ kc, T* __restrict__ vc, int64_t maxlen, const int32_t* __restrict__ slots,
+                                                             int position_id, int32_t* __restrict__ row_token, int2* __restrict__ tile_tokens, int64_t kvLen,
+                                                             unsigned tables, unsigned head_groups, float* __restrict__ turns) {
+    constexpr int S = 128, kHeads = 32;
+    __shared__ __align__(16) float turn[4][S];
+    if (blockIdx.x < tables) {
+        fill_row_tokens(reinterpret_cast<int32_t*>(turn), qL, slots, row_token, tile_tokens, kvLen);
+        return;
+    }
+    const unsigned item = blockIdx.x - tables, bl = item / head_groups, group = item - bl * head_groups, b = bl / (unsigned)qL, l = bl - b * (unsigned)qL;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c4 = 4 * (threadIdx.x & 15);
+    const int slot = slots[l];
+    const bool slot_ok = slot >= 0 && slot < maxlen;  // (as above)
+    float4 kl[2], kh[2], vl[2], vh[2];
+    const size_t base = ((size_t)bl * H) * S + c4;
+    int head[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        head[u] = (int)(group * kHeads) + 16 * u + (threadIdx.x >> 4);
+        const size_t at = base + (size_t)min(head[u], H - 1) * S;  // (heads past the last re-read that one and store nothing)
+        kl[u] = load4(k + at), kh[u] = load4(k + at + S / 2);
+        vl[u] = load4(v + at), vh[u] = load4(v + at + S / 2);
+    }
+    const float xita = inv_freq[lane] * (float)((int)l + position_id);
+    const float cs = cosf(xita), sn = sinf(xita);
+    turn[wave][lane] = cs, turn[wave][S / 2 + lane] = sn;
+    if (b == 0 && group == 0 && wave == 0) turns[(size_t)l * S + lane] = cs, turns[(size_t)l * S + S / 2 + lane] = sn;
+    __syncthreads();
+    const float4 c = load4(&turn[wave][c4]), s = load4(&turn[wave][S / 2 + c4]);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        if (head[u] >= H) continue;
+        const size_t at = base + (size_t)head[u] * S;
+        rotate4(kl[u], kh[u], c, s);
+        store4(k + at, kl[u]), store4(k + at + S / 2, kh[u]);
+        if (slot_ok) {
+            const size_t row = (((size_t)b * H + head[u]) * maxlen + slot) * S + c4;
+            store4(kc + row, kl[u]), store4(kc + row + S / 2, kh[u]);
+            store4(vc + row, vl[u]), store4(vc + row + S / 2, vh[u]);
+        }
+    }
 }
 
 // ---- split-KV attention of few query tokens over a short cache ----
@@ -1180,7 +1247,7 @@ template <typename T>
 __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __restrict__ kc, const T* __restrict__ vc,
                                                           int64_t qL, int64_t H, int64_t maxlen, int64_t kvLen,
                                                           const int32_t* __restrict__ row_token, const int2* __restrict__ tile_tokens, int qtiles, int kv_span,
-                                                          float* __restrict__ part, int nsplit) {
+                                                          float* __restrict__ part, int nsplit, const float* __restrict__ turns) {
     constexpr bool LO = sizeof(T) == 4;  // an fp16 cache holds no low halves
     constexpr int S = 128, BQ = 128, BK = 32, KSB = 272, VSB = 80;
     extern __shared__ __align__(16) uint8_t smem_raw[];
@@ -1266,18 +1333,35 @@ __global__ __launch_bounds__(512) void attn_prefill_kernel(float* q, const T* __
     // barrier per pass: behind it the pass's buffer is complete and nobody reads the other buffer any more, which
     // the pass then fills -- set 0 after its own products, set 1 before them -- from the registers that the loads of the pass before filled.
     LLMOPS_STAGE_LOAD(kv_begin + set * BK);
-    // The queries: every second row of the workgroup's by each set, a row by half a wave, through LDS into the lane's share of its own
+    // The queries, a row by sixteen lanes that hold the two halves of its rotary pairs, through LDS into the lane's share of its own
     // row as halves (step i covers dims 16i + 8*hf .. +7).  (Each lane fetching from its own row, 64 rows apart in one load: 4 us.)
     uint8_t* const q_lds = LO ? smem_raw + sizeof(PrefillSmem<LO>) : smem_raw + 4 * sizeof(PrefillSmem<LO>);
     constexpr int kQHalf = LO ? 2 * (int)sizeof(PrefillSmem<LO>) : 64 * kPrefillRow;  // rows 64 .. from here on
-    const int trow = 2 * wave8 + hf, tcol = c32;
     {
+        const int qrow = threadIdx.x >> 4, qcol = 4 * (threadIdx.x & 15);  // rows qrow + 32u, columns qcol .. and 64 + qcol ..
         float4 t[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) t[u] = *reinterpret_cast<const float4*>(q0 + min(trow + 16 * u, q_rows - 1) * (H * S) + 4 * tcol);
+        for (int u = 0; u < 4; u++) {
+            const float* at = q0 + min(qrow + 32 * u, q_rows - 1) * (H * S) + qcol;
+            t[2 * u] = load4(at), t[2 * u + 1] = load4(at + 64);
+        }
+        if (turns != nullptr) {  // (q as the caller left it: see attn_prep_rows_kernel)
+            const float* const turns0 = turns + (int64_t)qt * (BQ * S) + qcol;
+            float4 c[4], s[4];
 #pragma unroll
-        for (int u = 0; u < 8; u++)
-            *reinterpret_cast<float4*>(q_lds + (u >> 2) * kQHalf + (trow + 16 * (u & 3)) * kPrefillRow + 16 * tcol) = t[u];
+            for (int u = 0; u < 4; u++) {
+                const float* at = turns0 + min(qrow + 32 * u, q_rows - 1) * S;
+                c[u] = load4(at), s[u] = load4(at + 64);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) rotate4(t[2 * u], t[2 * u + 1], c[u], s[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            uint8_t* at = q_lds + (u >> 1) * kQHalf + (qrow + 32 * (u & 1)) * kPrefillRow + 4 * qcol;
+            *reinterpret_cast<float4*>(at) = t[2 * u];
+            *reinterpret_cast<float4*>(at + 256) = t[2 * u + 1];
+        }
     }
     // The last cache tile that any query of the workgroup may see bounds the walk (rows of later tokens and rows
     // beyond it are masked anyway; without the bound an early query tile would stage, barrier by barrier, all the
@@ -1739,7 +1823,14 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
     // (beside it the token ranges of the tiles, ahead of the records, of which there are at least a row's more than any plan takes)
     const unsigned tables = tiled ? (unsigned)((kvLen + 63) / 64) : 0;
     int2* const tile_tokens = reinterpret_cast<int2*>(part);
-    part += align_up((size_t)tables * 2 * sizeof(int2), 256) / sizeof(float);
+    const size_t tile_bytes = align_up((size_t)tables * 2 * sizeof(int2), 256), turn_bytes = (size_t)qL * S * sizeof(float);
+    part += tile_bytes / sizeof(float);
+    // q is rotated by the tiled kernel where all dimensions rotate and the angles' table fits ahead of the records (a record's place per
+    // query and head is free: it does in any workspace of the size asked for)
+    float* const turns = part;
+    const bool late_q = tiled && half == 64 && B * qL * ((H + 31) / 32) < ((int64_t)1 << 30) && H < ((int64_t)1 << 31) &&
+                        tile_bytes + turn_bytes + (nchunks > 1 ? (size_t)bhq * nchunks * (S + 2) * sizeof(float) : 0) <= workspace_bytes - part_off;
+    if (late_q) part += turn_bytes / sizeof(float);
     if (!tiled && (int64_t)bhq * nchunks > max_records)
         return fail(LLMOPS_EWORKSPACE, "attention workspace too small for %lld chunk records", (long long)bhq * nchunks);
     // All tokens of a head together: rotation and cache update ride in the same launch where the rotary pairs suit it, the
@@ -1756,7 +1847,11 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
         LLMOPS_LAUNCH_CHECK();
         return LLMOPS_OK;
     }
-    if (tiled) {
+    if (late_q) {
+        const unsigned head_groups = (unsigned)((H + 31) / 32);
+        attn_prep_rows_kernel<T><<<(unsigned)(B * qL) * head_groups + tables, 256, 0, st>>>(k, v, (int)qL, (int)H, inv_freq, kc, vc, maxlen, slots, position_id,
+                                                                                            row_token, tile_tokens, kvLen, tables, head_groups, turns);
+    } else if (tiled) {
         attn_prep_kernel<T, true><<<(unsigned)(B * qL * H) + tables, 64, 0, st>>>(q, k, v, qL, H, S, inv_freq, half, kc, vc, maxlen, slots,
                                                                                  position_id, row_token, tile_tokens, kvLen, tables);
     } else {
@@ -1777,7 +1872,7 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
             configured = true;
         }
         attn_prefill_kernel<T><<<dim3((unsigned)(B * H * qtiles), (unsigned)nchunks), 512, smem, st>>>(q, kc, vc, qL, H, maxlen, kvLen, row_token, tile_tokens,
-                                                                                                       qtiles, plan.rows, part, nchunks);
+                                                                                                       qtiles, plan.rows, part, nchunks, late_q ? turns : nullptr);
         LLMOPS_LAUNCH_CHECK();
         if (nchunks > 1) {
             const unsigned groups = (unsigned)((bhq + 7) / 8);

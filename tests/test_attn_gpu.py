@@ -523,6 +523,23 @@ def test_attention_prefill_at_the_reference_sweep_sizes(ops, orc, past, qL, half
     _prefill_case(ops, orc, rng, past, qL, 2048, half, heads=[0, 13, 31])
 
 
+@pytest.mark.parametrize("half", [64, 32])   # q rotated by the tiled kernel, q rotated ahead of it
+@pytest.mark.parametrize("B,qL,past,H", [(1, 32, 0, 1), (2, 33, 700, 5), (1, 129, 5, 35), (3, 97, 0, 64)])
+def test_attention_prefill_rotation_of_ragged_heads_and_tokens(ops, orc, B, qL, past, H, half):
+    """heads that do not fill a group of 32 (or 16), tokens that end inside a tile's 32 rows, a batch, a cache in pieces"""
+    rng = np.random.default_rng(qL + half)
+    S, maxlen = 128, 900
+    inv_freq = (1.0 / (10000.0 ** (np.arange(0, 2 * half, 2, dtype=np.float32) / np.float32(2 * half)))).astype(np.float32)
+    cache = rng.standard_normal((2, B, H, maxlen, S)).astype(np.float32)
+    q, k, v = (rng.standard_normal((B, qL, H * S)).astype(np.float32) for _ in range(3))
+    slots = ((past + np.arange(qL)) % maxlen).astype(np.int32)
+    g = dict(q=q, k=k, v=v, cache=cache, inv_freq=inv_freq, slots=slots, position_id=past, layer_id=0)
+    out, k_rot, cache_after = run_attention(ops, g)
+    want, k_ref, cache_ref = orc.attention(q, k, v, inv_freq, cache, slots, past, 0)
+    assert max_rel_err(out, want) <= 1e-4   # (as the prompts above)
+    assert np.abs(k_rot - k_ref).max() <= 1e-5 and np.abs(cache_after - cache_ref).max() <= 1e-5
+
+
 def test_attention_prefill_long_chunk_wrapping_the_ring(ops, orc):
     """a 1024-token chunk whose slots wrap around a cache of 2048 rows that is already full"""
     rng = np.random.default_rng(77)

@@ -171,14 +171,23 @@ def attention(m, rows, H, past, maxlen, half):
     m.touch("rotation", "slots", rows * 4, 0, (rows - 1) * 4 + 4)
     for what, lo in (("k rows of the cache", 0), ("v rows of the cache", plane)):
         m.touch("rotation", what, (lo, lo + plane), lo + int(slot.min()) * S * e, lo + ((H - 1) * maxlen + int(slot.max())) * S * e + S * e)
-    for what in ("q", "k", "v"):
-        m.touch("rotation", what, q_bytes, 0, (((rows - 1) * H + H - 1) * S + S - 1) * 4 + 4)
+    # behind that table the tiles' token ranges, the angles' cosines and sines, the records (what the launch asks the workspace for)
+    turns = part + up(tables * 16)
+    records = turns + rows * S * 4
+    assert records + (H * rows * n.value * 520 if n.value > 1 else 0) <= ws_bytes
+    m.touch("rotation", "token ranges of the tiles", (part, turns), part, part + tables * 16)
+    m.touch("rotation", "cosines and sines", (turns, records), turns, turns + ((rows - 1) * S + 64 + 63) * 4 + 4)
+    group_heads = np.arange(-(-H // 32) * 32)
+    for what in ("k", "v"):
+        m.touch("rotation", what, q_bytes, 0, (((rows - 1) * H + np.minimum(group_heads, H - 1).max()) * S + 64 + 60) * 4 + 16)
     name = "attention, %d pieces of %d rows" % (n.value, r.value)
     for what, lo in (("k rows of the cache", 0), ("v rows of the cache", plane)):
         m.touch(name, what, (lo, lo + plane), lo, lo + ((H - 1) * maxlen + kv - 1) * S * e + S * e)
     m.touch(name, "token of a cache row", (head, head + kv * 4), head, head + (kv - 1) * 4 + 4)  # (what the table's workgroups wrote)
+    m.touch(name, "q", q_bytes, 0, ((rows - 1) * H + H - 1) * S * 4 + (64 + 60) * 4 + 16)
+    m.touch(name, "cosines and sines", (turns, records), turns, turns + ((rows - 1) * S + 64 + 60) * 4 + 16)
     if n.value > 1:
-        m.touch(name, "records", (part, ws_bytes), part, part + ((H * rows - 1) * n.value + n.value - 1) * 520 + 520)
+        m.touch(name, "records", (records, ws_bytes), records, records + ((H * rows - 1) * n.value + n.value - 1) * 520 + 520)
     m.touch(name, "output", q_bytes, 0, ((rows - 1) * H + H - 1) * S * 4 + S * 4)
 
 
@@ -327,3 +336,20 @@ def test_streamed_products_stay_inside(Ng, Kg, N, parts):
     finally:
         lib.llmops_test_fc_stream_set(0, 0, 0, 0)
     assert not m.bad, m.bad
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_an_attention_workspace_of_the_size_asked_holds_the_angles_beside_the_records(half):
+    """The tiled prompt kernel rotates q from a table of angles that lies ahead of the records: whatever the heads, tokens and cache,
+    a workspace of exactly the size asked has the room."""
+    from llmops import _lib
+    lib = _lib.load()
+    for H in (1, 2, 3, 32):
+        for rows in (32, 33, 127, 129, 500, 2048):
+            for maxlen in (1, 33, 64, 128, 129, 192, 193, 256, 300, 1000, 4096):
+                for past in (0, 1, 100, maxlen // 2, 2 * maxlen):
+                    k, r, n = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+                    assert lib.llmops_test_attn_plan(1, rows, H, maxlen, past, int(half), ctypes.byref(k), ctypes.byref(r), ctypes.byref(n)) == 0
+                    tables = -(-min(past + rows, maxlen) // 64)
+                    need = 65536 + up(maxlen * 4) + up(tables * 16) + rows * 512 + (H * rows * n.value * 520 if n.value > 1 else 0)
+                    assert k.value == 3 and need <= lib.llmops_attention_workspace_bytes(1, rows, H, 128, maxlen), (H, rows, maxlen, past)
