@@ -1,7 +1,7 @@
 // Rotary embedding, KV-cache update and attention over the cache
 // (attention_rope2 / attention_rope, /root/reference/ops/op_attn.hpp:721-1029 and :518-718).
 //
-// One query token: attn_decode_kernel (everything in one launch) and attn_merge_kernel.  More:
+// One query token: attn_decode_kernel (everything in one launch) and the merge of 3.  More:
 //   1. attn_prep_kernel   rotate q and k in place (rope_embed, ops/op_attn.hpp:44-94), write the
 //                         rotated k and the v rows into the cache at slots[p] (:764-773), and
 //                         from 32 tokens on record which cache rows were written by which token of this call
@@ -10,7 +10,7 @@
 //   2. below 32 tokens    attn_split_kernel or attn_few_kernel: a workgroup takes a chunk of cache rows and leaves
 //                         per query the chunk's score maximum, its sum of exponentials and its weighted V sum.
 //      from 32 on         attn_prefill_kernel: 128 queries to a workgroup, the cache rows in one piece or in several.
-//   3. attn_merge_kernel  merges the chunks of a query with the usual max/sum rescaling and
+//   3. merge_records      (attn_merge_rows_kernel or attn_merge_kernel) merges the chunks of a query with the usual max/sum rescaling and
 //                         overwrites q with the result (:1018-1025).
 // The cache element type is fp32 (reference layout) or fp16 (all arithmetic still fp32).
 //
@@ -762,12 +762,13 @@ __global__ __launch_bounds__(128) void attn_merge_kernel(float* __restrict__ q, 
     q[((b * qL + pq) * H + h) * S + threadIdx.x] = r;
 }
 
-// The same for up to N records of a query and many queries (the pieces of attn_prefill_kernel): half a wave to a query, 16 bytes to a
-// lane, all records of eight queries asked for at once.  (512 tokens behind 1500, 32 heads, two records each: 20 us by
-// attn_merge_kernel's workgroup per query, 7.)
+// The same, bit for bit, for up to N records of a query whose number is known: half a wave to a query, 16 bytes to a lane, all records of
+// eight queries asked for at once.  Bound by one round trip to memory with few queries, by the records with many.  (512 tokens behind 1500,
+// 32 heads, two records each: 20 us by attn_merge_kernel's workgroup per query, 7; fewer tokens: at merge_records.)
 template <int N>
 __global__ __launch_bounds__(256) void attn_merge_rows_kernel(float* __restrict__ q, const float* __restrict__ part, int qL, int H,
                                                                unsigned queries, int nchunks) {
+#pragma clang fp contract(off)  // (the products of den are rounded as those of attn_merge_kernel are)
     constexpr int S = 128;
     const unsigned bhq = blockIdx.x * 8 + (threadIdx.x >> 5);
     const int at = 4 * (threadIdx.x & 31);
@@ -781,15 +782,19 @@ __global__ __launch_bounds__(256) void attn_merge_rows_kernel(float* __restrict_
         lo[c] = *reinterpret_cast<const float2*>(rc + 2 + at);
         hi[c] = *reinterpret_cast<const float2*>(rc + 4 + at);
     }
-    float M = -FLT_MAX, den = 0.0f, w[N];
+    float M = -FLT_MAX, den[N], w[N];
 #pragma unroll
     for (int c = 0; c < N; c++) M = fmaxf(M, st[c].x);  // (records past the last are copies of it)
 #pragma unroll
     for (int c = 0; c < N; c++) {
         w[c] = c >= nchunks || st[c].y == 0.0f ? 0.0f : expf(st[c].x - M);
-        den += w[c] * st[c].y;
+        den[c] = w[c] * st[c].y;
     }
-    const float inv = 1.0f / den;
+#pragma unroll
+    for (int o = N / 2; o > 0; o >>= 1)  // (the order of wave_sum: the bits of attn_merge_kernel)
+#pragma unroll
+        for (int c = 0; c < o; c++) den[c] += den[c + o];
+    const float inv = 1.0f / den[0];
     float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
     for (int c = 0; c < N; c++) {
@@ -1749,6 +1754,20 @@ extern "C" size_t llmops_attention_workspace_bytes(int64_t B, int64_t qL, int64_
            (size_t)records * (S + 2) * sizeof(float);
 }
 
+// Merging the records where their number is known here: up to eight by half waves whatever the queries; up to sixteen from 512 queries on
+// (attn_merge_kernel asks for 32 records however few there are, but has a workgroup to every query: with 64 queries of 16 records, 2 tokens
+// behind 1000, it is 0.3 us the faster one).  us for the whole call in a graph, 32 heads, by attn_merge_kernel / so: 3 tokens 11.5 / 10.4, 31 behind 97
+// 20.8 / 19.1, 16 behind 1500 24.9 / 24.9, batches 8 x 31 behind 100 halves 39.8 / 32.8, 8 x 31 behind 400 55.9 / 49.8, 4 x 16 behind 60 20.4 / 17.6,
+// 4 x 20 behind 900 45.0 / 43.4; one token behind 100 9.5 / 8.9, of eight sequences behind 100 halves 11.9 / 10.7, behind 500 halves 18.9 / 18.0.
+static void merge_records(float* q, const float* part, int64_t bhq, int64_t qL, int64_t H, int records, hipStream_t st) {
+    const unsigned groups = (unsigned)((bhq + 7) / 8);
+    if (records <= 2) attn_merge_rows_kernel<2><<<groups, 256, 0, st>>>(q, part, (int)qL, (int)H, (unsigned)bhq, records);
+    else if (records <= 4) attn_merge_rows_kernel<4><<<groups, 256, 0, st>>>(q, part, (int)qL, (int)H, (unsigned)bhq, records);
+    else if (records <= 8) attn_merge_rows_kernel<8><<<groups, 256, 0, st>>>(q, part, (int)qL, (int)H, (unsigned)bhq, records);
+    else if (records <= 16 && bhq >= 512) attn_merge_rows_kernel<16><<<groups, 256, 0, st>>>(q, part, (int)qL, (int)H, (unsigned)bhq, records);
+    else attn_merge_kernel<<<(unsigned)bhq, 128, 0, st>>>(q, part, qL, H, records);
+}
+
 template <typename T>
 static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t qL, int64_t H, int64_t S,
                           const float* inv_freq, int64_t half, T* cache, int64_t maxlen, const int32_t* slots,
@@ -1810,7 +1829,8 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
 #undef LLMOPS_DECODE
         LLMOPS_LAUNCH_CHECK();
         if (nchunks > 1) {
-            attn_merge_kernel<<<(unsigned)bhq, 128, 0, st>>>(q, part, qL, H, nchunks, 4 * p.pw, pos_dev, maxlen);
+            if (pos_dev != nullptr) attn_merge_kernel<<<(unsigned)bhq, 128, 0, st>>>(q, part, qL, H, nchunks, 4 * p.pw, pos_dev, maxlen);
+            else merge_records(q, part, bhq, qL, H, nchunks, st);
             LLMOPS_LAUNCH_CHECK();
         }
         return LLMOPS_OK;
@@ -1843,7 +1863,7 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
         attn_few_kernel<T, true><<<(unsigned)wgs_rope, 256, 0, st>>>(q, kc, vc, (int)qL, H, maxlen, (int)kvLen, slots, part,
                                                                                    nchunks + 1, k, v, inv_freq, position_id);
         LLMOPS_LAUNCH_CHECK();
-        attn_merge_kernel<<<(unsigned)bhq, 128, 0, st>>>(q, part, qL, H, nchunks + 1);
+        merge_records(q, part, bhq, qL, H, nchunks + 1, st);
         LLMOPS_LAUNCH_CHECK();
         return LLMOPS_OK;
     }
@@ -1875,11 +1895,7 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
                                                                                                        qtiles, plan.rows, part, nchunks, late_q ? turns : nullptr);
         LLMOPS_LAUNCH_CHECK();
         if (nchunks > 1) {
-            const unsigned groups = (unsigned)((bhq + 7) / 8);
-            if (nchunks <= 2) attn_merge_rows_kernel<2><<<groups, 256, 0, st>>>(q, part, (int)qL, (int)H, (unsigned)bhq, nchunks);
-            else if (nchunks <= 4) attn_merge_rows_kernel<4><<<groups, 256, 0, st>>>(q, part, (int)qL, (int)H, (unsigned)bhq, nchunks);
-            else if (nchunks <= 8) attn_merge_rows_kernel<8><<<groups, 256, 0, st>>>(q, part, (int)qL, (int)H, (unsigned)bhq, nchunks);
-            else attn_merge_kernel<<<(unsigned)bhq, 128, 0, st>>>(q, part, qL, H, nchunks);
+            merge_records(q, part, bhq, qL, H, nchunks, st);
             LLMOPS_LAUNCH_CHECK();
         }
         return LLMOPS_OK;
@@ -1894,7 +1910,7 @@ static int attention_impl(float* q, float* k, const float* v, int64_t B, int64_t
     else
         attn_split_kernel<T, 4><<<(unsigned)(bhq * nchunks), 256, 0, st>>>(q, kc, vc, qL, H, maxlen, kvLen, slots, part, nchunks);
     LLMOPS_LAUNCH_CHECK();
-    attn_merge_kernel<<<(unsigned)bhq, 128, 0, st>>>(q, part, qL, H, nchunks);
+    merge_records(q, part, bhq, qL, H, nchunks, st);
     LLMOPS_LAUNCH_CHECK();
     return LLMOPS_OK;
 }

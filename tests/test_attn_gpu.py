@@ -523,6 +523,15 @@ def test_attention_prefill_at_the_reference_sweep_sizes(ops, orc, past, qL, half
     _prefill_case(ops, orc, rng, past, qL, 2048, half, heads=[0, 13, 31])
 
 
+@pytest.mark.parametrize("B,qL,kv,H", [(1, 3, 40, 5), (1, 1, 100, 3), (8, 1, 200, 32), (8, 1, 511, 32), (1, 16, 1500, 32), (1, 20, 1900, 26),
+                                       (1, 16, 1500, 31), (1, 17, 2050, 32), (1, 1, 129, 1)])
+@pytest.mark.parametrize("cache_dtype", [torch.float32, torch.float16])
+def test_attention_few_tokens_records_merged(ops, B, qL, kv, H, cache_dtype):
+    """One and more tokens whose records are merged by half waves (up to eight; nine to sixteen from 512 queries on) and by a workgroup per
+    query (fewer queries, more records), the last workgroup partly filled."""
+    _tokens_behind_a_cache(ops, B, qL, kv, H, cache_dtype, "in order")
+
+
 @pytest.mark.parametrize("half", [64, 32])   # q rotated by the tiled kernel, q rotated ahead of it
 @pytest.mark.parametrize("B,qL,past,H", [(1, 32, 0, 1), (2, 33, 700, 5), (1, 129, 5, 35), (3, 97, 0, 64)])
 def test_attention_prefill_rotation_of_ragged_heads_and_tokens(ops, orc, B, qL, past, H, half):
