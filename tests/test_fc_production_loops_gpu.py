@@ -5,7 +5,7 @@
   here bit for bit with the oracle's FC_dynamic_quantize_x / integer core (ops/op_fc.hpp:221-272,337-363;
   quant_row_q8_0 ops/utils.hpp:200-220).  The raw group sum is a tree sum in that kernel (it feeds only the
   fp32 output, ops/op_fc.hpp:408) and is compared to rounding.
-* The weight-streaming int8 MFMA kernel of 3..32 rows: its int32 sums (fc_Q4A_partials, use_mfma=3).
+* The weight-streaming int8 MFMA kernel: its int32 sums (fc_Q4A_partials, use_mfma=3).
 * Config 3 (group 128, M in {16,128,512,2048}, 4096->11008 and 11008->4096): the GPU output against the oracle
   on a sample of rows (FC rows are independent), and the int32 sums of its 128-row tiles at 2048 rows.
 
@@ -137,8 +137,7 @@ def test_decode_kernel_pass_distribution(orc, G, N, kgs):
 @pytest.mark.parametrize("rows", [3, 9, 16, 17, 32])
 @pytest.mark.parametrize("N,K", [(4096, 4096), (4096, 11008), (12288, 4096), (2080, 1024)])
 def test_streaming_mfma_kernel_int32_sums(orc, rows, N, K):
-    """fc_rows_mfma_kernel (3..32 rows, group 128): every workgroup shape the launcher picks -- two k-halves per
-    strip below 256 strips, 16 waves for long runs, two row tiles per wave from 17 rows on"""
+    """fc_stream_kernel (group 128) in the builds that the launcher picks at these sizes"""
     import llmops
     rng = np.random.default_rng(rows + N + K)
     wq = orc.quant_w((rng.standard_normal((N, K)) * 0.02).astype(np.float32), 128)
