@@ -137,6 +137,12 @@ bool llmops::streams(int64_t rows, int64_t Ng, int64_t Kg, int group_k) {
     const double ahead = rows > 512 ? 2.0 : Kg < 12 ? 4.75 : 7.0;
     return stream_estimate(rows, Ng, Kg, LLMOPS_FC_COUNTER_BYTES - kTicketBytes) <= gemm_tile_estimate(rows, Ng, Kg) + ahead;
 }
+// An input that does not start on 16 bytes takes the general quantization, whose codes lie row by row: more than 32 such rows are the tiled
+// kernel's (tiled / streaming, us: 32 x 11008 x 4096 15.4 / 12.7, 64 x 11008 x 4096 17.8 / 18.5, 128 x 11008 x 4096 22.8 / 26.9, 500 x 4096 x 11008
+// 55.1 / 69.9; 64 x 2048^2 10.5 / 6.8 goes with them).
+static bool streams_input(const float* x, int64_t rows, int64_t Ng, int64_t Kg, int group_k) {
+    return (rows <= 32 || aligned(x, 16) || stream_forced()) && streams(rows, Ng, Kg, group_k);
+}
 
 // the product for activations that a quantization launch has left in the workspace (more rows than the streaming
 // kernel that quantizes on the fly takes); streamed: what streams() says; tiled: the codes are in the order of tile_code_offset
@@ -183,7 +189,7 @@ static int fc_impl(const float* x, int64_t rows, int64_t K, const int8_t* weiq, 
         if (rc_t == 0 && residual != nullptr) rc_t = launch_add(y, residual, rows * N, st);
         return rc_t;
     }
-    const bool streamed = streams(rows, Ng, Kg, group_k);
+    const bool streamed = streams_input(x, rows, Ng, Kg, group_k);
     if (rows <= kMaxGemvRows && !(streamed && rows >= rows_from(Ng, Kg)))  // (one launch)
         return launch_gemv_fused(w, x, y, part, counters, rows, Ng, Kg, group_k, N, residual, nullptr, 0.0f, 0, nullptr, 0,
                                  nullptr, st);
@@ -291,7 +297,7 @@ static int fc_decode_impl(const float* x, int64_t rows, int64_t K, const int8_t*
         float* xd = reinterpret_cast<float*>(ws + lay.off_xd);
         float* gs = reinterpret_cast<float*>(ws + lay.off_gs);
         float2* xst = reinterpret_cast<float2*>(ws + lay.off_xst);
-        const bool streamed = streams(rows, Ng, Kg, group_k);
+        const bool streamed = streams_input(x, rows, Ng, Kg, group_k);
         bool tiled = streamed;
         int rc = (norm_w != nullptr || glu == 2)
                      ? launch_quant_x_fused(x, rows, K, group_k, norm_w, eps, glu == 2, xq, xst, tiled, st)

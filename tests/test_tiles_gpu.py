@@ -139,6 +139,18 @@ def test_streaming_product_exact_and_with_a_producer(ops, orc, rows, N, K):
     assert torch.equal(ops.fc_Q4A_decode(gu, pw, N, glu_in=True), ops.fc_Q4A(ops.silu_mul(gu), pw, N))
 
 
+@pytest.mark.parametrize("rows", [4, 32, 33, 128])
+def test_input_that_does_not_start_on_16_bytes(ops, orc, rows):
+    """The general quantization (codes row by row), on either side of the 32 rows from which the tiled kernel takes such an input."""
+    x, w, res = _inputs(rows, 300, 1024, rows)
+    pw = orc.quant_w(w, 128)
+    flat = torch.empty(x.size + 2, device="cuda")
+    flat[2:] = dev(x).flatten()
+    view = flat[2:].view(x.shape)
+    assert max_rel_err(ops.fc_Q4A(view, dev(pw), 300).cpu().numpy(), orc.fc(x, pw, 300)) <= 1e-5
+    assert max_rel_err(ops.fc_Q4A(view, dev(pw), 300, residual=dev(res)).cpu().numpy(), orc.fc(x, pw, 300) + res) <= 1e-5
+
+
 @pytest.mark.parametrize("N,Kg", [(70, 11), (96, 12), (4096, 32), (4128, 32), (8224, 31), (8224, 32)])
 def test_rows_either_side_of_the_streaming_kernel(ops, orc, N, Kg):
     """fc_Q4A on either side of the lines between the kernel that quantizes on the fly (2 to 4 rows) and the weight-streaming one, and
