@@ -285,11 +285,13 @@ __global__ __launch_bounds__(256, 3) void fc_gemm_g32_kernel(const uint8_t* __re
     }
 }
 
-// Split-K factor.  Estimated time in us: a workgroup's run of stages, 0.95 us each, times how many workgroups a compute unit
-// has to run (three fit; two together take 1.3, three 1.53 times what one does alone); the second launch that adds the partial
-// sums 0.44 us per four splits (its loads in flight) and their traffic.  Against every factor of 1 .. 6, 8, 10, 12, 16, 20, 24 at 19
-// row counts from 9 to 2048 of seven shapes: 1.3 % slower than the best on average, 10 % at worst (32 x 22016 x 4096, 8 splits
-// where 4 are best; the rule of two workgroups to a compute unit: 2.3 %, 23 %).
+// Split-K factor.  Estimated time in us: a workgroup's run of stages and 3.6 more for what it does around them, 0.95 us each, times
+// how many workgroups a compute unit has to run (three fit; two together take 1.19, three 1.45 times what one does alone); the
+// second launch that adds the partial sums 1.8 us, 0.77 more per four splits (its loads in flight) and their traffic.  Against up to
+// thirteen factors from 1 to 24 at up to 30 row counts from 9 to 2048 of eighteen shapes from 1024 x 512 to 22016 x 4096: 0.7 % slower than the
+// best on average, 8 % at worst (65 x 22016 x 4096, 2 splits where 5 are best).  (With nothing for the ends of a run and 0.44 us for the
+// second launch 2.0 % and 22 %: us, 9 x 12288 x 4096 22.4 in 16 splits / 19.4 in 8, 32 x 22016 x 4096 31.5 / 30.2 in 4, 300 x 8192 x 2048
+// 36.7 in 2 / 34.7 in one, 1024 x 2048^2 33.5 in 2 / 29.7 in one.)
 // Partial sums never take a workspace that fits the built-in scratch of llmops_fc_Q4A_noalloc beyond it.
 int plan_gemm_g32(int64_t rows, int64_t Ng, int64_t Kg, int force_split, int* st_per_split) {
     const int64_t nst = (Kg + kG32Gps - 1) / kG32Gps;
@@ -303,8 +305,8 @@ int plan_gemm_g32(int64_t rows, int64_t Ng, int64_t Kg, int force_split, int* st
         const int64_t per = (nst + s - 1) / s, S = (nst + per - 1) / per;
         if (S > 1 && room >= 0 && S * rows * Ng * kGroupN * 4 > room && force_split <= 0) continue;
         const int64_t full = tiles * S / 768, rest = tiles * S % 768;
-        double t = 0.95 * (double)per * ((double)full * 1.53 + (rest == 0 ? 0.0 : rest <= 256 ? 1.0 : rest <= 512 ? 1.3 : 1.53));
-        if (S > 1) t += 0.44 * (double)((S + 3) / 4) + 1.16e-6 * (double)S * (double)rows * (double)(Ng * kGroupN);
+        double t = 0.95 * ((double)per + 3.6) * ((double)full * 1.45 + (rest == 0 ? 0.0 : rest <= 256 ? 1.0 : rest <= 512 ? 1.19 : 1.45));
+        if (S > 1) t += 1.8 + 0.77 * (double)((S + 3) / 4) + 1.05e-6 * (double)S * (double)rows * (double)(Ng * kGroupN);
         if (best == 0.0 || t < best) best = t, best_s = S, best_per = per;
     }
     *st_per_split = (int)best_per;
