@@ -1656,14 +1656,14 @@ static TokensPlan plan_tokens(int64_t bh, int64_t qL, int64_t kvLen, bool half_c
     if (qL >= g_prefill_min_tokens) {
         // A workgroup takes a compute unit: with fewer query tiles than those, ns workgroups share a tile's cache rows, at
         // least 128 each.  A row costs a tile 0.0365 us (halves 0.0305: two products instead of three); the launch that merges the
-        // records costs 2.6 us and 0.165 us per 1000 records.  (us, one piece / as planned, 32 heads: 32 tokens behind 100 17.4 / 17.4
-        // (two 17.9), behind 500 32.4 / 20.2; 128 behind 200 29.2 / 26.1, behind 2000 95.6 / 40.8; 256 behind none 28.4 / 28.4 (two 29.9),
-        // halves 24.1 / 24.2 (27.7); 384 behind 300 48.8 / 42.9; 512 behind none 41.5 / 40.1, behind 1500 108.8 / 79.2; 8 heads, 2048 tokens
-        // 97.9 / 68.2; 128 heads, 128 behind 1500 91.4 / 78.3.  Of 30 sizes two are 2 to 5 % slower than with the best number of pieces.)
-        // Beside halves a record is priced at 0.35 us per 1000, above what it costs: the planner's test holds 200 and 256 tokens behind 300 to
-        // one piece there (256: 35.2, in four 30.8; 384 behind 300 43.3, in two 40.0).
+        // records costs 2.6 us and 0.15 us per 1000 records, beside either cache.  Against every number of pieces at 710 sizes of each
+        // cache (8 to 256 heads in all, 32 to 2048 tokens behind 0 to 3500): 0.03 % slower than the best on average and 3 % at worst, beside
+        // halves 0.13 % and 8 %.  (us with the copy that puts q and k back, one piece / several, 32 heads: 32 tokens behind 100 19.3 / 19.6, behind
+        // 500 34.7 / 21.4; 128 behind 200 30.7 / 27.2, behind 2500 114 / 41; 256 behind none 30.45 / 30.5, behind 300 42.7 / 33.2; 512 behind none
+        // 43.4 / 40.8, behind 1500 98 / 75; 8 heads, 2048 tokens 100 / 70.  Halves: 64 behind 100 19.1 / 19.9, 200 behind 300 34.7 / 28.6; 256 behind
+        // none 26.9 / 28.6, behind 300 37.9 / 31.4; 512 behind 300 50.8 / 45.3; 16 heads, 512 behind 100 39.7 / 32.1.)
         p.kernel = 3;
-        const double row = half_cache ? 0.0305 : 0.0365, record = half_cache ? 0.35e-3 : 0.165e-3;
+        const double row = half_cache ? 0.0305 : 0.0365, record = 0.15e-3;
         int64_t ns = 256 / (bh * ((qL + 127) / 128));
         if (ns > (kvLen + 127) / 128) ns = (kvLen + 127) / 128;
         if (ns < 2 || bhq * ns > max_records || row * (double)(kvLen - kvLen / ns) < 2.6 + record * (double)(bhq * ns)) ns = 1;

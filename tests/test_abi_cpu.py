@@ -270,9 +270,9 @@ def test_attention_planner_measured_sizes(half):
 
 
 @pytest.mark.parametrize("heads,tokens,past,pieces32,pieces16", [
-    (32, 32, 500, True, True), (32, 64, 100, False, False), (32, 256, 0, False, False), (32, 256, 300, True, False),
-    (32, 200, 300, True, False), (16, 384, 64, None, False), (16, 1024, 400, True, True), (32, 512, 1500, True, True),
-    (32, 2048, 0, False, False), (128, 512, 3500, False, False)])
+    (32, 32, 500, True, True), (32, 64, 100, False, False), (32, 256, 0, None, False), (32, 256, 300, True, True),
+    (32, 200, 300, True, True), (16, 384, 100, True, True), (16, 512, 100, True, True), (16, 1024, 400, True, True), (32, 512, 300, True, True),
+    (32, 512, 1500, True, True), (32, 2048, 0, False, False), (128, 512, 3500, False, False)])
 def test_attention_planner_pieces_of_the_tiled_kernel(heads, tokens, past, pieces32, pieces16):
     """From 32 query tokens: the cache rows of a tile in several workgroups or in one, at sizes where one of the two measured
     faster (or where the tiles fill the chip); None: the same within 3 %."""
