@@ -93,13 +93,14 @@ static int g_rows_from_small = 0, g_rows_from_large = 0;
 //   4096x11008:             2 rows 8.7 / 10.8, 3 10.7 / 10.9 (from a cache 12.2 / 10.9), 4 12.4 / 10.4, 8 19.6 / 10.6; 2500x11008: 3 14.9 / 9.7
 //   1500x2048, 2048x2048:   4 rows 5.7 / 5.5, 8 8.3 / 5.5
 //   1024x512 .. 4096x1024:  4 rows 4.2 / 5.0, 8 6.3 / 5.3 (call by call 6.3 / 8.6)
-//   512x4096 (16):          3 rows 6.8 / 6.0, 6 8.3 / 6.0 (call by call 8.3 / 8.4), 8 9.1 / 6.0; 600x11008: 3 8.6 / 7.7, 4 9.2 / 7.7, 8 12.4 / 7.8
-//   Under 16 strips the first kernel stays up to 8 rows: the bits of its dump build are those of fc_Q4A there.
+//   1 to 64 strips, within 15 % whatever their number: x 2048 4 rows 5.6 / 5.5, 8 8.5 / 5.7 (call by call 8.3 / 6.5 to 8.4); x 4096 3 rows 6.9 / 6.0,
+//   6 8.6 / 6.6, 8 9.3 / 6.7 (9.0 / 6.4 to 8.4); x 8192 4 rows 8.4 / 7.9, 8 11.2 / 8.1; x 11008 4 rows with 8 strips 8.6 / 9.1, with 16 9.2 / 9.2,
+//   with 47 14.4 / 9.6; 5 with 8 strips 10.0 / 9.1
 static int rows_from(int64_t Ng, int64_t Kg) {
     const int forced = Ng > 256 ? g_rows_from_large : g_rows_from_small;
     if (forced > 0) return forced;
-    if (Ng < 16 || Kg < 12) return kMaxGemvRows + 1;
-    if (Ng < 64) return Kg < 24 ? kMaxGemvRows + 1 : Kg < 64 ? 6 : 4;
+    if (Kg < 12) return kMaxGemvRows + 1;
+    if (Ng < 64) return Kg < 24 ? kMaxGemvRows + 1 : Kg < 64 ? 6 : Ng < 16 ? 5 : 4;
     if (Ng > 256 || Kg >= 64) return 3;
     return Kg < 24 ? 5 : 4;
 }

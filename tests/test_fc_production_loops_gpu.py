@@ -58,8 +58,15 @@ def check_dump(orc, x, wq, N, G):
     assert np.array_equal(xd.view(np.uint32), od.view(np.uint32)), "activation scales differ"
     assert np.abs(gs - og).max() <= 1e-5 * max(1.0, float(np.abs(x).max()) * G)
     assert np.array_equal(acc, orc.fc_partials(oq, wq)), "int32 sums of the decode kernel differ"
-    # the dump build computes the same outputs as the kernel llmops.fc_Q4A launches, and both meet the oracle
-    prod = llmops.fc_Q4A(dev(x[None]), dev(wq), N)[0].cpu().numpy()
+    # the dump build computes the same outputs as the kernel llmops.fc_Q4A launches where it does so in one launch (the row count from
+    # which it quantizes first is set beyond 8 here), and both meet the oracle
+    from llmops import _lib
+    lib = _lib.load()
+    lib.llmops_test_fc_set_row_routing(9, 9)
+    try:
+        prod = llmops.fc_Q4A(dev(x[None]), dev(wq), N)[0].cpu().numpy()
+    finally:
+        lib.llmops_test_fc_set_row_routing(0, 0)
     assert np.array_equal(y.view(np.uint32), prod.view(np.uint32))
     assert max_rel_err(y, orc.fc(x[None], wq, N)[0]) <= 1e-3
     return xq
@@ -125,9 +132,7 @@ def test_decode_kernel_pass_distribution(orc, G, N, kgs):
     for Kg in kgs:
         K = Kg * G
         wq = orc.quant_w((rng.standard_normal((N, K)) * 0.02).astype(np.float32), G)
-        # (3..8 rows run 8-wave workgroups; with 64 strips or more and group 128 fc_Q4A sends them to the MFMA kernel,
-        # whose output check_dump could not compare bit for bit)
-        for rows in ((1, 2, 3, 5, 8) if (N < 2048 or G == 32) else (1, 2)):
+        for rows in (1, 2, 3, 5, 8):   # (3..8 rows run 8-wave workgroups)
             x = rng.standard_normal((rows, K)).astype(np.float32)
             x[0, :8] = TIE
             x[0, 8:G] = 0

@@ -163,6 +163,26 @@ def test_rows_either_side_of_the_streaming_kernel(ops, orc, N, Kg):
         assert max_rel_err(ops.fc_Q4A(dev(x), dev(pw), N, residual=dev(res)).cpu().numpy(), want + res) <= 1e-5
 
 
+@pytest.mark.parametrize("N,Kg,first", [(20, 24, 6), (33, 32, 6), (480, 63, 6), (256, 64, 5), (480, 64, 5), (512, 64, 4), (250, 23, 9), (96, 11, 9)])
+def test_rows_from_which_few_strips_are_streamed(ops, orc, N, Kg, first):
+    """Tensors of fewer than 64 strips: fc_Q4A quantizes first from `first` rows on (9: never, up to 8): the bits of that kernel from
+    there, of the one-launch kernel below; both against the oracle."""
+    from llmops import _lib
+    lib = _lib.load()
+    for rows in {max(2, first - 1), min(first, 8)}:
+        x, w, _ = _inputs(rows, N, 128 * Kg, rows + Kg)
+        pw = orc.quant_w(w, 128)
+        got = {}
+        for routing in (0, 9, 2):
+            lib.llmops_test_fc_set_row_routing(routing, routing)
+            try:
+                got[routing] = ops.fc_Q4A(dev(x), dev(pw), N)
+            finally:
+                lib.llmops_test_fc_set_row_routing(0, 0)
+            assert max_rel_err(got[routing].cpu().numpy(), orc.fc(x, pw, N)) <= 1e-5
+        assert torch.equal(got[0], got[2 if rows >= first else 9]) and not torch.equal(got[2], got[9])
+
+
 @pytest.mark.parametrize("rows", [3, 16, 17, 32])
 @pytest.mark.parametrize("N,Kg", [(2048, 1), (2050, 15), (2048, 16), (2080, 35), (2048, 49), (8224, 33), (8224, 66)])
 def test_few_row_product_runs(ops, orc, rows, N, Kg):
