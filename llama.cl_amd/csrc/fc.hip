@@ -428,7 +428,7 @@ extern "C" int llmops_fc_Q4A_partials(const int8_t* xq, int64_t rows, const int8
     const uint8_t* w = reinterpret_cast<const uint8_t*>(weiq);
     LLMOPS_REQUIRE(use_mfma >= 0 && use_mfma <= 3 && (use_mfma < 2 || group_k == 128));
     if (use_mfma == 3) {
-        LLMOPS_REQUIRE(rows <= 32);
+        LLMOPS_REQUIRE(rows <= 1024);  // (what streams() sends there)
         return launch_fc_rows_partials(w, xq, acc, rows, Ng, Kg, as_stream(stream));
     }
     if (use_mfma) return launch_gemm_partials(w, xq, acc, rows, Ng, Kg, group_k, use_mfma == 2, as_stream(stream));

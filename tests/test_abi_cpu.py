@@ -77,6 +77,9 @@ def test_argument_validation_without_device(lib):
     for use_mfma, groups in ((1, 1 << 19), (2, 1 << 18)):
         rc = lib.llmops_fc_Q4A_partials(vp(256), i64(64), vp(256), i64(1), i64(groups), 128, vp(256), use_mfma, vp(0))
         assert rc == 1 and b"K must be below" in lib.llmops_last_error()
+    # .. by the weight-streaming kernel: up to the 1024 rows that it takes
+    rc = lib.llmops_fc_Q4A_partials(vp(256), i64(1025), vp(256), i64(1), i64(4), 128, vp(256), 3, vp(0))
+    assert rc == 1 and b"rows <= 1024" in lib.llmops_last_error()
     rc = lib.llmops_fc_workspace_reset(vp(0), ctypes.c_size_t(1 << 20), vp(0))
     assert rc == 1 and b"workspace != nullptr" in lib.llmops_last_error()
     # the entry point that allocates nothing validates its arguments before it enqueues anything (no device here:

@@ -1,5 +1,7 @@
 """Edges of the tiled product, of the weight-streaming one and of the launches that were folded together, against the oracle.
 Outputs are fp32 sums of exact int32 group sums: 1e-5 of the largest, as elsewhere."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -56,8 +58,30 @@ def test_tiled_product_edges(ops, orc, tile, rows, N, Kg, split):
     assert max_rel_err(got_res, want + res) <= 1e-5
 
 
+@pytest.fixture(params=["tiled", "tiled, split", "streaming 1 1 8 0", "streaming 2 2 4 1", "streaming 3 1 4 0", "streaming 4 2 8 1"])
+def product(request):
+    """A product of more than 8 rows (group 128) pinned: the tiled kernel as planned or K in three, builds of the streaming kernel (row tiles,
+    strips, waves, K in halves)."""
+    from llmops import _lib
+    lib, kind = _lib.load(), request.param.split()
+    try:
+        if kind[0] == "streaming":
+            lib.llmops_test_fc_stream_set(*map(int, kind[1:]))
+        else:
+            lib.llmops_test_gemm_set_tuning(-1)
+            lib.llmops_test_gemm_set_split(3 if len(kind) > 1 else 0)
+        build = [ctypes.c_int(-1) for _ in range(4)]
+        assert lib.llmops_test_fc_stream_plan(100, 16, 8, *[ctypes.byref(b) for b in build]) == 0
+        assert [b.value for b in build] == (list(map(int, kind[1:])) if kind[0] == "streaming" else [0, -1, -1, -1])
+        yield request.param
+    finally:
+        lib.llmops_test_fc_stream_set(0, 0, 0, 0)
+        lib.llmops_test_gemm_set_tuning(0)
+        lib.llmops_test_gemm_set_split(0)
+
+
 @pytest.mark.parametrize("rows", [40, 300])
-def test_tiled_product_sums_that_overflow(ops, orc, rows):
+def test_product_sums_that_overflow(ops, orc, rows, product):
     """A row whose group sum is beyond fp32 although its values are not: infinite outputs where the min says so, in that
     row and nowhere else."""
     x, w, _ = _inputs(rows, 96, 640, 3)
@@ -68,6 +92,28 @@ def test_tiled_product_sums_that_overflow(ops, orc, rows):
     assert np.isinf(want[0, 7]).all() and np.array_equal(got[0, 7], want[0, 7])
     other = np.arange(rows) != 7
     assert max_rel_err(got[0, other], want[0, other]) <= 1e-5
+
+
+@pytest.mark.parametrize("rows,Kg", [(37, 8), (131, 17)])
+def test_product_rows_stay_their_own(ops, orc, rows, Kg, product):
+    """Rows of ordinary, tiny, huge and zero activations side by side: each to 1e-5 of its own largest output (sums of Kg products carry
+    Kg * 2^-24).  An infinity or a NaN in one row leaves the bits of all others as they are and no value of its own finite."""
+    x, w, _ = _inputs(rows, 290, 128 * Kg, rows + Kg)
+    x[0, 2:6] *= 1e-4
+    x[0, 6:10] *= 30000.0
+    x[0, 10] = 0.0
+    x[0, 1, 128:256] = 0.0
+    x[0, 17:20] *= 3000.0
+    x[0, rows - 1] *= 1e-6
+    pw = orc.quant_w(w, 128)
+    want = orc.fc(x, pw, 290)[0]
+    got = ops.fc_Q4A(dev(x), dev(pw), 290)[0]
+    err, scale = np.abs(got.cpu().numpy() - want).max(axis=1), np.abs(want).max(axis=1)
+    assert (err <= 1e-5 * scale).all() and (got[10] == 0.0).all()
+    x[0, 3, 77], x[0, 35, 1000] = np.inf, np.nan
+    hurt = ops.fc_Q4A(dev(x), dev(pw), 290)[0]
+    rest = [r for r in range(rows) if r not in (3, 35)]
+    assert torch.equal(hurt[rest], got[rest]) and not torch.isfinite(hurt[[3, 35]]).any()
 
 
 @pytest.mark.parametrize("rows,N", [(9, 70), (33, 300)])
@@ -98,7 +144,7 @@ def test_group32_product_last_stage(ops, orc, rows, N, Kg):
 def test_streaming_product_every_build(ops, orc, row_tiles, strips, waves, halves):
     """Every build of the weight-streaming product, forced: rows that end inside a row tile, one past it and past a row block, columns
     inside a strip, strips inside a pair (and fewer than the eight of a round of the XCDs), waves with no k-group, one and several; K in
-    halves; residual, in place too; results in parts; the same bits again (the exchange slots are left empty)."""
+    halves; residual; results in parts; the same bits again (the exchange slots are left empty); the int32 sums."""
     from llmops import _lib
     lib = _lib.load()
     lib.llmops_test_fc_stream_set(row_tiles, strips, waves, halves)
@@ -120,6 +166,12 @@ def test_streaming_product_every_build(ops, orc, row_tiles, strips, waves, halve
             flat = torch.empty(tx.numel() + 2, device="cuda")
             flat[2:] = tx.flatten()
             assert max_rel_err(ops.fc_Q4A(flat[2:].view(tx.shape), tw, N).cpu().numpy(), want) <= 1e-5
+            # the int32 sums: of codes row by row by themselves, of codes in the order of the loads through outputs that are exact
+            xq = np.random.default_rng(rows).integers(-127, 128, (rows, 128 * Kg)).astype(np.int8)
+            assert np.array_equal(ops.fc_Q4A_partials(dev(xq), tw, use_mfma=3).cpu().numpy(), orc.fc_partials(xq, pw))
+            xe, we = oracle.closed_form_fc_inputs(rows, N, 128 * Kg, seed=rows)
+            got = ops.fc_Q4A(dev(xe.reshape(1, rows, 128 * Kg)), ops.offline_FC_quant_Q4A(dev(we), 128), N).cpu().numpy()
+            assert np.array_equal(got[0], (xe.astype(np.float64) @ we.astype(np.float64).T).astype(np.float32))
     finally:
         lib.llmops_test_fc_stream_set(0, 0, 0, 0)
 
