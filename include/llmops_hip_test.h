@@ -34,7 +34,8 @@ void llmops_test_fc_set_tuning(int target_workgroups, int waves_per_workgroup);
 
 /* prefill GEMM planner knob: force the row-tile factor of the LDS-tiled MFMA kernel (1, 2 or 4:
  * 32, 64 or 128 rows per workgroup); 0 (and what is none of these) = choose per shape; -1 = choose
- * per shape and send 9..32 rows to the tiled kernel too instead of the weight-streaming MFMA kernel */
+ * per shape and send whatever the weight-streaming MFMA kernel would take to the tiled kernel too (2..8 rows: to the
+ * kernel that quantizes on the fly) */
 void llmops_test_gemm_set_tuning(int row_tile_factor);
 
 /* prefill GEMM with split-K: the product kernel adds the partial sums itself (the last split of a tile to

@@ -502,7 +502,7 @@ struct GemmPlan {
     bool lds;
 };
 
-static int g_gemm_rt = 0;  // 0 = choose per shape; 1, 2, 4 = that tile; -1 = also keep 9..32 rows on the tiled kernel
+static int g_gemm_rt = 0;  // 0 = choose per shape; 1, 2, 4 = that tile; -1 = also what the weight-streaming kernel would take
 static int g_gemm_fused_reduce = 1;  // split-K partial sums added by the product kernel itself (0: by a second launch)
 static int g_gemm_force_split = 0;   // > 0: the split-K factor to use whatever the estimate says (tests)
 bool gemm_rows_kernel_enabled() { return g_gemm_rt >= 0; }

@@ -2,6 +2,8 @@
 the `llmops` module (ctypes -> C ABI -> HIP kernels).  Bit-exact: packed bytes, Q8 codes, scales,
 group sums, int32 partial sums.  fp32 outputs: max|err|/max|ref| <= 1e-3 (the stated contract;
 observed errors are ~1e-6)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -535,10 +537,9 @@ def test_fc_two_k_splits_both_handoffs(ops, orc, rows, N, K):
 @pytest.mark.parametrize("rows", [3, 5, 8, 9, 13, 16, 17, 24, 32])
 @pytest.mark.parametrize("N,K", [(4096, 11008), (4090, 4096), (2070, 2048), (3000, 2176)])
 def test_fc_rows_kernel_two_k_halves(ops, orc, rows, N, K):
-    """The weight-streaming MFMA kernel on tensors with fewer than 256 strips: two workgroups per strip with
-    half of K each, meeting through one 64-bit exchange per output, against one workgroup per strip: both
-    against the oracle, bit-equal over repeated launches, with and without the residual; ragged N, odd
-    k-group counts (17 = 8 + 9)."""
+    """The weight-streaming MFMA kernel with two workgroups per strip that have half of K each and meet through one 64-bit
+    exchange per output, against one workgroup per strip (both forced): either against the oracle, bit-equal over repeated
+    launches, with and without the residual; ragged N, odd k-group counts (17 = 8 + 9)."""
     from llmops import _lib
     lib = _lib.load()
     rng = np.random.default_rng(rows + N)
@@ -547,17 +548,28 @@ def test_fc_rows_kernel_two_k_halves(ops, orc, rows, N, K):
     res = rng.standard_normal((1, rows, N)).astype(np.float32)
     pw = dev(orc.quant_w(w, 128))
     want = orc.fc(x, host(pw), N)
+    build, got = [ctypes.c_int(-1) for _ in range(4)], []
     try:
-        for on in (1, 0, 1):
-            lib.llmops_test_fc_rows_set_split(on)
+        lib.llmops_test_fc_set_row_routing(2, 2)
+        for halves in (1, 0, 1):
+            lib.llmops_test_fc_stream_set((rows + 15) // 16, 1, 8, halves)
+            assert lib.llmops_test_fc_stream_plan(rows, (N + 31) // 32, K // 128, *[ctypes.byref(o) for o in build]) == 0
+            assert [o.value for o in build] == [(rows + 15) // 16, 1, 8, halves]
             a = ops.fc_Q4A(dev(x), pw, N)
             b = ops.fc_Q4A(dev(x), pw, N)
             c = ops.fc_Q4A(dev(x), pw, N, residual=dev(res))
             assert torch.equal(a, b)
             assert max_rel_err(host(a), want) <= 1e-5
             assert max_rel_err(host(c), want + res) <= 1e-5
+            got.append(a)
+        assert torch.equal(got[0], got[2]) and not torch.equal(got[0], got[1])
+        lib.llmops_test_fc_stream_set(0, 0, 0, 0)
+        lib.llmops_test_fc_rows_set_split(0)   # (what the planner chooses is then whole)
+        assert lib.llmops_test_fc_stream_plan(rows, (N + 31) // 32, K // 128, *[ctypes.byref(o) for o in build]) == 0 and build[3].value == 0
     finally:
+        lib.llmops_test_fc_stream_set(0, 0, 0, 0)
         lib.llmops_test_fc_rows_set_split(1)
+        lib.llmops_test_fc_set_row_routing(0, 0)
 
 
 @pytest.mark.parametrize("rows", [2, 3, 4, 6, 8])
@@ -566,7 +578,7 @@ def test_fc_few_rows_either_kernel(ops, orc, rows, N, K):
     """2..8 rows at group 128 can run the streaming kernel that quantizes on the fly or the weight-streaming
     MFMA kernel behind a quantization launch (the row count at which the second takes over is a tuning
     knob): both against the oracle, with and without the residual, for a tensor on either side of 256
-    strips and one whose 35 k-groups per workgroup take the MFMA kernel's 16-wave form."""
+    strips and one whose waves have runs of several k-groups."""
     from llmops import _lib
     lib = _lib.load()
     rng = np.random.default_rng(rows * 7 + N)
@@ -588,21 +600,31 @@ def test_fc_few_rows_either_kernel(ops, orc, rows, N, K):
 
 @pytest.mark.parametrize("rows", [17, 48, 100, 128, 129, 200, 256])
 @pytest.mark.parametrize("N,K", [(2070, 1024), (4096, 640), (2048, 2816)])
-def test_fc_prefill_mid_rows_vs_oracle(ops, orc, rows, N, K):
-    """17..256 rows at group 128 as the planner runs them (tiling and split-K factor chosen per shape):
-    ragged rows, N not a multiple of 32, k-group counts 8, 5 and 22 (splits of unequal length): output
+@pytest.mark.parametrize("kernel", ["streaming", "tiled"])
+def test_fc_prefill_mid_rows_vs_oracle(ops, orc, rows, N, K, kernel):
+    """17..256 rows at group 128 as the planners run them: the weight-streaming kernel, which takes these sizes, and the tiled one, to
+    which they are sent (its tiling and split-K factor chosen per shape): ragged rows, N not a multiple of 32, k-group counts 8, 5 and 22 (splits of unequal length): output
     and residual epilogue against the oracle, the closed-form construction exactly."""
+    from llmops import _lib
+    lib = _lib.load()
     rng = np.random.default_rng(rows + N)
     x = rng.standard_normal((1, rows, K)).astype(np.float32)
     w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
     res = rng.standard_normal((1, rows, N)).astype(np.float32)
     pw = orc.quant_w(w, 128)
     want = orc.fc(x, pw, N)
-    assert max_rel_err(host(ops.fc_Q4A(dev(x), dev(pw), N)), want) <= 1e-5
-    assert max_rel_err(host(ops.fc_Q4A(dev(x), dev(pw), N, residual=dev(res))), want + res) <= 1e-5
-    xe, we = oracle.closed_form_fc_inputs(rows, N, K, seed=rows)
-    ye = host(ops.fc_Q4A(dev(xe.reshape(1, rows, K)), ops.offline_FC_quant_Q4A(dev(we), 128), N))
-    assert np.array_equal(ye, (xe.astype(np.float64) @ we.astype(np.float64).T).astype(np.float32).reshape(1, rows, N))
+    build = [ctypes.c_int(-1) for _ in range(4)]
+    lib.llmops_test_gemm_set_tuning(-1 if kernel == "tiled" else 0)
+    try:
+        assert lib.llmops_test_fc_stream_plan(rows, (N + 31) // 32, K // 128, *[ctypes.byref(b) for b in build]) == 0
+        assert (build[0].value == 0) == (kernel == "tiled")
+        assert max_rel_err(host(ops.fc_Q4A(dev(x), dev(pw), N)), want) <= 1e-5
+        assert max_rel_err(host(ops.fc_Q4A(dev(x), dev(pw), N, residual=dev(res))), want + res) <= 1e-5
+        xe, we = oracle.closed_form_fc_inputs(rows, N, K, seed=rows)
+        ye = host(ops.fc_Q4A(dev(xe.reshape(1, rows, K)), ops.offline_FC_quant_Q4A(dev(we), 128), N))
+        assert np.array_equal(ye, (xe.astype(np.float64) @ we.astype(np.float64).T).astype(np.float32).reshape(1, rows, N))
+    finally:
+        lib.llmops_test_gemm_set_tuning(0)
 
 
 @pytest.mark.parametrize("tiling", [1, 2, 4])
@@ -783,8 +805,7 @@ def test_fc_group32_non_finite_rows_stay_theirs(ops, orc):
 @pytest.mark.parametrize("rows", [9, 12, 16])
 @pytest.mark.parametrize("N,K", [(2070, 1024), (4096, 4096)])
 def test_fc_rows_9_to_16_streaming_mfma(ops, orc, rows, N, K):
-    """9..16 rows at group 128 with at least 64 strips take the weight-streaming MFMA kernel
-    (one strip per workgroup): output and residual epilogue against the oracle, N not a multiple of 32."""
+    """9..16 rows at group 128 take the weight-streaming MFMA kernel: output and residual epilogue against the oracle, N not a multiple of 32."""
     rng = np.random.default_rng(rows + N)
     x = rng.standard_normal((1, rows, K)).astype(np.float32)
     w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
@@ -830,6 +851,10 @@ def test_gemm_split_k_reduced_in_kernel_equals_second_launch(ops, M, N, K):
     x = dev(rng.standard_normal((1, M, K)).astype(np.float32))
     res = dev(rng.standard_normal((1, M, N)).astype(np.float32))
     try:
+        lib.llmops_test_gemm_set_tuning(-1)                       # the tiled kernel whatever the rows, its tile and splits as planned
+        build, rt, splits = [ctypes.c_int(-1) for _ in range(4)], ctypes.c_int(), ctypes.c_int()
+        assert lib.llmops_test_fc_stream_plan(M, (N + 31) // 32, K // 128, *[ctypes.byref(b) for b in build]) == 0 and build[0].value == 0
+        assert lib.llmops_test_gemm_plan(M, (N + 31) // 32, K // 128, 128, ctypes.byref(rt), ctypes.byref(splits)) == 0 and splits.value > 1
         lib.llmops_test_gemm_set_reduce(0)
         want, want_res = ops.fc_Q4A(x, wq, N), ops.fc_Q4A(x, wq, N, residual=res)
         for mode in (1, 100):                                     # default rule; every split count (several load batches)
@@ -845,6 +870,7 @@ def test_gemm_split_k_reduced_in_kernel_equals_second_launch(ops, M, N, K):
                 assert torch.equal(ops.fc_Q4A(x, wq, N, residual=res), first_res)
     finally:
         lib.llmops_test_gemm_set_reduce(1)
+        lib.llmops_test_gemm_set_tuning(0)
     # and the decode kernels, which share the counters, still find them at zero
     y1 = ops.fc_Q4A(x[:, :1].contiguous(), wq, N)
     assert torch.equal(y1, ops.fc_Q4A(x[:, :1].contiguous(), wq, N))
