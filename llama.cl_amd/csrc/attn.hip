@@ -144,12 +144,6 @@ __device__ __forceinline__ float4 load4(const __half* p) {
     return make_float4(fa.x, fa.y, fb.x, fb.y);
 }
 
-__device__ __forceinline__ float2 load2(const float* p) { return *reinterpret_cast<const float2*>(p); }
-__device__ __forceinline__ float2 load2(const __half* p) {
-    const uint32_t u = *reinterpret_cast<const uint32_t*>(p);
-    return __half22float2(*reinterpret_cast<const __half2*>(&u));
-}
-
 // a value as the cache holds it
 template <typename T>
 __device__ __forceinline__ float cache_round(float v);

@@ -60,7 +60,7 @@ static FcWorkspace fc_layout(int64_t rows, int64_t Ng, int64_t Kg, int G, size_t
     w.off_gs = o;
     o = align_up(o + (size_t)rows * Kg * sizeof(float), 256);
     w.off_xst = o;
-    // (+256: the weight-streaming MFMA kernel fetches the pairs of whole 16-row tiles, up to 31 pairs past the last row)
+    // (+256: no kernel reads behind the last pair; the sizes that callers have asked for count it)
     o = align_up(o + (size_t)rows * Kg * 2 * sizeof(float) + 256, 256);
     w.off_part = o;
     w.room = limit == 0 ? INT64_MAX : (int64_t)limit - (int64_t)o;  // (multiples of 256 both)
@@ -122,14 +122,16 @@ static int fc_check_args(const float* x, int64_t rows, int64_t K, const int8_t* 
 // Whether the product of quantized activations (group 128) is the weight-streaming kernel's or the tiled one's.  Up to 16
 // rows are bound by the weight stream (tiled / streaming, us: 9 x 1024 x 512 7.6 / 5.0, 16 x 512 x 4096 9.6 / 6.5).  Above, the
 // streaming kernel fetches every row's codes for each strip again, the tiled one shares them between four strips but needs splits
-// of K and barriers: whichever is estimated to take less, with 7 us on the tiled side, which its estimate leaves out.  Of 190 sizes (17 ..
-// 512 rows of 13 shapes from 1024 x 512 to 11008 x 11008) two are up to 5 % slower than by the other kernel (384 x 4096 x 11008 43.7 /
-// 45.8) and six stay up to 20 % behind it (96 x 22016 x 4096 35.3 / 29.5): 64 x 4096^2 14.1 / 9.0, 128 x 4096 x 11008 25.1 / 22.6, 256 x
-// 4096^2 20.9 / 16.3, 512 x 2048^2 15.5 / 12.8; 256 x 22016 x 4096 48.1 / 57.3, 128 x 11008 x 11008 43.6 / 49.1.  Up to 11 k-groups
-// the tiled path's quantization costs less and most of this kernel's time is its results: 4.75 (40 x 4096 x 512 8.8 / 5.7,
-// 384 x 4096 x 512 10.0 / 9.5; 448 rows 10.05 / 10.7, 300 x 6000 x 512 10.4 / 10.7).  From 513 rows on the estimates are less even:
-// 2 (600 x 512 x 4096 17.0 / 13.3, 900 x 2048^2 19.6 / 17.8, 1000 x 1500 x 3072 26.4 / 21.0; 1000 x 600 x 11008 34.7 / 35.4,
-// 800 x 600 x 11008 31.0 / 33.8, 600 x 4096^2 does not come near); beyond 1024 rows what there is to gain is a few percent.
+// of K and barriers: whichever is estimated to take less, with 7 us on the tiled side, which its estimate leaves out (first fetch, finish,
+// quantization); 4.75 up to 11 k-groups, where the quantization costs less and most of this kernel's time is its results; 2 from 513 rows on,
+// where both estimates are less even.  Beyond 1024 rows what there is to gain is a few percent.  Of 687 sizes (17 .. 1024 rows of fifteen shapes
+// from 1024 x 512 to 22016 x 4096 and 11008 x 11008, both kernels in turn, weights from memory) none that is streamed would be more than 1.7 % faster in
+// tiles (768 x 600 x 11008 29.8 / 30.3); 37 that are tiled would be 2 % and more faster streamed, most of them within 8 % (us, tiled / streaming:
+// 192 x 12288 x 4096 35.0 / 29.9, 96 x 22016 x 4096 34.8 / 30.5, 192 x 11008 x 4096 31.1 / 29.0, 576 x 4096^2 33.5 / 31.1, 832 x 2000 x 8192 44.0 / 40.4).
+// Some times: 64 x 4096^2 13.8 / 8.5, 128 x 4096 x 11008 25.4 / 22.6, 256 x 4096^2 20.2 / 16.0, 512 x 2048^2 16.0 / 12.5, 384 x 4096 x 512 10.4 / 10.0,
+// 448 10.5 / 11.2, 256 x 22016 x 4096 48.1 / 57.5, 128 x 11008 x 11008 40.6 / 46.2, 1024 x 1500 x 3072 25.4 / 22.4.  Neither is ahead from one row count on:
+// tiles, splits and row blocks come in steps, 4096 x 11008 at 256 rows 35.9 / 31.2, 272 40.1 / 43.4, 304 40.7 / 41.5, 336 43.2 / 42.6, 384 45.8 / 45.2, 512
+// 54.0 / 52.2, 544 64.9 / 66.4.
 bool llmops::streams(int64_t rows, int64_t Ng, int64_t Kg, int group_k) {
     if (group_k != 128 || rows > 1024 || !gemm_rows_kernel_enabled() || !stream_fits(rows, Kg)) return false;
     if (rows <= 16) return true;

@@ -246,7 +246,8 @@ __global__ __launch_bounds__(NW * 64, (RT * SW > 4 ? 2 : RT * SW > 2 ? 3 : 4)) v
 // take together, 0.114 SW + 0.073 RT each; 0.35 RT * SW per workgroup of the compute unit at the end; halves 0.6 us and 4.9 us
 // per million outputs; a workgroup that follows another alone on its compute unit 1.4 us; the weights 0.10 us per MB.  Fitted
 // to all of these at 3 .. 512 rows of 13 shapes from 1024 x 512 to 22016 x 4096 and 11008 x 11008, weights from memory: the choices are
-// 0.8 % slower than the best measured on average, 11 % at worst (384 x 4096 x 11008, 56.0 against 50.4; the tiled kernel's 43.7 is taken).
+// 0.8 % slower than the best measured on average, 14 % at worst (256 x 4096 x 512, two strips where one is better, 9.3 against 8.2; above 4
+// k-groups 8 %, 16 x 4096^2 in halves 7.3 against 6.7).
 struct StreamPlan {
     int RT, SW, NW;
     bool split;
