@@ -130,8 +130,8 @@ size_t llmops_fc_Q4A_noalloc_scratch_bytes(void);
 int llmops_fc_Q4A_noalloc(const float* x, int64_t rows, int64_t K, const int8_t* weiq, int64_t Ng, int64_t Kg,
                           int group_k, int64_t N, float* y, llmops_stream_t stream);
 
-/* fc_Q4A followed by iadd(y, residual) (ops/op_misc.hpp:55-79) in one launch for rows <= 8:
- * y = fc_Q4A(x) + residual, residual fp32 [rows,N].  The decode step uses it for the o and down
+/* fc_Q4A followed by iadd(y, residual) (ops/op_misc.hpp:55-79), with the launches of fc_Q4A alone: the add rides in the
+ * product's stores.  y = fc_Q4A(x) + residual, residual fp32 [rows,N].  The decode step uses it for the o and down
  * projections (chatllama/main.py:355-357,372-375).  residual may be y itself (the add in place the
  * reference does), except when K is not a multiple of group_k and rows <= 8: that combination adds
  * the residual in a second launch and is refused with LLMOPS_EINVAL if the two alias. */

@@ -222,24 +222,24 @@ extern "C" int llmops_fc_Q4A_residual(const float* x, int64_t rows, int64_t K, c
 // (64 strips x 4 k-groups) to 3 us (688 x 32) and more with a producer, hardly anything the other way, where the second
 // launch costs 1.5 to 3 us and the sums 1.9.  In a graph, weights not from a cache, us, streaming / separate launches, at
 // rows either side of where the line lies (strips x k-groups):
-//   residual:             16x32 4 rows 7.8 / 6.3, 5 8.3 / 6.8; 48x86 3 13.2 / 9.8; 64x4 4 4.5 / 5.1, 5 5.5 / 5.2; 64x16 4 5.8 / 6.3, 5 7.3 / 6.4; 128x32 3
+//   residual:             64x4 4 rows 4.5 / 5.1, 5 5.5 / 5.2; 64x16 4 5.8 / 6.3, 5 7.3 / 6.4; 128x32 3
 //                         7.4 / 7.3; 128x86 3 10.4 / 11.4, 4 11.5 / 10.8; 256x32 3 8.0 / 9.0, 4 8.8 / 8.5; 384x32 2 9.3 / 12.3, 3 13.3 / 12.3;
 //                         688x32 3 20.1 / 16.4
-//   .. and sums:          16x32 6 rows 9.0 / 8.8, 7 9.4 / 8.6; 48x86 3 13.7 / 11.7; 64x4 8 6.9 / 7.2; 64x16 6 8.0 / 8.5, 8 9.2 / 8.4; 128x32 5 9.3 / 9.4, 6
+//   .. and sums:          64x4 8 rows 6.9 / 7.2; 64x16 6 8.0 / 8.5, 8 9.2 / 8.4; 128x32 5 9.3 / 9.4, 6
 //                         9.7 / 9.4; 128x86 4 12.3 / 12.7, 5 15.9 / 12.9; 256x32 4 9.2 / 10.5, 5 11.4 / 10.6; 384x32 2 9.6 / 13.2, 3 14.1 / 13.5
-//   rmsnorm:              8x32 2 rows 7.8 / 6.7, 3 11.4 / 6.8; 64x4 2 5.9 / 5.2, 3 8.1 / 5.3; 128x32 2 8.3 / 7.7, 3 12.1 / 7.8; 128x86 2 11.0 / 12.8, 3
+//   rmsnorm:              64x4 2 rows 5.9 / 5.2, 3 8.1 / 5.3; 128x32 2 8.3 / 7.7, 3 12.1 / 7.8; 128x86 2 11.0 / 12.8, 3
 //                         15.2 / 13.0; 384x32 2 15.7 / 11.7; 688x32 2 23.3 / 15.8
-//   .. and sums:          16x16 2 rows 6.8 / 7.9, 3 9.6 / 8.0; 64x16 2 7.0 / 8.6, 3 9.9 / 8.6; 128x32 2 8.6 / 9.9, 3 12.2 / 9.8; 384x32 2 16.5 / 13.7
-//   .. sums handed in:    16x32 3 rows 8.9 / 6.9, 5 9.6 / 7.5; 64x4 4 5.2 / 5.3, 5 6.6 / 5.5; 64x16 4 7.0 / 6.5, 5 9.4 / 6.7; 128x32 2 6.6 / 7.7, 3 9.3 / 7.8;
+//   .. and sums:          64x16 2 rows 7.0 / 8.6, 3 9.9 / 8.6; 128x32 2 8.6 / 9.9, 3 12.2 / 9.8; 384x32 2 16.5 / 13.7
+//   .. sums handed in:    64x4 4 rows 5.2 / 5.3, 5 6.6 / 5.5; 64x16 4 7.0 / 6.5, 5 9.4 / 6.7; 128x32 2 6.6 / 7.7, 3 9.3 / 7.8;
 //                         128x86 3 11.9 / 13.1, 4 13.3 / 13.0; 256x32 2 7.0 / 8.9, 3 9.8 / 8.9; 384x32 2 10.7 / 11.7, 3 17.1 / 11.7; 688x32 2 14.7 / 15.8
-//   silu * up, residual:  16x32 4 rows 9.6 / 6.4, 5 9.2 / 6.8; 48x86 2 9.6 / 9.7, 3 14.9 / 9.8; 64x4 4 5.1 / 5.2, 5 6.2 / 5.2; 64x16 4 6.8 / 6.4; 128x32 2
+//   silu * up, residual:  64x4 4 rows 5.1 / 5.2, 5 6.2 / 5.2; 64x16 4 6.8 / 6.4; 128x32 2
 //                         6.5 / 7.2, 3 8.6 / 7.3; 128x86 2 9.4 / 10.7, 3 12.0 / 10.8; 384x32 2 10.5 / 11.3; 688x32 2 14.6 / 15.3
-//   .. and sums:          16x16 5 rows 8.9 / 7.8, 8 10.9 / 7.7; 64x4 7 7.6 / 7.2, 8 8.1 / 7.1; 64x16 5 9.1 / 8.5; 128x32 3 9.1 / 9.4, 4 10.2 / 9.2; 128x86 3
+//   .. and sums:          64x4 7 rows 7.6 / 7.2, 8 8.1 / 7.1; 64x16 5 9.1 / 8.5; 128x32 3 9.1 / 9.4, 4 10.2 / 9.2; 128x86 3
 //                         12.6 / 12.8; 256x32 3 9.5 / 10.5, 4 10.8 / 10.5; 384x32 2 11.2 / 13.3, 3 17.0 / 13.5
-// Fewer than 64 strips of fewer than 12 k-groups are one launch, as in fc_Q4A (16x4: residual 5 rows 5.3 / 5.1, 8 6.5 / 5.2, .. and sums 8 6.8 / 7.1,
-// silu * up 5 6.2 / 5.2; with a rmsnorm, 3 rows 8.0 / 5.2, the other way would be the faster one).
+// Fewer than 64 strips are one launch, as the header promises, also where the other way would be the faster one (16x4: residual 8 rows 6.5 / 5.2;
+// 16x32: residual 5 rows 8.3 / 6.8, .. and sums 7 9.4 / 8.6; 8x32: rmsnorm 3 rows 11.4 / 6.8; 48x86: silu * up 5 rows 20.0 / 9.8).
 static bool decode_quantizes_first(int64_t rows, int64_t K, int64_t Ng, int64_t Kg, int group_k, bool norm, bool sums_in, int glu, bool sums_out) {
-    if ((Ng < 64 && Kg < 12) || rows > kMaxGemvRows || !streams(rows, Ng, Kg, group_k) || glu == 1 || (norm && K > 16384)) return false;
+    if (Ng < 64 || rows > kMaxGemvRows || !streams(rows, Ng, Kg, group_k) || glu == 1 || (norm && K > 16384)) return false;
     const bool large = Ng > 256;
     const int64_t blocks = Ng * Kg;
     int from = large ? (g_rows_from_large > 0 ? g_rows_from_large : 3) : g_rows_from_small > 0 ? g_rows_from_small : 4;

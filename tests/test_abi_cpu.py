@@ -152,13 +152,13 @@ def test_gemm_planner_choices(lib):
 
 @pytest.mark.parametrize("form,sizes", [
     # (strips, k-groups): the last row count that measured faster in one launch, the first that did in separate ones
-    ("residual", {(16, 16): (4, 5), (16, 32): (2, 5), (48, 86): (2, 4), (64, 4): (4, 6), (64, 16): (4, 5), (128, 32): (3, 4), (128, 86): (3, 4), (256, 32): (3, 4), (384, 32): (2, 3), (688, 32): (2, 3)}),
-    ("residual sums", {(16, 16): (6, 9), (16, 32): (6, 7), (48, 86): (2, 6), (64, 4): (8, 9), (64, 16): (6, 8), (128, 32): (5, 6), (128, 86): (4, 5), (256, 32): (4, 5), (384, 32): (2, 3), (688, 32): (2, 3)}),
-    ("norm", {(8, 32): (1, 3), (16, 16): (1, 3), (48, 86): (1, 3), (64, 4): (1, 3), (64, 16): (1, 3), (128, 32): (1, 3), (128, 86): (2, 3), (256, 32): (1, 3), (384, 32): (1, 2), (688, 32): (1, 2)}),
-    ("norm sums", {(16, 16): (2, 3), (16, 32): (2, 3), (64, 4): (2, 3), (64, 16): (2, 3), (128, 32): (2, 3), (128, 86): (2, 3), (256, 32): (2, 3), (384, 32): (1, 2), (688, 32): (1, 2)}),
-    ("norm sums_in", {(16, 16): (3, 5), (16, 32): (2, 5), (48, 86): (2, 3), (64, 4): (4, 5), (64, 16): (3, 5), (128, 32): (2, 3), (256, 32): (2, 3), (384, 32): (2, 3), (688, 32): (1, 2)}),
-    ("glu", {(16, 16): (3, 5), (16, 32): (2, 5), (48, 86): (2, 3), (64, 4): (4, 5), (64, 16): (3, 5), (128, 32): (2, 3), (128, 86): (2, 3), (256, 32): (2, 3), (384, 32): (1, 2), (688, 32): (1, 2)}),
-    ("glu sums", {(16, 16): (4, 8), (16, 32): (3, 6), (48, 86): (2, 4), (64, 4): (6, 8), (64, 16): (4, 6), (128, 32): (2, 4), (128, 86): (2, 4), (256, 32): (3, 4), (384, 32): (2, 3), (688, 32): (2, 3)})])
+    ("residual", {(64, 4): (4, 6), (64, 16): (4, 5), (128, 32): (3, 4), (128, 86): (3, 4), (256, 32): (3, 4), (384, 32): (2, 3), (688, 32): (2, 3)}),
+    ("residual sums", {(64, 4): (8, 9), (64, 16): (6, 8), (128, 32): (5, 6), (128, 86): (4, 5), (256, 32): (4, 5), (384, 32): (2, 3), (688, 32): (2, 3)}),
+    ("norm", {(64, 4): (1, 3), (64, 16): (1, 3), (128, 32): (1, 3), (128, 86): (2, 3), (256, 32): (1, 3), (384, 32): (1, 2), (688, 32): (1, 2)}),
+    ("norm sums", {(64, 4): (2, 3), (64, 16): (2, 3), (128, 32): (2, 3), (128, 86): (2, 3), (256, 32): (2, 3), (384, 32): (1, 2), (688, 32): (1, 2)}),
+    ("norm sums_in", {(64, 4): (4, 5), (64, 16): (3, 5), (128, 32): (2, 3), (256, 32): (2, 3), (384, 32): (2, 3), (688, 32): (1, 2)}),
+    ("glu", {(64, 4): (4, 5), (64, 16): (3, 5), (128, 32): (2, 3), (128, 86): (2, 3), (256, 32): (2, 3), (384, 32): (1, 2), (688, 32): (1, 2)}),
+    ("glu sums", {(64, 4): (6, 8), (64, 16): (4, 6), (128, 32): (2, 4), (128, 86): (2, 4), (256, 32): (3, 4), (384, 32): (2, 3), (688, 32): (2, 3)})])
 def test_rows_from_which_a_decode_projection_is_quantized_first(lib, form, sizes):
     opts, first = form.split(), ctypes.c_int(-1)
     i64 = ctypes.c_int64
@@ -171,7 +171,7 @@ def test_rows_from_which_a_decode_projection_is_quantized_first(lib, form, sizes
     for (strips, groups), (one, many) in sizes.items():
         assert [separate(r, strips, groups) for r in (1, one, many, 9)] == [0, 0, 1, 1], (form, strips, groups)
         # what the quantization and the product behind it do not take: one launch up to 8 rows
-        assert not separate(8, strips, groups, group_k=32) and not separate(8, 63, 11)
+        assert not separate(8, 63, groups) and not separate(8, strips, groups, group_k=32)
         assert not separate(8, strips, groups, glu=1)
         if opts == ["norm"]:  # the FC in front hands on its sums of squares where this one is a single launch
             for rows in range(1, 10):
