@@ -41,9 +41,10 @@ MEASURED_TRAFFIC_PROFILE = "profiles/fc_gemv_fused_kernel__hbm_traffic_pmc.md"
 PROFILE_SOURCES = {
     "profiles/fc_gemv_fused_kernel__hbm_traffic_pmc.md": (("fc_gemv.hip", "gemv_device.h"), "dcfc69057e8a4660"),
     "profiles/fc_gemv_fused_kernel__vector_alu_pmc.md": (("fc_gemv.hip", "gemv_device.h"), "dcfc69057e8a4660"),
-    "profiles/fc_gemm_kernels__prefill_g128_pmc.md": (("fc_gemm.hip", "gemm_device.h", "fc_rows.hip", "q8_act.hip"), "8e44e870f12329a7"),
-    "profiles/attn_prefill_kernel__prompt_2048_pmc.md": (("attn.hip",), "b8d23a92c7c2c397"),
-    "profiles/fc_gemm_g32_attn_few_quant_w_kernels__pmc.md": (("fc_gemm_g32.hip", "gemm_device.h", "attn.hip", "q4_pack.hip"), "ddfe6c3880745663"),
+    "profiles/fc_gemm_kernels__prefill_g128_pmc.md": (("fc_gemm.hip", "gemm_device.h"), "34529b812da70895"),
+    "profiles/fc_stream_kernel__pmc.md": (("fc_rows.hip", "gemm_device.h", "gemv_device.h"), "ec234d8e69254553"),
+    "profiles/attn_prefill_kernel__prompt_2048_pmc.md": (("attn.hip",), "4eee8c437d2125e2"),
+    "profiles/fc_gemm_g32_attn_few_quant_w_kernels__pmc.md": (("fc_gemm_g32.hip", "gemm_device.h", "attn.hip", "q4_pack.hip"), "a126a036e6091770"),
 }
 MEASURED_TRAFFIC_KERNEL_SHA16 = PROFILE_SOURCES[MEASURED_TRAFFIC_PROFILE][1]
 G = 128
